@@ -58,7 +58,7 @@ extern "C" {
 
 enum { MOBA_DTYPE_BF16 = 0, MOBA_DTYPE_F16 = 1 };
 
-#define MOBA_ABI_VERSION 115 /* the signatures below; moba_version() returns the number the library was built with */
+#define MOBA_ABI_VERSION 116 /* the signatures below; moba_version() returns the number the library was built with */
 int moba_version(void);
 const char* moba_strerror(int code);
 
@@ -314,14 +314,20 @@ int moba_bwd(const void* dout, const void* q, const void* k, const void* v, cons
              int dq_key_split, const int64_t* strides, int32_t* queues, void* dkv_scratch, int64_t dkv_scratch_bytes,
              float softmax_scale, int dtype, void* stream);
 
-/* Decode: one query token per sequence against the key/value cache.  Replaces the
- * flash_attn_func call of the adapter's decode branch, moba/wrapper.py:76-82 (full attention
- * over the cache, grouped-query heads).
- *   q [B,H,D]: element strides q_stride_b, q_stride_h, D contiguous
- *   k, v [B,Hkv,Skv,D]: element strides kv_stride_b, kv_stride_h; key rows contiguous and D apart
- *   out [B,H,D] elem, contiguous
- *   part_o [B*H*splits, D] fp32 and part_lse [B*H*splits] fp32 scratch, splits = moba_decode_splits()
- * H/Hkv in {1,2,4,8}; strides multiples of 8 elements; scale = softmax scale. */
+/* Decode: the last nq tokens of every sequence against its key/value cache.  Replaces the
+ * flash_attn_func call of the adapter's decode branch, moba/wrapper.py:76-82 (grouped-query heads, bottom-right
+ * aligned causal mask: token j of the nq sees the keys up to position Skv - nq + j).  The cache is read once for all
+ * the query rows of a key/value head.
+ *   q [B,H,nq,D], k, v [B,Hkv,Skv,D]; D contiguous, key rows D apart
+ *   strides: {q batch, q head, q token, k/v batch, k/v head} in elements, multiples of 8
+ *   out [B,nq,H,D] elem, contiguous
+ *   part_o [B*nq*H*splits, D] fp32 and part_lse [B*nq*H*splits] fp32 scratch,
+ *   splits = moba_tail_splits(B, Hkv, H / Hkv, nq, Skv)
+ * scale = softmax scale. */
+int moba_tail_splits(int B, int Hkv, int rep, int nq, int Skv);
+int moba_tail(const void* q, const void* k, const void* v, void* out, float* part_o, float* part_lse, int B, int H,
+              int Hkv, int nq, int Skv, int D, const int64_t* strides, float scale, int dtype, void* stream);
+/* The same for one token (q [B,H,D]; H/Hkv at most 32; splits = moba_decode_splits()). */
 int moba_decode_splits(int B, int Hkv, int Skv);
 int moba_decode(const void* q, const void* k, const void* v, void* out, float* part_o, float* part_lse, int B, int H,
                 int Hkv, int Skv, int D, int64_t q_stride_b, int64_t q_stride_h, int64_t kv_stride_b,

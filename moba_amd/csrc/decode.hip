@@ -1,172 +1,273 @@
-// Decode attention: one new query token per sequence against the whole key/value cache,
-// the branch of the reference adapter that calls flash_attn_func with a single query
-// (moba/wrapper.py:76-82).  Full attention (every cached key is visible), grouped-query
-// heads handled in place, softmax scale supplied by the caller.
+// Decode attention: the last `nq` tokens of every sequence against its key/value cache, the branch of the
+// reference adapter that calls flash_attn_func with few query tokens (moba/wrapper.py:76-82).  Token j of the nq
+// sees the keys up to its own position Skv - nq + j; grouped-query heads are handled in place; the softmax scale is
+// the caller's.
 //
-// HBM-bound: K and V of the cache are read exactly once, 16 bytes per lane.  The key range
-// of a (batch, kv head) is cut into splits, one workgroup each; a 16-lane group owns one
-// key at a time (8 head dimensions per lane), so a wave streams 4 keys per load.  All
-// REP query heads of the kv head are served from the same loads.  Each lane group keeps
-// its own online softmax state; groups, waves and finally splits are combined with the
-// usual log-sum-exp algebra (the running maximum moves lazily, so the common step is
-// p = exp2(s - m); acc += p * v).
+// HBM-bound: K and V of the cache are to be read once.  The nq * rep query rows that share a key/value head are the
+// 32 columns of a matrix product (S^T = K Q^T, O^T += V^T P^T with v_mfma_f32_32x32x16), so one pass over the cache
+// serves them all: a kernel that gives every row its own dot products is bound by the vector unit from a handful of
+// rows on, and one that runs once per new token reads the cache that often.  A workgroup takes a range of the keys
+// (a split); its four waves take different keys of it, or different blocks of 32 rows once there are more than 32.
+// A wave copies its own K and V blocks of 32 keys global -> LDS (two stages of 16 KiB, no barrier: the wait for a
+// block counts the wave's own copies) while it computes the block before: 64 to 128 KiB per compute unit in flight,
+// where about 40 KiB cover the latency at the full rate.  One workgroup per compute unit (128 KiB of LDS); the
+// splits are chosen so that the workgroups come out just below a multiple of the units.
 //
-//   decode_partial_kernel   part_o[b, hq, split, :] (normalised, fp32), part_lse (log2 domain)
-//   decode_merge_kernel     out[b, hq, :]
-#include "common.h"
+// Measured (32 query heads on 8): 131072 keys, one token: 97 us a call (107 with a vector-unit kernel of 128 splits);
+// 16 x 8191 keys, fp16: 95 us = 5.6 TB/s (101); 4 x 20000 keys, 5 tokens: 64 us = 5.1 TB/s (342, once per token).
+// Beyond 128 rows per key/value head it is bound by its own instruction chain (one wave per SIMD), 0.45 PFLOP/s.
+//
+// Precision: the scores' products are exact, their sums fp32.  A probability is fed to the second product as the
+// sum of two elements (its rounded value and the rounded rest), so that it keeps 16 (bf16) or 22 (fp16) bits: the
+// matrix pipe has the time, and one element alone would double the error of the result.
+//
+//   tail_partial_kernel   part_o[row, split, :] (normalised, fp32), part_lse (log2 domain); one split: out itself
+//   tail_merge_kernel     out[row, :]
+#include "attn_common.h"
 
 namespace moba {
 
-constexpr int kDecodeMaxSplits = 128;
+constexpr int kTailKeys = 32;                                 // keys a wave handles per step
+constexpr int kTailTile = kTailKeys * kHeadDim * 2;           // bytes of its K (or V) block
+constexpr int kTailWaveLds = 4 * kTailTile;                   // two stages of K and V
+constexpr int kTailLds = 4 * kTailWaveLds;
+constexpr int kTailRedRow = kHeadDim + 4;                     // floats per row when the waves' sums meet in LDS
+constexpr int kTailRedStats = 4 * 32 * kTailRedRow * 4;       // byte offset of [4 waves][32 rows] maxima, then sums
+static_assert(kTailRedStats + 2 * 4 * 32 * 4 <= kTailLds, "the waves' sums fit the stages");
+constexpr int kTailMaxSplits = 128;
 
-// sum over the 16 lanes of a DPP row, delivered to all of them, without LDS traffic:
-// row mirror (i <-> 15-i), half-row mirror (i <-> 7-i), then the two quad permutations
-template <int CTRL>
-__device__ __forceinline__ float dpp_move(float x) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xF, 0xF, true));
-}
-__device__ __forceinline__ float sum_row16(float x) {
-  x += dpp_move<0x140>(x);  // row_mirror
-  x += dpp_move<0x141>(x);  // row_half_mirror
-  x += dpp_move<0xB1>(x);   // quad_perm [1,0,3,2]
-  x += dpp_move<0x4E>(x);   // quad_perm [2,3,0,1]
-  return x;
-}
+template <class E>
+struct TailParams {
+  const typename E::elem* q;
+  const typename E::elem* k;
+  const typename E::elem* v;
+  typename E::elem* out;  // [B, nq, H, D]
+  float* part_o;          // [B*nq*H, nsplit, D]
+  float* part_lse;        // [B*nq*H, nsplit]
+  int64_t q_stride_b, q_stride_h, q_stride_t, kv_stride_b, kv_stride_h;  // elements
+  int Hkv, rep, Skv, nq;
+  int wr_log2;            // log2 of the row blocks of a workgroup (its other waves split the keys)
+  int keys_per_split, nsplit;
+  float scale_log2;
+};
 
-template <class E, int REP>
-__global__ __launch_bounds__(256) void decode_partial_kernel(
-    const typename E::elem* __restrict__ q, const typename E::elem* __restrict__ k,
-    const typename E::elem* __restrict__ v, float* __restrict__ part_o, float* __restrict__ part_lse, int Hkv,
-    int Skv, int64_t q_stride_b, int64_t q_stride_h, int64_t kv_stride_b, int64_t kv_stride_h, int keys_per_split,
-    int nsplit, float scale_log2) {
+// fp16 probabilities are kept 2^7 times larger (the running maximum may lag by 2^8: they stay below 2^15), so that
+// those far below the maximum stay above the type's smallest number; the factor cancels
+template <class E> struct TailShift { static constexpr float value = 0.f; };
+template <> struct TailShift<F16> { static constexpr float value = 7.f; };
+constexpr float kTailMaxLag = 8.f;
+
+template <class E>
+__global__ __launch_bounds__(256, 1) void tail_partial_kernel(const TailParams<E> p) {
   MOBA_ELEM_TYPES(E)
-  __shared__ float red_o[4][REP][kHeadDim];
-  __shared__ float red_m[4][REP], red_l[4][REP];
-  const int split = blockIdx.x, hkv = blockIdx.y, b = blockIdx.z;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int g = lane >> 4, c = lane & 15;
-  const int key_lo = split * keys_per_split;
-  const int key_hi = min(Skv, key_lo + keys_per_split);
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 31, hh = lane >> 5;
+  const int split = blockIdx.x, b = blockIdx.z;
+  const int group = blockIdx.y / p.Hkv, hkv = blockIdx.y - group * p.Hkv;
+  const int wr_n = 1 << p.wr_log2, wk_n = 4 >> p.wr_log2;
+  const int wr = wave & (wr_n - 1), wk = wave >> p.wr_log2;
+  const int rows = p.nq * p.rep;
+  const int row0 = (group * wr_n + wr) * 32;
+  const int row = min(row0 + n, rows - 1);  // (rows past the last repeat it and are not written)
+  const int j = row / p.rep, g = row - j * p.rep;
+  const int key_lo = split * p.keys_per_split, key_hi = min(p.Skv, key_lo + p.keys_per_split);
+  const int limit = min(p.Skv - p.nq + j, key_hi - 1);          // the row's last visible key in this split
+  const int first_masked = min(p.Skv - p.nq, key_hi - 1);       // keys up to here are visible to every row
+  const int nblk = (key_hi - key_lo + kTailKeys - 1) / kTailKeys;
+  const int mine = row0 < rows ? (nblk - wk + wk_n - 1) / wk_n : 0;  // blocks wk, wk + wk_n, ... are this wave's
 
-  float qf[REP][8];
+  // K/V loader: one instruction copies 4 keys x 256 bytes; lane i lands at 16*i, so it picks the global column whose
+  // swizzled place that is
+  const uint32_t lds_base = lds_addr(smem) + wave * kTailWaveLds;
+  const int ld_kin = lane >> 4, ld_pc = lane & 15;
+  uint32_t ld_off[8];
 #pragma unroll
-  for (int r = 0; r < REP; ++r) {
-    const elem8 x = *reinterpret_cast<const elem8*>(q + b * q_stride_b + (int64_t)(hkv * REP + r) * q_stride_h + 8 * c);
+  for (int i = 0; i < 8; ++i) ld_off[i] = (4 * i + ld_kin) * 256 + sw_col16(4 * i + ld_kin, ld_pc) * 16;
+  const char* k_head = (const char*)(p.k + b * p.kv_stride_b + (int64_t)hkv * p.kv_stride_h);
+  const char* v_head = (const char*)(p.v + b * p.kv_stride_b + (int64_t)hkv * p.kv_stride_h);
+  auto issue = [&](int it, int stage) __attribute__((always_inline)) {
+    const int key0 = key_lo + (wk + it * wk_n) * kTailKeys;
+    const uint32_t kdst = lds_base + stage * 2 * kTailTile, vdst = kdst + kTailTile;
+    if (key0 + kTailKeys <= key_hi) {
+      const int64_t off = (int64_t)key0 * 256;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) qf[r][e] = (float)x[e] * scale_log2;
-  }
-  float m[REP], l[REP], acc[REP][8];
+      for (int i = 0; i < 8; ++i) async_copy16_sv(k_head + off, ld_off[i], kdst + i * 1024);
 #pragma unroll
-  for (int r = 0; r < REP; ++r) {
-    m[r] = -1e30f;  // finite: exp2(m - m_new) stays defined before the first key
-    l[r] = 0.f;
+      for (int i = 0; i < 8; ++i) async_copy16_sv(v_head + off, ld_off[i], vdst + i * 1024);
+    } else {  // (keys past the end: the last key again; their scores are masked)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) acc[r][e] = 0.f;
-  }
-  const elem* kb = k + b * kv_stride_b + (int64_t)hkv * kv_stride_h + 8 * c;
-  const elem* vb = v + b * kv_stride_b + (int64_t)hkv * kv_stride_h + 8 * c;
-
-  // 16 keys per workgroup step (4 waves x 4 lane groups), kUnroll steps (8 row loads per lane) in flight
-  constexpr int kUnroll = 4;
-  for (int key0 = key_lo + 4 * wave + g; key0 < key_hi; key0 += 16 * kUnroll) {
-    elem8 kf[kUnroll], vf[kUnroll];
-    bool ok[kUnroll];
+      for (int i = 0; i < 8; ++i) {
+        const int64_t off = (int64_t)min(key0 + 4 * i + ld_kin, key_hi - 1) * 256 + (ld_off[i] & 255);
+        async_copy16(k_head + off, kdst + i * 1024);
+      }
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-      const int key = key0 + 16 * u;
-      ok[u] = key < key_hi;
-      const int64_t off = (int64_t)(ok[u] ? key : key_lo) * kHeadDim;
-      kf[u] = __builtin_nontemporal_load(reinterpret_cast<const elem8*>(kb + off));
-      vf[u] = __builtin_nontemporal_load(reinterpret_cast<const elem8*>(vb + off));
+      for (int i = 0; i < 8; ++i) {
+        const int64_t off = (int64_t)min(key0 + 4 * i + ld_kin, key_hi - 1) * 256 + (ld_off[i] & 255);
+        async_copy16(v_head + off, vdst + i * 1024);
+      }
     }
+  };
+
+  // Q^T operand: lane (n, hh) holds q[row n][16*s8 + 8*hh .. +7]
+  elem8 bq[8];
+  {
+    const elem* src = p.q + b * p.q_stride_b + (int64_t)(hkv * p.rep + g) * p.q_stride_h + j * p.q_stride_t + 8 * hh;
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-      float s[REP];
+    for (int s8 = 0; s8 < 8; ++s8) bq[s8] = *reinterpret_cast<const elem8*>(src + 16 * s8);
+  }
+  if (mine > 0) issue(0, 0);
+  if (mine > 1) issue(1, 1);
+
+  // fragment addresses inside stage 0 (see the forward kernel)
+  uint32_t koff[8], voffA[4], voffB[4];
+  {
+    const int k_sw = ((n & 3) << 2) ^ ((n >> 2) & 3);
 #pragma unroll
-      for (int r = 0; r < REP; ++r) {
-        float d = 0.f;
+    for (int s8 = 0; s8 < 8; ++s8) koff[s8] = lds_base + n * 256 + (((2 * s8 + hh) ^ k_sw) << 4);
+    const int g16 = lane >> 4, i0 = (lane & 15) >> 2, i1 = lane & 3;
+    const int v_c16 = 2 * (g16 & 1) + (i1 >> 1), v_sub = (i1 & 1) * 8;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) d += qf[r][e] * (float)kf[u][e];
-        d = sum_row16(d);
-        s[r] = ok[u] ? d : -INFINITY;
-      }
-      bool grow = false;
-#pragma unroll
-      for (int r = 0; r < REP; ++r) grow |= s[r] > m[r];
-      if (__any(grow)) {  // rare once the maximum has settled
-#pragma unroll
-        for (int r = 0; r < REP; ++r) {
-          const float m_new = fmaxf(m[r], s[r]);
-          const float alpha = fast_exp2(m[r] - m_new);
-          m[r] = m_new;
-          l[r] *= alpha;
-#pragma unroll
-          for (int e = 0; e < 8; ++e) acc[r][e] *= alpha;
-        }
-      }
-#pragma unroll
-      for (int r = 0; r < REP; ++r) {
-        const float p = fast_exp2(s[r] - m[r]);
-        l[r] += p;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) acc[r][e] += p * (float)vf[u][e];
-      }
+    for (int db = 0; db < 4; ++db) {
+      const int c16 = 4 * db + v_c16;
+      voffA[db] = lds_base + kTailTile + (4 * hh + i0) * 256 + ((c16 ^ (i0 << 2) ^ hh) << 4) + v_sub;
+      voffB[db] = lds_base + kTailTile + (4 * hh + i0 + 8) * 256 + ((c16 ^ (i0 << 2) ^ (hh + 2)) << 4) + v_sub;
     }
   }
 
-  // combine the four lane groups of the wave, then the four waves
+  f32x16 oacc[4];
 #pragma unroll
-  for (int r = 0; r < REP; ++r) {
+  for (int db = 0; db < 4; ++db)
 #pragma unroll
-    for (int o = 16; o <= 32; o <<= 1) {
-      const float m_o = __shfl_xor(m[r], o, 64);
-      const float l_o = __shfl_xor(l[r], o, 64);
-      const float m_new = fmaxf(m[r], m_o);
-      const float a = fast_exp2(m[r] - m_new), a_o = fast_exp2(m_o - m_new);
-      l[r] = l[r] * a + l_o * a_o;
+    for (int e = 0; e < 16; ++e) oacc[db][e] = 0.f;
+  float m_run = -1e30f, l_run = 0.f;  // (finite: exp2(m - m_new) stays defined before the first visible key)
+
+  for (int it = 0; it < mine; ++it) {
+    const uint32_t st = (it & 1) * 2 * kTailTile;
+    // this block's 16 copies have landed (the next block's 16 may still be in flight)
+    if (it + 1 < mine) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    f32x16 s;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) acc[r][e] = acc[r][e] * a + __shfl_xor(acc[r][e], o, 64) * a_o;
-      m[r] = m_new;
+    for (int e = 0; e < 16; ++e) s[e] = 0.f;
+    elem8 ka[8];
+#pragma unroll
+    for (int s8 = 0; s8 < 8; ++s8) ka[s8] = *lds_ptr<const elem8>(koff[s8] + st);
+#pragma unroll
+    for (int s8 = 0; s8 < 8; ++s8) s = mfma32(ka[s8], bq[s8], s);
+    // the V^T fragments travel while the softmax runs
+    elem8 va[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int j2 = i >> 2, db = i & 3;
+      const elem4 a = lds_read_tr<elem4>(voffA[db] + st + 16 * j2 * 256);
+      const elem4 c = lds_read_tr<elem4>(voffB[db] + st + 16 * j2 * 256);
+      va[i] = __builtin_shufflevector(a, c, 0, 1, 2, 3, 4, 5, 6, 7);
     }
-    if (g == 0) {
+    const int key0 = key_lo + (wk + it * wk_n) * kTailKeys;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) red_o[wave][r][8 * c + e] = acc[r][e];
-      if (c == 0) {
-        red_m[wave][r] = m[r];
-        red_l[wave][r] = l[r];
-      }
+    for (int e = 0; e < 16; ++e) s[e] *= p.scale_log2;
+    if (key0 + kTailKeys - 1 > first_masked) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        if (key0 + 8 * (e >> 2) + 4 * hh + (e & 3) > limit) s[e] = -INFINITY;
     }
+    float mx = s[0];
+#pragma unroll
+    for (int e = 1; e < 16; ++e) mx = fmaxf(mx, s[e]);
+    mx = max_xhalf(mx);
+    if (__any(mx > m_run + kTailMaxLag)) {  // rare once the maximum has settled
+      const float m_new = mx > m_run + kTailMaxLag ? mx : m_run;
+      const float alpha = fast_exp2(m_run - m_new);
+      m_run = m_new;
+      l_run *= alpha;
+#pragma unroll
+      for (int db = 0; db < 4; ++db)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) oacc[db][e] *= alpha;
+    }
+    const float ref = m_run - TailShift<E>::value;
+    elem8 hi[2], lo[2];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const float pe = fast_exp2(s[e] - ref);
+      l_run += pe;
+      const elem h = (elem)pe;
+      hi[e >> 3][e & 7] = h;
+      lo[e >> 3][e & 7] = (elem)(pe - (float)h);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) oacc[i & 3] = mfma32(va[i], hi[i >> 2], oacc[i & 3]);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) oacc[i & 3] = mfma32(va[i], lo[i >> 2], oacc[i & 3]);
+    if (it + 2 < mine) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // every fragment of this stage is in registers
+      issue(it + 2, it & 1);
+    }
+  }
+  l_run = sum_xhalf(l_run);
+
+  // The waves that hold the same rows meet in LDS.  Element e of lane (n, hh) is O[row n][32*db + 8*(e/4) + 4*hh + e%4].
+  __syncthreads();  // every wave has read its last fragments
+  float* red = reinterpret_cast<float*>(smem);
+  float* red_m = reinterpret_cast<float*>(smem + kTailRedStats);
+  float* red_l = red_m + 4 * 32;
+#pragma unroll
+  for (int db = 0; db < 4; ++db)
+#pragma unroll
+    for (int g4 = 0; g4 < 4; ++g4)
+      *reinterpret_cast<f32x4*>(red + (wave * 32 + n) * kTailRedRow + 32 * db + 8 * g4 + 4 * hh) =
+          f32x4{oacc[db][4 * g4], oacc[db][4 * g4 + 1], oacc[db][4 * g4 + 2], oacc[db][4 * g4 + 3]};
+  if (hh == 0) {
+    red_m[wave * 32 + n] = m_run;
+    red_l[wave * 32 + n] = l_run;
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < REP * kHeadDim; i += 256) {
-    const int r = i / kHeadDim, d = i % kHeadDim;
-    float mm = red_m[0][r];
+  const int rows_here = min(32 * wr_n, rows - group * wr_n * 32);
+  for (int i = tid; i < rows_here * 32; i += 256) {
+    const int rr = i >> 5, d = (i & 31) * 4;      // row of the workgroup, dimension
+    const int w0 = rr >> 5, nn = rr & 31;         // its row block (= its first wave), its row in there
+    float mm = red_m[w0 * 32 + nn];
+    for (int w = 1; w < wk_n; ++w) mm = fmaxf(mm, red_m[(w0 + (w << p.wr_log2)) * 32 + nn]);
+    float ll = 0.f;
+    f32x4 oo = {0.f, 0.f, 0.f, 0.f};
+    for (int w = 0; w < wk_n; ++w) {
+      const int at = (w0 + (w << p.wr_log2)) * 32 + nn;
+      const float a = fast_exp2(red_m[at] - mm);
+      ll += red_l[at] * a;
+      const f32x4 x = *reinterpret_cast<const f32x4*>(red + at * kTailRedRow + d);
 #pragma unroll
-    for (int w = 1; w < 4; ++w) mm = fmaxf(mm, red_m[w][r]);
-    float ll = 0.f, oo = 0.f;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      const float a = fast_exp2(red_m[w][r] - mm);
-      ll += red_l[w][r] * a;
-      oo += red_o[w][r][d] * a;
+      for (int e = 0; e < 4; ++e) oo[e] += x[e] * a;
     }
-    const int64_t row = ((int64_t)b * Hkv * REP + hkv * REP + r) * nsplit + split;
-    // a split without keys cannot occur (the host sizes the splits), so ll > 0
-    part_o[row * kHeadDim + d] = oo / ll;
-    if (d == 0) part_lse[row] = mm + fast_log2(ll);
+    const int rg = group * wr_n * 32 + rr;
+    const int jj = rg / p.rep, gg = rg - jj * p.rep;
+    const int64_t orow = ((int64_t)b * p.nq + jj) * (p.Hkv * p.rep) + hkv * p.rep + gg;
+    // (a row may see no key of its split: the causal limit; never without another split that it does see)
+    const float inv = ll > 0.f ? 1.f / ll : 0.f;
+    if (p.nsplit == 1) {
+      u32x2 w;
+      w[0] = pack2<E>(oo[0] * inv, oo[1] * inv);
+      w[1] = pack2<E>(oo[2] * inv, oo[3] * inv);
+      *reinterpret_cast<u32x2*>(p.out + orow * kHeadDim + d) = w;
+    } else {
+      const int64_t prow = orow * p.nsplit + split;
+      *reinterpret_cast<f32x4*>(p.part_o + prow * kHeadDim + d) = f32x4{oo[0] * inv, oo[1] * inv, oo[2] * inv, oo[3] * inv};
+      if (d == 0) p.part_lse[prow] = ll > 0.f ? mm - TailShift<E>::value + fast_log2(ll) : -INFINITY;
+    }
   }
 }
 
-// One workgroup per (batch, query head): four waves take a quarter of the splits each, a lane owns
-// two head dimensions; the four partial sums meet in LDS.
+// One workgroup per output row: four waves take a quarter of the splits each, a lane owns two head dimensions; the
+// four partial sums meet in LDS.
 template <class E>
-__global__ __launch_bounds__(256) void decode_merge_kernel(const float* __restrict__ part_o,
-                                                           const float* __restrict__ part_lse,
-                                                           typename E::elem* __restrict__ out, int nsplit) {
+__global__ __launch_bounds__(256) void tail_merge_kernel(const float* __restrict__ part_o,
+                                                         const float* __restrict__ part_lse,
+                                                         typename E::elem* __restrict__ out, int nsplit) {
   typedef typename E::elem elem;
   __shared__ float red[4][kHeadDim];
   __shared__ float red_l[4];
-  const int64_t row = blockIdx.x;  // b * Hq + hq
+  const int64_t row = blockIdx.x;  // (b * nq + j) * H + h
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const float* pl = part_lse + row * nsplit;
   float mm = -INFINITY;
@@ -197,68 +298,98 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(const float* __restri
 
 using namespace moba;
 
-// Number of key splits the kernels will use for this problem: the caller sizes
-// part_o [B*Hq*splits, D] fp32 and part_lse [B*Hq*splits] fp32 with it.
-static int decode_split(int B, int Hkv, int Skv, int* keys_per_split) {
-  const int64_t groups = (int64_t)B * Hkv;
-  int64_t want = (1024 + groups - 1) / groups;        // enough workgroups to fill 256 CUs several times
-  const int64_t by_len = (Skv + 255) / 256;           // at least 256 keys per split
-  if (want > by_len) want = by_len;
-  if (want > kDecodeMaxSplits) want = kDecodeMaxSplits;
-  if (want < 1) want = 1;
-  const int per = (int)((Skv + want - 1) / want);
-  *keys_per_split = per;
-  return (Skv + per - 1) / per;                        // no empty split
+struct TailSplit {
+  int wr_log2, groups, keys_per_split, nsplit;  // groups: workgroups per (sequence, key/value head, split)
+};
+
+// How the work is cut: row blocks over the waves of a workgroup, then the keys over workgroups.  A workgroup's time
+// is its steps (kTailKeys keys per wave that splits the keys) plus about one more for start and end, and a compute
+// unit holds one workgroup: the number of splits is the one that gives the shortest rounds * steps.
+static TailSplit tail_split(int B, int Hkv, int rows, int Skv) {
+  TailSplit t;
+  t.wr_log2 = rows <= 32 ? 0 : (rows <= 64 ? 1 : 2);
+  t.groups = (rows + (32 << t.wr_log2) - 1) / (32 << t.wr_log2);
+  const int unit = kTailKeys * (4 >> t.wr_log2);
+  const int steps = (Skv + unit - 1) / unit;
+  const int64_t wgs = (int64_t)B * Hkv * t.groups;
+  int cus = compute_units();
+  if (cus <= 0) cus = 256;
+  int64_t best = 0;
+  t.nsplit = 1;
+  t.keys_per_split = steps * unit;
+  for (int ns = 1; ns <= steps && ns <= kTailMaxSplits; ++ns) {
+    const int per = (steps + ns - 1) / ns, n = (steps + per - 1) / per;  // (no empty split)
+    const int64_t cost = ((wgs * n + cus - 1) / cus) * (per + 1);
+    if (ns == 1 || cost < best) {
+      best = cost;
+      t.nsplit = n;
+      t.keys_per_split = per * unit;
+    }
+  }
+  return t;
 }
 
+// The caller sizes part_o [B*nq*Hkv*rep*splits, D] fp32 and part_lse with it.
+extern "C" int moba_tail_splits(int B, int Hkv, int rep, int nq, int Skv) {
+  if (B <= 0 || Hkv <= 0 || rep <= 0 || nq <= 0 || nq > Skv || (int64_t)rep * nq > (1 << 20)) return 0;
+  return tail_split(B, Hkv, rep * nq, Skv).nsplit;
+}
 extern "C" int moba_decode_splits(int B, int Hkv, int Skv) {
-  if (B <= 0 || Hkv <= 0 || Skv <= 0) return 0;
-  int per;
-  return decode_split(B, Hkv, Skv, &per);
+  return moba_tail_splits(B, Hkv, 1, 1, Skv);  // (the same for every group of up to 32 query heads)
 }
 
-template <class E, int REP>
-static void launch_decode(const void* q, const void* k, const void* v, void* out, float* part_o, float* part_lse,
-                          int B, int Hkv, int Skv, int64_t qsb, int64_t qsh, int64_t kvsb, int64_t kvsh, int nsplit,
-                          int per, float scale_log2, hipStream_t st) {
+template <class E>
+static int launch_tail(const void* q, const void* k, const void* v, void* out, float* part_o, float* part_lse,
+                       const TailSplit& ts, int B, int Hkv, int rep, int nq, int Skv, const int64_t* strides, float scale,
+                       hipStream_t st) {
+  LaunchCheck launch_check;
   typedef typename E::elem elem;
-  hipLaunchKernelGGL((decode_partial_kernel<E, REP>), dim3(nsplit, Hkv, B), dim3(256), 0, st, (const elem*)q,
-                     (const elem*)k, (const elem*)v, part_o, part_lse, Hkv, Skv, qsb, qsh, kvsb, kvsh, per, nsplit,
-                     scale_log2);
-  hipLaunchKernelGGL(decode_merge_kernel<E>, dim3((unsigned)(B * Hkv * REP)), dim3(256), 0, st,
-                     (const float*)part_o, (const float*)part_lse, (elem*)out, nsplit);
+  TailParams<E> p;
+  p.q = (const elem*)q; p.k = (const elem*)k; p.v = (const elem*)v; p.out = (elem*)out;
+  p.part_o = part_o; p.part_lse = part_lse;
+  p.q_stride_b = strides[0]; p.q_stride_h = strides[1]; p.q_stride_t = strides[2];
+  p.kv_stride_b = strides[3]; p.kv_stride_h = strides[4];
+  p.Hkv = Hkv; p.rep = rep; p.Skv = Skv; p.nq = nq;
+  p.wr_log2 = ts.wr_log2; p.keys_per_split = ts.keys_per_split; p.nsplit = ts.nsplit;
+  p.scale_log2 = scale * 1.4426950408889634f;
+  static bool allowed[kMaxDevices];
+  if (!allow_dynamic_lds((const void*)tail_partial_kernel<E>, kTailLds, allowed)) return MOBA_ERR_LAUNCH;
+  hipLaunchKernelGGL(tail_partial_kernel<E>, dim3(ts.nsplit, Hkv * ts.groups, B), dim3(256), kTailLds, st, p);
+  if (ts.nsplit > 1)
+    hipLaunchKernelGGL(tail_merge_kernel<E>, dim3((unsigned)((int64_t)B * nq * Hkv * rep)), dim3(256), 0, st,
+                       (const float*)part_o, (const float*)part_lse, (elem*)out, ts.nsplit);
+  return launch_check.result();
 }
 
-// q [B, H, D] (strides q_stride_b, q_stride_h in elements, D contiguous); k, v [B, Hkv, Skv, D]
-// (strides kv_stride_b, kv_stride_h; a key row is D contiguous elements and rows are D apart);
-// out [B, H, D] contiguous.  H / Hkv must be 1, 2, 4 or 8.
+// q [B, H, nq, D] with the strides (elements) {batch, head, token}, D contiguous; k, v [B, Hkv, Skv, D] with the
+// strides {batch, head}, a key row D contiguous elements and rows D apart: strides[5] holds the five.
+// out [B, nq, H, D] contiguous.
+extern "C" int moba_tail(const void* q, const void* k, const void* v, void* out, float* part_o, float* part_lse, int B,
+                         int H, int Hkv, int nq, int Skv, int D, const int64_t* strides, float scale, int dtype,
+                         void* stream) {
+  if (!q || !k || !v || !out || !part_o || !part_lse || !strides) return MOBA_ERR_ARG;
+  if (B <= 0 || H <= 0 || Hkv <= 0 || Skv <= 0 || nq <= 0 || nq > Skv || H % Hkv != 0 || B > 65535) return MOBA_ERR_ARG;
+  if (D != kHeadDim || (dtype != MOBA_DTYPE_BF16 && dtype != MOBA_DTYPE_F16)) return MOBA_ERR_UNSUPPORTED;
+  if (((uintptr_t)q & 15) || ((uintptr_t)k & 15) || ((uintptr_t)v & 15) || ((uintptr_t)out & 15) ||
+      ((uintptr_t)part_o & 15))
+    return MOBA_ERR_ARG;
+  for (int i = 0; i < 5; ++i)
+    if (strides[i] & 7) return MOBA_ERR_ARG;  // 16-byte loads
+  const int rep = H / Hkv;
+  if ((int64_t)rep * nq > (1 << 20)) return MOBA_ERR_LIMIT;
+  const TailSplit ts = tail_split(B, Hkv, rep * nq, Skv);
+  if ((int64_t)Hkv * ts.groups > 65535 || (int64_t)B * nq * H >= 0x7fffffffLL) return MOBA_ERR_LIMIT;
+  hipStream_t st = (hipStream_t)stream;
+  return dtype == MOBA_DTYPE_F16
+             ? launch_tail<F16>(q, k, v, out, part_o, part_lse, ts, B, Hkv, rep, nq, Skv, strides, scale, st)
+             : launch_tail<Bf16>(q, k, v, out, part_o, part_lse, ts, B, Hkv, rep, nq, Skv, strides, scale, st);
+}
+
+// One token: q [B, H, D] (strides q_stride_b, q_stride_h in elements), out [B, H, D] contiguous.  H / Hkv at most 32.
 extern "C" int moba_decode(const void* q, const void* k, const void* v, void* out, float* part_o, float* part_lse,
                            int B, int H, int Hkv, int Skv, int D, int64_t q_stride_b, int64_t q_stride_h,
                            int64_t kv_stride_b, int64_t kv_stride_h, float scale, int dtype, void* stream) {
-  LaunchCheck launch_check;
-  if (!q || !k || !v || !out || !part_o || !part_lse) return MOBA_ERR_ARG;
-  if (B <= 0 || H <= 0 || Hkv <= 0 || Skv <= 0 || H % Hkv != 0 || B > 65535 || Hkv > 65535) return MOBA_ERR_ARG;
-  if (D != kHeadDim || (dtype != MOBA_DTYPE_BF16 && dtype != MOBA_DTYPE_F16)) return MOBA_ERR_UNSUPPORTED;
-  if (((uintptr_t)q & 15) || ((uintptr_t)k & 15) || ((uintptr_t)v & 15)) return MOBA_ERR_ARG;
-  if ((q_stride_b | q_stride_h | kv_stride_b | kv_stride_h) & 7) return MOBA_ERR_ARG;  // 16-byte loads
-  const int rep = H / Hkv;
-  int per;
-  const int nsplit = decode_split(B, Hkv, Skv, &per);
-  const float sl2 = scale * 1.4426950408889634f;
-  hipStream_t st = (hipStream_t)stream;
-#define MOBA_DECODE(EL, R)                                                                                      \
-  launch_decode<EL, R>(q, k, v, out, part_o, part_lse, B, Hkv, Skv, q_stride_b, q_stride_h, kv_stride_b,       \
-                       kv_stride_h, nsplit, per, sl2, st)
-#define MOBA_DECODE_REP(EL)                 \
-  switch (rep) {                            \
-    case 1: MOBA_DECODE(EL, 1); break;      \
-    case 2: MOBA_DECODE(EL, 2); break;      \
-    case 4: MOBA_DECODE(EL, 4); break;      \
-    case 8: MOBA_DECODE(EL, 8); break;      \
-    default: return MOBA_ERR_UNSUPPORTED;   \
-  }
-  if (dtype == MOBA_DTYPE_F16) { MOBA_DECODE_REP(F16) } else { MOBA_DECODE_REP(Bf16) }
-#undef MOBA_DECODE_REP
-#undef MOBA_DECODE
-  return launch_check.result();
+  if (Hkv > 0 && H / Hkv > 32) return MOBA_ERR_UNSUPPORTED;  // (moba_decode_splits knows groups of up to 32 only)
+  const int64_t strides[5] = {q_stride_b, q_stride_h, 0, kv_stride_b, kv_stride_h};
+  return moba_tail(q, k, v, out, part_o, part_lse, B, H, Hkv, 1, Skv, D, strides, scale, dtype, stream);
 }

@@ -1,9 +1,8 @@
 """Decode attention on MI355X: new query tokens against the key/value cache (the adapter's decode
 branch, moba/wrapper.py:76-82, which calls flash_attn_func in the reference: every cached key is
-visible to a new token up to its own position).  One token: the HIP decode kernel reads K and V of
-the cache once, in place, with grouped-query heads.  A few tokens: that kernel once per token.  Many
-tokens (chunked prefill against a cache): the forward attention kernel's causal tiles on the tail of
-the sequence."""
+visible to a new token up to its own position).  One token or a few: the HIP decode kernel reads K and V of
+the cache once, in place, for all query rows of a key/value head.  Many tokens (chunked prefill against a cache):
+the forward attention kernel's causal tiles on the tail of the sequence."""
 
 from __future__ import annotations
 
@@ -19,56 +18,8 @@ SUPPORTED_GROUP_SIZES = (1, 2, 4, 8)
 
 def supported(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor) -> bool:
     """True when decode_attention can take these tensors ([B,H,1,D] and [B,Hkv,Skv,D])."""
-    if not (query.is_cuda and key.is_cuda and value.is_cuda):
-        return False
-    if query.dtype not in (torch.bfloat16, torch.float16) or key.dtype != query.dtype or value.dtype != query.dtype:
-        return False
-    if query.dim() != 4 or key.dim() != 4 or key.shape != value.shape:
-        return False
-    b, h, q_len, d = query.shape
-    if q_len != 1 or d != 128 or key.shape[0] != b or key.shape[3] != d or key.shape[2] == 0:
-        return False
-    return key.shape[1] > 0 and h % key.shape[1] == 0 and h // key.shape[1] in SUPPORTED_GROUP_SIZES
-
-
-def _rows_in_place(t: torch.Tensor) -> torch.Tensor:
-    """A [B,Hkv,Skv,D] tensor whose key rows are contiguous and D apart, with 16-byte friendly strides."""
-    d = t.shape[3]
-    ok = t.stride(3) == 1 and t.stride(2) == d and t.stride(0) % 8 == 0 and t.stride(1) % 8 == 0 and t.data_ptr() % 16 == 0
-    return t if ok else t.contiguous()
-
-
-def decode_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
-                     scaling: Optional[float] = None) -> torch.Tensor:
-    """query [B,H,1,D], key/value [B,Hkv,Skv,D] -> [B,1,H,D] (the layout the adapter returns).
-    Softmax scale ``scaling`` (default D**-0.5); every cached key is visible."""
-    if not supported(query, key, value):
-        raise ValueError("decode_attention needs bf16/fp16 GPU tensors, one query token, head_dim 128 and "
-                         "1, 2, 4 or 8 query heads per key/value head")
-    lib = _lib.load()
-    b, h, _, d = query.shape
-    hkv, skv = key.shape[1], key.shape[2]
-    q = query if (query.stride(3) == 1 and query.stride(0) % 8 == 0 and query.stride(1) % 8 == 0
-                  and query.data_ptr() % 16 == 0) else query.contiguous()
-    k, v = _rows_in_place(key), _rows_in_place(value)
-    if k.stride() != v.stride():
-        k, v = k.contiguous(), v.contiguous()
-    splits = lib.moba_decode_splits(b, hkv, skv)
-    dev = query.device
-    part_o = torch.empty((b * h * splits, d), dtype=torch.float32, device=dev)
-    part_lse = torch.empty((b * h * splits,), dtype=torch.float32, device=dev)
-    out = torch.empty((b, 1, h, d), dtype=query.dtype, device=dev)
-    scale = float(scaling) if scaling is not None else d ** -0.5
-    dtype = _lib.DTYPE_F16 if query.dtype == torch.float16 else _lib.DTYPE_BF16
-    stream = ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
-    p = lambda t: ctypes.c_void_p(t.data_ptr())
-    _lib.check(lib.moba_decode(p(q), p(k), p(v), p(out), p(part_o), p(part_lse), b, h, hkv, skv, d,
-                               q.stride(0), q.stride(1), k.stride(0), k.stride(1), scale, dtype, stream),
-               "moba_decode")
-    return out
-
-
-SHORT_QUERY = 16   # up to this many new tokens: one launch of the decode kernel per token
+    return (chunk_supported(query, key, value) and query.shape[2] == 1
+            and query.shape[1] // key.shape[1] in SUPPORTED_GROUP_SIZES)
 
 
 def chunk_supported(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor) -> bool:
@@ -83,6 +34,55 @@ def chunk_supported(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor)
     if d != 128 or key.shape[0] != b or key.shape[3] != d or not 0 < q_len <= key.shape[2]:
         return False
     return key.shape[1] > 0 and h % key.shape[1] == 0
+
+
+def _rows_in_place(t: torch.Tensor) -> torch.Tensor:
+    """A [B,Hkv,Skv,D] tensor whose key rows are contiguous and D apart, with 16-byte friendly strides."""
+    d = t.shape[3]
+    ok = t.stride(3) == 1 and t.stride(2) == d and t.stride(0) % 8 == 0 and t.stride(1) % 8 == 0 and t.data_ptr() % 16 == 0
+    return t if ok else t.contiguous()
+
+
+def _tail(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, scaling: Optional[float]) -> torch.Tensor:
+    """[B,H,q_len,D] against [B,Hkv,Skv,D] -> [B,q_len,H,D] on the decode kernel: the cache is read once for all
+    query rows of a key/value head."""
+    lib = _lib.load()
+    b, h, q_len, d = query.shape
+    hkv, skv = key.shape[1], key.shape[2]
+    qs = query.stride()
+    q = query if (qs[3] == 1 and not (qs[0] | qs[1] | qs[2]) & 7 and query.data_ptr() % 16 == 0) else query.contiguous()
+    k, v = _rows_in_place(key), _rows_in_place(value)
+    if k.stride() != v.stride():
+        k, v = k.contiguous(), v.contiguous()
+    dev = query.device
+    out = torch.empty((b, q_len, h, d), dtype=query.dtype, device=dev)
+    rows = b * q_len * h * lib.moba_tail_splits(b, hkv, h // hkv, q_len, skv)
+    part = torch.empty(rows * (d + 1), dtype=torch.float32, device=dev)   # partial outputs, then their log-sum-exps
+    part_o = part.data_ptr()
+    scale = float(scaling) if scaling is not None else d ** -0.5
+    dtype = _lib.DTYPE_F16 if query.dtype == torch.float16 else _lib.DTYPE_BF16
+    qs, ks = q.stride(), k.stride()
+    _lib.check(lib.moba_tail(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), part_o, part_o + rows * d * 4, b, h,
+                             hkv, q_len, skv, d, (ctypes.c_int64 * 5)(qs[0], qs[1], qs[2], ks[0], ks[1]), scale, dtype,
+                             torch.cuda.current_stream(dev).cuda_stream), "moba_tail")
+    return out
+
+
+def decode_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
+                     scaling: Optional[float] = None) -> torch.Tensor:
+    """query [B,H,1,D], key/value [B,Hkv,Skv,D] -> [B,1,H,D] (the layout the adapter returns).
+    Softmax scale ``scaling`` (default D**-0.5); every cached key is visible."""
+    if not supported(query, key, value):
+        raise ValueError("decode_attention needs bf16/fp16 GPU tensors, one query token, head_dim 128 and "
+                         "1, 2, 4 or 8 query heads per key/value head")
+    return _tail(query, key, value, scaling)
+
+
+# Up to this many new tokens the decode kernel takes them, more go to the forward kernel's causal tiles.  Measured at 512
+# new tokens, decode kernel / tiles: 0.62 / 0.75 ms (34816 keys, 32 heads on 8), 1.51 / 1.78 ms (4 sequences of 20000
+# keys), 0.056 / 0.18 ms (8000 keys, 8 heads on 8); at 2048 tokens the tiles do 34816 keys in 1.0 ms, which the decode
+# kernel's 0.45 PFLOP/s would take 2.3 ms for.
+TAIL_TOKENS = 512
 
 
 _TAIL_TABLES = {}  # (kv_len, row tiles skipped, device) -> int32 tables of the causal tiles of a sequence's tail
@@ -111,10 +111,8 @@ def chunk_decode_attention(query: torch.Tensor, key: torch.Tensor, value: torch.
                          "keys and a whole number of query heads per key/value head")
     b, h, q_len, d = query.shape
     hkv, kv_len = key.shape[1], key.shape[2]
-    if q_len <= SHORT_QUERY and h // hkv in SUPPORTED_GROUP_SIZES:
-        first = kv_len - q_len + 1
-        return torch.cat([decode_attention(query[:, :, j:j + 1], key[:, :, :first + j], value[:, :, :first + j], scaling)
-                          for j in range(q_len)], dim=1)
+    if q_len <= TAIL_TOKENS:
+        return _tail(query, key, value, scaling)
     from . import moba_efficient as E
     lib = _lib.load()
     dev = query.device

@@ -134,3 +134,39 @@ def test_adapter_decodes_several_tokens_with_the_kernels():
         b, _ = moba_layer(moba_attn_varlen_naive, cfg, Mod(), q, k, v, None)    # SDPA with the bottom-right mask
         assert calls == [1] and a.shape == b.shape == (2, q_len, 8, 128)
         assert (a.float() - b.float()).abs().max() < 2e-2
+
+
+@pytest.mark.parametrize("B,H,Hkv,dtype", [(1, 8, 2, torch.bfloat16), (2, 3, 1, torch.float16), (1, 2, 2, torch.bfloat16)])
+@pytest.mark.parametrize("Skv,q_len", [(1, 1), (31, 5), (32, 32), (33, 8), (129, 9), (300, 16), (1025, 17), (700, 33), (2113, 129)])
+def test_decode_kernel_at_the_edges_of_its_blocks(B, H, Hkv, dtype, Skv, q_len):
+    """Key counts around the 32-key steps and the splits, row counts around 32, 64 and 128 rows per key/value head (one,
+    two and four row blocks per workgroup, several workgroups), a group of three heads, q as a slice of a fused
+    projection.  Errors: the result is rounded once to the element type (2^-9 / 2^-12 of values up to about 4)."""
+    from moba_amd.decode import chunk_decode_attention
+    print("block case", B, H, Hkv, Skv, q_len, dtype, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(Skv * 131 + q_len)
+    q = torch.randn((B, q_len, H + 2 * Hkv, 128), generator=g, device="cuda").to(dtype)[:, :, :H].transpose(1, 2)
+    k = torch.randn((B, Hkv, Skv + 7, 128), generator=g, device="cuda").to(dtype)[:, :, :Skv]
+    v = torch.randn((B, Hkv, Skv + 7, 128), generator=g, device="cuda").to(dtype)[:, :, :Skv]
+    out = chunk_decode_attention(q, k, v)
+    want = _ref_tail(q, k, v, 128 ** -0.5)
+    err = (out.float() - want).abs()
+    bound = (4.0 if dtype == torch.bfloat16 else 0.5) * 2.0 ** -8
+    assert torch.isfinite(out.float()).all() and err.max() < bound, err.max().item()
+
+
+def test_decode_kernel_keeps_small_probabilities():
+    """One key far above 100000 others whose probabilities are 2^-22 to 2^-16 of its own and together weigh a quarter of it:
+    they must not fall below the element type (fp16's smallest number is 2^-24) or be rounded away."""
+    from moba_amd.decode import chunk_decode_attention
+    for dtype in (torch.float16, torch.bfloat16):
+        q = torch.zeros((1, 1, 1, 128), device="cuda", dtype=dtype)
+        q[..., 0] = 1.0
+        k = torch.zeros((1, 1, 100001, 128), device="cuda", dtype=dtype)
+        k[0, 0, 1:, 0] = -torch.linspace(16, 22, 100000, device="cuda").to(dtype)
+        v = torch.ones((1, 1, 100001, 128), device="cuda", dtype=dtype)
+        v[0, 0, 0] = 0
+        out = chunk_decode_attention(q, k, v, 0.6931471805599453)     # (a score of -x is a probability of 2^-x)
+        p = torch.exp2(k[0, 0, :, 0].double())
+        want = (p[1:].sum() / p.sum()).item()
+        assert abs(out.float().mean().item() - want) < 2.0 ** -7 * want, (dtype, out.float().mean().item(), want)
