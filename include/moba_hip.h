@@ -258,6 +258,18 @@ int moba_fwd_partials(const void* q, const void* k, const void* v, void* part_o,
                       float* lse, int64_t S, int H, int Hkv, int D, int K, int F, int N, int B, int64_t hist_bound,
                       int64_t self_tiles, int key_split, const int64_t* strides, int32_t* queues, int32_t* redo,
                       float softmax_scale, int dtype, int self_tile_skip, int64_t q_tok_shift, void* stream);
+/* The same on tile tables (self_tile_prefix, self_tile_chunk, tile_off, tile_seg, hist_bound, self_tiles) for tiles of
+ * tile_rows rows: moba_fwd_tile_rows(), or moba_bwd_tile_rows(), whose tiles run one workgroup each, two side by side
+ * on a compute unit, for problems of short chunks or few tiles.  queues is then not used; redo, if given, has redo[0]
+ * zeroed by the caller and receives the tiles that were computed again with a running maximum, for information. */
+int moba_fwd_partials_rows(const void* q, const void* k, const void* v, void* part_o, float* part_lse,
+                           const int32_t* seg_off, const int32_t* tile_off, const int32_t* seg_dest,
+                           const int32_t* fchunk_tok, const int32_t* chunk_tok, const int32_t* self_tile_prefix,
+                           const int32_t* tile_seg, const int32_t* self_tile_chunk, const int32_t* chunk_direct, void* out,
+                           float* lse, int64_t S, int H, int Hkv, int D, int K, int F, int N, int B, int64_t hist_bound,
+                           int64_t self_tiles, int key_split, const int64_t* strides, int32_t* queues, int32_t* redo,
+                           float softmax_scale, int dtype, int self_tile_skip, int64_t q_tok_shift, int tile_rows,
+                           void* stream);
 int moba_fwd_merge(const void* part_o, const float* part_lse, const int32_t* sel, void* out, float* lse, int64_t S,
                    int H, int D, int K, int key_split, const int32_t* mrg_start, const int32_t* mrg_prefix, int nranges,
                    int64_t merge_tokens, int dtype, void* stream);

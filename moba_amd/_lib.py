@@ -42,6 +42,9 @@ _SIGNATURES = {
     "moba_fwd_partials": (c_int, [c_void_p] * 16 + [c_int64, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int64,
                                                    c_int64, c_int, c_strides, c_void_p, c_void_p, c_float, c_int,
                                                    c_int, c_int64, c_void_p]),
+    "moba_fwd_partials_rows": (c_int, [c_void_p] * 16 + [c_int64, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
+                                                        c_int64, c_int64, c_int, c_strides, c_void_p, c_void_p, c_float,
+                                                        c_int, c_int, c_int64, c_int, c_void_p]),
     "moba_fwd_merge": (c_int, [c_void_p] * 5 + [c_int64, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_int, c_int64,
                                                c_int, c_void_p]),
     "moba_fwd_key_split": (c_int, [c_int64, c_int, c_int, c_int, c_int64, c_int64]),

@@ -14,7 +14,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(CSRC, "build")
 LIB = os.path.join(HERE, "libmoba_hip.so")
-SOURCES = ["chunk_mean.hip", "gate_topk.hip", "lists.hip", "fwd.hip", "bwd.hip", "decode.hip", "plan.hip", "probe.hip", "capi.hip"]
+SOURCES = ["chunk_mean.hip", "gate_topk.hip", "lists.hip", "fwd.hip", "fwd_tile.hip", "bwd.hip", "decode.hip", "plan.hip", "probe.hip", "capi.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -27,13 +27,14 @@ FLAGS = [
 
 # per-source extra flags: the attention kernels never produce NaN from finite inputs, and
 # telling the compiler so removes the canonicalisation of every MFMA result before a max
-EXTRA = {"fwd.hip": ["-fno-honor-nans"]}
+EXTRA = {"fwd.hip": ["-fno-honor-nans"], "fwd_tile.hip": ["-fno-honor-nans"]}
 
 
 def _compile(src: str, force: bool) -> str:
     path = os.path.join(CSRC, src)
     obj = os.path.join(OBJ, src.replace(".hip", ".o"))
-    deps = [path, os.path.join(CSRC, "common.h"), os.path.join(CSRC, "attn_common.h"), os.path.abspath(__file__)]
+    headers = [os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith(".h")]
+    deps = [path, *headers, os.path.abspath(__file__)]
     if not force and os.path.exists(obj) and all(os.path.getmtime(obj) > os.path.getmtime(d) for d in deps):
         return obj
     cmd = [HIPCC, *FLAGS, *EXTRA.get(src, []), "-c", path, "-o", obj]

@@ -121,9 +121,13 @@ static __global__ void zero_queues_kernel(int* queues, int* also) {
 // Workgroup ids are dealt round-robin to the 8 XCDs; give each XCD runs of 1 << block_log2 (at most kXcdBlock)
 // consecutive logical tiles so that tiles sharing a K/V chunk share an L2.  (A grid of few tiles takes shorter
 // runs: whole runs of 64 would leave some XCDs with twice the tiles of others, or with none.)
+// Every other round of runs goes to the XCDs in reverse: causal tiles come longest first head by head, and where a
+// head is a whole number of runs the same XCDs would otherwise get the long half of every head (16384 tokens, 32
+// heads, full causal attention: 2.45 -> 2.07 ms).
 __device__ __forceinline__ int logical_tile_id(int block_log2) {
-  const int x = blockIdx.x & 7, y = blockIdx.x >> 3;
-  return ((((y >> block_log2) << 3) + x) << block_log2) + (y & ((1 << block_log2) - 1));
+  const int y = blockIdx.x >> 3, round = y >> block_log2;
+  const int x = (round & 1) ? 7 - (blockIdx.x & 7) : (blockIdx.x & 7);
+  return (((round << 3) + x) << block_log2) + (y & ((1 << block_log2) - 1));
 }
 
 // Tile decoding in steps, so that a kernel can start the key/value copies (which need only the

@@ -19,7 +19,7 @@
 // MFMA rate.  Compulsory HBM traffic is q, k, v once, the partials once each way.
 #include <cstddef>
 #include <type_traits>
-#include "attn_common.h"
+#include "fwd_common.h"
 
 namespace moba {
 
@@ -33,33 +33,10 @@ constexpr int kFwdEntries = 2 * kFwdStages * kTileBytes, kFwdIdSlot = kFwdEntrie
 constexpr int kFwdRedoWord = kFwdIdSlot + 8;  // set by a wave whose rows left the range of the fixed-reference softmax
 constexpr int kFwdLds = kFwdIdSlot + 16;
 
-template <class E>
-struct FwdParams {
-  const typename E::elem* q;
-  const typename E::elem* k;
-  const typename E::elem* v;
-  typename E::elem* part_o;  // [S*H*K1, D]
-  float* part_lse;  // [S*H*K1], log2 domain
-  typename E::elem* out;     // [S*H, D]: where the tiles of chunks without history slots (TileTables::chunk_direct) write
-  float* lse;                // [S*H], natural log
-  TileTables t;
-  float scale_log2;  // D^-0.5 * log2(e)
-  int* queues;       // [8] tile counters, one per XCD, zero when the kernel starts
-  int* redo;         // [1 + tiles] count and ids of the tiles to be computed again (see kFixedRef); count zero at the start
-};
-
-constexpr float kRescaleThreshold = 8.f;  // log2 units: the running max may lag the true max by this much
-// Fixed-reference softmax: a row's sum of exponentials (relative to the row maximum of the tile's first key
-// block) at or beyond this, or not a number, sends the tile to the kernel that tracks the maximum; so does an
-// accumulator of the row that is not finite (a probability beyond the element type's range -- 2^16 for fp16 --
-// or products with large |v| that left fp32).
-constexpr float kFixedRefMaxSum = 0x1p96f;
-
-// how a workgroup comes by its tiles
+// how a resident workgroup comes by its tiles
 enum : int {
-  kTilePerGroup = 0,  // one tile, the id from the workgroup id (small problems)
-  kTilesQueued = 1,   // resident workgroups drawing ids from the per-XCD queues
-  kTilesListed = 2,   // resident workgroups walking the list FwdParams::redo
+  kTilesQueued,   // drawing ids from the per-XCD queues
+  kTilesListed,   // walking the list FwdParams::redo
 };
 
 // The loop is software pipelined by hand at the granularity of a 32-key block u:
@@ -72,9 +49,9 @@ enum : int {
 // One barrier per key tile, at its top: a wave first waits for its own copies of tile t+1 (issued a whole tile
 // earlier), and once all eight waves have passed the barrier tile t+1 is complete in LDS and nobody reads tile
 // t-1 any more, so its stage takes tile t+2.
-// kMode: resident workgroups that draw tiles from the queues (large problems), or one tile per workgroup,
-// the id from the workgroup id: with few tiles the queue protocol's start-up and wind-down (three passes
-// to fill the look-ahead, eight empty draws to know that nothing is left) would dominate.
+// The workgroups are resident and draw their tiles from queues: large problems.  With few tiles the queue protocol's
+// start-up and wind-down (three passes to fill the look-ahead, eight empty draws to know that nothing is left) would
+// dominate: those, and short chunks, run one workgroup per tile (fwd_tile.hip).
 // kFixedRef (queued): the softmax of a tile is taken relative to one fixed reference per row, the row
 // maximum of the tile's first 32-key block, instead of a running maximum.  A bf16 probability has the
 // exponent range of fp32, so later scores may exceed the reference by almost 2^7 before anything overflows
@@ -247,7 +224,6 @@ __global__ __launch_bounds__(512, 2) void moba_fwd_kernel(const FwdParams<E> p) 
   int dest_done = 0, rows_done = 0, id_done = 0;
   bool valid_done = false, direct_done = false;  // (direct: the tile's rows go straight to the outputs)
   int list_pos = blockIdx.x;  // kTilesListed: position in the list of the next tile
-  int key_part = 0;           // kTilePerGroup: which part of a history tile's keys this workgroup takes
   if constexpr (kFixedRef) {
     if (tid == 0) *reinterpret_cast<int*>(smem + kFwdRedoWord) = 0;  // first read many barriers from here
   }
@@ -350,12 +326,6 @@ __global__ __launch_bounds__(512, 2) void moba_fwd_kernel(const FwdParams<E> p) 
   // ================= tile switch =================
   // The next tile's first copies and loads are issued before the finished tile's partial is written: they
   // travel while the partial is normalised and stored.
-  if constexpr (kMode == kTilePerGroup) {
-    if (have_partial) {
-      write_partial();
-      return;
-    }
-  }
   int drawn = 0;  // wave 0, lane 0: the value of the queue's counter
   {
     const FwdParams<E> pn = kernarg_now<FwdParams<E>>(0);
@@ -364,32 +334,13 @@ __global__ __launch_bounds__(512, 2) void moba_fwd_kernel(const FwdParams<E> p) 
     const int er = (tx >> 6) * 32 + (tx & 31);
     if constexpr (kQueued) {
       t = t1;  // the next tile becomes the current one: its rows' gather-list entries are in LDS by now
-    } else if constexpr (kMode == kTilesListed) {
+    } else {
       t.row_count = 0;
       t.nkeys = -1;  // unless there is another tile in the list
       if (list_pos < pn.redo[0]) {  // (uniform; the count is final: the kernel that wrote it has ended)
         const int listed = pn.redo[1 + list_pos];
         list_pos += gridDim.x;
         if (!decode_tile_head(pn.t, listed, t, kFwdTileRows)) t.nkeys = -1;  // (cannot happen: listed ids are tiles)
-      }
-    } else {
-      // the parts of the history tiles (hist_bound << ks ids, the part in the low bits) and the self tiles,
-      // whichever kind takes longer first: workgroups start in the order of their ids
-      int logical = logical_tile_id(pn.t.xcd_block_log2);
-      const int ks = pn.t.key_split_log2;
-      const int parts_end = pn.t.hist_bound << ks;
-      int hist_part = pn.t.self_first ? logical - pn.t.self_total : (logical < parts_end ? logical : -1);
-      if (hist_part >= parts_end) return;
-      if (hist_part >= 0) {
-        key_part = hist_part & ((1 << ks) - 1);
-        logical = hist_part >> ks;
-      } else {
-        logical = pn.t.hist_bound + (pn.t.self_first ? logical : logical - parts_end);
-      }
-      if (!decode_tile_head(pn.t, logical, t, kFwdTileRows)) return;
-      if (t.base >= 0) {  // this part's share of the chunk's keys
-        t.nkeys >>= ks;
-        t.kv_tok0 += key_part * t.nkeys;
       }
     }
     int q_tok = 0, q_head = 0;  // token and head of this lane's query row
@@ -413,7 +364,6 @@ __global__ __launch_bounds__(512, 2) void moba_fwd_kernel(const FwdParams<E> p) 
       // the per-row half (queued: decoded when the Q rows were requested, see prefetch_q), then the Q rows
       if constexpr (!kQueued) {
         decode_tile_rows(pn.t, tx >> 6, er, decode_tile_row_entry(pn.t, er, t), t);
-        if constexpr (kMode == kTilePerGroup) t.dest += key_part * pn.t.part_stride;  // (part 0 for a self tile)
       }
       limit = t.limit;
       min_limit = __builtin_amdgcn_readfirstlane(t.wave_min_limit);
@@ -859,9 +809,9 @@ static int fwd_xcd_block_log2(int64_t total) {  // runs of at most an eighth of 
   while (b < 6 && (128LL << b) <= total) ++b;
   return b;
 }
-static int64_t fwd_grid(int64_t total, int cus) {
+static int64_t fwd_grid(int64_t total, int cus, int tile_rows) {
   int64_t grid = ((int64_t)cus + 7) / 8 * 8;
-  if (total < 8 * grid) {
+  if (tile_rows != kFwdTileRows || total < 8 * grid) {
     const int64_t run = 8LL << fwd_xcd_block_log2(total);
     grid = -((total + run - 1) / run * run);
   }
@@ -873,7 +823,7 @@ static int64_t fwd_grid(int64_t total, int cus) {
 extern "C" int moba_fwd_is_queued(int64_t hist_bound, int64_t self_tiles, int H) {
   const int cus = resident_compute_units();
   if (cus <= 0 || hist_bound < 0 || self_tiles < 0 || H <= 0) return 0;
-  return fwd_grid(hist_bound + self_tiles * H, cus) > 0 ? 1 : 0;
+  return fwd_grid(hist_bound + self_tiles * H, cus, kFwdTileRows) > 0 ? 1 : 0;
 }
 
 // Into how many parts moba_fwd_partials should cut the keys of every history tile: 1 unless the problem is so
@@ -894,8 +844,8 @@ extern "C" int moba_fwd_key_split(int64_t S, int H, int K, int B, int64_t hist_b
 
 template <class E>
 static int launch_partials(const void* q, const void* k, const void* v, void* part_o, float* part_lse, void* out,
-                           float* lse, const TileTables& t, int D, float softmax_scale, int64_t grid, int* queues,
-                           int* redo, hipStream_t st) {
+                           float* lse, const TileTables& t, int D, float softmax_scale, int64_t grid, int tile_rows,
+                           int* queues, int* redo, hipStream_t st) {
   LaunchCheck launch_check;
   FwdParams<E> p;
   p.q = (const typename E::elem*)q; p.k = (const typename E::elem*)k; p.v = (const typename E::elem*)v;
@@ -906,14 +856,14 @@ static int launch_partials(const void* q, const void* k, const void* v, void* pa
                                      : (float)(1.4426950408889634 / sqrt((double)D));
   p.queues = queues;
   p.redo = redo;
-  static bool allowed[4][kMaxDevices];  // one set of arrays per element type
+  static bool allowed[3][kMaxDevices];  // one set of arrays per element type
   if (grid > 0) {  // resident workgroups drawing from the queues
     hipLaunchKernelGGL(zero_queues_kernel, dim3(1), dim3(8), 0, st, queues, redo);  // a kernel, not a memset: graph safe
     {
       if (redo) {
         // fixed-reference softmax, then the tiles it could not serve (normally none) with the tracked maximum
-        if (!allow_dynamic_lds((const void*)moba_fwd_kernel<E, kTilesQueued, true>, kFwdLds, allowed[2]) ||
-            !allow_dynamic_lds((const void*)moba_fwd_kernel<E, kTilesListed, false>, kFwdLds, allowed[3]))
+        if (!allow_dynamic_lds((const void*)moba_fwd_kernel<E, kTilesQueued, true>, kFwdLds, allowed[0]) ||
+            !allow_dynamic_lds((const void*)moba_fwd_kernel<E, kTilesListed, false>, kFwdLds, allowed[2]))
           return MOBA_ERR_LAUNCH;
         hipLaunchKernelGGL((moba_fwd_kernel<E, kTilesQueued, true>), dim3((unsigned)grid), dim3(512), kFwdLds, st, p);
         hipLaunchKernelGGL((moba_fwd_kernel<E, kTilesListed, false>), dim3((unsigned)grid), dim3(512), kFwdLds, st, p);
@@ -923,14 +873,15 @@ static int launch_partials(const void* q, const void* k, const void* v, void* pa
     if (!allow_dynamic_lds((const void*)moba_fwd_kernel<E, kTilesQueued, false>, kFwdLds, allowed[1])) return MOBA_ERR_LAUNCH;
     hipLaunchKernelGGL((moba_fwd_kernel<E, kTilesQueued, false>), dim3((unsigned)grid), dim3(512), kFwdLds, st, p);
   } else {         // one workgroup per tile id
-    if (!allow_dynamic_lds((const void*)moba_fwd_kernel<E, kTilePerGroup, false>, kFwdLds, allowed[0])) return MOBA_ERR_LAUNCH;
-    hipLaunchKernelGGL((moba_fwd_kernel<E, kTilePerGroup, false>), dim3((unsigned)-grid), dim3(512), kFwdLds, st, p);
+    if (tile_rows == kFwdTileRows) p.redo = nullptr;  // (not cleared by this call, not needed)
+    const int rc = launch_fwd_tiles<E>(p, tile_rows, -grid, st);
+    if (rc != MOBA_OK) return rc;
   }
   return launch_check.result();
 }
 
-// hist_bound: any upper bound on the number of history tiles (floor(M/128) + F*H is one).
-extern "C" int moba_fwd_partials(const void* q, const void* k, const void* v, void* part_o, float* part_lse,
+// hist_bound: any upper bound on the number of history tiles (floor(M/tile_rows) + F*H is one).
+extern "C" int moba_fwd_partials_rows(const void* q, const void* k, const void* v, void* part_o, float* part_lse,
                                  const int32_t* seg_off, const int32_t* tile_off, const int32_t* seg_dest,
                                  const int32_t* fchunk_tok, const int32_t* chunk_tok,
                                  const int32_t* self_tile_prefix, const int32_t* tile_seg,
@@ -938,12 +889,13 @@ extern "C" int moba_fwd_partials(const void* q, const void* k, const void* v, vo
                                  int64_t S, int H, int Hkv, int D, int K, int F,
                                  int N, int B, int64_t hist_bound, int64_t self_tiles, int key_split,
                                  const int64_t* strides, int32_t* queues, int32_t* redo, float softmax_scale,
-                                 int dtype, int self_tile_skip, int64_t q_tok_shift, void* stream) {
+                                 int dtype, int self_tile_skip, int64_t q_tok_shift, int tile_rows, void* stream) {
+  if (tile_rows != kFwdTileRows && tile_rows != TM) return MOBA_ERR_ARG;
   if (!q || !k || !v || !part_o || !part_lse || !chunk_tok || !self_tile_prefix || !self_tile_chunk || !queues)
     return MOBA_ERR_ARG;
   if (chunk_direct && (!out || !lse || ((uintptr_t)out & 15))) return MOBA_ERR_ARG;
   // queries that are the tail of their sequence: plain causal attention whose rows all go straight to the outputs
-  if (self_tile_skip < 0 || q_tok_shift < 0 || q_tok_shift > (int64_t)self_tile_skip * kFwdTileRows) return MOBA_ERR_ARG;
+  if (self_tile_skip < 0 || q_tok_shift < 0 || q_tok_shift > (int64_t)self_tile_skip * tile_rows) return MOBA_ERR_ARG;
   if (self_tile_skip > 0 && (K != 0 || !chunk_direct || (strides && strides[4] != 0))) return MOBA_ERR_ARG;
   if (Hkv <= 0 || H % Hkv != 0) return MOBA_ERR_ARG;
   if (K > 0 && (!seg_off || !tile_off || !seg_dest || !fchunk_tok || !tile_seg)) return MOBA_ERR_ARG;
@@ -963,7 +915,7 @@ extern "C" int moba_fwd_partials(const void* q, const void* k, const void* v, vo
   if (cus <= 0) return MOBA_ERR_LAUNCH;
   // with fewer than a few tiles per resident workgroup the queues do not pay: one workgroup per id then
   // (a negative grid tells the launcher)
-  const int64_t grid = fwd_grid(total, cus);
+  const int64_t grid = fwd_grid(total, cus, tile_rows);
   // the parts are tiles of the one-workgroup-per-id form only, whole key tiles each
   if (key_split > 1 && (grid > 0 || B % (TN * key_split) != 0)) return MOBA_ERR_ARG;
   TileTables t;
@@ -983,8 +935,23 @@ extern "C" int moba_fwd_partials(const void* q, const void* k, const void* v, vo
   t.self_skip = self_tile_skip; t.q_shift = (int)q_tok_shift;
   hipStream_t st = (hipStream_t)stream;
   return dtype == MOBA_DTYPE_F16
-             ? launch_partials<F16>(q, k, v, part_o, part_lse, out, lse, t, D, softmax_scale, grid, queues, redo, st)
-             : launch_partials<Bf16>(q, k, v, part_o, part_lse, out, lse, t, D, softmax_scale, grid, queues, redo, st);
+             ? launch_partials<F16>(q, k, v, part_o, part_lse, out, lse, t, D, softmax_scale, grid, tile_rows, queues, redo, st)
+             : launch_partials<Bf16>(q, k, v, part_o, part_lse, out, lse, t, D, softmax_scale, grid, tile_rows, queues, redo, st);
+}
+
+extern "C" int moba_fwd_partials(const void* q, const void* k, const void* v, void* part_o, float* part_lse,
+                                 const int32_t* seg_off, const int32_t* tile_off, const int32_t* seg_dest,
+                                 const int32_t* fchunk_tok, const int32_t* chunk_tok,
+                                 const int32_t* self_tile_prefix, const int32_t* tile_seg,
+                                 const int32_t* self_tile_chunk, const int32_t* chunk_direct, void* out, float* lse,
+                                 int64_t S, int H, int Hkv, int D, int K, int F,
+                                 int N, int B, int64_t hist_bound, int64_t self_tiles, int key_split,
+                                 const int64_t* strides, int32_t* queues, int32_t* redo, float softmax_scale,
+                                 int dtype, int self_tile_skip, int64_t q_tok_shift, void* stream) {
+  return moba_fwd_partials_rows(q, k, v, part_o, part_lse, seg_off, tile_off, seg_dest, fchunk_tok, chunk_tok,
+                                self_tile_prefix, tile_seg, self_tile_chunk, chunk_direct, out, lse, S, H, Hkv, D, K, F, N,
+                                B, hist_bound, self_tiles, key_split, strides, queues, redo, softmax_scale, dtype,
+                                self_tile_skip, q_tok_shift, kFwdTileRows, stream);
 }
 
 // mrg_start [nranges], mrg_prefix [nranges + 1], merge_tokens = mrg_prefix[nranges]: the tokens to merge, for a

@@ -1,0 +1,419 @@
+// Forward attention, one workgroup per tile: the form of the forward kernel for problems of few tiles and of short
+// chunks.  Tiles, slots and results are those of moba_fwd_kernel (fwd.hip); what differs is how a compute unit is
+// kept busy.  There one workgroup of eight waves walks tile after tile, and the switch from one to the next (partial
+// out, lookups, first copies, first products: about 14000 cycles) is paid in the open, which a tile of 2048 or 4096
+// keys hides and one of 256 or 512 keys (8000 to 16000 cycles of matrix work) does not.  Here a workgroup is four
+// waves (128 rows) and two of them share a compute unit (80 KiB of LDS each): one's switch runs under the other's
+// matrix instructions.
+//
+// LDS: a ring of three K stages and two of V, 64 keys each.  At the top of key tile t a wave waits for its own copies
+// of V(t) and K(t+1), issued a tile earlier; behind the barrier both are complete, nobody reads K(t-1) and V(t-1) any
+// more, and their stages take K(t+2) and V(t+1).
+//
+// Measured, attention kernel alone: 3 x 2001 tokens, 32 heads, chunk 256, fp16: 160 -> 104 us; 20480 tokens in five
+// sequences, 8 heads, chunk 512: 163 -> 130 us; 8191 tokens, 32 heads, chunk 512: 374 -> 269 us.  Beyond a few
+// milliseconds the chip's power limit decides and the doubled L2 -> LDS traffic costs 3 to 8 %: those stay with
+// moba_fwd_kernel (the rule stands with the caller's choice of the tile height).
+//
+// Softmax: relative to the row maximum of the tile's first 32 keys (see fwd.hip); a tile in which a row leaves the
+// range that is safe is computed again on the spot with a running maximum, by the same workgroup.
+#include <cstddef>
+#include <type_traits>
+#include "fwd_common.h"
+
+namespace moba {
+
+template <int NW>
+struct FwdTileShape {
+  static constexpr int kVBase = 3 * kTileBytes;
+  static constexpr int kLds = 5 * kTileBytes;       // two workgroups of four waves fill the unit's 160 KiB exactly
+  static constexpr int kFlags = kLds - 4 * NW;      // a word per wave; in the second V stage, free when it is used
+};
+
+template <class E, int NW>
+__global__ __launch_bounds__(NW * 64, 2) void fwd_tile_kernel(const FwdParams<E> p) {
+  MOBA_ELEM_TYPES(E)
+  using Shape = FwdTileShape<NW>;
+  constexpr int kRows = 32 * NW, kCopies = 16 / NW;  // rows of a tile; copy instructions per wave and K or V tile
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 31, hh = lane >> 5;
+
+  // ---- which tile: the parts of the history tiles (hist_bound << ks ids, the part in the low bits) and the self
+  // tiles, whichever kind takes longer first: workgroups start in the order of their ids ----
+  Tile t;
+  int key_part = 0;
+  {
+    int logical = logical_tile_id(p.t.xcd_block_log2);
+    const int ks = p.t.key_split_log2;
+    const int parts_end = p.t.hist_bound << ks;
+    const int hist_part = p.t.self_first ? logical - p.t.self_total : (logical < parts_end ? logical : -1);
+    if (hist_part >= parts_end) return;
+    if (hist_part >= 0) {
+      key_part = hist_part & ((1 << ks) - 1);
+      logical = hist_part >> ks;
+    } else {
+      logical = p.t.hist_bound + (p.t.self_first ? logical : logical - parts_end);
+    }
+    if (!decode_tile_head(p.t, logical, t, kRows)) return;
+    if (t.base >= 0) {  // this part's share of the chunk's keys
+      t.nkeys >>= ks;
+      t.kv_tok0 += key_part * t.nkeys;
+    }
+  }
+  const int h = t.h, nkeys = t.nkeys;
+  const int nkt = (nkeys + TN - 1) / TN;
+
+  // ---- K/V loader: wave w copies the slabs w, w + NW, ... of a tile's 16 (4 keys x 256 bytes each) ----
+  const int64_t row_bytes = p.t.kv_tok_b;
+  const uint32_t lds_base = lds_addr(smem);
+  const int ld_kin = lane >> 4, ld_pc = lane & 15;
+  uint32_t ld_off[kCopies];
+#pragma unroll
+  for (int i = 0; i < kCopies; ++i) {
+    const int key = 4 * (NW * i + wave) + ld_kin;
+    ld_off[i] = (uint32_t)(key * row_bytes + sw_col16(key, ld_pc) * 16);
+  }
+  const int64_t kv_off = kv_tok_bytes(p.t, t.kv_tok0) + (h / p.t.rep) * p.t.kv_head_b;
+  const char* k_head = (const char*)p.k + kv_off;
+  const char* v_head = (const char*)p.v + kv_off;
+  auto issue = [&](const char* head, int kt, uint32_t dst) __attribute__((always_inline)) {
+    const int key0 = kt * TN;
+    if (key0 + TN <= nkeys) {
+      const char* base = head + (int64_t)key0 * row_bytes;
+#pragma unroll
+      for (int i = 0; i < kCopies; ++i) async_copy16_sv(base, ld_off[i], dst + (NW * i + wave) * 1024);
+    } else {
+      // (keys past the end of the range: the last key again -- their scores are masked, their V rows cleared)
+#pragma unroll
+      for (int i = 0; i < kCopies; ++i) {
+        const int slab = NW * i + wave, key = 4 * slab + ld_kin;
+        async_copy16(head + (int64_t)min(key0 + key, nkeys - 1) * row_bytes + sw_col16(key, ld_pc) * 16, dst + slab * 1024);
+      }
+    }
+  };
+  auto issue_k = [&](int kt) __attribute__((always_inline)) {
+    if (kt < nkt) issue(k_head, kt, lds_base + (kt % 3) * kTileBytes);
+  };
+  auto issue_v = [&](int kt) __attribute__((always_inline)) {
+    if (kt < nkt) issue(v_head, kt, lds_base + Shape::kVBase + (kt & 1) * kTileBytes);
+  };
+  // rows of V past the end of the key range must not reach the matrix pipe (0 * NaN): clear them
+  auto scrub_v = [&](int kt) __attribute__((always_inline)) {
+    const int key0 = kt * TN;
+    if (key0 + TN <= nkeys) return;
+    char* vdst = smem + Shape::kVBase + (kt & 1) * kTileBytes;
+#pragma unroll
+    for (int i = 0; i < kCopies; ++i) {
+      const int slab = NW * i + wave;
+      if (key0 + 4 * slab + ld_kin >= nkeys) *reinterpret_cast<u32x4*>(vdst + slab * 1024 + lane * 16) = u32x4{0, 0, 0, 0};
+    }
+  };
+  auto first_copies = [&]() __attribute__((always_inline)) {
+    issue_k(0);
+    issue_v(0);
+    issue_k(1);
+  };
+  first_copies();
+
+  // ---- this lane's row, its Q^T operand ----
+  const int r = wave * 32 + n;
+  decode_tile_rows(p.t, wave, r, decode_tile_row_entry(p.t, r, t), t);
+  const int dest = t.dest + key_part * p.t.part_stride;  // (part 0 for a self tile)
+  const int limit = t.limit;
+  const int min_limit = __builtin_amdgcn_readfirstlane(t.wave_min_limit);
+  const bool row_valid = r < t.row_count;
+  elem8 bq[8];
+  {
+    const elem* src = reinterpret_cast<const elem*>((const char*)p.q + q_tok_bytes(p.t, t.tok) + h * p.t.q_head_b) + 8 * hh;
+#pragma unroll
+    for (int s8 = 0; s8 < 8; ++s8) bq[s8] = *reinterpret_cast<const elem8*>(src + 16 * s8);
+  }
+
+  // ---- fragment addresses inside stage 0 (see fwd.hip) ----
+  uint32_t koff[8], voffA[4], voffB[4];
+  {
+    const int k_sw = ((n & 3) << 2) ^ ((n >> 2) & 3);
+#pragma unroll
+    for (int s8 = 0; s8 < 8; ++s8) koff[s8] = lds_base + n * 256 + (((2 * s8 + hh) ^ k_sw) << 4);
+    const int g16 = lane >> 4, i0 = (lane & 15) >> 2, i1 = lane & 3;
+    const int v_c16 = 2 * (g16 & 1) + (i1 >> 1), v_sub = (i1 & 1) * 8;
+#pragma unroll
+    for (int db = 0; db < 4; ++db) {
+      const int c16 = 4 * db + v_c16;
+      voffA[db] = lds_base + Shape::kVBase + (4 * hh + i0) * 256 + ((c16 ^ (i0 << 2) ^ hh) << 4) + v_sub;
+      voffB[db] = lds_base + Shape::kVBase + (4 * hh + i0 + 8) * 256 + ((c16 ^ (i0 << 2) ^ (hh + 2)) << 4) + v_sub;
+    }
+  }
+  // the addresses move with the ring: K by one stage after the first half of every key tile (the second half already
+  // reads the next tile's), V by one after the second
+  auto k_frag = [&](int kb, int s8) __attribute__((always_inline)) { return *lds_ptr<const elem8>(koff[s8] + (uint32_t)(kb * 8192)); };
+  auto v_frag = [&](int kb, int j2, int db) __attribute__((always_inline)) {
+    const elem4 va = lds_read_tr<elem4>(voffA[db] + (uint32_t)((32 * kb + 16 * j2) * 256));
+    const elem4 vb = lds_read_tr<elem4>(voffB[db] + (uint32_t)((32 * kb + 16 * j2) * 256));
+    return __builtin_shufflevector(va, vb, 0, 1, 2, 3, 4, 5, 6, 7);
+  };
+
+  f32x16 oacc[4];
+  float m_run, l_run;
+  const float sl2 = p.scale_log2;
+  auto mask_block = [&](f32x16& s, int key0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e)
+      if (key0 + 8 * (e >> 2) + 4 * hh + (e & 3) > limit) s[e] = -INFINITY;
+  };
+  auto row_max = [&](const f32x16& s) __attribute__((always_inline)) {
+    float mx = s[0];
+#pragma unroll
+    for (int e = 1; e < 16; ++e) mx = fmaxf(mx, s[e]);
+    return max_xhalf(mx) * sl2;
+  };
+#define MOBA_PIN(x) asm volatile("" : "+v"(x))
+
+  // All keys of the tile; kFixed: relative to the first block's row maximum, otherwise with a running maximum.
+  // Pipelined by hand over 32-key blocks like the loop of fwd.hip: S^T of the next block under the exponentials of
+  // this one, O^T += V^T P^T of this one under the first exponentials of the next.
+  auto all_keys = [&](auto fixed_c) __attribute__((always_inline)) {
+    constexpr bool kFixed = decltype(fixed_c)::value;
+#pragma unroll
+    for (int db = 0; db < 4; ++db)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) oacc[db][e] = 0.f;
+    wait_vmem();
+    scrub_v(0);
+    __syncthreads();
+    f32x16 s0, s1;
+    elem8 pb[2], kpre[4];
+    {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) s0[e] = 0.f;
+#pragma unroll
+      for (int s8 = 0; s8 < 8; ++s8) s0 = mfma32(k_frag(0, s8), bq[s8], s0);
+      if (31 > min_limit) mask_block(s0, 0);
+      // (every row has a key in this block: key 0 of a causal tile, any key of a history tile)
+      m_run = row_max(s0);
+      l_run = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float pe = fast_exp2(s0[e] * sl2 - m_run);
+        l_run += pe;
+        pb[0][e] = (elem)pe;
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) kpre[i] = k_frag(1, i);
+    }
+    // One step on key block kb of the tile: sc its S^T, elements 0..7 already in pb[0]; sn receives S^T of the next
+    // block, block nkb of the tile koff points to; kpre holds the first four K fragments of it and receives those of
+    // the block after (block 1 - nkb, after the addresses have moved if `move`).
+    auto step = [&](f32x16& sc, f32x16& sn, int nkb, int next_key0, auto has_next_c, bool masked, int kb, bool pre,
+                    auto move_k) __attribute__((always_inline)) {
+      constexpr bool has_next = decltype(has_next_c)::value;
+      elem8 ka[8], va[8];
+      float pf[8], rs = 0.f;
+      if constexpr (has_next) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ka[i] = kpre[i];
+      }
+#pragma unroll
+      for (int s8 = 0; s8 < 8; ++s8) {
+        if constexpr (has_next) {
+          if (s8 + 4 < 8) ka[s8 + 4] = k_frag(nkb, s8 + 4);
+          if (s8 == 0) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) sn[e] = 0.f;
+          }
+          sn = mfma32(ka[s8], bq[s8], sn);
+        }
+        pf[s8] = fast_exp2(sc[8 + s8] * sl2 - m_run);
+        if (s8 > 0) rs += pf[s8 - 1];
+        MOBA_PIN(pf[s8]);
+        MOBA_PIN(rs);
+        if (s8 >= 4 && s8 < 6) {
+          va[2 * (s8 - 4)] = v_frag(kb, 0, 2 * (s8 - 4));
+          va[2 * (s8 - 4) + 1] = v_frag(kb, 0, 2 * (s8 - 4) + 1);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      move_k();
+      l_run += rs + pf[7];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) pb[1][e] = (elem)pf[e];
+      if constexpr (has_next) {
+        if (masked) mask_block(sn, next_key0);
+      }
+      float pg[8], rn = 0.f;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        if (k + 4 < 8) va[k + 4] = v_frag(kb, 1, k & 3);
+        if (k >= 4 && pre) kpre[k - 4] = k_frag(1 - nkb, k - 4);
+        oacc[k & 3] = mfma32(va[k], pb[k >> 2], oacc[k & 3]);
+        if constexpr (has_next && kFixed) {
+          if (k == 1) {
+            pg[0] = fast_exp2(sn[0] * sl2 - m_run);
+            pg[1] = fast_exp2(sn[1] * sl2 - m_run);
+            MOBA_PIN(pg[0]);
+            MOBA_PIN(pg[1]);
+          } else if (k >= 2) {
+            pg[k] = fast_exp2(sn[k] * sl2 - m_run);
+            rn = (k == 2) ? pg[0] + pg[1] : rn + pg[k - 1];
+            MOBA_PIN(pg[k]);
+            MOBA_PIN(rn);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if constexpr (has_next && !kFixed) {  // the rare form: no slots
+        const float mx = row_max(sn);
+        const float m_new = mx > m_run + kRescaleThreshold ? mx : m_run;
+        const float alpha = fast_exp2(m_run - m_new);
+        m_run = m_new;
+        l_run *= alpha;
+#pragma unroll
+        for (int db = 0; db < 4; ++db)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) oacc[db][e] *= alpha;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          pg[e] = fast_exp2(sn[e] * sl2 - m_run);
+          if (e < 7) rn += pg[e];
+        }
+      }
+      if constexpr (has_next) {
+        l_run += rn + pg[7];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) pb[0][e] = (elem)pg[e];
+      }
+    };
+    int kstage = 0;
+    auto move_k = [&]() __attribute__((always_inline)) {
+      const uint32_t d = kstage == 2 ? (uint32_t)(-2 * kTileBytes) : (uint32_t)kTileBytes;
+      kstage = kstage == 2 ? 0 : kstage + 1;
+#pragma unroll
+      for (int s8 = 0; s8 < 8; ++s8) koff[s8] += d;
+    };
+    auto stay = [] __attribute__((always_inline)) {};
+    auto tile_body = [&](int it, auto more_c) __attribute__((always_inline)) {
+      constexpr bool more = decltype(more_c)::value;  // a key tile follows this one
+      const int key0 = it * TN;
+      if (it > 0) {
+        wait_vmem();
+        scrub_v(it);
+        __syncthreads();
+      }
+      if constexpr (more) {
+        issue_k(it + 2);
+        issue_v(it + 1);
+      }
+      step(s0, s1, 1, key0 + 32, std::true_type{}, key0 + 63 > min_limit, 0, more, move_k);
+      step(s1, s0, 0, key0 + TN, more_c, more && key0 + TN + 31 > min_limit, 1, more, stay);
+      const uint32_t d = (it & 1) ? (uint32_t)(-kTileBytes) : (uint32_t)kTileBytes;
+#pragma unroll
+      for (int db = 0; db < 4; ++db) {
+        voffA[db] += d;
+        voffB[db] += d;
+      }
+    };
+    int it = 0;
+    for (; it + 1 < nkt; ++it) tile_body(it, std::true_type{});
+    tile_body(it, std::false_type{});
+    __syncthreads();  // every wave has read its last fragments: the stages are free
+  };
+#undef MOBA_PIN
+
+  all_keys(std::true_type{});
+  float l_tot = sum_xhalf(l_run);
+  {
+    // compared as bit patterns (the file is compiled without NaN semantics): infinities, every NaN and negative sums
+    // all read as "too large"; the largest magnitude among the row's accumulators likewise
+    uint32_t worst = 0;
+#pragma unroll
+    for (int db = 0; db < 4; ++db)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) worst = max(worst, __builtin_bit_cast(uint32_t, oacc[db][e]) & 0x7fffffffu);
+    const bool bad = row_valid && (__builtin_bit_cast(uint32_t, l_tot) >= __builtin_bit_cast(uint32_t, kFixedRefMaxSum) ||
+                                   worst >= 0x7f800000u);
+    volatile int* flags = reinterpret_cast<volatile int*>(smem + Shape::kFlags);
+    const bool any_bad = __any(bad);
+    if (lane == 0) flags[wave] = any_bad ? 1 : 0;
+    __syncthreads();
+    int again = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) again |= flags[w];
+    if (__builtin_amdgcn_readfirstlane(again)) {
+      __syncthreads();  // (every wave has read the flags)
+      // back to stage 0: nkt tiles moved K by nkt stages, V by nkt
+      const uint32_t dk = (uint32_t)((nkt % 3) * kTileBytes), dv = (uint32_t)((nkt & 1) * kTileBytes);
+#pragma unroll
+      for (int s8 = 0; s8 < 8; ++s8) koff[s8] -= dk;
+#pragma unroll
+      for (int db = 0; db < 4; ++db) {
+        voffA[db] -= dv;
+        voffB[db] -= dv;
+      }
+      first_copies();
+      all_keys(std::false_type{});
+      l_tot = sum_xhalf(l_run);
+      if (p.redo && tid == 0) {  // (listed for a caller that asks which tiles these were)
+        const int at = __hip_atomic_fetch_add(p.redo, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        p.redo[1 + at] = t.id;
+      }
+    }
+  }
+
+  // ---- normalise, write: through 4 KiB of LDS per wave, half a row at a time, so that the rows leave as 128-byte
+  // pieces, eight rows per store instruction (see fwd.hip) ----
+  {
+    const float inv = 1.f / l_tot;
+    char* stage = smem + wave * 4096;
+    char* wrow = stage + n * 128 + 8 * hh;
+    const int wsw = (n >> 1) & 7;
+    elem* const o_base = t.direct ? p.out : p.part_o;
+    if (row_valid && hh == 0) {
+      const float l2 = m_run + fast_log2(l_tot);
+      if (t.direct) p.lse[dest] = l2 * 0.6931471805599453f;
+      else p.part_lse[dest] = l2;
+    }
+    const int c16 = lane & 7;
+    const int rows_here = t.row_count - wave * 32;
+    int d4[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) d4[i] = __shfl(dest, 8 * i + (lane >> 3), 64);
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+#pragma unroll
+      for (int d2 = 0; d2 < 2; ++d2)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const int db = 2 * half + d2;
+          u32x2 w;
+          w[0] = pack2<E>(oacc[db][4 * g + 0] * inv, oacc[db][4 * g + 1] * inv);
+          w[1] = pack2<E>(oacc[db][4 * g + 2] * inv, oacc[db][4 * g + 3] * inv);
+          *reinterpret_cast<u32x2*>(wrow + (((4 * d2 + g) ^ wsw) << 4)) = w;
+        }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int row = 8 * i + (lane >> 3);
+        const u32x4 x = *reinterpret_cast<const u32x4*>(stage + row * 128 + ((c16 ^ ((row >> 1) & 7)) << 4));
+        if (row < rows_here) *reinterpret_cast<u32x4*>(o_base + (int64_t)d4[i] * kHeadDim + 64 * half + c16 * 8) = x;
+      }
+    }
+  }
+}
+
+template <class E, int NW>
+static int launch(const FwdParams<E>& p, int64_t workgroups, hipStream_t st) {
+  static bool allowed[kMaxDevices];
+  if (!allow_dynamic_lds((const void*)fwd_tile_kernel<E, NW>, FwdTileShape<NW>::kLds, allowed)) return MOBA_ERR_LAUNCH;
+  hipLaunchKernelGGL((fwd_tile_kernel<E, NW>), dim3((unsigned)workgroups), dim3(NW * 64), FwdTileShape<NW>::kLds, st, p);
+  return MOBA_OK;
+}
+
+template <class E>
+int launch_fwd_tiles(const FwdParams<E>& p, int tile_rows, int64_t workgroups, hipStream_t st) {
+  return tile_rows == 128 ? launch<E, 4>(p, workgroups, st) : launch<E, 8>(p, workgroups, st);
+}
+template int launch_fwd_tiles<Bf16>(const FwdParams<Bf16>&, int, int64_t, hipStream_t);
+template int launch_fwd_tiles<F16>(const FwdParams<F16>&, int, int64_t, hipStream_t);
+
+}  // namespace moba

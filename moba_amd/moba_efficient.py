@@ -297,13 +297,22 @@ class _Geometry:
 
     def __init__(self, plan: MobaPlan, lib, H: int, D: int, esize: int):
         S, K = plan.S, plan.K
+        # rows per tile of the forward (forward_tile_rows); tiles of the backward's height share its tables
+        self.rows_per_tile = forward_tile_rows(plan, H)
+        tall = self.rows_per_tile == FWD_TILE_ROWS
+        self.self_tiles = plan.fwd_self_tiles if tall else plan.self_tiles
+        self.self_names = (("fwd_" if tall else "") + "self_tile_prefix", ("fwd_" if tall else "") + "self_tile_chunk")
         self.tptr = {name: _ptr(t) for name, t in plan.tables.items()}
         self.null = ctypes.c_void_p(0)
-        self.bound = plan.hist_tile_bound(H, FWD_TILE_ROWS)
+        self.bound = plan.hist_tile_bound(H, self.rows_per_tile)
         if plan.fallback:
             self.split = 1
         else:
-            self.split = int(lib.moba_fwd_key_split(S, H, K, plan.chunk_size, self.bound, plan.fwd_self_tiles))
+            # (two of the short tiles share a compute unit: they count half.  16384 tokens, 2 heads, chunk 4096 in two parts:
+            # 149 -> 130 us; 8192 tokens, 4 heads, chunk 1024: 57 -> 49 us; with twice as many tiles the merge of the
+            # parts takes what they gain)
+            n = 1 if tall else 2
+            self.split = int(lib.moba_fwd_key_split(S, H, K, plan.chunk_size, -(-self.bound // n), -(-self.self_tiles // n)))
         # lists: cnt, seg_off, tile_off, seg_dest, tile_seg (int32, each start a multiple of 4 ints)
         sizes = [plan.P * H + 1, plan.F * H + 1, plan.F * H + 1, max(plan.pairs_per_head * H, 1), self.bound]
         self.list_sizes = sizes
@@ -311,20 +320,41 @@ class _Geometry:
         for n in sizes:
             starts.append(starts[-1] + (n + 3) // 4 * 4)
         self.list_starts = starts
-        # ... and, for a call that a backward will follow, the backward kernels' tile tables behind them
+        # ... and, for a call that a backward will follow, the backward kernels' tile tables behind them, unless the
+        # forward's tiles have the same height
         self.bwd_bound = plan.hist_tile_bound(H, TILE_ROWS)
-        self.bwd_starts = [starts[-1], starts[-1] + (plan.F * H + 1 + 3) // 4 * 4]
-        self.list_ints_with_bwd = self.bwd_starts[1] + self.bwd_bound
+        if tall:
+            self.bwd_starts = [starts[-1], starts[-1] + (plan.F * H + 1 + 3) // 4 * 4]
+            self.list_ints_with_bwd = self.bwd_starts[1] + self.bwd_bound
+        else:
+            self.bwd_starts = [starts[2], starts[4]]
+            self.list_ints_with_bwd = starts[-1]
         # attention scratch: per-slot partial outputs, their log-sum-exps, the kernel's 8 tile counters, then
         # the list of tiles its fixed-reference softmax hands to the kernel that tracks the running maximum
         # (count first; the call zeroes the counters and the count)
         rows = S * H * (K + 1) * self.split
         self.rows = rows
         self.part_o_bytes = rows * D * esize
-        self.scratch_ints = 8 + 1 + self.bound + plan.fwd_self_tiles * H
+        self.scratch_ints = 8 + 1 + self.bound + self.self_tiles * H
         self.ws_bytes = self.part_o_bytes + rows * 4 + self.scratch_ints * 4
         self.mean_ws = {}  # kv heads -> fp64 elements of the chunk mean's workspace
         self.bwd = {}      # kv heads -> sizes of the backward's scratch
+
+
+# Which of its two forms the forward attention kernel takes: tiles of TILE_ROWS rows, one workgroup each, two side by side
+# on a compute unit, or tiles of FWD_TILE_ROWS rows drawn by one resident workgroup per unit.  The first hides a tile's
+# start and end under its neighbour, the second moves half the bytes from L2 to LDS.  Chunks of 512 keys and less always
+# gain from the first (3 x 2001 tokens, 32 heads, chunk 256: 160 -> 104 us; 196608 tokens, chunk 512: 6.42 -> 6.37 ms,
+# chunk 256: 5.05 -> 4.64 ms); longer ones while the call is short (16384 tokens, chunk 2048: 1.29 -> 1.13 ms; 49152
+# tokens: 3.87 ms both ways; 98304 tokens: 7.93 against 8.26 ms).
+SHORT_TILES_CHUNK = 512
+SHORT_TILES_FLOPS = 4e12
+
+
+def forward_tile_rows(plan: MobaPlan, H: int) -> int:
+    """Rows per tile of the forward attention kernel for this plan and number of heads."""
+    short_chunks = not plan.fallback and plan.chunk_size <= SHORT_TILES_CHUNK
+    return TILE_ROWS if short_chunks or plan.flops_per_head * HEAD_DIM * H <= SHORT_TILES_FLOPS else FWD_TILE_ROWS
 
 
 def _geometry(plan: MobaPlan, lib, H: int, D: int, esize: int) -> _Geometry:
@@ -335,7 +365,18 @@ def _geometry(plan: MobaPlan, lib, H: int, D: int, esize: int) -> _Geometry:
     return g
 
 
-def _forward(q, k, v, plan: MobaPlan, timer: Optional[StageTimer] = None, scale: float = 0.0, bwd_tables=None):
+def _forward(q, k, v, plan: MobaPlan, timer: Optional[StageTimer] = None, scale: float = 0.0):
+    """As _run_forward; tile_off and tile_seg are those of tiles of FWD_TILE_ROWS rows, whatever the kernel took."""
+    res = _run_forward(q, k, v, plan, timer, scale)
+    S, H, D = _dims(q)
+    if plan.fallback or forward_tile_rows(plan, H) == FWD_TILE_ROWS:
+        return res
+    out, lse, sel, seg_off, _, seg_dest, _ = res
+    tile_off, tile_seg = tile_tables(seg_off, plan, H, FWD_TILE_ROWS)
+    return out, lse, sel, seg_off, tile_off, seg_dest, tile_seg
+
+
+def _run_forward(q, k, v, plan: MobaPlan, timer: Optional[StageTimer] = None, scale: float = 0.0, bwd_tables=None):
     """q, k, v: [tokens, heads, 128], or batched [batch, heads, tokens, 128] (read in place, see _dims), already
     addressable (_in_place).  Returns (out, lse, sel, seg_off, tile_off, seg_dest, tile_seg).
     bwd_tables: a list that receives the backward kernels' (tile_off, tile_seg), made on the way.
@@ -364,11 +405,11 @@ def _forward(q, k, v, plan: MobaPlan, timer: Optional[StageTimer] = None, scale:
         lists = torch.empty(g.list_starts[-1] if bwd_tables is None else g.list_ints_with_bwd, dtype=torch.int32,
                             device=dev)
         base = lists.data_ptr()
-        if bwd_tables is None:
-            bwd_args = (0, null, null, 0)
-        else:
+        bwd_args = (0, null, null, 0)
+        if bwd_tables is not None:
             b0, b1 = g.bwd_starts
             bwd_tables += [lists[b0:b0 + plan.F * H + 1], lists[b1:b1 + g.bwd_bound]]
+        if bwd_tables is not None and g.rows_per_tile != TILE_ROWS:
             bwd_args = (TILE_ROWS, ctypes.c_void_p(base + 4 * b0), ctypes.c_void_p(base + 4 * b1), g.bwd_bound)
         cntp, seg_offp, tile_offp, seg_destp, tile_segp = (ctypes.c_void_p(base + 4 * a) for a in g.list_starts[:5])
         seg_off, tile_off, seg_dest, tile_seg = (lists[a:a + n] for a, n in zip(g.list_starts[1:5], g.list_sizes[1:]))
@@ -384,7 +425,7 @@ def _forward(q, k, v, plan: MobaPlan, timer: Optional[StageTimer] = None, scale:
         with span("build_lists"):
             _lib.check(lib.moba_build_lists(selp, tp["chunk_tok"], tp["chunk_fb"], tp["chunk_local"], tp["pair_off"],
                                             cntp, seg_offp, tile_offp, seg_destp, tile_segp, S, H, K, plan.N, plan.F,
-                                            plan.P, plan.cmax, FWD_TILE_ROWS, g.bound, 1, *bwd_args, plan.dense_local,
+                                            plan.P, plan.cmax, g.rows_per_tile, g.bound, 1, *bwd_args, plan.dense_local,
                                             stream), "moba_build_lists")
     out = torch.empty((S, H, D), dtype=q.dtype, device=dev)
     lse = torch.empty((S, H), dtype=torch.float32, device=dev)
@@ -394,16 +435,20 @@ def _forward(q, k, v, plan: MobaPlan, timer: Optional[StageTimer] = None, scale:
     part_lsep = ctypes.c_void_p(base + g.part_o_bytes)
     queuesp = ctypes.c_void_p(base + g.part_o_bytes + g.rows * 4)
     redop = ctypes.c_void_p(base + g.part_o_bytes + g.rows * 4 + 32) if FIXED_REFERENCE else null
+    if g.rows_per_tile == TILE_ROWS and not KEEP_SCRATCH:
+        redop = null    # (these tiles need no list: their workgroups compute them again themselves)
     if KEEP_SCRATCH:
         at = g.part_o_bytes + g.rows * 4 + 32
-        last_scratch["redo"] = ws2[at:at + 4 * (g.scratch_ints - 8)].view(torch.int32) if FIXED_REFERENCE else None
+        redo = last_scratch["redo"] = ws2[at:at + 4 * (g.scratch_ints - 8)].view(torch.int32) if FIXED_REFERENCE else None
+        if redo is not None:
+            redo[0] = 0
     with span("fwd_partials"):
-        _lib.check(lib.moba_fwd_partials(qp, kp, vp, part_op, part_lsep, seg_offp, tile_offp, seg_destp,
-                                         tp.get("fchunk_tok", null), tp["achunk_tok"], tp["fwd_self_tile_prefix"],
-                                         tile_segp, tp["fwd_self_tile_chunk"], tp["achunk_direct"] if DIRECT_ROWS else null,
-                                         _ptr(out), _ptr(lse), S, H, Hkv, D, K, plan.F, plan.NA,
-                                         plan.chunk_size, g.bound, plan.fwd_self_tiles, g.split, strides, queuesp,
-                                         redop, scale, code, 0, 0, stream), "moba_fwd_partials")
+        _lib.check(lib.moba_fwd_partials_rows(qp, kp, vp, part_op, part_lsep, seg_offp, tile_offp, seg_destp,
+                                              tp.get("fchunk_tok", null), tp["achunk_tok"], tp[g.self_names[0]],
+                                              tile_segp, tp[g.self_names[1]], tp["achunk_direct"] if DIRECT_ROWS else null,
+                                              _ptr(out), _ptr(lse), S, H, Hkv, D, K, plan.F, plan.NA,
+                                              plan.chunk_size, g.bound, g.self_tiles, g.split, strides, queuesp,
+                                              redop, scale, code, 0, 0, g.rows_per_tile, stream), "moba_fwd_partials_rows")
     if not DIRECT_ROWS:
         with span("fwd_merge"):
             _lib.check(lib.moba_fwd_merge(part_op, part_lsep, selp, _ptr(out), _ptr(lse), S, H, D, K, g.split,
@@ -474,7 +519,7 @@ class _MobaAttention(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, plan, timer=None, scale=0.0):
         tables = []  # the backward's tile tables, made by the forward's list stage
-        out, lse, sel, seg_off, _, seg_dest, _ = _forward(q, k, v, plan, timer, scale, bwd_tables=tables)
+        out, lse, sel, seg_off, _, seg_dest, _ = _run_forward(q, k, v, plan, timer, scale, bwd_tables=tables)
         ctx.plan = plan
         ctx.scale = scale
         ctx.aux = (sel, seg_off, seg_dest, tables)
@@ -542,8 +587,8 @@ def _forward_in_groups(q, k, v, plan, groups, timer, scale, keep):
     for h0, h1 in groups:
         group_plan = _choose_plan(plan, h1 - h0)
         tables = [] if keep is not None else None
-        res = _forward(q[:, h0:h1], k[:, h0 // rep:h1 // rep], v[:, h0 // rep:h1 // rep], group_plan, timer, scale,
-                       bwd_tables=tables)
+        res = _run_forward(q[:, h0:h1], k[:, h0 // rep:h1 // rep], v[:, h0 // rep:h1 // rep], group_plan, timer,
+                           scale, bwd_tables=tables)
         out[:, h0:h1] = res[0]
         lse[:, h0:h1] = res[1]
         if keep is not None:
@@ -601,7 +646,7 @@ def _attend(q, k, v, plan, timer=None, scale=0.0):
     plan = _choose_plan(plan, H)
     if grad:
         return _MobaAttention.apply(q, k, v, plan, timer, scale)
-    return _forward(q, k, v, plan, timer, scale)[:2]
+    return _run_forward(q, k, v, plan, timer, scale)[:2]
 
 
 def moba_attn_varlen(

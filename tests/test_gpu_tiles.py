@@ -1,0 +1,72 @@
+"""The two tile heights of the forward attention kernel against each other and against the dense oracle: 128 rows, one
+workgroup per tile (short chunks and short calls), and 256 rows, by resident workgroups or one workgroup each."""
+
+import numpy as np
+import pytest
+import torch
+
+from test_gpu_queued import test_queued_kernels_against_the_dense_oracle as queued_case
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def tile_rows(monkeypatch):
+    """Sets the tile height; plans keep what was derived from it, so their caches start and end empty."""
+    from moba_amd import moba_efficient as E
+    from moba_amd import plan as P
+
+    def forget():
+        P._BY_VALUE.clear()
+        P._BY_TENSOR.clear()
+
+    def choose(rows):
+        monkeypatch.setattr(E, "forward_tile_rows", lambda plan, H: rows)
+        forget()
+
+    yield choose
+    forget()
+
+
+@pytest.mark.parametrize("dense,dtype,spread", [(True, torch.bfloat16, 1.0), (False, torch.bfloat16, 8.0),
+                                                (True, torch.float16, 8.0)])
+def test_resident_workgroups_against_the_dense_oracle(dense, dtype, spread, tile_rows, monkeypatch):
+    """The shape of the queued kernels' test, whose chunks are short, on the resident workgroups all the same."""
+    tile_rows(256)
+    queued_case(dense, dtype, spread, monkeypatch)
+
+
+@pytest.mark.parametrize("lens,heads,kv_heads,B,topk,dtype", [
+    ([128], 1, 1, 64, 2, torch.bfloat16),
+    ([129, 127, 1, 257], 2, 1, 65, 3, torch.float16),      # one-row tiles, a key tile of one key
+    ([640, 63], 3, 3, 128, 2, torch.bfloat16),
+    ([2048], 4, 2, 512, 1, torch.float16),                 # full causal attention
+    ([4096], 1, 1, 2048, 3, torch.bfloat16),               # history tiles cut along their keys
+    ([3000], 2, 2, 192, 3, torch.bfloat16),
+])
+@pytest.mark.parametrize("spread", [1.0, 8.0])
+def test_tile_heights_agree(lens, heads, kv_heads, B, topk, dtype, spread, tile_rows):
+    """A row's result does not depend on the tile it lies in (bit for bit) unless some row of a tile leaves the range of
+    the fixed-reference softmax (spread 8): the two softmax forms then differ by their roundings, at most a few of the
+    element type's steps at values of up to about 4."""
+    from moba_amd import moba_efficient as E
+    cu = [0] + np.cumsum(lens).tolist()
+    S = cu[-1]
+    print("tile case", lens, heads, B, topk, dtype, spread, flush=True)
+    g = torch.Generator().manual_seed(S + heads)
+    q = (torch.randn((S, heads, 128), generator=g) * spread).to(dtype).cuda()
+    k = (torch.randn((S, kv_heads, 128), generator=g) * spread).to(dtype).cuda()
+    v = torch.randn((S, kv_heads, 128), generator=g).to(dtype).cuda()
+    got = []
+    for rows in (128, 256):
+        tile_rows(rows)
+        cu_t = torch.tensor(cu, dtype=torch.int32, device="cuda")
+        got.append(E.moba_attn_varlen_with_lse(q, k, v, cu_t, max(lens), B, topk, gqa=True))
+    (out_a, lse_a), (out_b, lse_b) = got
+    assert torch.isfinite(out_a.float()).all() and torch.isfinite(lse_a).all()
+    if spread == 1.0 and not (len(lens) == 1 and B == 2048):   # (parts: their number follows from the number of tiles)
+        assert torch.equal(out_a, out_b) and torch.equal(lse_a, lse_b)
+    else:
+        step = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+        assert (out_a.float() - out_b.float()).abs().max() < 4 * 4 * step
+        assert (lse_a - lse_b).abs().max() < 1e-3 * max(1.0, spread * spread)
