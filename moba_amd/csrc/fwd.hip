@@ -664,18 +664,20 @@ __global__ __launch_bounds__(512, 2) void moba_fwd_kernel(const FwdParams<E> p) 
 // two.  (An absent slot's bytes are whatever the buffer holds; they are dropped by selection, not multiplied by
 // a zero weight.)  Slots are accumulated in ascending order, as in the general form below.  For up to 8 slots:
 // with 16 in registers too few waves fit a compute unit, and the kernel takes three times as long.
-template <class E, int NV>
+template <class E, int D, int NV>
 __device__ __forceinline__ void merge_few_slots(const typename E::elem* __restrict__ po, const float* __restrict__ pl,
                                                 const int* __restrict__ ps, typename E::elem* __restrict__ out,
                                                 float* __restrict__ lse, int64_t row, bool row_ok, int c8, int K1,
                                                 int parts, int nvirt, int part_rows) {
   MOBA_ELEM_TYPES(E)
-  elem8 x[NV];
+  constexpr int kPer = D / 16;  // elements per lane
+  using vec = typename std::conditional<kPer == 8, elem8, elem4>::type;
+  vec x[NV];
 #pragma unroll
   for (int u = 0; u < NV; ++u) {
     const int part = parts == 1 ? 0 : u / K1, j = u - part * K1;
     if (u < nvirt)
-      x[u] = __builtin_nontemporal_load(reinterpret_cast<const elem8*>(po + (int64_t)(part * part_rows + j) * kHeadDim));
+      x[u] = __builtin_nontemporal_load(reinterpret_cast<const vec*>(po + (int64_t)(part * part_rows + j) * D));
   }
   const int part = parts == 1 ? 0 : c8 / K1, j = c8 - part * K1;
   const bool ok = c8 < nvirt && (j == 0 ? part == 0 : ps[j - 1] >= 0);
@@ -684,9 +686,9 @@ __device__ __forceinline__ void merge_few_slots(const typename E::elem* __restri
 #pragma unroll
   for (int o = 8; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 16));
   const float wl = ok ? fast_exp2(l - mx) : 0.f;
-  float acc[8];
+  float acc[kPer];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) acc[e] = 0.f;
+  for (int e = 0; e < kPer; ++e) acc[e] = 0.f;
   float wsum = 0.f;
 #pragma unroll
   for (int u = 0; u < NV; ++u) {
@@ -694,14 +696,14 @@ __device__ __forceinline__ void merge_few_slots(const typename E::elem* __restri
     const float w = __shfl(wl, u, 16);
     wsum += w;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) acc[e] += w > 0.f ? w * (float)x[u][e] : 0.f;
+    for (int e = 0; e < kPer; ++e) acc[e] += w > 0.f ? w * (float)x[u][e] : 0.f;
   }
   if (!row_ok) return;
   const float inv = 1.f / wsum;
-  elem8 o;
+  vec o;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) o[e] = (elem)(acc[e] * inv);
-  __builtin_nontemporal_store(o, reinterpret_cast<elem8*>(out + row * kHeadDim + c8 * 8));
+  for (int e = 0; e < kPer; ++e) o[e] = (elem)(acc[e] * inv);
+  __builtin_nontemporal_store(o, reinterpret_cast<vec*>(out + row * D + c8 * kPer));
   if (c8 == 0) lse[row] = (mx + fast_log2(wsum)) * 0.6931471805599453f;
 }
 
@@ -710,7 +712,7 @@ __device__ __forceinline__ void merge_few_slots(const typename E::elem* __restri
 // With token ranges (mrg_start / mrg_prefix [nranges(+1)]: range b holds the tokens mrg_start[b] + i for
 // i < mrg_prefix[b+1] - mrg_prefix[b]) only the rows of those tokens are merged, `rows` counting them: the others
 // were written by the attention kernel itself.  Null: every row of [0, rows).
-template <class E>
+template <class E, int D>
 __global__ __launch_bounds__(256) void moba_merge_kernel(const typename E::elem* __restrict__ part_o,
                                                          const float* __restrict__ part_lse,
                                                          const int* __restrict__ sel, typename E::elem* __restrict__ out,
@@ -718,6 +720,8 @@ __global__ __launch_bounds__(256) void moba_merge_kernel(const typename E::elem*
                                                          int64_t all_rows, const int* __restrict__ mrg_start,
                                                          const int* __restrict__ mrg_prefix, int nranges, int H) {
   MOBA_ELEM_TYPES(E)
+  constexpr int kPer = D / 16;  // elements per lane
+  using vec = typename std::conditional<kPer == 8, elem8, elem4>::type;
   const int64_t row_raw = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
   const bool row_ok = row_raw < rows;
   int64_t row = row_ok ? row_raw : rows - 1;  // whole 16-lane groups stay active for the shuffles
@@ -730,7 +734,7 @@ __global__ __launch_bounds__(256) void moba_merge_kernel(const typename E::elem*
   const int K = K1 - 1;
   const float* pl = part_lse + row * K1;
   const int* ps = sel + row * K;
-  const elem* po = part_o + row * K1 * kHeadDim + c8 * 8;  // the self slot: always written
+  const elem* po = part_o + row * K1 * D + c8 * kPer;  // the self slot: always written
   // Lane c8 of the row's group fetches the LSE and the presence of slot j0 + c8, so the slot
   // statistics cost one round trip per 16 slots; weights travel by lane shuffles.  Absent slots
   // are redirected to the self slot with weight 0, so the partial-output loads are unconditional and
@@ -742,7 +746,7 @@ __global__ __launch_bounds__(256) void moba_merge_kernel(const typename E::elem*
   const int nvirt = parts * K1;
   const int part_rows = (int)(all_rows * K1);
   if (nvirt <= 8) {  // (uniform)
-    merge_few_slots<E, 8>(po, pl, ps, out, lse, row, row_ok, c8, K1, parts, nvirt, part_rows);
+    merge_few_slots<E, D, 8>(po, pl, ps, out, lse, row, row_ok, c8, K1, parts, nvirt, part_rows);
     return;
   }
   float mx = -INFINITY;
@@ -755,9 +759,9 @@ __global__ __launch_bounds__(256) void moba_merge_kernel(const typename E::elem*
   }
 #pragma unroll
   for (int o = 8; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 16));
-  float acc[8];
+  float acc[kPer];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) acc[e] = 0.f;
+  for (int e = 0; e < kPer; ++e) acc[e] = 0.f;
   float wsum = 0.f;
   for (int v0 = 0; v0 < nvirt; v0 += 16) {
     const int v = v0 + c8;
@@ -768,30 +772,30 @@ __global__ __launch_bounds__(256) void moba_merge_kernel(const typename E::elem*
     const int at_ok = ok ? at : 0;
     const int nslot = min(16, nvirt - v0);
     for (int u0 = 0; u0 < nslot; u0 += 8) {
-      elem8 x[8];
+      vec x[8];
       float w[8];
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
         w[u] = __shfl(wl, u0 + u, 16);           // 0 for slots past the last too (their lanes computed ok = false)
         const int where = parts == 1 ? (w[u] > 0.f ? v0 + u0 + u : 0) : __shfl(at_ok, u0 + u, 16);
         if (u0 + u < nslot)                      // uniform: no loads for slots that do not exist
-          x[u] = __builtin_nontemporal_load(reinterpret_cast<const elem8*>(po + (int64_t)where * kHeadDim));
+          x[u] = __builtin_nontemporal_load(reinterpret_cast<const vec*>(po + (int64_t)where * D));
       }
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
         if (u0 + u >= nslot) break;
         wsum += w[u];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) acc[e] += w[u] * (float)x[u][e];
+        for (int e = 0; e < kPer; ++e) acc[e] += w[u] * (float)x[u][e];
       }
     }
   }
   if (!row_ok) return;
   const float inv = 1.f / wsum;
-  elem8 o;
+  vec o;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) o[e] = (elem)(acc[e] * inv);
-  __builtin_nontemporal_store(o, reinterpret_cast<elem8*>(out + row * kHeadDim + c8 * 8));
+  for (int e = 0; e < kPer; ++e) o[e] = (elem)(acc[e] * inv);
+  __builtin_nontemporal_store(o, reinterpret_cast<vec*>(out + row * D + c8 * kPer));
   if (c8 == 0) lse[row] = (mx + fast_log2(wsum)) * 0.6931471805599453f;
 }
 
@@ -874,7 +878,7 @@ static int launch_partials(const void* q, const void* k, const void* v, void* pa
     hipLaunchKernelGGL((moba_fwd_kernel<E, kTilesQueued, false>), dim3((unsigned)grid), dim3(512), kFwdLds, st, p);
   } else {         // one workgroup per tile id
     if (tile_rows == kFwdTileRows) p.redo = nullptr;  // (not cleared by this call, not needed)
-    const int rc = launch_fwd_tiles<E>(p, tile_rows, -grid, st);
+    const int rc = launch_fwd_tiles<E>(p, D, tile_rows, -grid, st);
     if (rc != MOBA_OK) return rc;
   }
   return launch_check.result();
@@ -899,7 +903,7 @@ extern "C" int moba_fwd_partials_rows(const void* q, const void* k, const void* 
   if (self_tile_skip > 0 && (K != 0 || !chunk_direct || (strides && strides[4] != 0))) return MOBA_ERR_ARG;
   if (Hkv <= 0 || H % Hkv != 0) return MOBA_ERR_ARG;
   if (K > 0 && (!seg_off || !tile_off || !seg_dest || !fchunk_tok || !tile_seg)) return MOBA_ERR_ARG;
-  if (D != kHeadDim || (dtype != MOBA_DTYPE_BF16 && dtype != MOBA_DTYPE_F16)) return MOBA_ERR_UNSUPPORTED;
+  if ((D != kHeadDim && !(D == 64 && tile_rows == TM)) || (dtype != MOBA_DTYPE_BF16 && dtype != MOBA_DTYPE_F16)) return MOBA_ERR_UNSUPPORTED;
   if (S <= 0 || H <= 0 || K < 0 || F < 0 || N <= 0 || B <= 0 || hist_bound < 0 || self_tiles <= 0) return MOBA_ERR_ARG;
   if (((uintptr_t)q & 15) || ((uintptr_t)k & 15) || ((uintptr_t)v & 15) || ((uintptr_t)part_o & 15)) return MOBA_ERR_ARG;
   int key_split_log2 = 0;
@@ -926,6 +930,7 @@ extern "C" int moba_fwd_partials_rows(const void* q, const void* k, const void* 
   t.Hkv = Hkv; t.rep = H / Hkv;
   t.hist_bound = (K > 0) ? (int)hist_bound : 0;
   t.self_total = (int)(self_tiles * H);
+  if (!strides && D != kHeadDim) return MOBA_ERR_ARG;  // (packed is said for 128 only)
   if (!set_layout(t, strides)) return MOBA_ERR_ARG;
   t.key_split_log2 = key_split_log2;
   t.part_stride = (int)(S * H * (K + 1));
@@ -963,7 +968,7 @@ extern "C" int moba_fwd_merge(const void* part_o, const float* part_lse, const i
   if (!part_o || !part_lse || !out || !lse || (K > 0 && !sel)) return MOBA_ERR_ARG;
   if (key_split < 1 || key_split > kMaxKeySplit) return MOBA_ERR_ARG;
   if (K == 0) key_split = 1;
-  if (D != kHeadDim || (dtype != MOBA_DTYPE_BF16 && dtype != MOBA_DTYPE_F16)) return MOBA_ERR_UNSUPPORTED;
+  if ((D != kHeadDim && D != 64) || (dtype != MOBA_DTYPE_BF16 && dtype != MOBA_DTYPE_F16)) return MOBA_ERR_UNSUPPORTED;
   if (S <= 0 || H <= 0 || K < 0 || ((uintptr_t)part_o & 15) || ((uintptr_t)out & 15)) return MOBA_ERR_ARG;
   if (mrg_start ? (!mrg_prefix || nranges <= 0 || merge_tokens < 0 || merge_tokens > S)
                 : (mrg_prefix || merge_tokens != S))
@@ -971,12 +976,15 @@ extern "C" int moba_fwd_merge(const void* part_o, const float* part_lse, const i
   if (merge_tokens == 0) return MOBA_OK;  // every row was written by the attention kernel
   const int64_t rows = merge_tokens * H;
   const dim3 grid((unsigned)((rows + 15) / 16));
-  if (dtype == MOBA_DTYPE_F16)
-    hipLaunchKernelGGL(moba_merge_kernel<F16>, grid, dim3(256), 0, (hipStream_t)stream, (const f16*)part_o, part_lse,
-                       sel, (f16*)out, lse, rows, K + 1, key_split, S * H, mrg_start, mrg_prefix, nranges, H);
-  else
-    hipLaunchKernelGGL(moba_merge_kernel<Bf16>, grid, dim3(256), 0, (hipStream_t)stream, (const bf16*)part_o,
-                       part_lse, sel, (bf16*)out, lse, rows, K + 1, key_split, S * H, mrg_start, mrg_prefix, nranges, H);
+#define MOBA_MERGE(EL, DIM)                                                                                          \
+  hipLaunchKernelGGL((moba_merge_kernel<EL, DIM>), grid, dim3(256), 0, (hipStream_t)stream, (const EL::elem*)part_o,  \
+                     part_lse, sel, (EL::elem*)out, lse, rows, K + 1, key_split, S * H, mrg_start, mrg_prefix, nranges, H)
+  if (dtype == MOBA_DTYPE_F16) {
+    if (D == 64) MOBA_MERGE(F16, 64); else MOBA_MERGE(F16, 128);
+  } else {
+    if (D == 64) MOBA_MERGE(Bf16, 64); else MOBA_MERGE(Bf16, 128);
+  }
+#undef MOBA_MERGE
   return launch_check.result();
 }
 

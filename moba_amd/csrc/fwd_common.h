@@ -26,8 +26,9 @@ struct FwdParams {
 constexpr float kFixedRefMaxSum = 0x1p96f;
 constexpr float kRescaleThreshold = 8.f;  // log2 units: the running max may lag the true max by this much
 
-// one workgroup per tile (fwd_tile.hip); tile_rows: 128 or 256.  Returns an error code of common.h.
+// one workgroup per tile (fwd_tile.hip); head_dim 128 with tile_rows 128 or 256, or 64 with 128.  Returns an error code
+// of common.h.
 template <class E>
-int launch_fwd_tiles(const FwdParams<E>& p, int tile_rows, int64_t workgroups, hipStream_t st);
+int launch_fwd_tiles(const FwdParams<E>& p, int head_dim, int tile_rows, int64_t workgroups, hipStream_t st);
 
 }  // namespace moba

@@ -15,6 +15,11 @@
 // milliseconds the chip's power limit decides and the doubled L2 -> LDS traffic costs 3 to 8 %: those stay with
 // moba_fwd_kernel (the rule stands with the caller's choice of the tile height).
 //
+// Heads of 64 elements (the only kernel that takes them unpadded) need half the LDS and 147 registers: three workgroups
+// to a compute unit.  The exponentials weigh twice as much against the products there, so the rate in FLOP/s stays
+// below that of 128 elements, but half the work is gone: 8191 tokens, 32 heads, chunk 512, whole operator: 401 us padded to 128, 217 us here; 131072 tokens, chunk
+// 4096, 12 chunks: 64.8 -> 43.6 ms.
+//
 // Softmax: relative to the row maximum of the tile's first 32 keys (see fwd.hip); a tile in which a row leaves the
 // range that is safe is computed again on the spot with a running maximum, by the same workgroup.
 #include <cstddef>
@@ -23,18 +28,34 @@
 
 namespace moba {
 
-template <int NW>
+template <int D, int NW>
 struct FwdTileShape {
-  static constexpr int kVBase = 3 * kTileBytes;
-  static constexpr int kLds = 5 * kTileBytes;       // two workgroups of four waves fill the unit's 160 KiB exactly
+  static constexpr int kRowBytes = 2 * D;
+  static constexpr int kStage = TN * kRowBytes;     // bytes of a K or V tile
+  static constexpr int kVBase = 3 * kStage;
+  // D = 128: two workgroups of four waves fill the unit's 160 KiB exactly; D = 64: half of that, three fit by registers
+  static constexpr int kLds = 5 * kStage;
   static constexpr int kFlags = kLds - 4 * NW;      // a word per wave; in the second V stage, free when it is used
+  static constexpr int kCols = D / 8;               // 16-byte columns of a row
+  static constexpr int kSlabRows = 1024 / kRowBytes;  // rows that one copy instruction of a wave brings
+  static constexpr int kCopies = TN / kSlabRows / NW;  // copy instructions per wave and K or V tile
+  static constexpr int kWavesPerSimd = D == 128 ? 2 : 3;
 };
 
-template <class E, int NW>
-__global__ __launch_bounds__(NW * 64, 2) void fwd_tile_kernel(const FwdParams<E> p) {
+// The swizzle of the 16-byte columns: that of the 256-byte rows, or for 128-byte rows (two of them to the 256 bytes the
+// banks span) one under which 16 consecutive rows still put the same column into 16 different places, and so do the
+// 4 rows x 64 bytes of a transposed read.
+template <int D>
+__device__ __forceinline__ int tile_sw(int row) {
+  return D == 128 ? ((row & 3) << 2) ^ ((row >> 2) & 3) : ((row & 2) << 1) | ((row >> 2) & 3);
+}
+
+template <class E, int D, int NW>
+__global__ __launch_bounds__(NW * 64, (FwdTileShape<D, NW>::kWavesPerSimd)) void fwd_tile_kernel(const FwdParams<E> p) {
   MOBA_ELEM_TYPES(E)
-  using Shape = FwdTileShape<NW>;
-  constexpr int kRows = 32 * NW, kCopies = 16 / NW;  // rows of a tile; copy instructions per wave and K or V tile
+  using Shape = FwdTileShape<D, NW>;
+  constexpr int kRows = 32 * NW, kCopies = Shape::kCopies, kStage = Shape::kStage, kRowBytes = Shape::kRowBytes;
+  constexpr int kKs = D / 16, kDb = D / 32;  // matrix steps along the head dimension of S^T, row blocks of O^T
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -65,15 +86,15 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_tile_kernel(const FwdParams<E>
   const int h = t.h, nkeys = t.nkeys;
   const int nkt = (nkeys + TN - 1) / TN;
 
-  // ---- K/V loader: wave w copies the slabs w, w + NW, ... of a tile's 16 (4 keys x 256 bytes each) ----
+  // ---- K/V loader: wave w copies the 1 KiB slabs w, w + NW, ... of a tile ----
   const int64_t row_bytes = p.t.kv_tok_b;
   const uint32_t lds_base = lds_addr(smem);
-  const int ld_kin = lane >> 4, ld_pc = lane & 15;
+  const int ld_kin = lane / Shape::kCols, ld_pc = lane % Shape::kCols;
   uint32_t ld_off[kCopies];
 #pragma unroll
   for (int i = 0; i < kCopies; ++i) {
-    const int key = 4 * (NW * i + wave) + ld_kin;
-    ld_off[i] = (uint32_t)(key * row_bytes + sw_col16(key, ld_pc) * 16);
+    const int key = Shape::kSlabRows * (NW * i + wave) + ld_kin;
+    ld_off[i] = (uint32_t)(key * row_bytes + (ld_pc ^ tile_sw<D>(key)) * 16);
   }
   const int64_t kv_off = kv_tok_bytes(p.t, t.kv_tok0) + (h / p.t.rep) * p.t.kv_head_b;
   const char* k_head = (const char*)p.k + kv_off;
@@ -88,26 +109,26 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_tile_kernel(const FwdParams<E>
       // (keys past the end of the range: the last key again -- their scores are masked, their V rows cleared)
 #pragma unroll
       for (int i = 0; i < kCopies; ++i) {
-        const int slab = NW * i + wave, key = 4 * slab + ld_kin;
-        async_copy16(head + (int64_t)min(key0 + key, nkeys - 1) * row_bytes + sw_col16(key, ld_pc) * 16, dst + slab * 1024);
+        const int slab = NW * i + wave, key = Shape::kSlabRows * slab + ld_kin;
+        async_copy16(head + (int64_t)min(key0 + key, nkeys - 1) * row_bytes + (ld_pc ^ tile_sw<D>(key)) * 16, dst + slab * 1024);
       }
     }
   };
   auto issue_k = [&](int kt) __attribute__((always_inline)) {
-    if (kt < nkt) issue(k_head, kt, lds_base + (kt % 3) * kTileBytes);
+    if (kt < nkt) issue(k_head, kt, lds_base + (kt % 3) * kStage);
   };
   auto issue_v = [&](int kt) __attribute__((always_inline)) {
-    if (kt < nkt) issue(v_head, kt, lds_base + Shape::kVBase + (kt & 1) * kTileBytes);
+    if (kt < nkt) issue(v_head, kt, lds_base + Shape::kVBase + (kt & 1) * kStage);
   };
   // rows of V past the end of the key range must not reach the matrix pipe (0 * NaN): clear them
   auto scrub_v = [&](int kt) __attribute__((always_inline)) {
     const int key0 = kt * TN;
     if (key0 + TN <= nkeys) return;
-    char* vdst = smem + Shape::kVBase + (kt & 1) * kTileBytes;
+    char* vdst = smem + Shape::kVBase + (kt & 1) * kStage;
 #pragma unroll
     for (int i = 0; i < kCopies; ++i) {
       const int slab = NW * i + wave;
-      if (key0 + 4 * slab + ld_kin >= nkeys) *reinterpret_cast<u32x4*>(vdst + slab * 1024 + lane * 16) = u32x4{0, 0, 0, 0};
+      if (key0 + Shape::kSlabRows * slab + ld_kin >= nkeys) *reinterpret_cast<u32x4*>(vdst + slab * 1024 + lane * 16) = u32x4{0, 0, 0, 0};
     }
   };
   auto first_copies = [&]() __attribute__((always_inline)) {
@@ -124,38 +145,37 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_tile_kernel(const FwdParams<E>
   const int limit = t.limit;
   const int min_limit = __builtin_amdgcn_readfirstlane(t.wave_min_limit);
   const bool row_valid = r < t.row_count;
-  elem8 bq[8];
+  elem8 bq[kKs];
   {
     const elem* src = reinterpret_cast<const elem*>((const char*)p.q + q_tok_bytes(p.t, t.tok) + h * p.t.q_head_b) + 8 * hh;
 #pragma unroll
-    for (int s8 = 0; s8 < 8; ++s8) bq[s8] = *reinterpret_cast<const elem8*>(src + 16 * s8);
+    for (int s8 = 0; s8 < kKs; ++s8) bq[s8] = *reinterpret_cast<const elem8*>(src + 16 * s8);
   }
 
   // ---- fragment addresses inside stage 0 (see fwd.hip) ----
-  uint32_t koff[8], voffA[4], voffB[4];
+  uint32_t koff[kKs], voffA[kDb], voffB[kDb];
   {
-    const int k_sw = ((n & 3) << 2) ^ ((n >> 2) & 3);
 #pragma unroll
-    for (int s8 = 0; s8 < 8; ++s8) koff[s8] = lds_base + n * 256 + (((2 * s8 + hh) ^ k_sw) << 4);
+    for (int s8 = 0; s8 < kKs; ++s8) koff[s8] = lds_base + n * kRowBytes + (((2 * s8 + hh) ^ tile_sw<D>(n)) << 4);
     const int g16 = lane >> 4, i0 = (lane & 15) >> 2, i1 = lane & 3;
     const int v_c16 = 2 * (g16 & 1) + (i1 >> 1), v_sub = (i1 & 1) * 8;
 #pragma unroll
-    for (int db = 0; db < 4; ++db) {
-      const int c16 = 4 * db + v_c16;
-      voffA[db] = lds_base + Shape::kVBase + (4 * hh + i0) * 256 + ((c16 ^ (i0 << 2) ^ hh) << 4) + v_sub;
-      voffB[db] = lds_base + Shape::kVBase + (4 * hh + i0 + 8) * 256 + ((c16 ^ (i0 << 2) ^ (hh + 2)) << 4) + v_sub;
+    for (int db = 0; db < kDb; ++db) {
+      const int c16 = 4 * db + v_c16, row = 4 * hh + i0;
+      voffA[db] = lds_base + Shape::kVBase + row * kRowBytes + ((c16 ^ tile_sw<D>(row)) << 4) + v_sub;
+      voffB[db] = lds_base + Shape::kVBase + (row + 8) * kRowBytes + ((c16 ^ tile_sw<D>(row + 8)) << 4) + v_sub;
     }
   }
   // the addresses move with the ring: K by one stage after the first half of every key tile (the second half already
   // reads the next tile's), V by one after the second
-  auto k_frag = [&](int kb, int s8) __attribute__((always_inline)) { return *lds_ptr<const elem8>(koff[s8] + (uint32_t)(kb * 8192)); };
+  auto k_frag = [&](int kb, int s8) __attribute__((always_inline)) { return *lds_ptr<const elem8>(koff[s8] + (uint32_t)(kb * 32 * kRowBytes)); };
   auto v_frag = [&](int kb, int j2, int db) __attribute__((always_inline)) {
-    const elem4 va = lds_read_tr<elem4>(voffA[db] + (uint32_t)((32 * kb + 16 * j2) * 256));
-    const elem4 vb = lds_read_tr<elem4>(voffB[db] + (uint32_t)((32 * kb + 16 * j2) * 256));
+    const elem4 va = lds_read_tr<elem4>(voffA[db] + (uint32_t)((32 * kb + 16 * j2) * kRowBytes));
+    const elem4 vb = lds_read_tr<elem4>(voffB[db] + (uint32_t)((32 * kb + 16 * j2) * kRowBytes));
     return __builtin_shufflevector(va, vb, 0, 1, 2, 3, 4, 5, 6, 7);
   };
 
-  f32x16 oacc[4];
+  f32x16 oacc[kDb];
   float m_run, l_run;
   const float sl2 = p.scale_log2;
   auto mask_block = [&](f32x16& s, int key0) __attribute__((always_inline)) {
@@ -177,19 +197,19 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_tile_kernel(const FwdParams<E>
   auto all_keys = [&](auto fixed_c) __attribute__((always_inline)) {
     constexpr bool kFixed = decltype(fixed_c)::value;
 #pragma unroll
-    for (int db = 0; db < 4; ++db)
+    for (int db = 0; db < kDb; ++db)
 #pragma unroll
       for (int e = 0; e < 16; ++e) oacc[db][e] = 0.f;
     wait_vmem();
     scrub_v(0);
     __syncthreads();
     f32x16 s0, s1;
-    elem8 pb[2], kpre[4];
+    elem8 pb[2], kpre[kKs / 2];
     {
 #pragma unroll
       for (int e = 0; e < 16; ++e) s0[e] = 0.f;
 #pragma unroll
-      for (int s8 = 0; s8 < 8; ++s8) s0 = mfma32(k_frag(0, s8), bq[s8], s0);
+      for (int s8 = 0; s8 < kKs; ++s8) s0 = mfma32(k_frag(0, s8), bq[s8], s0);
       if (31 > min_limit) mask_block(s0, 0);
       // (every row has a key in this block: key 0 of a causal tile, any key of a history tile)
       m_run = row_max(s0);
@@ -201,7 +221,7 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_tile_kernel(const FwdParams<E>
         pb[0][e] = (elem)pe;
       }
 #pragma unroll
-      for (int i = 0; i < 4; ++i) kpre[i] = k_frag(1, i);
+      for (int i = 0; i < kKs / 2; ++i) kpre[i] = k_frag(1, i);
     }
     // One step on key block kb of the tile: sc its S^T, elements 0..7 already in pb[0]; sn receives S^T of the next
     // block, block nkb of the tile koff points to; kpre holds the first four K fragments of it and receives those of
@@ -209,29 +229,32 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_tile_kernel(const FwdParams<E>
     auto step = [&](f32x16& sc, f32x16& sn, int nkb, int next_key0, auto has_next_c, bool masked, int kb, bool pre,
                     auto move_k) __attribute__((always_inline)) {
       constexpr bool has_next = decltype(has_next_c)::value;
-      elem8 ka[8], va[8];
+      elem8 ka[kKs], va[2 * kDb];
       float pf[8], rs = 0.f;
       if constexpr (has_next) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) ka[i] = kpre[i];
+        for (int i = 0; i < kKs / 2; ++i) ka[i] = kpre[i];
       }
 #pragma unroll
-      for (int s8 = 0; s8 < 8; ++s8) {
+      for (int s8 = 0; s8 < kKs; ++s8) {
         if constexpr (has_next) {
-          if (s8 + 4 < 8) ka[s8 + 4] = k_frag(nkb, s8 + 4);
+          if (s8 + kKs / 2 < kKs) ka[s8 + kKs / 2] = k_frag(nkb, s8 + kKs / 2);
           if (s8 == 0) {
 #pragma unroll
             for (int e = 0; e < 16; ++e) sn[e] = 0.f;
           }
           sn = mfma32(ka[s8], bq[s8], sn);
         }
-        pf[s8] = fast_exp2(sc[8 + s8] * sl2 - m_run);
-        if (s8 > 0) rs += pf[s8 - 1];
-        MOBA_PIN(pf[s8]);
-        MOBA_PIN(rs);
-        if (s8 >= 4 && s8 < 6) {
-          va[2 * (s8 - 4)] = v_frag(kb, 0, 2 * (s8 - 4));
-          va[2 * (s8 - 4) + 1] = v_frag(kb, 0, 2 * (s8 - 4) + 1);
+#pragma unroll
+        for (int e = s8 * (8 / kKs); e < (s8 + 1) * (8 / kKs); ++e) {
+          pf[e] = fast_exp2(sc[8 + e] * sl2 - m_run);
+          if (e > 0) rs += pf[e - 1];
+          MOBA_PIN(pf[e]);
+          MOBA_PIN(rs);
+        }
+        if (s8 >= kKs / 2 && s8 < kKs / 2 + 2) {  // half of the first V fragments each
+#pragma unroll
+          for (int db = (s8 - kKs / 2) * (kDb / 2); db < (s8 - kKs / 2 + 1) * (kDb / 2); ++db) va[db] = v_frag(kb, 0, db);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -244,21 +267,25 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_tile_kernel(const FwdParams<E>
       }
       float pg[8], rn = 0.f;
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        if (k + 4 < 8) va[k + 4] = v_frag(kb, 1, k & 3);
-        if (k >= 4 && pre) kpre[k - 4] = k_frag(1 - nkb, k - 4);
-        oacc[k & 3] = mfma32(va[k], pb[k >> 2], oacc[k & 3]);
+      for (int k = 0; k < 2 * kDb; ++k) {
+        if (k < kDb) va[k + kDb] = v_frag(kb, 1, k);
+        if (k >= kDb && pre) {
+#pragma unroll
+          for (int i = (k - kDb) * kKs / (2 * kDb); i < (k - kDb + 1) * kKs / (2 * kDb); ++i) kpre[i] = k_frag(1 - nkb, i);
+        }
+        oacc[k % kDb] = mfma32(va[k], pb[k / kDb], oacc[k % kDb]);
         if constexpr (has_next && kFixed) {
-          if (k == 1) {
-            pg[0] = fast_exp2(sn[0] * sl2 - m_run);
-            pg[1] = fast_exp2(sn[1] * sl2 - m_run);
-            MOBA_PIN(pg[0]);
-            MOBA_PIN(pg[1]);
-          } else if (k >= 2) {
-            pg[k] = fast_exp2(sn[k] * sl2 - m_run);
-            rn = (k == 2) ? pg[0] + pg[1] : rn + pg[k - 1];
-            MOBA_PIN(pg[k]);
-            MOBA_PIN(rn);
+          // the eight exponentials spread over the slots behind the first, which is left to the last S^T product's result
+          const int e0 = k == 0 ? 0 : (k == 1 ? 0 : (kDb == 4 ? k : 3 * k - 4));
+          const int e1 = k == 0 ? 0 : (k == 1 ? 2 : (kDb == 4 ? k + 1 : 3 * k - 1));
+#pragma unroll
+          for (int e = e0; e < e1; ++e) {
+            pg[e] = fast_exp2(sn[e] * sl2 - m_run);
+            MOBA_PIN(pg[e]);
+            if (e > 1) {
+              rn = e == 2 ? pg[0] + pg[1] : rn + pg[e - 1];
+              MOBA_PIN(rn);
+            }
           }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -270,7 +297,7 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_tile_kernel(const FwdParams<E>
         m_run = m_new;
         l_run *= alpha;
 #pragma unroll
-        for (int db = 0; db < 4; ++db)
+        for (int db = 0; db < kDb; ++db)
 #pragma unroll
           for (int e = 0; e < 16; ++e) oacc[db][e] *= alpha;
 #pragma unroll
@@ -287,10 +314,10 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_tile_kernel(const FwdParams<E>
     };
     int kstage = 0;
     auto move_k = [&]() __attribute__((always_inline)) {
-      const uint32_t d = kstage == 2 ? (uint32_t)(-2 * kTileBytes) : (uint32_t)kTileBytes;
+      const uint32_t d = kstage == 2 ? (uint32_t)(-2 * kStage) : (uint32_t)kStage;
       kstage = kstage == 2 ? 0 : kstage + 1;
 #pragma unroll
-      for (int s8 = 0; s8 < 8; ++s8) koff[s8] += d;
+      for (int s8 = 0; s8 < kKs; ++s8) koff[s8] += d;
     };
     auto stay = [] __attribute__((always_inline)) {};
     auto tile_body = [&](int it, auto more_c) __attribute__((always_inline)) {
@@ -307,9 +334,9 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_tile_kernel(const FwdParams<E>
       }
       step(s0, s1, 1, key0 + 32, std::true_type{}, key0 + 63 > min_limit, 0, more, move_k);
       step(s1, s0, 0, key0 + TN, more_c, more && key0 + TN + 31 > min_limit, 1, more, stay);
-      const uint32_t d = (it & 1) ? (uint32_t)(-kTileBytes) : (uint32_t)kTileBytes;
+      const uint32_t d = (it & 1) ? (uint32_t)(-kStage) : (uint32_t)kStage;
 #pragma unroll
-      for (int db = 0; db < 4; ++db) {
+      for (int db = 0; db < kDb; ++db) {
         voffA[db] += d;
         voffB[db] += d;
       }
@@ -328,7 +355,7 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_tile_kernel(const FwdParams<E>
     // all read as "too large"; the largest magnitude among the row's accumulators likewise
     uint32_t worst = 0;
 #pragma unroll
-    for (int db = 0; db < 4; ++db)
+    for (int db = 0; db < kDb; ++db)
 #pragma unroll
       for (int e = 0; e < 16; ++e) worst = max(worst, __builtin_bit_cast(uint32_t, oacc[db][e]) & 0x7fffffffu);
     const bool bad = row_valid && (__builtin_bit_cast(uint32_t, l_tot) >= __builtin_bit_cast(uint32_t, kFixedRefMaxSum) ||
@@ -343,11 +370,11 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_tile_kernel(const FwdParams<E>
     if (__builtin_amdgcn_readfirstlane(again)) {
       __syncthreads();  // (every wave has read the flags)
       // back to stage 0: nkt tiles moved K by nkt stages, V by nkt
-      const uint32_t dk = (uint32_t)((nkt % 3) * kTileBytes), dv = (uint32_t)((nkt & 1) * kTileBytes);
+      const uint32_t dk = (uint32_t)((nkt % 3) * kStage), dv = (uint32_t)((nkt & 1) * kStage);
 #pragma unroll
-      for (int s8 = 0; s8 < 8; ++s8) koff[s8] -= dk;
+      for (int s8 = 0; s8 < kKs; ++s8) koff[s8] -= dk;
 #pragma unroll
-      for (int db = 0; db < 4; ++db) {
+      for (int db = 0; db < kDb; ++db) {
         voffA[db] -= dv;
         voffB[db] -= dv;
       }
@@ -380,7 +407,7 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_tile_kernel(const FwdParams<E>
 #pragma unroll
     for (int i = 0; i < 4; ++i) d4[i] = __shfl(dest, 8 * i + (lane >> 3), 64);
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {
+    for (int half = 0; half < D / 64; ++half) {
 #pragma unroll
       for (int d2 = 0; d2 < 2; ++d2)
 #pragma unroll
@@ -395,25 +422,27 @@ __global__ __launch_bounds__(NW * 64, 2) void fwd_tile_kernel(const FwdParams<E>
       for (int i = 0; i < 4; ++i) {
         const int row = 8 * i + (lane >> 3);
         const u32x4 x = *reinterpret_cast<const u32x4*>(stage + row * 128 + ((c16 ^ ((row >> 1) & 7)) << 4));
-        if (row < rows_here) *reinterpret_cast<u32x4*>(o_base + (int64_t)d4[i] * kHeadDim + 64 * half + c16 * 8) = x;
+        if (row < rows_here) *reinterpret_cast<u32x4*>(o_base + (int64_t)d4[i] * D + 64 * half + c16 * 8) = x;
       }
     }
   }
 }
 
-template <class E, int NW>
+template <class E, int D, int NW>
 static int launch(const FwdParams<E>& p, int64_t workgroups, hipStream_t st) {
+  using Shape = FwdTileShape<D, NW>;
   static bool allowed[kMaxDevices];
-  if (!allow_dynamic_lds((const void*)fwd_tile_kernel<E, NW>, FwdTileShape<NW>::kLds, allowed)) return MOBA_ERR_LAUNCH;
-  hipLaunchKernelGGL((fwd_tile_kernel<E, NW>), dim3((unsigned)workgroups), dim3(NW * 64), FwdTileShape<NW>::kLds, st, p);
+  if (!allow_dynamic_lds((const void*)fwd_tile_kernel<E, D, NW>, Shape::kLds, allowed)) return MOBA_ERR_LAUNCH;
+  hipLaunchKernelGGL((fwd_tile_kernel<E, D, NW>), dim3((unsigned)workgroups), dim3(NW * 64), Shape::kLds, st, p);
   return MOBA_OK;
 }
 
 template <class E>
-int launch_fwd_tiles(const FwdParams<E>& p, int tile_rows, int64_t workgroups, hipStream_t st) {
-  return tile_rows == 128 ? launch<E, 4>(p, workgroups, st) : launch<E, 8>(p, workgroups, st);
+int launch_fwd_tiles(const FwdParams<E>& p, int head_dim, int tile_rows, int64_t workgroups, hipStream_t st) {
+  if (head_dim == 64) return launch<E, 64, 4>(p, workgroups, st);
+  return tile_rows == 128 ? launch<E, 128, 4>(p, workgroups, st) : launch<E, 128, 8>(p, workgroups, st);
 }
-template int launch_fwd_tiles<Bf16>(const FwdParams<Bf16>&, int, int64_t, hipStream_t);
-template int launch_fwd_tiles<F16>(const FwdParams<F16>&, int, int64_t, hipStream_t);
+template int launch_fwd_tiles<Bf16>(const FwdParams<Bf16>&, int, int, int64_t, hipStream_t);
+template int launch_fwd_tiles<F16>(const FwdParams<F16>&, int, int, int64_t, hipStream_t);
 
 }  // namespace moba

@@ -55,7 +55,7 @@ __device__ __forceinline__ int find_seq(const int* __restrict__ cu, int nseq, in
 
 // (up to 12 picks the kernel is held to the registers of three waves per SIMD: it is bound by its vector
 // instructions, which the waves of a SIMD issue in turn while others wait for memory, LDS and barriers)
-template <class E, int KMAX>
+template <class E, int KMAX, int D>
 __global__ __launch_bounds__(256, KMAX <= 12 ? 3 : 1) void gate_topk_kernel(
     const typename E::elem* __restrict__ q, const typename E::elem* __restrict__ kbar, const int* __restrict__ cu_seqlens,
     const int* __restrict__ seq_fbase, int* __restrict__ sel, float* __restrict__ scores_out,
@@ -94,21 +94,21 @@ __global__ __launch_bounds__(256, KMAX <= 12 ? 3 : 1) void gate_topk_kernel(
 
   if (fhi > 0) {  // wave-uniform (and block-uniform)
     // Q^T operand: lane (n, hh) holds q[token n (+32)][16*ks + 8*hh .. +7]
-    elem8 bq[2][8];
+    elem8 bq[2][D / 16];
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) {
       const int tok = min(tok0 + 32 * qb + n, S - 1);
       const int be = batch_rows ? tok / batch_rows : 0;  // batch entry of the token in a batched layout
       const elem* src = q + (be * q_batch_stride + (tok - be * batch_rows) * q_tok_stride + hc * q_head_stride) + 8 * hh;
 #pragma unroll
-      for (int ks = 0; ks < 8; ++ks) bq[qb][ks] = *reinterpret_cast<const elem8*>(src + 16 * ks);
+      for (int ks = 0; ks < D / 16; ++ks) bq[qb][ks] = *reinterpret_cast<const elem8*>(src + 16 * ks);
     }
     for (int f0 = flo; f0 < fhi; f0 += 32) {
       const int fr = min(f0 + n, F - 1);
-      const elem* src = kbar + ((int64_t)fr * Hkv + hc / (H / Hkv)) * kHeadDim + 8 * hh;
+      const elem* src = kbar + ((int64_t)fr * Hkv + hc / (H / Hkv)) * D + 8 * hh;
       f32x16 acc0 = {0}, acc1 = {0};
 #pragma unroll
-      for (int ks = 0; ks < 8; ++ks) {
+      for (int ks = 0; ks < D / 16; ++ks) {
         const elem8 a = *reinterpret_cast<const elem8*>(src + 16 * ks);
         acc0 = mfma32(a, bq[0][ks], acc0);
         acc1 = mfma32(a, bq[1][ks], acc1);
@@ -260,10 +260,10 @@ extern "C" int moba_gate_topk(const void* q, const void* kbar, const int32_t* cu
   if (dtype != MOBA_DTYPE_BF16 && dtype != MOBA_DTYPE_F16) return MOBA_ERR_UNSUPPORTED;
   if (S <= 0 || S > 0x7fffffff - 64 || H <= 0 || nseq <= 0 || F <= 0 || B <= 0 || K <= 0) return MOBA_ERR_ARG;
   if (dense_local < 0 || dense_local > K) return MOBA_ERR_ARG;
-  if (D != kHeadDim) return MOBA_ERR_UNSUPPORTED;
+  if (D != kHeadDim && D != 64) return MOBA_ERR_UNSUPPORTED;
   if (((uintptr_t)q & 15) || ((uintptr_t)kbar & 15)) return MOBA_ERR_ARG;
-  // strides (elements): {q token, q head, ., ., rows per batch entry, q batch, .}; null = packed [S, H, 128]
-  const int64_t qts = strides ? strides[0] : (int64_t)H * kHeadDim, qhs = strides ? strides[1] : kHeadDim;
+  // strides (elements): {q token, q head, ., ., rows per batch entry, q batch, .}; null = packed [S, H, D]
+  const int64_t qts = strides ? strides[0] : (int64_t)H * D, qhs = strides ? strides[1] : D;
   if (strides && (strides[4] < 0 || strides[4] > 0x7fffffffLL)) return MOBA_ERR_ARG;  // (before it is narrowed)
   const int qbr = strides ? (int)strides[4] : 0;
   const int64_t qbs = strides ? strides[5] : 0;
@@ -271,17 +271,19 @@ extern "C" int moba_gate_topk(const void* q, const void* kbar, const int32_t* cu
   if (qbr < 0 || (qbr > 0 && (qbs <= 0 || (qbs & 7)))) return MOBA_ERR_ARG;
   dim3 grid((unsigned)((S + 63) / 64), (unsigned)((H + 3) / 4));
   hipStream_t st = (hipStream_t)stream;
-#define CALL(KM)                                                                                               \
-  if (dtype == MOBA_DTYPE_F16)                                                                                 \
-    hipLaunchKernelGGL((gate_topk_kernel<F16, KM>), grid, dim3(256), 0, st, (const f16*)q, (const f16*)kbar,   \
-                       cu_seqlens, seq_fbase, sel, scores_out, (int)S, H, Hkv, nseq, F, B, K, qts, qhs, qbr, qbs, \
-                       pair_off, cnt, dense_local);                                                            \
-  else                                                                                                         \
-    hipLaunchKernelGGL((gate_topk_kernel<Bf16, KM>), grid, dim3(256), 0, st, (const bf16*)q, (const bf16*)kbar, \
-                       cu_seqlens, seq_fbase, sel, scores_out, (int)S, H, Hkv, nseq, F, B, K, qts, qhs, qbr, qbs, \
-                       pair_off, cnt, dense_local)
+#define GATE(EL, KM, DIM)                                                                                             \
+  hipLaunchKernelGGL((gate_topk_kernel<EL, KM, DIM>), grid, dim3(256), 0, st, (const EL::elem*)q, (const EL::elem*)kbar, \
+                     cu_seqlens, seq_fbase, sel, scores_out, (int)S, H, Hkv, nseq, F, B, K, qts, qhs, qbr, qbs,       \
+                     pair_off, cnt, dense_local)
+#define CALL(KM)                                                       \
+  if (dtype == MOBA_DTYPE_F16) {                                       \
+    if (D == 64) GATE(F16, KM, 64); else GATE(F16, KM, 128);           \
+  } else {                                                             \
+    if (D == 64) GATE(Bf16, KM, 64); else GATE(Bf16, KM, 128);         \
+  }
   MOBA_DISPATCH_K(K, CALL)
 #undef CALL
+#undef GATE
   return launch_check.result();
 }
 

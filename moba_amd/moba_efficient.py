@@ -23,6 +23,7 @@ from . import _lib
 from .plan import FWD_TILE_ROWS, MobaPlan, TILE_ROWS, make_plan
 
 HEAD_DIM = 128
+NARROW_HEAD_DIM = 64   # the forward's kernels also take heads of this width as they are
 # MOBA_FIXED_REFERENCE=0 keeps the forward kernel on its running-maximum softmax for every problem (the
 # fixed-reference form, with its redo list, is otherwise used where the C ABI's `redo` argument says)
 FIXED_REFERENCE = os.environ.get("MOBA_FIXED_REFERENCE", "1") != "0"
@@ -298,7 +299,7 @@ class _Geometry:
     def __init__(self, plan: MobaPlan, lib, H: int, D: int, esize: int):
         S, K = plan.S, plan.K
         # rows per tile of the forward (forward_tile_rows); tiles of the backward's height share its tables
-        self.rows_per_tile = forward_tile_rows(plan, H)
+        self.rows_per_tile = forward_tile_rows(plan, H, D)
         tall = self.rows_per_tile == FWD_TILE_ROWS
         self.self_tiles = plan.fwd_self_tiles if tall else plan.self_tiles
         self.self_names = (("fwd_" if tall else "") + "self_tile_prefix", ("fwd_" if tall else "") + "self_tile_chunk")
@@ -351,8 +352,10 @@ SHORT_TILES_CHUNK = 512
 SHORT_TILES_FLOPS = 4e12
 
 
-def forward_tile_rows(plan: MobaPlan, H: int) -> int:
+def forward_tile_rows(plan: MobaPlan, H: int, D: int = HEAD_DIM) -> int:
     """Rows per tile of the forward attention kernel for this plan and number of heads."""
+    if D == NARROW_HEAD_DIM:
+        return TILE_ROWS    # (the only form for such heads)
     short_chunks = not plan.fallback and plan.chunk_size <= SHORT_TILES_CHUNK
     return TILE_ROWS if short_chunks or plan.flops_per_head * HEAD_DIM * H <= SHORT_TILES_FLOPS else FWD_TILE_ROWS
 
@@ -369,7 +372,7 @@ def _forward(q, k, v, plan: MobaPlan, timer: Optional[StageTimer] = None, scale:
     """As _run_forward; tile_off and tile_seg are those of tiles of FWD_TILE_ROWS rows, whatever the kernel took."""
     res = _run_forward(q, k, v, plan, timer, scale)
     S, H, D = _dims(q)
-    if plan.fallback or forward_tile_rows(plan, H) == FWD_TILE_ROWS:
+    if plan.fallback or forward_tile_rows(plan, H, D) == FWD_TILE_ROWS:
         return res
     out, lse, sel, seg_off, _, seg_dest, _ = res
     tile_off, tile_seg = tile_tables(seg_off, plan, H, FWD_TILE_ROWS)
@@ -465,6 +468,10 @@ def _backward(dout, q, k, v, out, lse, sel, seg_off, seg_dest, plan: MobaPlan, s
     """tables: the backward kernels' (tile_off, tile_seg) if the forward made them (made here otherwise)."""
     lib = _lib.load()
     S, H, D = _dims(q)
+    if D < HEAD_DIM:   # (the backward's kernels take heads of 128 elements)
+        dout, q, k, v, out = (torch.nn.functional.pad(x, (0, HEAD_DIM - D)) for x in (dout, q, k, v, out))
+        grads = _backward(dout, q, k, v, out, lse, sel, seg_off, seg_dest, plan, scale or D ** -0.5, tables)
+        return tuple(x[..., :D].contiguous() for x in grads)
     Hkv = _dims(k)[1]
     dev = q.device
     K = plan.K
@@ -668,8 +675,9 @@ def moba_attn_varlen(
     Returns:
         [seqlen, heads, head_dim] in q's dtype.  Softmax scale is head_dim ** -0.5.
 
-    The kernels are built for head_dim 128.  Narrower heads are padded with zeros to 128 (the scores, the
-    gate and the softmax scale head_dim ** -0.5 are those of the narrow heads; the padding costs the work
+    The kernels are built for head_dim 128, and those of the forward for 64 too.  Other heads are padded with zeros to
+    the next of the two, and for the backward to 128 (the scores, the gate and the softmax scale head_dim ** -0.5 are
+    those of the narrow heads; the padding costs the work
     and memory of 128); wider heads are refused.
     """
     return moba_attn_varlen_with_lse(q, k, v, cu_seqlens, max_seqlen, moba_chunk_size, moba_topk)[0]
@@ -689,14 +697,14 @@ def moba_attn_batched(query, key, value, moba_chunk_size, moba_topk):
     [batch, kv_heads, seqlen, head_dim], every batch entry one sequence.  The tensors are read where they lie
     (no transposing copies, which ``hf_to_fa`` costs for batch > 1, moba/wrapper.py:56-58; no key/value head
     expansion); returns [batch * seqlen, heads, head_dim] like the packed operator.  Layouts the kernels cannot
-    address, and head_dim below 128, go through packed copies."""
+    address, and head_dim other than 128 and 64, go through packed copies."""
     from .wrapper import _cu_seqlens_for, hf_to_fa
     b, h, l, d = query.shape
     if key.shape != value.shape or key.dim() != 4 or key.shape[0] != b or key.shape[2] != l or key.shape[3] != d:
         raise ValueError("query must be [batch, heads, seqlen, head_dim] and key, value [batch, kv_heads, seqlen, head_dim]")
     cu_seqlens = _cu_seqlens_for(b, l, query.device)
     make_plan(cu_seqlens, moba_chunk_size, moba_topk, host_lengths=range(0, (b + 1) * l, l))
-    in_place = (d == HEAD_DIM and _addressable(query) and _addressable(key) and _addressable(value)
+    in_place = (d in (HEAD_DIM, NARROW_HEAD_DIM) and _addressable(query) and _addressable(key) and _addressable(value)
                 and _row_strides(key) == _row_strides(value) and _batch_stride(key) == _batch_stride(value))
     if not in_place:
         return moba_attn_varlen_gqa(hf_to_fa(query), hf_to_fa(key), hf_to_fa(value), cu_seqlens, l, moba_chunk_size,
@@ -724,8 +732,8 @@ def moba_attn_varlen_with_lse(q, k, v, cu_seqlens, max_seqlen, moba_chunk_size, 
     if plan.S != q.shape[0]:
         raise ValueError(f"cu_seqlens ends at {plan.S} but q has {q.shape[0]} tokens")
     head_dim = q.shape[2]
-    if head_dim < HEAD_DIM:
-        pad = (0, HEAD_DIM - head_dim)
+    if head_dim not in (HEAD_DIM, NARROW_HEAD_DIM):
+        pad = (0, (NARROW_HEAD_DIM if head_dim < NARROW_HEAD_DIM else HEAD_DIM) - head_dim)
         q, k, v = (torch.nn.functional.pad(x, pad) for x in (q, k, v))
         out, lse = _attend(q, k, v, plan, timer, head_dim ** -0.5)
         return out[..., :head_dim].contiguous(), lse

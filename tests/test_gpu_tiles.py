@@ -21,7 +21,7 @@ def tile_rows(monkeypatch):
         P._BY_TENSOR.clear()
 
     def choose(rows):
-        monkeypatch.setattr(E, "forward_tile_rows", lambda plan, H: rows)
+        monkeypatch.setattr(E, "forward_tile_rows", lambda plan, H, D=128: rows)
         forget()
 
     yield choose
@@ -70,3 +70,34 @@ def test_tile_heights_agree(lens, heads, kv_heads, B, topk, dtype, spread, tile_
         step = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
         assert (out_a.float() - out_b.float()).abs().max() < 4 * 4 * step
         assert (lse_a - lse_b).abs().max() < 1e-3 * max(1.0, spread * spread)
+
+
+@pytest.mark.parametrize("lens,heads,kv_heads,B,topk,dtype", [
+    ([128], 1, 1, 64, 2, torch.bfloat16),
+    ([129, 127, 1, 257], 2, 1, 65, 3, torch.float16),
+    ([2048], 4, 2, 512, 1, torch.float16),
+    ([4096], 1, 1, 2048, 3, torch.bfloat16),
+    ([3000], 5, 1, 192, 13, torch.bfloat16),
+])
+@pytest.mark.parametrize("spread", [1.0, 8.0])
+def test_heads_of_64_are_those_of_128_padded(lens, heads, kv_heads, B, topk, dtype, spread, tile_rows):
+    """The forward's kernels for 64-element heads form the same sums as those for 128 on zero-padded heads (zeros add
+    nothing): selection, output and log-sum-exp bit for bit, on the packed and on the batched layout."""
+    from moba_amd import moba_efficient as E
+    cu = [0] + np.cumsum(lens).tolist()
+    S = cu[-1]
+    print("narrow case", lens, heads, B, topk, dtype, spread, flush=True)
+    g = torch.Generator().manual_seed(S + heads)
+    q = (torch.randn((S, heads, 64), generator=g) * spread).to(dtype).cuda()
+    k = (torch.randn((S, kv_heads, 64), generator=g) * spread).to(dtype).cuda()
+    v = torch.randn((S, kv_heads, 64), generator=g).to(dtype).cuda()
+    tile_rows(128)
+    cu_t = torch.tensor(cu, dtype=torch.int32, device="cuda")
+    out, lse = E.moba_attn_varlen_with_lse(q, k, v, cu_t, max(lens), B, topk, gqa=True)
+    wide = [torch.nn.functional.pad(x, (0, 64)) for x in (q, k, v)]
+    want, want_lse = E._attend(*wide, E.make_plan(cu_t, B, topk), None, 64 ** -0.5)
+    assert out.shape == q.shape and torch.isfinite(out.float()).all()
+    assert torch.equal(out, want[..., :64]) and torch.equal(lse, want_lse)
+    if len(lens) == 1:
+        one = E.moba_attn_batched(*(x.transpose(0, 1)[None] for x in (q, k, v)), B, topk)
+        assert torch.equal(one, out)
