@@ -4,7 +4,7 @@
 //
 //   pass 1  count    one workgroup per (query chunk, head): how many of its tokens
 //                    picked each earlier chunk of the sequence -> cnt[(f, h, query chunk)]
-//   pass 2  scan     exclusive prefix sum of cnt in (f, h, query chunk) order: that is
+//   pass 2  scan     exclusive prefix sum (one workgroup, or two launches of many) of cnt in (f, h, query chunk) order: that is
 //                    the list position of the first such token, because query chunks
 //                    of a sequence are visited in ascending token order
 //   pass 3  fill     same decomposition as pass 1; inside a workgroup the four waves own
@@ -189,18 +189,16 @@ __global__ __launch_bounds__(NW * 64) void lists_fill_kernel(
                           dense_local, lds);
 }
 
-// exclusive prefix sum of a[0..n) in place, total stored at a[n]; one workgroup.
-__global__ __launch_bounds__(1024) void scan_kernel(int* __restrict__ a, int n) {
-  __shared__ int wsum[16];
-  __shared__ int carry_s;
+// exclusive prefix sum of a[lo..hi) in place, starting from `carry`, by a workgroup of 1024; returns the total
+__device__ __forceinline__ int scan_range(int* __restrict__ a, int lo, int hi, int carry) {
+  __shared__ int wsum[2][16];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  if (tid == 0) carry_s = 0;
-  __syncthreads();
-  for (int base = 0; base < n; base += 4096) {
+  int half = 0;  // (two sets of wave sums in turn: one barrier per 4096 elements)
+  for (int base = lo; base < hi; base += 4096, half ^= 1) {
     const int i0 = base + tid * 4;
     int v[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = (i0 + e < n) ? a[i0 + e] : 0;
+    for (int e = 0; e < 4; ++e) v[e] = (i0 + e < hi) ? a[i0 + e] : 0;
     const int tsum = v[0] + v[1] + v[2] + v[3];
     int inc = tsum;  // inclusive scan across the wave
 #pragma unroll
@@ -208,27 +206,63 @@ __global__ __launch_bounds__(1024) void scan_kernel(int* __restrict__ a, int n) 
       const int t = __shfl_up(inc, o, 64);
       if (lane >= o) inc += t;
     }
-    if (lane == 63) wsum[wave] = inc;
+    if (lane == 63) wsum[half][wave] = inc;
     __syncthreads();
     int woff = 0, total = 0;
 #pragma unroll
     for (int w = 0; w < 16; ++w) {
-      const int x = wsum[w];
+      const int x = wsum[half][w];
       if (w < wave) woff += x;
       total += x;
     }
-    const int carry = carry_s;
     int run = carry + woff + inc - tsum;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      if (i0 + e < n) a[i0 + e] = run;
+      if (i0 + e < hi) a[i0 + e] = run;
       run += v[e];
     }
-    __syncthreads();
-    if (tid == 0) carry_s = carry + total;
-    __syncthreads();
+    carry += total;
   }
-  if (tid == 0) a[n] = carry_s;
+  return carry;
+}
+
+// exclusive prefix sum of a[0..n) in place, total stored at a[n]; one workgroup.
+__global__ __launch_bounds__(1024) void scan_kernel(int* __restrict__ a, int n) {
+  const int total = scan_range(a, 0, n, 0);
+  if (threadIdx.x == 0) a[n] = total;
+}
+
+// The same by many workgroups of `per` elements each, in two launches: the sums of the ranges, then every workgroup adds
+// up the sums before its own and scans its range.  One workgroup alone is bound by its own round trips (4096 elements
+// in about 2.5 us): 9.4 million counts -- 196608 tokens, 32 heads, chunks of 256 -- took it 5.8 ms of a call of 14 ms.
+__global__ __launch_bounds__(1024) void scan_sums_kernel(const int* __restrict__ a, int n, int per, int* __restrict__ sums) {
+  __shared__ int wsum[16];
+  const int lo = blockIdx.x * per, hi = min(n, lo + per);
+  int s = 0;
+  for (int i = lo + threadIdx.x; i < hi; i += 1024) s += a[i];
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o, 64);
+  if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < 16; ++w) s += wsum[w];
+    sums[blockIdx.x] = s;
+  }
+}
+__global__ __launch_bounds__(1024) void scan_apply_kernel(int* __restrict__ a, int n, int per, const int* __restrict__ sums) {
+  __shared__ int wsum[16];
+  int s = 0;
+  for (int i = threadIdx.x; i < (int)blockIdx.x; i += 1024) s += sums[i];
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o, 64);
+  if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = s;
+  __syncthreads();
+  int carry = 0;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) carry += wsum[w];
+  const int lo = blockIdx.x * per, hi = min(n, lo + per);
+  const int total = scan_range(a, lo, hi, carry);
+  if (blockIdx.x + 1 == gridDim.x && threadIdx.x == 0) a[n] = total;
 }
 
 // per (f, h): list start and number of row tiles
@@ -420,6 +454,22 @@ __global__ __launch_bounds__(1024) void lists_fill_tail_kernel(
 
 using namespace moba;
 
+// scratch: scratch_ints ints that nobody needs until the scan is done.  Up to 16384 elements (four of its steps) one
+// workgroup costs no more than the second launch.
+static void launch_scan(int* a, int n, int* scratch, int64_t scratch_ints, hipStream_t st) {
+  int64_t groups = ((int64_t)n + 4095) / 4096;
+  if (groups > scratch_ints) groups = scratch_ints;
+  if (n <= 16384 || groups < 2) {
+    hipLaunchKernelGGL(scan_kernel, dim3(1), dim3(1024), 0, st, a, n);
+    return;
+  }
+  const int64_t steps = ((int64_t)n + groups * 4096 - 1) / (groups * 4096);  // per workgroup
+  const int per = (int)(steps * 4096);
+  const dim3 grid((unsigned)(((int64_t)n + per - 1) / per));
+  hipLaunchKernelGGL(scan_sums_kernel, grid, dim3(1024), 0, st, (const int*)a, n, per, scratch);
+  hipLaunchKernelGGL(scan_apply_kernel, grid, dim3(1024), 0, st, a, n, per, (const int*)scratch);
+}
+
 static void launch_tile_tables(const int32_t* seg_off, int32_t* tile_off, int32_t* tile_seg, int H, int F,
                                int tile_rows, int64_t hist_bound, hipStream_t st) {
   if ((int64_t)F * H < kTailMaxSegments && hist_bound <= kTailMaxTiles) {
@@ -429,7 +479,7 @@ static void launch_tile_tables(const int32_t* seg_off, int32_t* tile_off, int32_
   }
   hipLaunchKernelGGL(lists_tile_counts_kernel, dim3((F * H + 255) / 256), dim3(256), 0, st, seg_off, tile_off, F * H,
                      tile_rows);
-  hipLaunchKernelGGL(scan_kernel, dim3(1), dim3(1024), 0, st, tile_off, F * H);
+  launch_scan(tile_off, F * H, tile_seg, hist_bound, st);
   hipLaunchKernelGGL(lists_tile_seg_kernel, dim3((unsigned)((hist_bound + 255) / 256)), dim3(256), 0, st,
                      (const int*)tile_off, tile_seg, F * H, (int)hist_bound);
 }
@@ -474,7 +524,7 @@ extern "C" int moba_build_lists(const int32_t* sel, const int32_t* chunk_tok, co
   if (!counted)
     hipLaunchKernelGGL(lists_count_kernel<256>, grid, dim3(256), (size_t)cmax * 4, st, sel, chunk_tok, chunk_fb,
                        chunk_local, pair_off, cnt, H, K, dense_local);
-  hipLaunchKernelGGL(scan_kernel, dim3(1), dim3(1024), 0, st, cnt, P * H);
+  launch_scan(cnt, P * H, tile_off, (int64_t)F * H, st);
   // more than 64 KiB of dynamic LDS has to be asked for explicitly
   // (LDS: 12 bytes per wave and candidate chunk)
   const bool wide = S / N >= 1024 && (size_t)cmax * 192 <= 64 * 1024;  // long chunks: 16 waves per (chunk, head)
@@ -509,7 +559,7 @@ extern "C" int moba_build_lists(const int32_t* sel, const int32_t* chunk_tok, co
   } else {
     hipLaunchKernelGGL(lists_segments_kernel, dim3((F * H + 1 + 255) / 256), dim3(256), 0, st, (const int*)cnt,
                        pair_off, seg_off, tile_off, F, H, tile_rows);
-    hipLaunchKernelGGL(scan_kernel, dim3(1), dim3(1024), 0, st, tile_off, F * H);
+    launch_scan(tile_off, F * H, tile_seg, hist_bound, st);
     hipLaunchKernelGGL(lists_tile_seg_kernel, dim3((unsigned)((hist_bound + 255) / 256)), dim3(256), 0, st,
                        (const int*)tile_off, tile_seg, F * H, (int)hist_bound);
   }
