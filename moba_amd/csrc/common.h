@@ -81,6 +81,10 @@ __device__ __forceinline__ void mfma32_into_vgprs(f32x16& d, f16x8 a, f16x8 b, b
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ __forceinline__ float fast_log2(float x) { return __builtin_amdgcn_logf(x); }
 
+// The bits of a float.  A function of a value on purpose: __builtin_bit_cast of an element of a vector variable reads
+// element 0, whatever the index.
+__device__ __forceinline__ uint32_t float_bits(float x) { return __builtin_bit_cast(uint32_t, x); }
+
 // two floats rounded (to nearest even) to the element type, packed into 32 bits
 template <class E>
 __device__ __forceinline__ uint32_t pack2(float lo, float hi) {

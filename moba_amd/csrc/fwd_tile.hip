@@ -357,7 +357,7 @@ __global__ __launch_bounds__(NW * 64, (FwdTileShape<D, NW>::kWavesPerSimd)) void
 #pragma unroll
     for (int db = 0; db < kDb; ++db)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) worst = max(worst, __builtin_bit_cast(uint32_t, oacc[db][e]) & 0x7fffffffu);
+      for (int e = 0; e < 16; ++e) worst = max(worst, float_bits(oacc[db][e]) & 0x7fffffffu);
     const bool bad = row_valid && (__builtin_bit_cast(uint32_t, l_tot) >= __builtin_bit_cast(uint32_t, kFixedRefMaxSum) ||
                                    worst >= 0x7f800000u);
     volatile int* flags = reinterpret_cast<volatile int*>(smem + Shape::kFlags);

@@ -101,3 +101,28 @@ def test_heads_of_64_are_those_of_128_padded(lens, heads, kv_heads, B, topk, dty
     if len(lens) == 1:
         one = E.moba_attn_batched(*(x.transpose(0, 1)[None] for x in (q, k, v)), B, topk)
         assert torch.equal(one, out)
+
+
+@pytest.mark.parametrize("rows", [128, 256])
+def test_overflow_in_any_dimension_is_found(rows, tile_rows):
+    """Probabilities of 2^68 to 2^96 (relative to the fixed reference) times values of 2^60 leave fp32 in the accumulators of
+    some dimensions only: v is zero in dimensions 0 and 4 of every 32, those of the first accumulator registers.  Such
+    tiles have to be computed again with a running maximum all the same; scaling v by a power of two scales the result."""
+    from moba_amd import moba_efficient as E
+    S, H, B, topk = 32768, 8, 1024, 3
+    print("overflow case", rows, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(17)
+    q, k, v = (torch.randn((S, H, 128), generator=g, device="cuda") for _ in range(3))
+    q, k, v = (q * 4.5).to(torch.bfloat16), (k * 4.5).to(torch.bfloat16), v.to(torch.bfloat16)
+    v[..., 0::32] = 0
+    v[..., 4::32] = 0
+    tile_rows(rows)
+    cu_t = torch.tensor([0, S], dtype=torch.int32, device="cuda")
+    small = E.moba_attn_varlen(q, k, v, cu_t, S, B, topk)
+    large = E.moba_attn_varlen(q, k, (v.float() * 2.0 ** 60).to(torch.bfloat16), cu_t, S, B, topk)
+    assert torch.isfinite(large.float()).all()
+    err = (large.float() * 2.0 ** -60 - small.float()).abs()
+    # Near one-hot rows: values of up to about 4.5 on both sides, each rounded to 8 bits three times (probabilities,
+    # partial result, result): 2 * 3 * 2^-9 * 4.5 = 5.3e-2 at most; in the mean (values of about 0.8, roundings of either
+    # sign, half a rounding on average) below 2 * 3 * 2^-10 * 0.8 = 4.7e-3.
+    assert err.max() < 5.3e-2 and err.mean() < 4.7e-3, (err.max().item(), err.mean().item())
