@@ -10,10 +10,15 @@
 // chunks 0..d of every sequence (which would pick every earlier chunk) get no picks
 // at all: the attention kernels serve them through one causal pass over the prefix.
 //
-// One wave handles 64 consecutive tokens of one head: the score tile
-// (32 chunks x 64 tokens) is two 32x32x16 MFMA accumulators, staged through LDS
-// so that each lane then owns one token and runs an insertion top-k held in
-// registers.  Scores never reach HBM (except through the optional debug output).
+// One wave handles 64 consecutive tokens of one head: the score tile (32 chunks x 64 tokens) is two 32x32x16 MFMA
+// accumulators.  Sixteen lane-half swaps leave the 32 scores of token `lane` in lane `lane`; a lane marks those that
+// beat the worst entry of its list (three instructions each, no LDS) and inserts them one per pass, lowest id first, in
+// a top-k held in registers.  Scores never reach HBM (except through the optional debug output).
+//
+// Bound: Q is read once (HBM) for few candidates; with many the vector instructions per candidate decide.  Measured at
+// 196608 tokens, 32 heads on 8, up to 767 candidates, 2 picks: 2.20 ms with the tile transposed through LDS and a
+// barrier on either side of it, 1.39 ms here; 302060 tokens, up to 147 candidates: 1.12 -> 0.91 ms; 65536 tokens, 16
+// heads, up to 511 candidates, 11 picks: 422 -> 333 us.
 #include "common.h"
 
 namespace moba {
@@ -53,16 +58,19 @@ __device__ __forceinline__ int find_seq(const int* __restrict__ cu, int nseq, in
   return upper_row(cu, nseq, s);
 }
 
-// (up to 12 picks the kernel is held to the registers of three waves per SIMD: it is bound by its vector
-// instructions, which the waves of a SIMD issue in turn while others wait for memory, LDS and barriers)
+// (up to 4 picks the kernel is held to the registers of three waves per SIMD, whose waves issue their vector
+// instructions while others wait; longer lists would spill there: 11 picks, 31 candidates: 422 us held to three, 337 to
+// two)
 template <class E, int KMAX, int D>
-__global__ __launch_bounds__(256, KMAX <= 12 ? 3 : 1) void gate_topk_kernel(
+__global__ __launch_bounds__(256, KMAX <= 4 ? 3 : (KMAX <= 16 ? 2 : 1)) void gate_topk_kernel(
     const typename E::elem* __restrict__ q, const typename E::elem* __restrict__ kbar, const int* __restrict__ cu_seqlens,
     const int* __restrict__ seq_fbase, int* __restrict__ sel, float* __restrict__ scores_out,
     int S, int H, int Hkv, int nseq, int F, int B, int K, int64_t q_tok_stride, int64_t q_head_stride,
     int batch_rows, int64_t q_batch_stride, const int* __restrict__ pair_off, int* __restrict__ cnt, int dense_local) {
   MOBA_ELEM_TYPES(E)
-  __shared__ float sc[4][64][33];
+  // a lane's 32 scores, for the passes that take one of them by its number (rows 136 bytes apart: 8-byte writes, and reads of
+  // one number by all lanes, spread over the banks); later the staged lists and the histograms
+  __shared__ __attribute__((aligned(16))) float sc[4][64][34];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int n = lane & 31, hh = lane >> 5;
   const int tok0 = blockIdx.x * 64;
@@ -103,55 +111,83 @@ __global__ __launch_bounds__(256, KMAX <= 12 ? 3 : 1) void gate_topk_kernel(
 #pragma unroll
       for (int ks = 0; ks < D / 16; ++ks) bq[qb][ks] = *reinterpret_cast<const elem8*>(src + 16 * ks);
     }
+    const elem* const kb_head = kbar + (hc / (H / Hkv)) * D + 8 * hh;
+    elem8 a[D / 16];  // the chunk representatives of the block to come
+    auto load_block = [&](int f0) __attribute__((always_inline)) {
+      const elem* src = kb_head + (int64_t)min(f0 + n, F - 1) * Hkv * D;
+#pragma unroll
+      for (int ks = 0; ks < D / 16; ++ks) a[ks] = *reinterpret_cast<const elem8*>(src + 16 * ks);
+    };
+    constexpr bool kAhead = KMAX <= 16;  // (longer lists leave it no registers: 32 picks 400 us with it, 277 without)
+    if constexpr (kAhead) load_block(flo);
+    float* const mine = &sc[wave][lane][0];
     for (int f0 = flo; f0 < fhi; f0 += 32) {
-      const int fr = min(f0 + n, F - 1);
-      const elem* src = kbar + ((int64_t)fr * Hkv + hc / (H / Hkv)) * D + 8 * hh;
+      if constexpr (!kAhead) load_block(f0);
       f32x16 acc0 = {0}, acc1 = {0};
 #pragma unroll
       for (int ks = 0; ks < D / 16; ++ks) {
-        const elem8 a = *reinterpret_cast<const elem8*>(src + 16 * ks);
-        acc0 = mfma32(a, bq[0][ks], acc0);
-        acc1 = mfma32(a, bq[1][ks], acc1);
+        acc0 = mfma32(a[ks], bq[0][ks], acc0);
+        acc1 = mfma32(a[ks], bq[1][ks], acc1);
       }
+      if constexpr (kAhead) {
+        if (f0 + 32 < fhi) load_block(f0 + 32);  // (travels while this block is gone through)
+      }
+      // Lane (n, hh) holds the scores of chunks 8*(e/4) + 4*hh + e%4 for tokens n (acc0) and 32 + n (acc1).  Swapping
+      // acc1 of the lower half with acc0 of the upper one gives lane l token l: chunks 8*(e/4) + e%4 in acc0 and
+      // 4 more than that in acc1.
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        const int ch = 8 * (e >> 2) + 4 * hh + (e & 3);
-        sc[wave][n][ch] = acc0[e];
-        sc[wave][32 + n][ch] = acc1[e];
+        const auto r = __builtin_amdgcn_permlane32_swap(float_bits(acc0[e]), float_bits(acc1[e]), false, false);
+        acc0[e] = __builtin_bit_cast(float, (uint32_t)r[0]);
+        acc1[e] = __builtin_bit_cast(float, (uint32_t)r[1]);
       }
-      __syncthreads();
-      if (f0 == flo || scores_out) {  // (uniform) the first candidates: every one of them enters the list
+      auto score = [&](int j) __attribute__((always_inline)) {  // of chunk f0 + j (j a constant once unrolled)
+        return (j & 4) ? acc1[4 * (j >> 3) + (j & 3)] : acc0[4 * (j >> 3) + (j & 3)];
+      };
+      const int lo = max(fb - f0, 0), hi = min(fb + c - f0, 32);  // chunks f0 + lo .. f0 + hi - 1 are the token's to pick
+      auto to_lds = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int g = 0; g < 8; ++g) {
+          *reinterpret_cast<float2*>(mine + 8 * (g >> 1) + 2 * (g & 1)) = make_float2(acc0[2 * g], acc0[2 * g + 1]);
+          *reinterpret_cast<float2*>(mine + 8 * (g >> 1) + 4 + 2 * (g & 1)) = make_float2(acc1[2 * g], acc1[2 * g + 1]);
+        }
+      };
+      if (scores_out) {  // (uniform)
+        to_lds();
+        for (int j = lo; j < hi; ++j)
+          if (head_ok) scores_out[((int64_t)s * H + h) * F + f0 + j] = mine[j];
+      }
+      if (f0 == flo) {  // (uniform) the first candidates: every one of them enters the list
+        if constexpr (KMAX <= 16) {
+#pragma unroll
+          for (int j = 0; j < 32; ++j) {
+            const float x = score(j);
+            if (j >= lo && j < hi) top.push(x, f0 + j);
+          }
+        } else {  // (32 copies of a long insertion would not fit the instruction cache)
+          to_lds();
 #pragma unroll 4
-        for (int j = 0; j < 32; ++j) {
-          const int f = f0 + j;
-          const float x = sc[wave][lane][j];
-          const bool valid = (f >= fb) && (f < fb + c);
-          if (valid) {
-            top.push(x, f);
-            if (scores_out && head_ok) scores_out[((int64_t)s * H + h) * F + f] = x;
-          }
+          for (int j = 0; j < 32; ++j)
+            if (j >= lo && j < hi) top.push(mine[j], f0 + j);
         }
-      } else {
-        // Later candidates: few beat the worst entry a lane's list holds by now (it only rises), so the lanes
-        // first mark those that do, then insert them in ascending order, one per pass, until no lane has any
-        // left -- a handful of insertions per 32 candidates instead of 32.
-        const float worst = top.val[KMAX - 1];
-        uint32_t beat = 0;
-#pragma unroll 8
-        for (int j = 0; j < 32; ++j) {
-          const int f = f0 + j;
-          const bool valid = (f >= fb) && (f < fb + c);
-          beat |= (valid && sc[wave][lane][j] > worst) ? 1u << j : 0u;
-        }
-        while (__ballot(beat != 0)) {  // (wave-uniform)
-          if (beat) {
-            const int j = __ffs(beat) - 1;
-            beat &= beat - 1;
-            top.push(sc[wave][lane][j], f0 + j);
-          }
+        continue;
+      }
+      // the candidates that beat the list's worst entry as the block begins (it only rises), chunk f0 + j in bit 31 - j;
+      // a -inf or NaN score beats nothing
+      const float worst = top.val[KMAX - 1];
+      uint32_t beat = 0;
+#pragma unroll
+      for (int j = 0; j < 32; ++j) beat = beat + beat + (score(j) > worst ? 1u : 0u);
+      beat &= hi > lo ? (0xffffffffu >> lo) & (0xffffffffu << (32 - hi)) : 0u;
+      if (!__ballot(beat != 0)) continue;  // (wave-uniform)
+      to_lds();
+      while (__ballot(beat != 0)) {  // (wave-uniform) one insertion per lane and pass, in ascending order of the ids
+        if (beat) {
+          const int j = __clz(beat);
+          beat &= ~(0x80000000u >> j);
+          top.push(mine[j], f0 + j);
         }
       }
-      __syncthreads();
     }
   }
   // The four waves hold the lists of four consecutive heads of the same 64 tokens: K ints per (token, head) that
