@@ -240,15 +240,7 @@ __global__ __launch_bounds__(512, 2) void moba_fwd_kernel(const FwdParams<E> p) 
     const float l_tot = sum_xhalf(l_run);
     const float inv = 1.f / l_tot;
     if constexpr (kFixedRef) {
-      // compared as bit patterns (the file is compiled without NaN semantics): infinities, every NaN and
-      // negative sums all read as "too large"; the largest magnitude among the row's accumulators likewise
-      uint32_t worst = 0;
-#pragma unroll
-      for (int db = 0; db < 4; ++db)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) worst = max(worst, float_bits(oacc[db][e]) & 0x7fffffffu);
-      const bool bad = valid_done && (__builtin_bit_cast(uint32_t, l_tot) >= __builtin_bit_cast(uint32_t, kFixedRefMaxSum) ||
-                                      worst >= 0x7f800000u);
+      const bool bad = valid_done && (beyond_fixed_range(l_tot) || any_not_finite(oacc));
       if (__any(bad) && ln == 0) *reinterpret_cast<volatile int*>(smem + kFwdRedoWord) = 1;
     }
     char* stage = smem + (wave_u < 4 ? 2 * kTileBytes + wave_u * 4096 : kFwdVBase + 2 * kTileBytes + (wave_u - 4) * 4096);
@@ -428,7 +420,8 @@ __global__ __launch_bounds__(512, 2) void moba_fwd_kernel(const FwdParams<E> p) 
     id_word ^= 1;
     const int64_t id = ((int64_t)(j / kQueueRun) * 8 + queue) * kQueueRun + (j % kQueueRun);
     if (id < (int64_t)tt.hist_bound + tt.self_total) {
-      id3 = (int)id;
+      // (self_first: the self tiles take the first of the numbers drawn)
+      id3 = !tt.self_first ? (int)id : (id < tt.self_total ? (int)id + tt.hist_bound : (int)id - tt.self_total);
       empty_queues = 0;
     } else {
       queue = (queue + 1) & 7;
@@ -935,7 +928,10 @@ extern "C" int moba_fwd_partials_rows(const void* q, const void* k, const void* 
   t.key_split_log2 = key_split_log2;
   t.part_stride = (int)(S * H * (K + 1));
   t.xcd_block_log2 = fwd_xcd_block_log2(total);
-  t.self_first = key_split > 1;
+  // Which kind of tile comes first: the longer one, so that short tiles are left for the end.  History tiles have the
+  // chunk's keys (or a part of them); self tiles up to the chunk's, unless an attention chunk is longer than a chunk --
+  // a dense prefix -- which shows in there being too few of them to cover the tokens otherwise.
+  t.self_first = key_split > 1 || (int64_t)N * B < S;
   t.chunk_direct = chunk_direct;
   t.self_skip = self_tile_skip; t.q_shift = (int)q_tok_shift;
   hipStream_t st = (hipStream_t)stream;

@@ -351,15 +351,7 @@ __global__ __launch_bounds__(NW * 64, (FwdTileShape<D, NW>::kWavesPerSimd)) void
   all_keys(std::true_type{});
   float l_tot = sum_xhalf(l_run);
   {
-    // compared as bit patterns (the file is compiled without NaN semantics): infinities, every NaN and negative sums
-    // all read as "too large"; the largest magnitude among the row's accumulators likewise
-    uint32_t worst = 0;
-#pragma unroll
-    for (int db = 0; db < kDb; ++db)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) worst = max(worst, float_bits(oacc[db][e]) & 0x7fffffffu);
-    const bool bad = row_valid && (__builtin_bit_cast(uint32_t, l_tot) >= __builtin_bit_cast(uint32_t, kFixedRefMaxSum) ||
-                                   worst >= 0x7f800000u);
+    const bool bad = row_valid && (beyond_fixed_range(l_tot) || any_not_finite(oacc));
     volatile int* flags = reinterpret_cast<volatile int*>(smem + Shape::kFlags);
     const bool any_bad = __any(bad);
     if (lane == 0) flags[wave] = any_bad ? 1 : 0;
