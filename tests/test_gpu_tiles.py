@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 import torch
 
+from oracle import moba_oracle as O
 from test_gpu_queued import test_queued_kernels_against_the_dense_oracle as queued_case
 
 pytestmark = pytest.mark.gpu
@@ -126,3 +127,23 @@ def test_overflow_in_any_dimension_is_found(rows, tile_rows):
     # partial result, result): 2 * 3 * 2^-9 * 4.5 = 5.3e-2 at most; in the mean (values of about 0.8, roundings of either
     # sign, half a rounding on average) below 2 * 3 * 2^-10 * 0.8 = 4.7e-3.
     assert err.max() < 5.3e-2 and err.mean() < 4.7e-3, (err.max().item(), err.mean().item())
+
+
+@pytest.mark.parametrize("S,H,B,D", [
+    (20, 3, 1, 128), (50, 1, 7, 64), (900, 2, 127, 128), (1100, 2, 300, 128), (2400, 1, 777, 64),   # fewer and more than
+    (9000, 1, 4096, 128), (5000, 4, 1024, 128),          # eight tokens per lane; one workgroup of 1024, a chunk that needs two stages
+    (3000, 37, 100, 128), (33000, 2, 8, 128), (8200, 9, 8, 64),   # many workgroups; very many short chunks (two stages)
+])
+def test_chunk_mean_forms(S, H, B, D):
+    """Every form of the chunk mean gives the rounded exact mean, whatever its number of threads and token lanes."""
+    from moba_amd import moba_efficient as E
+    print("mean case", S, H, B, D, flush=True)
+    g = torch.Generator().manual_seed(S)
+    k = torch.randn((S, H, D), generator=g).to(torch.bfloat16)
+    plan = E.make_plan([0, S], B, 3, device="cuda")
+    want = O.chunk_mean(k, [0, S], B)
+    clear = torch.full((1000,), 7, dtype=torch.int32, device="cuda")
+    got = E.chunk_mean(k.cuda(), plan, clear=clear)
+    assert torch.equal(got.cpu().view(torch.int16), want.view(torch.int16)) and int(clear.abs().max()) == 0
+    strided = k.transpose(0, 1).contiguous().cuda().transpose(0, 1)      # [heads, tokens, dim] seen token-first
+    assert torch.equal(E.chunk_mean(strided, plan), got)
