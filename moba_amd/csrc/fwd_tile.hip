@@ -375,7 +375,8 @@ __global__ __launch_bounds__(NW * 64, (FwdTileShape<D, NW>::kWavesPerSimd)) void
       l_tot = sum_xhalf(l_run);
       if (p.redo && tid == 0) {  // (listed for a caller that asks which tiles these were)
         const int at = __hip_atomic_fetch_add(p.redo, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        p.redo[1 + at] = t.id;
+        // (every part of a cut tile counts: more of them than the array has entries are counted only)
+        if (at < p.t.hist_bound + p.t.self_total) p.redo[1 + at] = t.id;
       }
     }
   }

@@ -147,3 +147,36 @@ def test_chunk_mean_forms(S, H, B, D):
     assert torch.equal(got.cpu().view(torch.int16), want.view(torch.int16)) and int(clear.abs().max()) == 0
     strided = k.transpose(0, 1).contiguous().cuda().transpose(0, 1)      # [heads, tokens, dim] seen token-first
     assert torch.equal(E.chunk_mean(strided, plan), got)
+
+
+def test_list_of_tiles_computed_again_is_bounded(tile_rows, monkeypatch):
+    """With history tiles cut along their keys more parts than tiles can leave the fixed reference's range: they are all
+    counted, and nothing is written behind the list (here, and in every call, the end of the scratch allocation)."""
+    from moba_amd import moba_efficient as E
+    S, H, B, topk = 8192, 1, 4096, 2
+    tile_rows(128)
+    cu_t = torch.tensor([0, S], dtype=torch.int32, device="cuda")
+    plan = E.make_plan(cu_t, B, topk)
+    g = E._geometry(plan, E._lib.load(), H, 128, 2)
+    entries = g.scratch_ints - 9
+    guard = g.split * (g.bound + g.self_tiles) * 4
+    assert g.split * (S - B) // 128 > entries     # (every token of the second chunk attends the first: full tiles)
+    monkeypatch.setattr(g, "ws_bytes", g.ws_bytes + guard)
+    monkeypatch.setattr(E, "KEEP_SCRATCH", True)
+    # scores that rise along the keys: every part's first 32 keys are far below its last ones
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    q, k, v = (torch.randn((S, H, 128), generator=gen, device="cuda") for _ in range(3))
+    q = q.abs() + 1
+    k = k * 0.1 + torch.arange(S, device="cuda")[:, None, None] % 512 * (8.0 / 512)
+    q, k, v = (x.to(torch.bfloat16) for x in (q, k, v))
+    torch.use_deterministic_algorithms(True)
+    try:
+        E._run_forward(q, k, v, plan)
+    finally:
+        torch.use_deterministic_algorithms(False)
+    redo = E.last_scratch["redo"]
+    whole = torch.empty(0, dtype=torch.uint8, device="cuda").set_(redo.untyped_storage())
+    torch.cuda.synchronize()
+    assert redo[0] > entries, (redo[0].item(), entries)
+    assert redo[1:].min() >= 0 and redo[1:].max() < g.bound + g.self_tiles * H
+    assert (whole[g.ws_bytes - guard:g.ws_bytes] == 255).all()
