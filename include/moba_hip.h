@@ -342,7 +342,12 @@ int moba_bwd(const void* dout, const void* q, const void* k, const void* v, cons
 int moba_tail_splits(int B, int Hkv, int rep, int nq, int Skv);
 int moba_tail(const void* q, const void* k, const void* v, void* out, float* part_o, float* part_lse, int B, int H,
               int Hkv, int nq, int Skv, int D, const int64_t* strides, float scale, int dtype, void* stream);
-/* The same for one token (q [B,H,D]; H/Hkv at most 32; splits = moba_decode_splits()). */
+/* The same for many tokens per head, on the forward kernel's causal tiles: no scratch, probabilities rounded to the
+ * element type.  strides, in elements, multiples of 8: {q batch, q head, q token, k/v batch, k/v head, k/v token}, the
+ * last at most 2^23; scale > 0. */
+int moba_tail_tiles(const void* q, const void* k, const void* v, void* out, int B, int H, int Hkv, int nq, int Skv,
+                    int D, const int64_t* strides, float scale, int dtype, void* stream);
+/* One token by moba_tail (q [B,H,D]; H/Hkv at most 32; splits = moba_decode_splits()). */
 int moba_decode_splits(int B, int Hkv, int Skv);
 int moba_decode(const void* q, const void* k, const void* v, void* out, float* part_o, float* part_lse, int B, int H,
                 int Hkv, int Skv, int D, int64_t q_stride_b, int64_t q_stride_h, int64_t kv_stride_b,

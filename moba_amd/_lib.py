@@ -59,6 +59,7 @@ _SIGNATURES = {
     "moba_mfma_probe": (c_int, [c_void_p, c_void_p, c_int, c_int, c_void_p]),
     "moba_tail_splits": (c_int, [c_int] * 5),
     "moba_tail": (c_int, [c_void_p] * 6 + [c_int] * 6 + [c_strides, c_float, c_int, c_void_p]),
+    "moba_tail_tiles": (c_int, [c_void_p] * 4 + [c_int] * 6 + [c_strides, c_float, c_int, c_void_p]),
     "moba_decode_splits": (c_int, [c_int, c_int, c_int]),
     "moba_decode": (c_int, [c_void_p] * 6 + [c_int] * 5 + [c_int64] * 4 + [c_float, c_int, c_void_p]),
 }

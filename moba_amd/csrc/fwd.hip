@@ -801,15 +801,10 @@ extern "C" int moba_fwd_tile_rows(void) { return kFwdTileRows; }
 constexpr int kMaxKeySplit = 8;
 // workgroups of the forward kernel: resident ones drawing from the queues (> 0), or one per tile id (< 0, see
 // moba_fwd_partials)
-static int fwd_xcd_block_log2(int64_t total) {  // runs of at most an eighth of an XCD's share of the ids
-  int b = 0;
-  while (b < 6 && (128LL << b) <= total) ++b;
-  return b;
-}
 static int64_t fwd_grid(int64_t total, int cus, int tile_rows) {
   int64_t grid = ((int64_t)cus + 7) / 8 * 8;
   if (tile_rows != kFwdTileRows || total < 8 * grid) {
-    const int64_t run = 8LL << fwd_xcd_block_log2(total);
+    const int64_t run = 8LL << tile_xcd_block_log2(total);
     grid = -((total + run - 1) / run * run);
   }
   return grid;
@@ -927,7 +922,7 @@ extern "C" int moba_fwd_partials_rows(const void* q, const void* k, const void* 
   if (!set_layout(t, strides)) return MOBA_ERR_ARG;
   t.key_split_log2 = key_split_log2;
   t.part_stride = (int)(S * H * (K + 1));
-  t.xcd_block_log2 = fwd_xcd_block_log2(total);
+  t.xcd_block_log2 = tile_xcd_block_log2(total);
   // Which kind of tile comes first: the longer one, so that short tiles are left for the end.  History tiles have the
   // chunk's keys (or a part of them); self tiles up to the chunk's, unless an attention chunk is longer than a chunk --
   // a dense prefix -- which shows in there being too few of them to cover the tokens otherwise.

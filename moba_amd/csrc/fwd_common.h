@@ -48,6 +48,12 @@ __device__ __forceinline__ bool beyond_fixed_range(float l_tot) {
 
 constexpr float kRescaleThreshold = 8.f;  // log2 units: the running max may lag the true max by this much
 
+// One workgroup per tile: ids reach the XCDs in runs of at most an eighth of an XCD's share of the ids (log2)
+inline int tile_xcd_block_log2(int64_t total) {
+  int b = 0;
+  while (b < 6 && (128LL << b) <= total) ++b;
+  return b;
+}
 // one workgroup per tile (fwd_tile.hip); head_dim 128 with tile_rows 128 or 256, or 64 with 128.  Returns an error code
 // of common.h.
 template <class E>

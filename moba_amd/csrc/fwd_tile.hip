@@ -50,7 +50,10 @@ __device__ __forceinline__ int tile_sw(int row) {
   return D == 128 ? ((row & 3) << 2) ^ ((row >> 2) & 3) : ((row & 2) << 1) | ((row >> 2) & 3);
 }
 
-template <class E, int D, int NW>
+// kTail: the queries are the last tokens of their sequences against a key/value cache (moba_tail_tiles below).  The
+// tiles follow from sizes alone, all sequences in one launch; TileTables then holds, besides heads and strides,
+//   S: query tokens per sequence, N: tiles per head of a sequence, q_shift: keys before the first query token
+template <class E, int D, int NW, bool kTail>
 __global__ __launch_bounds__(NW * 64, (FwdTileShape<D, NW>::kWavesPerSimd)) void fwd_tile_kernel(const FwdParams<E> p) {
   MOBA_ELEM_TYPES(E)
   using Shape = FwdTileShape<D, NW>;
@@ -65,7 +68,19 @@ __global__ __launch_bounds__(NW * 64, (FwdTileShape<D, NW>::kWavesPerSimd)) void
   // tiles, whichever kind takes longer first: workgroups start in the order of their ids ----
   Tile t;
   int key_part = 0;
-  {
+  int seq = 0, row0 = 0;  // kTail: sequence, first of its query tokens
+  if constexpr (kTail) {
+    const int logical = logical_tile_id(p.t.xcd_block_log2);
+    if (logical >= p.t.self_total) return;
+    const int sh = logical / p.t.N;
+    seq = sh / p.t.H;
+    row0 = (p.t.N - 1 - (logical - sh * p.t.N)) * kRows;  // (longest first)
+    t.id = logical;
+    t.h = sh - seq * p.t.H;
+    t.row_count = min(kRows, p.t.S - row0);
+    t.nkeys = p.t.q_shift + row0 + t.row_count;
+    t.direct = 1;
+  } else {
     int logical = logical_tile_id(p.t.xcd_block_log2);
     const int ks = p.t.key_split_log2;
     const int parts_end = p.t.hist_bound << ks;
@@ -96,7 +111,7 @@ __global__ __launch_bounds__(NW * 64, (FwdTileShape<D, NW>::kWavesPerSimd)) void
     const int key = Shape::kSlabRows * (NW * i + wave) + ld_kin;
     ld_off[i] = (uint32_t)(key * row_bytes + (ld_pc ^ tile_sw<D>(key)) * 16);
   }
-  const int64_t kv_off = kv_tok_bytes(p.t, t.kv_tok0) + (h / p.t.rep) * p.t.kv_head_b;
+  const int64_t kv_off = (kTail ? seq * p.t.kv_batch_b : kv_tok_bytes(p.t, t.kv_tok0)) + (h / p.t.rep) * p.t.kv_head_b;
   const char* k_head = (const char*)p.k + kv_off;
   const char* v_head = (const char*)p.v + kv_off;
   auto issue = [&](const char* head, int kt, uint32_t dst) __attribute__((always_inline)) {
@@ -140,14 +155,24 @@ __global__ __launch_bounds__(NW * 64, (FwdTileShape<D, NW>::kWavesPerSimd)) void
 
   // ---- this lane's row, its Q^T operand ----
   const int r = wave * 32 + n;
-  decode_tile_rows(p.t, wave, r, decode_tile_row_entry(p.t, r, t), t);
+  const char* q_row;
+  if constexpr (kTail) {
+    const int row = row0 + min(r, t.row_count - 1);
+    t.dest = (seq * p.t.S + row) * p.t.H + h;
+    t.limit = p.t.q_shift + row;
+    t.wave_min_limit = p.t.q_shift + row0 + min(wave * 32, t.row_count - 1);
+    q_row = (const char*)p.q + seq * p.t.q_batch_b + row * p.t.q_tok_b;
+  } else {
+    decode_tile_rows(p.t, wave, r, decode_tile_row_entry(p.t, r, t), t);
+    q_row = (const char*)p.q + q_tok_bytes(p.t, t.tok);
+  }
   const int dest = t.dest + key_part * p.t.part_stride;  // (part 0 for a self tile)
   const int limit = t.limit;
   const int min_limit = __builtin_amdgcn_readfirstlane(t.wave_min_limit);
   const bool row_valid = r < t.row_count;
   elem8 bq[kKs];
   {
-    const elem* src = reinterpret_cast<const elem*>((const char*)p.q + q_tok_bytes(p.t, t.tok) + h * p.t.q_head_b) + 8 * hh;
+    const elem* src = reinterpret_cast<const elem*>(q_row + h * p.t.q_head_b) + 8 * hh;
 #pragma unroll
     for (int s8 = 0; s8 < kKs; ++s8) bq[s8] = *reinterpret_cast<const elem8*>(src + 16 * s8);
   }
@@ -389,7 +414,7 @@ __global__ __launch_bounds__(NW * 64, (FwdTileShape<D, NW>::kWavesPerSimd)) void
     char* wrow = stage + n * 128 + 8 * hh;
     const int wsw = (n >> 1) & 7;
     elem* const o_base = t.direct ? p.out : p.part_o;
-    if (row_valid && hh == 0) {
+    if (!kTail && row_valid && hh == 0) {
       const float l2 = m_run + fast_log2(l_tot);
       if (t.direct) p.lse[dest] = l2 * 0.6931471805599453f;
       else p.part_lse[dest] = l2;
@@ -421,21 +446,83 @@ __global__ __launch_bounds__(NW * 64, (FwdTileShape<D, NW>::kWavesPerSimd)) void
   }
 }
 
-template <class E, int D, int NW>
+template <class E, int D, int NW, bool kTail>
 static int launch(const FwdParams<E>& p, int64_t workgroups, hipStream_t st) {
   using Shape = FwdTileShape<D, NW>;
   static bool allowed[kMaxDevices];
-  if (!allow_dynamic_lds((const void*)fwd_tile_kernel<E, D, NW>, Shape::kLds, allowed)) return MOBA_ERR_LAUNCH;
-  hipLaunchKernelGGL((fwd_tile_kernel<E, D, NW>), dim3((unsigned)workgroups), dim3(NW * 64), Shape::kLds, st, p);
+  if (!allow_dynamic_lds((const void*)fwd_tile_kernel<E, D, NW, kTail>, Shape::kLds, allowed)) return MOBA_ERR_LAUNCH;
+  hipLaunchKernelGGL((fwd_tile_kernel<E, D, NW, kTail>), dim3((unsigned)workgroups), dim3(NW * 64), Shape::kLds, st, p);
   return MOBA_OK;
 }
 
 template <class E>
 int launch_fwd_tiles(const FwdParams<E>& p, int head_dim, int tile_rows, int64_t workgroups, hipStream_t st) {
-  if (head_dim == 64) return launch<E, 64, 4>(p, workgroups, st);
-  return tile_rows == 128 ? launch<E, 128, 4>(p, workgroups, st) : launch<E, 128, 8>(p, workgroups, st);
+  if (head_dim == 64) return launch<E, 64, 4, false>(p, workgroups, st);
+  return tile_rows == 128 ? launch<E, 128, 4, false>(p, workgroups, st) : launch<E, 128, 8, false>(p, workgroups, st);
 }
 template int launch_fwd_tiles<Bf16>(const FwdParams<Bf16>&, int, int, int64_t, hipStream_t);
 template int launch_fwd_tiles<F16>(const FwdParams<F16>&, int, int, int64_t, hipStream_t);
 
+// Rows per tile of moba_tail_tiles, for `row_blocks` blocks of 128 query tokens in all or `tall` of 256.  Tall tiles move half
+// the bytes from L2 to LDS, but one fills a compute unit and a short one half of it.  In units of a full round of tall
+// tiles (one per unit), measured at 32 and 16 heads, 40000 keys: a full round of short ones (two per unit) 1.035, up to
+// one per unit 0.49 to 0.58, above that 0.82 to 1.035; up to half a round of tall ones 0.71, the rest 0.75 to 1.
+//   2048 tokens, 32 heads, 34816 keys: 1.04 ms short, 0.975 tall; 4 sequences x 1100 tokens, 16 heads, 40000 keys: 1.60
+//   short, 1.88 tall; 2048 tokens, 8 heads, 40000 keys: 0.54 short, 0.79 tall
+static int tail_tile_rows(int64_t blocks, int64_t tall, int cus) {
+  auto cost = [](int64_t n, int64_t round, double full, double few, double low) {
+    const int64_t rest = n % round;
+    const double part = (double)rest / (double)round;
+    return full * (double)(n / round) + (rest == 0 ? 0. : (2 * rest <= round ? few : low + (full - low) * part));
+  };
+  return cost(blocks, 2 * (int64_t)cus, 1.035, 0.55, 0.6) < cost(tall, cus, 1., 0.71, 0.5) ? 128 : 256;
+}
+
+template <class E>
+static int launch_tail_tiles(const void* q, const void* k, const void* v, void* out, const TileTables& t, float scale,
+                             int64_t workgroups, int tile_rows, hipStream_t st) {
+  LaunchCheck launch_check;
+  FwdParams<E> p = {};
+  p.q = (const typename E::elem*)q; p.k = (const typename E::elem*)k; p.v = (const typename E::elem*)v;
+  p.out = (typename E::elem*)out;
+  p.t = t;
+  p.scale_log2 = scale * 1.4426950408889634f;
+  const int rc = tile_rows == 128 ? launch<E, 128, 4, true>(p, workgroups, st) : launch<E, 128, 8, true>(p, workgroups, st);
+  return rc != MOBA_OK ? rc : launch_check.result();
+}
+
 }  // namespace moba
+
+using namespace moba;
+
+// The last nq tokens of B sequences against their keys and values, on the causal tiles of fwd_tile_kernel: token j sees
+// keys 0 .. Skv - nq + j.  q, k and v are read in place, all sequences in one launch: one launch per sequence left most
+// of the chip idle whenever heads * nq / 256 was below the number of compute units, and copied q and the result.
+// 4 sequences x 1024 tokens, 8 heads, 9000 keys: 836 -> 166 us; 4 x 2048, 32 heads, 9000 keys: 1771 -> 993 us; one of 2048
+// tokens, 32 heads, 34816 keys: 1018 -> 961 us (bound by the products: 1.18 PFLOP/s).
+extern "C" int moba_tail_tiles(const void* q, const void* k, const void* v, void* out, int B, int H, int Hkv, int nq,
+                               int Skv, int D, const int64_t* strides, float scale, int dtype, void* stream) {
+  if (!q || !k || !v || !out || !strides) return MOBA_ERR_ARG;
+  if (B <= 0 || H <= 0 || Hkv <= 0 || nq <= 0 || nq > Skv || H % Hkv != 0 || !(scale > 0.f)) return MOBA_ERR_ARG;
+  if (D != kHeadDim || (dtype != MOBA_DTYPE_BF16 && dtype != MOBA_DTYPE_F16)) return MOBA_ERR_UNSUPPORTED;
+  if (((uintptr_t)q & 15) || ((uintptr_t)k & 15) || ((uintptr_t)v & 15) || ((uintptr_t)out & 15)) return MOBA_ERR_ARG;
+  for (int i = 0; i < 6; ++i)
+    if (strides[i] < 0 || (strides[i] & 7)) return MOBA_ERR_ARG;  // 16-byte accesses
+  if (strides[5] > (1 << 23)) return MOBA_ERR_ARG;                // (a key tile's byte offsets fit 31 bits)
+  const int64_t heads = (int64_t)B * H;
+  if (heads >= 0x7fffffffLL || heads * nq >= 0x7fffffffLL) return MOBA_ERR_LIMIT;
+  const int cus = resident_compute_units();
+  if (cus <= 0) return MOBA_ERR_LAUNCH;
+  const int tile_rows = tail_tile_rows(heads * (((int64_t)nq + 127) / 128), heads * (((int64_t)nq + 255) / 256), cus);
+  const int64_t tiles = ((int64_t)nq + tile_rows - 1) / tile_rows, total = heads * tiles;
+  TileTables t = {};
+  t.S = nq; t.N = (int)tiles; t.q_shift = Skv - nq; t.self_total = (int)total;
+  t.H = H; t.Hkv = Hkv; t.rep = H / Hkv; t.K1 = 1;
+  t.q_batch_b = strides[0] * 2; t.q_head_b = strides[1] * 2; t.q_tok_b = strides[2] * 2;
+  t.kv_batch_b = strides[3] * 2; t.kv_head_b = strides[4] * 2; t.kv_tok_b = strides[5] * 2;
+  t.xcd_block_log2 = tile_xcd_block_log2(total);
+  const int64_t run = 8LL << t.xcd_block_log2, workgroups = (total + run - 1) / run * run;
+  if (workgroups >= 0x7fffffffLL) return MOBA_ERR_LIMIT;
+  return dtype == MOBA_DTYPE_F16 ? launch_tail_tiles<F16>(q, k, v, out, t, scale, workgroups, tile_rows, (hipStream_t)stream)
+                                 : launch_tail_tiles<Bf16>(q, k, v, out, t, scale, workgroups, tile_rows, (hipStream_t)stream);
+}

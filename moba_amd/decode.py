@@ -2,7 +2,7 @@
 branch, moba/wrapper.py:76-82, which calls flash_attn_func in the reference: every cached key is
 visible to a new token up to its own position).  One token or a few: the HIP decode kernel reads K and V of
 the cache once, in place, for all query rows of a key/value head.  Many tokens (chunked prefill against a cache):
-the forward attention kernel's causal tiles on the tail of the sequence."""
+the forward attention kernel's causal tiles on the tail of the sequences."""
 
 from __future__ import annotations
 
@@ -43,6 +43,17 @@ def _rows_in_place(t: torch.Tensor) -> torch.Tensor:
     return t if ok else t.contiguous()
 
 
+def _steps(t: torch.Tensor):
+    """Strides of batch, head and token; 0 for a dimension of one entry, whose stride says nothing."""
+    return [s if n > 1 else 0 for s, n in zip(t.stride()[:3], t.shape)]
+
+
+def _rows_addressable(t: torch.Tensor) -> bool:
+    """Whether the causal tiles can read a [B,heads,tokens,D] tensor in place: contiguous rows, 16-byte friendly strides."""
+    s = _steps(t)
+    return t.stride(3) == 1 and not (s[0] | s[1] | s[2]) & 7 and s[2] <= 1 << 23 and t.data_ptr() % 16 == 0
+
+
 def _tail(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, scaling: Optional[float]) -> torch.Tensor:
     """[B,H,q_len,D] against [B,Hkv,Skv,D] -> [B,q_len,H,D] on the decode kernel: the cache is read once for all
     query rows of a key/value head."""
@@ -78,11 +89,41 @@ def decode_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor
     return _tail(query, key, value, scaling)
 
 
-# Up to this many new tokens the decode kernel takes them, more go to the forward kernel's causal tiles.  Measured at 512
-# new tokens, decode kernel / tiles: 0.62 / 0.75 ms (34816 keys, 32 heads on 8), 1.51 / 1.78 ms (4 sequences of 20000
-# keys), 0.056 / 0.18 ms (8000 keys, 8 heads on 8); at 2048 tokens the tiles do 34816 keys in 1.0 ms, which the decode
-# kernel's 0.45 PFLOP/s would take 2.3 ms for.
-TAIL_TOKENS = 512
+def _tail_tiles(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, scaling: Optional[float]) -> torch.Tensor:
+    """As _tail, on the forward kernel's causal tiles, all sequences in one launch."""
+    lib = _lib.load()
+    b, h, q_len, d = query.shape
+    hkv, skv = key.shape[1], key.shape[2]
+    q, k, v = (t if _rows_addressable(t) else t.contiguous() for t in (query, key, value))
+    if _steps(k) != _steps(v):
+        k, v = k.contiguous(), v.contiguous()
+    out = torch.empty((b, q_len, h, d), dtype=query.dtype, device=query.device)
+    scale = float(scaling) if scaling is not None else d ** -0.5
+    dtype = _lib.DTYPE_F16 if query.dtype == torch.float16 else _lib.DTYPE_BF16
+    _lib.check(lib.moba_tail_tiles(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), b, h, hkv, q_len, skv, d,
+                                   (ctypes.c_int64 * 6)(*_steps(q), *_steps(k)), scale, dtype,
+                                   torch.cuda.current_stream(query.device).cuda_stream), "moba_tail_tiles")
+    return out
+
+
+def _takes_tiles(b: int, h: int, hkv: int, q_len: int) -> bool:
+    """Whether the causal tiles beat the decode kernel, by the number of 32-row blocks that one walks (rows of a key/value
+    head packed together, whole workgroups of 32, 64 or 128 rows) and of 128-row tiles of the other, both times the keys.
+    At 40000 keys a block takes 1.5 us; tiles take 540 us up to about one per compute unit and 2.25 us each in the long
+    run.  Decode kernel / tiles in us: 512 tokens, 32 heads on 8: 681 / 542; 256 tokens: 367 / 540; 4 sequences of 40
+    tokens: 405 / 584; of 100: 787 / 585; 4 x 4096 tokens, 1 head: 741 / 549; 4 x 2048: 402 / 551.  (Up to 16 tokens it is
+    always the decode kernel, whose probabilities are not rounded to the element type.)"""
+    rows = h // hkv * q_len
+    unit = 32 if rows <= 32 else 64 if rows <= 64 else 128
+    blocks = b * hkv * -(-rows // unit) * (unit // 32)
+    tiles = b * h * -(-q_len // 128)
+    return q_len > 16 and blocks > max(288, tiles * 3 // 2)
+
+
+# A single sequence of at least this many tiles of 256 rows goes to the forward kernel with resident workgroups, which
+# reads its tiles' tables: 32768 tokens, 32 heads, 131072 keys: 50.7 ms there, 51.2 on _tail_tiles; with 2048 tiles (8192
+# tokens, 64 heads) 13.72 and 13.74 ms at 65536 keys, 3.10 and 2.83 ms at 16384.
+RESIDENT_TILES = 4096
 
 
 _TAIL_TABLES = {}  # (kv_len, row tiles skipped, device) -> int32 tables of the causal tiles of a sequence's tail
@@ -111,8 +152,10 @@ def chunk_decode_attention(query: torch.Tensor, key: torch.Tensor, value: torch.
                          "keys and a whole number of query heads per key/value head")
     b, h, q_len, d = query.shape
     hkv, kv_len = key.shape[1], key.shape[2]
-    if q_len <= TAIL_TOKENS:
+    if not _takes_tiles(b, h, hkv, q_len) or (scaling is not None and not scaling > 0):
         return _tail(query, key, value, scaling)
+    if h * (q_len // 256) < RESIDENT_TILES:
+        return _tail_tiles(query, key, value, scaling)
     from . import moba_efficient as E
     lib = _lib.load()
     dev = query.device

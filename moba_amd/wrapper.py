@@ -126,7 +126,7 @@ def moba_layer(
         from .decode import decode_attention
         out = decode_attention(query, key, value, scaling)
     elif q_len < kv_len and dropout == 0.0 and _hip_decode(moba_impl, query, key, value, several=True):
-        # several new tokens against the cache: the decode kernel per token, or the forward kernel's causal tiles
+        # several new tokens against the cache: the decode kernel, or the forward kernel's causal tiles
         from .decode import chunk_decode_attention
         out = chunk_decode_attention(query, key, value, scaling)
     else:

@@ -170,3 +170,54 @@ def test_decode_kernel_keeps_small_probabilities():
         p = torch.exp2(k[0, 0, :, 0].double())
         want = (p[1:].sum() / p.sum()).item()
         assert abs(out.float().mean().item() - want) < 2.0 ** -7 * want, (dtype, out.float().mean().item(), want)
+
+
+@pytest.mark.parametrize("B,H,Hkv,Skv,q_len,dtype,spread", [
+    (1, 2, 1, 129, 129, torch.bfloat16, 1.0),       # one row in the last tile, no key before the first token
+    (3, 1, 1, 700, 127, torch.float16, 1.0),
+    (2, 6, 2, 1000, 300, torch.bfloat16, 8.0),      # tiles computed again with a running maximum
+    (1, 5, 5, 65, 64, torch.float16, 8.0),
+    (2, 32, 4, 777, 760, torch.bfloat16, 1.0),      # tiles of 256 rows, the last of 248
+    (2, 32, 4, 1100, 1024, torch.float16, 8.0),
+])
+@pytest.mark.parametrize("layout", ["cache", "fused", "expanded"])
+def test_causal_tiles_of_new_tokens(B, H, Hkv, Skv, q_len, dtype, spread, layout):
+    """The causal tiles read q, k and v in place, whatever their strides, and all sequences in one launch.  Errors: values of up
+    to about 4.5, the probabilities and the result each rounded to the element type, to half a step of a significand of 8
+    (bf16) or 11 bits: relative to the value at most u = 2^-8 or 2^-11 (just above a power of two), so at most 2 * 4.5 * u
+    together, and on average (half of that, over values of about 0.8) below 0.8 * u."""
+    import moba_amd.decode as D
+    print("new-token tiles", B, H, Hkv, Skv, q_len, dtype, spread, layout, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(Skv + q_len)
+    randn = lambda *s: torch.randn(s, generator=g, device="cuda")
+    q = (randn(B, q_len, H, 128) * spread).to(dtype).transpose(1, 2)
+    if layout == "cache":        # preallocated for more tokens
+        k = (randn(B, Hkv, Skv + 9, 128) * spread).to(dtype)[:, :, :Skv]
+        v = randn(B, Hkv, Skv + 9, 128).to(dtype)[:, :, :Skv]
+    elif layout == "fused":      # slices of one projection, heads beside heads
+        kv = randn(B, Skv, 2 * Hkv, 128).to(dtype)
+        kv[:, :, :Hkv] *= spread
+        k, v = kv[:, :, :Hkv].transpose(1, 2), kv[:, :, Hkv:].transpose(1, 2)
+    else:                        # one prompt under every sequence; values in another layout than keys
+        k = (randn(1, Hkv, Skv, 128) * spread).to(dtype).expand(B, -1, -1, -1)
+        v = randn(1, Skv, Hkv, 128).to(dtype).transpose(1, 2).expand(B, -1, -1, -1)
+    out = D._tail_tiles(q, k, v, None)
+    err = (out.float() - _ref_tail(q, k, v, 128 ** -0.5)).abs()
+    u = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    assert out.shape == (B, q_len, H, 128) and torch.isfinite(out.float()).all()
+    assert err.max() < 2 * 4.5 * u and err.mean() < 0.8 * u, (err.max().item(), err.mean().item())
+
+
+def test_routes_of_new_tokens(monkeypatch):
+    """Few tokens always take the decode kernel; the kernel for very many gives the tiles' result bit for bit."""
+    import moba_amd.decode as D
+    for b, h, hkv in ((1, 1, 1), (64, 32, 32), (8, 64, 4), (3, 45, 5), (1, 128, 1)):
+        assert not any(D._takes_tiles(b, h, hkv, n) for n in range(1, 17))
+    g = torch.Generator(device="cuda").manual_seed(8)
+    q = torch.randn((2, 32, 1500, 128), generator=g, device="cuda").to(torch.bfloat16)
+    k, v = (torch.randn((2, 8, 1777, 128), generator=g, device="cuda").to(torch.bfloat16) for _ in range(2))
+    assert D._takes_tiles(2, 32, 8, 1500)
+    tiles = D.chunk_decode_attention(q, k, v)
+    assert torch.equal(tiles, D._tail_tiles(q, k, v, None))
+    monkeypatch.setattr(D, "RESIDENT_TILES", 0)
+    assert torch.equal(tiles, D.chunk_decode_attention(q, k, v))
