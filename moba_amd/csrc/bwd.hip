@@ -63,7 +63,7 @@ struct BwdParams {
   uint32_t hk_magic;  // n / (H*K1) == (n * hk_magic) >> hk_shift for every n < 2^31
   uint32_t hk_shift;
   int* queues;        // [16] tile counters, one per XCD, of the dQ kernel and of the dK/dV kernel; zero at the start
-  // Small problems: every key tile of the dK/dV kernel is cut into dkv_split parts (its rows' stages in equal
+  // Small problems: every key tile of the dK/dV kernel is cut into dkv_split parts (its heads' stages in equal
   // shares) that run as tiles of their own and leave fp32 sums in part_dkv [tiles * dkv_split][2][128][128],
   // which bwd_dkv_reduce_kernel adds up in a fixed order.  dkv_split = 1: whole tiles, dk and dv written directly.
   float* part_dkv;
@@ -518,7 +518,9 @@ __global__ __launch_bounds__(256) void bwd_dq_reduce_kernel(const typename E::el
 // ------------------------------------------------------------------------------------ dK, dV
 // kBatched: q is a batched layout (rows of different batch entries are not an affine function of the token);
 // the common case has no division and no branch in the address of a gathered Q row.
-template <class E, bool kBatched>
+// kParts: tiles cut into dkv_split parts (a form of its own: the other has no scalar registers to
+// spare, 302060 tokens, 32 heads, forward and backward: 104.8 ms with both in one, 104.3 before, and no slower apart).
+template <class E, bool kBatched, bool kParts>
 __global__ __launch_bounds__(256, 1) void bwd_dkv_kernel(const BwdParams<E> p) {
   MOBA_ELEM_TYPES(E)
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -541,7 +543,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_kernel(const BwdParams<E> p) {
   __syncthreads();
   const int drawn = __builtin_amdgcn_readfirstlane(*reinterpret_cast<const int*>(smem + kDkvIdSlot));
   const int64_t id = (((int64_t)(drawn / kXcdBlock) << ql) + queue) * kXcdBlock + (drawn % kXcdBlock);
-  const int split = p.dkv_split;
+  const int split = kParts ? p.dkv_split : 1;
   if (id >= (int64_t)p.kv_total * split) {
     queue = (queue + 1) & qmask;
     if (++empty_queues > qmask) break;
@@ -799,10 +801,36 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_kernel(const BwdParams<E> p) {
     }
   };
 
+  // This part's share of the stages of all heads, one head's behind the other's: a head costs a part the start of a
+  // pipeline (lookups, first copies, first products: 3 us, two stages' time), so a part should meet few of them.  (A
+  // share of every head's stages instead: 271 us where this takes 253, 20480 tokens in five sequences, 8 heads on 2, chunk 512.)
+  int skip = 0, left = 0x7fffffff;  // stages before the part's first one, and how many it has
+  if constexpr (kParts) {
+    int total = nself * rep;
+    if (fid >= 0) {
+      const int* ends = p.t.seg_off + fid * H + hkv * rep;
+      int before = table_load(ends);
+      for (int i = 1; i <= rep; ++i) {
+        const int end = table_load(ends + i);
+        total += (end - before + TQ - 1) / TQ;
+        before = end;
+      }
+    }
+    skip = (int)((int64_t)total * part / split);
+    left = (int)((int64_t)total * (part + 1) / split) - skip;
+    // (vector registers, of which there are some left, hold the two across the stage loop: scalar ones are short there)
+    asm volatile("" : "+v"(skip));
+    asm volatile("" : "+v"(left));
+  }
   for (int hq = hkv * rep; hq < (hkv + 1) * rep; ++hq) {
   select_head(hq);
-  // this part's share of the head's stages
-  const int q_first = (int)((int64_t)ntile * part / split), q_end = (int)((int64_t)ntile * (part + 1) / split);
+  int q_first = 0, q_end = ntile;
+  if constexpr (kParts) {
+    q_first = min(__builtin_amdgcn_readfirstlane(skip), ntile);
+    q_end = q_first + min(__builtin_amdgcn_readfirstlane(left), ntile - q_first);
+    skip -= q_first;
+    left -= q_end - q_first;
+  }
   if (q_end == q_first) continue;  // (uniform)
   set_lane_bases();
   __syncthreads();  // every wave is done with the LDS stages of the previous head
@@ -868,7 +896,7 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_kernel(const BwdParams<E> p) {
   wait_vmem();  // (the copies past the last stage: nothing may be on its way into LDS when the workgroup ends)
   }  // query heads
 
-  if (split > 1) {
+  if constexpr (kParts) {
     // this part's sums, unscaled, in fp32: [dk, dv][key of the tile][128]
     float* dst = p.part_dkv + (int64_t)unit * (2 * TM * kHeadDim) + (wave * 32 + n) * kHeadDim + 4 * hh;
 #pragma unroll
@@ -964,11 +992,13 @@ static int launch_bwd(const void* dout, const void* q, const void* k, const void
   p.hk_shift = 31 + lg;
   p.hk_magic = (uint32_t)((1ull << p.hk_shift) / hk + 1);
 
-  static bool allowed_dq[kMaxDevices], allowed_dkv[2][kMaxDevices];  // one set per element type
-  const bool batched = t.batch_rows != 0;
+  static bool allowed_dq[kMaxDevices], allowed_dkv[4][kMaxDevices];  // one set per element type
+  typedef void (*DkvKernel)(const BwdParams<E>);
+  static const DkvKernel dkv_kernels[4] = {bwd_dkv_kernel<E, false, false>, bwd_dkv_kernel<E, false, true>,
+                                           bwd_dkv_kernel<E, true, false>, bwd_dkv_kernel<E, true, true>};
+  const int form = (t.batch_rows != 0 ? 2 : 0) + (dkv_split > 1 ? 1 : 0);
   if (!allow_dynamic_lds((const void*)bwd_dq_kernel<E>, kBwdDqLds, allowed_dq) ||
-      !(batched ? allow_dynamic_lds((const void*)bwd_dkv_kernel<E, true>, kBwdDkvLds, allowed_dkv[1])
-                : allow_dynamic_lds((const void*)bwd_dkv_kernel<E, false>, kBwdDkvLds, allowed_dkv[0])))
+      !allow_dynamic_lds((const void*)dkv_kernels[form], kBwdDkvLds, allowed_dkv[form]))
     return MOBA_ERR_LAUNCH;
   const int64_t rows = S * H;
   hipLaunchKernelGGL(bwd_delta_kernel<E>, dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, st, (const elem*)dout,
@@ -980,8 +1010,7 @@ static int launch_bwd(const void* dout, const void* q, const void* k, const void
                        (const elem*)part_dq, sel, (elem*)dq, sum_rows, K + 1, 1 << t.key_split_log2, rows, mrg_start,
                        mrg_prefix, nranges, H);
   }
-  if (batched) hipLaunchKernelGGL((bwd_dkv_kernel<E, true>), dim3((unsigned)grid_kv), dim3(256), kBwdDkvLds, st, p);
-  else hipLaunchKernelGGL((bwd_dkv_kernel<E, false>), dim3((unsigned)grid_kv), dim3(256), kBwdDkvLds, st, p);
+  hipLaunchKernelGGL(dkv_kernels[form], dim3((unsigned)grid_kv), dim3(256), kBwdDkvLds, st, p);
   if (dkv_split > 1)
     hipLaunchKernelGGL(bwd_dkv_reduce_kernel<E>, dim3((unsigned)p.kv_total * 16), dim3(256), 0, st, p);
   return launch_check.result();

@@ -385,6 +385,42 @@ def test_history_tiles_of_dq_cut_into_parts():
         assert e.max() < MAX_ABS * scale and e.mean() < MEAN_ABS, (e.max().item(), e.mean().item())
 
 
+@pytest.mark.parametrize("heads,kv_heads,lens,B,topk", [
+    (6, 2, [4500, 300, 1201], 256, 3),     # three heads over four or fewer parts: parts within a head and across heads
+    (8, 1, [5000], 640, 2),                # eight heads, ragged stages, four parts of two heads each
+    (7, 1, [4096, 1], 4096, 1),            # no history at all: only causal rows; a tile of one key
+])
+def test_parts_of_a_key_tile_span_heads(heads, kv_heads, lens, B, topk, monkeypatch):
+    """A part of a key tile takes a range of the stages of all query heads together.  dk and dv are fp32 sums rounded once
+    either way, so a part-wise sum may only move values across a rounding boundary: in norm far below 2^-9 of the
+    result, and no element by more than one step of 2^-7 of the largest."""
+    from moba_amd import _lib, moba_attn_varlen_gqa
+    lib = _lib.load()
+    print("parts across heads", heads, kv_heads, lens, B, topk, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(heads)
+    S = sum(lens)
+    q, k, v, do = (torch.randn((S, n, 128), generator=g, device="cuda").to(torch.bfloat16)
+                   for n in (heads, kv_heads, kv_heads, heads))
+    cu_t = torch.tensor([0] + np.cumsum(lens).tolist(), dtype=torch.int32, device="cuda")
+
+    def run():   # (a new plan each time: a plan keeps the sizes of its scratch)
+        from moba_amd import plan as P
+        P._BY_VALUE.clear()
+        P._BY_TENSOR.clear()
+        kg, vg = (x.clone().requires_grad_(True) for x in (k, v))
+        moba_attn_varlen_gqa(q, kg, vg, cu_t, max(lens), B, topk).backward(do)
+        return kg.grad.float(), vg.grad.float()
+
+    cut = run()
+    real, asked = lib.moba_bwd_dkv_scratch_bytes, []
+    monkeypatch.setattr(lib, "moba_bwd_dkv_scratch_bytes", lambda *a: asked.append(real(*a)) or 0)
+    whole = run()
+    assert asked and (asked[0] > 0 or "MOBA_RESIDENT_CUS" in os.environ)
+    for a, b in zip(cut, whole):
+        assert torch.isfinite(a).all()
+        assert (a - b).norm() < 2.0 ** -9 * b.norm() and (a - b).abs().max() <= 2.0 ** -7 * b.abs().max()
+
+
 def test_key_tiles_cut_into_parts():
     """With few key tiles (here 16384 tokens x 1 key/value head = 128 tiles on 256 compute units) the dK/dV kernel
     cuts every tile into parts that leave fp32 sums for a reduction kernel: grouped-query heads, three sequences
