@@ -521,7 +521,7 @@ __global__ __launch_bounds__(256) void bwd_dq_reduce_kernel(const typename E::el
 // kParts: tiles cut into dkv_split parts (a form of its own: the other has no scalar registers to
 // spare, 302060 tokens, 32 heads, forward and backward: 104.8 ms with both in one, 104.3 before, and no slower apart).
 template <class E, bool kBatched, bool kParts>
-__global__ __launch_bounds__(256, 1) void bwd_dkv_kernel(const BwdParams<E> p) {
+__device__ __forceinline__ void bwd_dkv_tiles(const BwdParams<E>& p) {
   MOBA_ELEM_TYPES(E)
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -927,6 +927,15 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_kernel(const BwdParams<E> p) {
 #undef MOBA_PIN
 }
 
+template <class E, bool kBatched>
+__global__ __launch_bounds__(256, 1) void bwd_dkv_kernel(const BwdParams<E> p) {
+  bwd_dkv_tiles<E, kBatched, false>(p);
+}
+template <class E, bool kBatched>
+__global__ __launch_bounds__(256, 1) void bwd_dkv_parts_kernel(const BwdParams<E> p) {
+  bwd_dkv_tiles<E, kBatched, true>(p);
+}
+
 // dk, dv of the 128-key tiles from the fp32 sums of their parts, added in the order of the parts.
 // Sixteen workgroups per tile; a thread owns four consecutive elements of one key (coalesced 16-byte loads).
 template <class E>
@@ -994,8 +1003,8 @@ static int launch_bwd(const void* dout, const void* q, const void* k, const void
 
   static bool allowed_dq[kMaxDevices], allowed_dkv[4][kMaxDevices];  // one set per element type
   typedef void (*DkvKernel)(const BwdParams<E>);
-  static const DkvKernel dkv_kernels[4] = {bwd_dkv_kernel<E, false, false>, bwd_dkv_kernel<E, false, true>,
-                                           bwd_dkv_kernel<E, true, false>, bwd_dkv_kernel<E, true, true>};
+  static const DkvKernel dkv_kernels[4] = {bwd_dkv_kernel<E, false>, bwd_dkv_parts_kernel<E, false>,
+                                           bwd_dkv_kernel<E, true>, bwd_dkv_parts_kernel<E, true>};
   const int form = (t.batch_rows != 0 ? 2 : 0) + (dkv_split > 1 ? 1 : 0);
   if (!allow_dynamic_lds((const void*)bwd_dq_kernel<E>, kBwdDqLds, allowed_dq) ||
       !allow_dynamic_lds((const void*)dkv_kernels[form], kBwdDkvLds, allowed_dkv[form]))

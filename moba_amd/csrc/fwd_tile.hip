@@ -17,8 +17,8 @@
 //
 // Heads of 64 elements (the only kernel that takes them unpadded) need half the LDS and 147 registers: three workgroups
 // to a compute unit.  The exponentials weigh twice as much against the products there, so the rate in FLOP/s stays
-// below that of 128 elements, but half the work is gone: 8191 tokens, 32 heads, chunk 512, whole operator: 401 us padded to 128, 217 us here; 131072 tokens, chunk
-// 4096, 12 chunks: 64.8 -> 43.6 ms.
+// below that of 128 elements, but half the work is gone: 8191 tokens, 32 heads, chunk 512, whole operator: 401 us padded
+// to 128, 205 us here; 131072 tokens, chunk 4096, 12 chunks: 64.8 -> 43.6 ms.
 //
 // Softmax: relative to the row maximum of the tile's first 32 keys (see fwd.hip); a tile in which a row leaves the
 // range that is safe is computed again on the spot with a running maximum, by the same workgroup.

@@ -53,3 +53,14 @@ def test_generated_dkv_kernel_keeps_its_distance():
         dist, count, where = asm_check.min_result_distance(asm, sym)
         assert count == 80          # 2 chains x 8 steps in each of the five places phase A is instantiated
         assert dist >= asm_check.MIN_DISTANCE, where
+
+
+@pytest.mark.skipif(not os.path.exists(build.HIPCC), reason="needs hipcc")
+def test_generated_dkv_parts_kernel_keeps_its_distance():
+    asm = asm_check.device_assembly(build.HIPCC, build.FLAGS, os.path.join(build.CSRC, "bwd.hip"))
+    symbols = asm_check.dkv_kernel_symbols(asm, "bwd_dkv_parts_kernel")
+    assert len(symbols) == 4
+    for sym in symbols:
+        dist, count, where = asm_check.min_result_distance(asm, sym)
+        assert count == 80 and dist >= asm_check.MIN_DISTANCE, where
+    assert all(sym in asm_check.check_dkv_kernel(asm) for sym in symbols)
