@@ -115,8 +115,11 @@ def _takes_tiles(b: int, h: int, hkv: int, q_len: int) -> bool:
     always the decode kernel, whose probabilities are not rounded to the element type.)"""
     rows = h // hkv * q_len
     unit = 32 if rows <= 32 else 64 if rows <= 64 else 128
-    blocks = b * hkv * -(-rows // unit) * (unit // 32)
+    groups = -(-rows // unit)
+    blocks = b * hkv * groups * (unit // 32)
     tiles = b * h * -(-q_len // 128)
+    if b > 65535 or hkv * groups > 65535 or rows > 1 << 20:   # (more than the decode kernel's grid takes)
+        return q_len > 16 or h // hkv not in SUPPORTED_GROUP_SIZES
     return q_len > 16 and blocks > max(288, tiles * 3 // 2)
 
 

@@ -213,6 +213,13 @@ def test_routes_of_new_tokens(monkeypatch):
     import moba_amd.decode as D
     for b, h, hkv in ((1, 1, 1), (64, 32, 32), (8, 64, 4), (3, 45, 5), (1, 128, 1)):
         assert not any(D._takes_tiles(b, h, hkv, n) for n in range(1, 17))
+    # more sequences than the decode kernel's grid takes
+    assert D._takes_tiles(70000, 1, 1, 17) and D._takes_tiles(70000, 3, 1, 5) and not D._takes_tiles(65535, 1, 1, 17)
+    q, k, v = (torch.randn((66000, 1, n, 128), device="cuda").to(torch.bfloat16) for n in (17, 18, 18))
+    out = D.chunk_decode_attention(q, k, v)
+    some = [0, 1, 32767, 65535, 65536, 65999]
+    assert (out[some].float() - _ref_tail(q[some], k[some], v[some], 128 ** -0.5)).abs().max() < 2e-2
+    del q, k, v, out
     g = torch.Generator(device="cuda").manual_seed(8)
     q = torch.randn((2, 32, 1500, 128), generator=g, device="cuda").to(torch.bfloat16)
     k, v = (torch.randn((2, 8, 1777, 128), generator=g, device="cuda").to(torch.bfloat16) for _ in range(2))
