@@ -17,9 +17,11 @@
 // 16 x 8191 keys, fp16: 95 us = 5.6 TB/s (101); 4 x 20000 keys, 5 tokens: 64 us = 5.1 TB/s (342, once per token).
 // Beyond 128 rows per key/value head it is bound by its own instruction chain (one wave per SIMD), 0.45 PFLOP/s.
 //
-// Precision: the scores' products are exact, their sums fp32.  A probability is fed to the second product as the
-// sum of two elements (its rounded value and the rounded rest), so that it keeps 16 (bf16) or 22 (fp16) bits: the
-// matrix pipe has the time, and one element alone would double the error of the result.
+// Precision: the scores' products are exact, their sums fp32.  A probability is fed to the second product as the sum
+// of three elements (its rounded value, the rounded rest, and the rest of that), which hold all 24 bits of it: the matrix
+// pipe has the time, and one element alone would double the error of the result.  Beyond kTailExactTokens tokens two
+// elements (16 or 22 bits): there the products are the bound, and the other kernel for such calls, the causal tiles,
+// rounds to one.
 //
 //   tail_partial_kernel   part_o[row, split, :] (normalised, fp32), part_lse (log2 domain); one split: out itself
 //   tail_merge_kernel     out[row, :]
@@ -35,6 +37,7 @@ constexpr int kTailRedRow = kHeadDim + 4;                     // floats per row 
 constexpr int kTailRedStats = 4 * 32 * kTailRedRow * 4;       // byte offset of [4 waves][32 rows] maxima, then sums
 static_assert(kTailRedStats + 2 * 4 * 32 * 4 <= kTailLds, "the waves' sums fit the stages");
 constexpr int kTailMaxSplits = 128;
+constexpr int kTailExactTokens = 16;  // up to so many new tokens the probabilities keep their 24 bits
 
 template <class E>
 struct TailParams {
@@ -189,18 +192,29 @@ __global__ __launch_bounds__(256, 1) void tail_partial_kernel(const TailParams<E
     }
     const float ref = m_run - TailShift<E>::value;
     elem8 hi[2], lo[2];
+    float rest[16];
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
       const float pe = fast_exp2(s[e] - ref);
       l_run += pe;
       const elem h = (elem)pe;
+      const float r = pe - (float)h;
+      const elem l = (elem)r;
       hi[e >> 3][e & 7] = h;
-      lo[e >> 3][e & 7] = (elem)(pe - (float)h);
+      lo[e >> 3][e & 7] = l;
+      rest[e] = r - (float)l;
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) oacc[i & 3] = mfma32(va[i], hi[i >> 2], oacc[i & 3]);
 #pragma unroll
     for (int i = 0; i < 8; ++i) oacc[i & 3] = mfma32(va[i], lo[i >> 2], oacc[i & 3]);
+    if (p.nq <= kTailExactTokens) {
+      elem8 last[2];
+#pragma unroll
+      for (int e = 0; e < 16; ++e) last[e >> 3][e & 7] = (elem)rest[e];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) oacc[i & 3] = mfma32(va[i], last[i >> 2], oacc[i & 3]);
+    }
     if (it + 2 < mine) {
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // every fragment of this stage is in registers
       issue(it + 2, it & 1);
