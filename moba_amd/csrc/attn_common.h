@@ -118,6 +118,24 @@ static __global__ void zero_queues_kernel(int* queues, int* also) {
   if (also && threadIdx.x == 0) *also = 0;
 }
 
+// Whether any of the lane's accumulators is an infinity or not a number.  Compared as bit patterns (the forward
+// kernels are compiled without NaN semantics): signed for the positive ones, unsigned for the negative ones, half a v_max3 per element
+// and comparison -- this runs in the open at the end of a tile.
+template <int DB>
+__device__ __forceinline__ bool any_not_finite(const f32x16 (&acc)[DB]) {
+  int top = 0;
+  uint32_t bottom = 0;
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int e = 0; e < 16; e += 2) {
+      const uint32_t a = float_bits(acc[db][e]), b = float_bits(acc[db][e + 1]);
+      top = max(max(top, (int)a), (int)b);
+      bottom = max(max(bottom, a), b);
+    }
+  return top >= 0x7f800000 || bottom >= 0xff800000u;
+}
+
 // Workgroup ids are dealt round-robin to the 8 XCDs; give each XCD runs of 1 << block_log2 (at most kXcdBlock)
 // consecutive logical tiles so that tiles sharing a K/V chunk share an L2.  (A grid of few tiles takes shorter
 // runs: whole runs of 64 would leave some XCDs with twice the tiles of others, or with none.)

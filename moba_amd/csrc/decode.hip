@@ -23,6 +23,11 @@
 // elements (16 or 22 bits): there the products are the bound, and the other kernel for such calls, the causal tiles,
 // rounds to one.
 //
+// Values that are not finite: a probability of 0 for a key that a row does not see still meets the key's value in the
+// products, and 0 * Inf and the split probabilities' parts times Inf are NaN; a maximum that lags overflows for values near
+// the end of bf16's range.  A wave whose accumulators are not finite at the end goes through its keys again one by one,
+// in fp32, relative to the exact maximum, every row with the keys it sees only.
+//
 //   tail_partial_kernel   part_o[row, split, :] (normalised, fp32), part_lse (log2 domain); one split: out itself
 //   tail_merge_kernel     out[row, :]
 #include "attn_common.h"
@@ -59,6 +64,7 @@ struct TailParams {
 template <class E> struct TailShift { static constexpr float value = 0.f; };
 template <> struct TailShift<F16> { static constexpr float value = 7.f; };
 constexpr float kTailMaxLag = 8.f;
+constexpr float kTailNoMax = -3e38f;  // before the first visible key (finite: exp2(m - m_new) stays defined)
 
 template <class E>
 __global__ __launch_bounds__(256, 1) void tail_partial_kernel(const TailParams<E> p) {
@@ -144,7 +150,7 @@ __global__ __launch_bounds__(256, 1) void tail_partial_kernel(const TailParams<E
   for (int db = 0; db < 4; ++db)
 #pragma unroll
     for (int e = 0; e < 16; ++e) oacc[db][e] = 0.f;
-  float m_run = -1e30f, l_run = 0.f;  // (finite: exp2(m - m_new) stays defined before the first visible key)
+  float m_run = kTailNoMax, l_run = 0.f;
 
   for (int it = 0; it < mine; ++it) {
     const uint32_t st = (it & 1) * 2 * kTailTile;
@@ -220,6 +226,45 @@ __global__ __launch_bounds__(256, 1) void tail_partial_kernel(const TailParams<E
       issue(it + 2, it & 1);
     }
   }
+  if (__any(any_not_finite(oacc))) {  // (never for values of ordinary size)
+    auto each_key = [&](auto use) __attribute__((always_inline)) {
+      for (int it = 0; it < mine; ++it) {
+        const int key0 = key_lo + (wk + it * wk_n) * kTailKeys, key1 = min(key0 + kTailKeys, key_hi);
+        for (int key = key0; key < key1; ++key) {
+          const elem* kr = (const elem*)(k_head + (int64_t)key * 256) + 8 * hh;
+          float d = 0.f;
+#pragma unroll
+          for (int s8 = 0; s8 < 8; ++s8) {
+            const elem8 x = *reinterpret_cast<const elem8*>(kr + 16 * s8);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) d += (float)bq[s8][e] * (float)x[e];
+          }
+          const float sc = sum_xhalf(d) * p.scale_log2;
+          if (key <= limit) use(key, sc);
+        }
+      }
+    };
+    m_run = kTailNoMax;
+    each_key([&](int, float sc) __attribute__((always_inline)) { m_run = fmaxf(m_run, sc); });
+    const float ref = m_run - TailShift<E>::value;
+    float l = 0.f;
+#pragma unroll
+    for (int db = 0; db < 4; ++db)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) oacc[db][e] = 0.f;
+    each_key([&](int key, float sc) __attribute__((always_inline)) {
+      const float pe = fast_exp2(sc - ref);
+      l += pe;
+      const elem* vr = (const elem*)(v_head + (int64_t)key * 256) + 4 * hh;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const elem4 x = *reinterpret_cast<const elem4*>(vr + 8 * i);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) oacc[i >> 2][4 * (i & 3) + e] += pe * (float)x[e];
+      }
+    });
+    l_run = hh == 0 ? l : 0.f;
+  }
   l_run = sum_xhalf(l_run);
 
   // The waves that hold the same rows meet in LDS.  Element e of lane (n, hh) is O[row n][32*db + 8*(e/4) + 4*hh + e%4].
@@ -258,7 +303,7 @@ __global__ __launch_bounds__(256, 1) void tail_partial_kernel(const TailParams<E
     const int jj = rg / p.rep, gg = rg - jj * p.rep;
     const int64_t orow = ((int64_t)b * p.nq + jj) * (p.Hkv * p.rep) + hkv * p.rep + gg;
     // (a row may see no key of its split: the causal limit; never without another split that it does see)
-    const float inv = ll > 0.f ? 1.f / ll : 0.f;
+    const float inv = ll > 0.f || p.nsplit == 1 ? 1.f / ll : 0.f;
     if (p.nsplit == 1) {
       u32x2 w;
       w[0] = pack2<E>(oo[0] * inv, oo[1] * inv);

@@ -24,24 +24,7 @@ struct FwdParams {
 // accumulator of the row that is not finite (a probability beyond the element type's range -- 2^16 for fp16 --
 // or products with large |v| that left fp32).
 constexpr float kFixedRefMaxSum = 0x1p96f;
-// Whether any of the lane's accumulators is an infinity or not a number.  Compared as bit patterns (the kernels are
-// compiled without NaN semantics): signed for the positive ones, unsigned for the negative ones, half a v_max3 per element
-// and comparison -- this runs in the open at the end of a tile.
-template <int DB>
-__device__ __forceinline__ bool any_not_finite(const f32x16 (&acc)[DB]) {
-  int top = 0;
-  uint32_t bottom = 0;
-#pragma unroll
-  for (int db = 0; db < DB; ++db)
-#pragma unroll
-    for (int e = 0; e < 16; e += 2) {
-      const uint32_t a = float_bits(acc[db][e]), b = float_bits(acc[db][e + 1]);
-      top = max(max(top, (int)a), (int)b);
-      bottom = max(max(bottom, a), b);
-    }
-  return top >= 0x7f800000 || bottom >= 0xff800000u;
-}
-// ... and whether a row's sum of exponentials left the range: infinities, NaNs and negative sums read as too large
+// Whether a row's sum of exponentials left that range: infinities, NaNs and negative sums read as too large
 __device__ __forceinline__ bool beyond_fixed_range(float l_tot) {
   return float_bits(l_tot) >= __builtin_bit_cast(uint32_t, kFixedRefMaxSum);
 }

@@ -30,6 +30,12 @@ def _exact(q, k, v, scale):
     return torch.stack(rows, dim=1)
 
 
+def _close(out, want, dtype, largest=5.0):
+    """Rounded once to the element type: half a step of a significand of 8 or 11 bits at values below `largest`."""
+    bound = 1.05 * largest * 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    return (out.double() - want).abs().max().item() < bound
+
+
 def _partials(q, k, v, scale):
     """moba_tail's result before it is rounded: its splits' partial outputs, put together in float64."""
     from moba_amd import _lib
@@ -67,3 +73,74 @@ def test_probabilities_keep_their_32_bits(dtype, q_len):
     v[:, :, :128] = torch.eye(128, device="cuda", dtype=dtype)
     got, want = _partials(q, k, v, 1.0), _exact(q, k, v, 1.0)
     assert ((got - want).abs() / want).max().item() < 2.0 ** -20
+
+
+@pytest.mark.parametrize("B,H,Hkv,Skv,q_len", [
+    (2, 8, 2, 1000, 3), (1, 4, 4, 40, 16), (1, 32, 8, 1025, 8), (1, 6, 2, 9000, 5), (2, 16, 4, 300, 13),
+    (1, 32, 4, 700, 9)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), float("-inf")])
+def test_a_later_tokens_values_do_not_reach_an_earlier_one(B, H, Hkv, Skv, q_len, dtype, bad):
+    from moba_amd.decode import chunk_decode_attention
+    _note("hidden values", B, H, Hkv, Skv, q_len, dtype, bad)
+    g = torch.Generator(device="cuda").manual_seed(Skv)
+    q, k, v = (_randn(g, B, h, n, 128).to(dtype) for h, n in ((H, q_len), (Hkv, Skv), (Hkv, Skv)))
+    want = _exact(q, k, v, 128 ** -0.5)
+    v[:, :, -1, 5] = bad
+    v[:, :, -2, 7] = bad
+    out = chunk_decode_attention(q, k, v)
+    others = [d for d in range(128) if d not in (5, 7)]
+    assert _close(out[..., others], want[..., others], dtype)
+    assert _close(out[:, :-1, :, 5], want[:, :-1, :, 5], dtype) and _close(out[:, :-2, :, 7], want[:, :-2, :, 7], dtype)
+    for hit in (out[:, -1, :, 5], out[:, -2:, :, 7]):
+        assert torch.isnan(hit).all() if bad != bad else (hit == bad).all()
+    # a key that is not a number: only the tokens that see it
+    v[:, :, -2:] = 1
+    k[:, :, -1] = bad
+    out = chunk_decode_attention(q, k, v)
+    assert torch.isfinite(out[:, :-1].float()).all() and torch.isnan(out[:, -1].float()).any()
+
+
+@pytest.mark.parametrize("B,H,Hkv,Skv,q_len", [(1, 32, 8, 4097, 1), (2, 2, 2, 50, 1), (3, 16, 2, 1000, 4)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_a_visible_infinity_stays_one(B, H, Hkv, Skv, q_len, dtype):
+    """As in fp32 arithmetic: its dimension becomes that infinity, two of opposite signs are not a number, and the other
+    dimensions are what they were."""
+    from moba_amd.decode import chunk_decode_attention
+    _note("visible infinity", B, H, Hkv, Skv, q_len, dtype)
+    g = torch.Generator(device="cuda").manual_seed(Skv)
+    q, k, v = (_randn(g, B, h, n, 128).to(dtype) for h, n in ((H, q_len), (Hkv, Skv), (Hkv, Skv)))
+    want = _exact(q, k, v, 128 ** -0.5)
+    v[:, :, 5, 3], v[:, :, 40, 9] = float("inf"), float("-inf")
+    v[:, :, 2, 100], v[:, :, 33, 100] = float("inf"), float("-inf")
+    out = chunk_decode_attention(q, k, v)
+    assert (out[..., 3] == float("inf")).all() and (out[..., 9] == float("-inf")).all()
+    assert torch.isnan(out[..., 100]).all()
+    others = [d for d in range(128) if d not in (3, 9, 100)]
+    assert _close(out[..., others], want[..., others], dtype)
+
+
+def test_large_values_stay_finite():
+    """Scores that rise by 2^7 after a wave's first keys: sums of 64 products of at most 2^119 fit fp32 with the maximum
+    taken out, and would not with a maximum that lags behind by that factor."""
+    from moba_amd.decode import decode_attention
+    q = torch.zeros((256, 1, 1, 128), device="cuda", dtype=torch.bfloat16)
+    q[..., 0] = 1
+    k = torch.zeros((256, 1, 256, 128), device="cuda", dtype=torch.bfloat16)
+    k[:, :, 128:, 0] = 7.0
+    v = torch.full((256, 1, 256, 128), 2.0 ** 119, device="cuda", dtype=torch.bfloat16)
+    out = decode_attention(q, k, v, 0.6931471805599453)
+    assert (out.double() / 2.0 ** 119 - 1).abs().max().item() < 2.0 ** -8
+
+
+def test_scores_far_below_zero():
+    """Every score below -1e30: the maximum is still found."""
+    from moba_amd.decode import decode_attention
+    g = torch.Generator(device="cuda").manual_seed(5)
+    q = torch.zeros((1, 4, 1, 128), device="cuda", dtype=torch.bfloat16)
+    q[..., 0] = 1e20
+    k = torch.zeros((1, 4, 100, 128), device="cuda", dtype=torch.bfloat16)
+    k[..., 0] = -1e14
+    v = _randn(g, 1, 4, 100, 128).to(torch.bfloat16)
+    out = decode_attention(q, k, v, 1.0)
+    assert _close(out, v.double().mean(2)[:, None], torch.bfloat16)
