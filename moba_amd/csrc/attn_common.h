@@ -315,22 +315,37 @@ __device__ __forceinline__ V4 lds_read_tr(uint32_t addr) {
 // Issued as inline assembly so that completion is tracked by the explicit wait_vmem()
 // before the tile barrier only (the copy must stay in flight across the compute phase).
 // The statement overwrites M0 and says so to the compiler.
+// kStream: the bytes are read once on the chip and need not stay in its caches
+template <bool kStream = false>
 __device__ __forceinline__ void async_copy16(const void* gsrc, uint32_t lds_wave_base) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
-               :
-               : "v"(gsrc), "s"(lds_wave_base)
-               : "memory", "m0");
+  if constexpr (kStream)
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt"
+                 :
+                 : "v"(gsrc), "s"(lds_wave_base)
+                 : "memory", "m0");
+  else
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
+                 :
+                 : "v"(gsrc), "s"(lds_wave_base)
+                 : "memory", "m0");
 }
 // same with the global address split into a wave-uniform base and a per-lane byte offset
+template <bool kStream = false>
 __device__ __forceinline__ void async_copy16_sv(const void* uniform_base, uint32_t lane_off, uint32_t lds_wave_base) {
   const uint64_t b = (uint64_t)uniform_base;
   const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)b);
   const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
   const uint64_t sb = ((uint64_t)hi << 32) | lo;
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               :
-               : "v"(lane_off), "s"(sb), "s"(lds_wave_base)
-               : "memory", "m0");
+  if constexpr (kStream)
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt"
+                 :
+                 : "v"(lane_off), "s"(sb), "s"(lds_wave_base)
+                 : "memory", "m0");
+  else
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :
+                 : "v"(lane_off), "s"(sb), "s"(lds_wave_base)
+                 : "memory", "m0");
 }
 // same for 4 bytes per lane: lane i fills lds_wave_base + 4*i
 __device__ __forceinline__ void async_copy4(const void* gsrc, uint32_t lds_wave_base) {

@@ -3,18 +3,21 @@
 // sees the keys up to its own position Skv - nq + j; grouped-query heads are handled in place; the softmax scale is
 // the caller's.
 //
-// HBM-bound: K and V of the cache are to be read once.  The nq * rep query rows that share a key/value head are the
-// 32 columns of a matrix product (S^T = K Q^T, O^T += V^T P^T with v_mfma_f32_32x32x16), so one pass over the cache
-// serves them all: a kernel that gives every row its own dot products is bound by the vector unit from a handful of
+// HBM-bound: K and V of the cache are to be read once.  The nq * rep query rows that share a key/value head are
+// columns of a matrix product (S^T = K Q^T, O^T += V^T P^T with v_mfma_f32_32x32x16), so that up to 32 of them take one
+// pass over the cache: a kernel that gives every row its own dot products is bound by the vector unit from a handful of
 // rows on, and one that runs once per new token reads the cache that often.  A workgroup takes a range of the keys
-// (a split); its four waves take different keys of it, or different blocks of 32 rows once there are more than 32.
+// (a split); its four waves take different keys of it, or different blocks of 32 rows once there are more than 32 (two or
+// four waves then copy the same keys, from L2); beyond 128 rows further workgroups walk the same range, a pass each.
 // A wave copies its own K and V blocks of 32 keys global -> LDS (two stages of 16 KiB, no barrier: the wait for a
 // block counts the wave's own copies) while it computes the block before: 64 to 128 KiB per compute unit in flight,
 // where about 40 KiB cover the latency at the full rate.  One workgroup per compute unit (128 KiB of LDS); the
 // splits are chosen so that the workgroups come out just below a multiple of the units.
+// Keys that one wave reads alone (up to 32 rows) are copied past the caches: 1 x 65536 keys, 64 heads: 368 us without, 314
+// with (6.8 TB/s); keys that several waves or workgroups read are not: 40000 keys, 128 rows: 69.4 us without, 75.6 with.
 //
-// Measured (32 query heads on 8): 131072 keys, one token: 97 us a call (107 with a vector-unit kernel of 128 splits);
-// 16 x 8191 keys, fp16: 95 us = 5.6 TB/s (101); 4 x 20000 keys, 5 tokens: 64 us = 5.1 TB/s (342, once per token).
+// Measured (32 query heads on 8): 131072 keys, one token: 86 us a call = 6.2 TB/s (108 with a vector-unit kernel of 128
+// splits); 16 x 8191 keys: 84 us = 6.4 TB/s (102); 4 x 20000 keys, 5 tokens: 60 us (348, once per token).
 // Beyond 128 rows per key/value head it is bound by its own instruction chain (one wave per SIMD), 0.45 PFLOP/s.
 //
 // Precision: the scores' products are exact, their sums fp32.  A probability is fed to the second product as the sum
@@ -66,7 +69,8 @@ template <> struct TailShift<F16> { static constexpr float value = 7.f; };
 constexpr float kTailMaxLag = 8.f;
 constexpr float kTailNoMax = -3e38f;  // before the first visible key (finite: exp2(m - m_new) stays defined)
 
-template <class E>
+// kOnce: one workgroup and one wave reads a key's rows (up to 32 query rows per key/value head): they pass the caches by
+template <class E, bool kOnce>
 __global__ __launch_bounds__(256, 1) void tail_partial_kernel(const TailParams<E> p) {
   MOBA_ELEM_TYPES(E)
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -102,19 +106,19 @@ __global__ __launch_bounds__(256, 1) void tail_partial_kernel(const TailParams<E
     if (key0 + kTailKeys <= key_hi) {
       const int64_t off = (int64_t)key0 * 256;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) async_copy16_sv(k_head + off, ld_off[i], kdst + i * 1024);
+      for (int i = 0; i < 8; ++i) async_copy16_sv<kOnce>(k_head + off, ld_off[i], kdst + i * 1024);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) async_copy16_sv(v_head + off, ld_off[i], vdst + i * 1024);
+      for (int i = 0; i < 8; ++i) async_copy16_sv<kOnce>(v_head + off, ld_off[i], vdst + i * 1024);
     } else {  // (keys past the end: the last key again; their scores are masked)
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const int64_t off = (int64_t)min(key0 + 4 * i + ld_kin, key_hi - 1) * 256 + (ld_off[i] & 255);
-        async_copy16(k_head + off, kdst + i * 1024);
+        async_copy16<kOnce>(k_head + off, kdst + i * 1024);
       }
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const int64_t off = (int64_t)min(key0 + 4 * i + ld_kin, key_hi - 1) * 256 + (ld_off[i] & 255);
-        async_copy16(v_head + off, vdst + i * 1024);
+        async_copy16<kOnce>(v_head + off, vdst + i * 1024);
       }
     }
   };
@@ -411,9 +415,11 @@ static int launch_tail(const void* q, const void* k, const void* v, void* out, f
   p.Hkv = Hkv; p.rep = rep; p.Skv = Skv; p.nq = nq;
   p.wr_log2 = ts.wr_log2; p.keys_per_split = ts.keys_per_split; p.nsplit = ts.nsplit;
   p.scale_log2 = scale * 1.4426950408889634f;
-  static bool allowed[kMaxDevices];
-  if (!allow_dynamic_lds((const void*)tail_partial_kernel<E>, kTailLds, allowed)) return MOBA_ERR_LAUNCH;
-  hipLaunchKernelGGL(tail_partial_kernel<E>, dim3(ts.nsplit, Hkv * ts.groups, B), dim3(256), kTailLds, st, p);
+  static bool allowed[2][kMaxDevices];  // one set per element type
+  const bool once = ts.wr_log2 == 0 && ts.groups == 1;
+  const auto kernel = once ? tail_partial_kernel<E, true> : tail_partial_kernel<E, false>;
+  if (!allow_dynamic_lds((const void*)kernel, kTailLds, allowed[once])) return MOBA_ERR_LAUNCH;
+  hipLaunchKernelGGL(kernel, dim3(ts.nsplit, Hkv * ts.groups, B), dim3(256), kTailLds, st, p);
   if (ts.nsplit > 1)
     hipLaunchKernelGGL(tail_merge_kernel<E>, dim3((unsigned)((int64_t)B * nq * Hkv * rep)), dim3(256), 0, st,
                        (const float*)part_o, (const float*)part_lse, (elem*)out, ts.nsplit);
