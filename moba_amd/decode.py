@@ -12,6 +12,7 @@ from typing import Optional
 import torch
 
 from . import _lib
+from .moba_efficient import _aligned
 
 SUPPORTED_GROUP_SIZES = (1, 2, 4, 8)
 
@@ -36,22 +37,33 @@ def chunk_supported(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor)
     return key.shape[1] > 0 and h % key.shape[1] == 0
 
 
-def _rows_in_place(t: torch.Tensor) -> torch.Tensor:
-    """A [B,Hkv,Skv,D] tensor whose key rows are contiguous and D apart, with 16-byte friendly strides."""
-    d = t.shape[3]
-    ok = t.stride(3) == 1 and t.stride(2) == d and t.stride(0) % 8 == 0 and t.stride(1) % 8 == 0 and t.data_ptr() % 16 == 0
-    return t if ok else t.contiguous()
+def _packed(t: torch.Tensor):
+    t = _aligned(t)
+    b, h, n, d = t.shape
+    return t, (h * n * d if b > 1 else 0, n * d if h > 1 else 0, d if n > 1 else 0)
 
 
-def _steps(t: torch.Tensor):
-    """Strides of batch, head and token; 0 for a dimension of one entry, whose stride says nothing."""
-    return [s if n > 1 else 0 for s, n in zip(t.stride()[:3], t.shape)]
+def _placed(t: torch.Tensor, row_step: int = 0):
+    """A [B,heads,tokens,D] tensor as the kernels will read it, and its strides of batch, head and token: untouched where
+    its rows are contiguous (and row_step apart, if given) and everything 16-byte friendly, a packed copy otherwise.
+    The stride of a dimension of one entry says nothing and is 0 here."""
+    b, h, n, _ = t.shape
+    sb, sh, sn, sd = t.stride()
+    steps = (sb if b > 1 else 0, sh if h > 1 else 0, sn if n > 1 else 0)
+    if (sd == 1 and not (steps[0] | steps[1] | steps[2]) & 7 and steps[2] <= 1 << 23 and t.data_ptr() % 16 == 0
+            and (sn == row_step or not row_step or n == 1)):
+        return t, steps
+    return _packed(t)
 
 
-def _rows_addressable(t: torch.Tensor) -> bool:
-    """Whether the causal tiles can read a [B,heads,tokens,D] tensor in place: contiguous rows, 16-byte friendly strides."""
-    s = _steps(t)
-    return t.stride(3) == 1 and not (s[0] | s[1] | s[2]) & 7 and s[2] <= 1 << 23 and t.data_ptr() % 16 == 0
+def _placed_three(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, row_step: int = 0):
+    """query, key and value by _placed, and the strides of the first and of the other two, which share theirs."""
+    q, qs = _placed(query)
+    k, ks = _placed(key, row_step)
+    v, vs = _placed(value, row_step)
+    if ks != vs:
+        (k, ks), (v, vs) = _packed(k), _packed(v)
+    return q, k, v, qs, ks
 
 
 def _tail(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, scaling: Optional[float]) -> torch.Tensor:
@@ -60,11 +72,7 @@ def _tail(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, scaling: 
     lib = _lib.load()
     b, h, q_len, d = query.shape
     hkv, skv = key.shape[1], key.shape[2]
-    qs = query.stride()
-    q = query if (qs[3] == 1 and not (qs[0] | qs[1] | qs[2]) & 7 and query.data_ptr() % 16 == 0) else query.contiguous()
-    k, v = _rows_in_place(key), _rows_in_place(value)
-    if k.stride() != v.stride():
-        k, v = k.contiguous(), v.contiguous()
+    q, k, v, qs, ks = _placed_three(query, key, value, d)
     dev = query.device
     out = torch.empty((b, q_len, h, d), dtype=query.dtype, device=dev)
     rows = b * q_len * h * lib.moba_tail_splits(b, hkv, h // hkv, q_len, skv)
@@ -72,9 +80,8 @@ def _tail(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, scaling: 
     part_o = part.data_ptr()
     scale = float(scaling) if scaling is not None else d ** -0.5
     dtype = _lib.DTYPE_F16 if query.dtype == torch.float16 else _lib.DTYPE_BF16
-    qs, ks = q.stride(), k.stride()
     _lib.check(lib.moba_tail(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), part_o, part_o + rows * d * 4, b, h,
-                             hkv, q_len, skv, d, (ctypes.c_int64 * 5)(qs[0], qs[1], qs[2], ks[0], ks[1]), scale, dtype,
+                             hkv, q_len, skv, d, (ctypes.c_int64 * 5)(*qs, ks[0], ks[1]), scale, dtype,
                              torch.cuda.current_stream(dev).cuda_stream), "moba_tail")
     return out
 
@@ -94,14 +101,12 @@ def _tail_tiles(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, sca
     lib = _lib.load()
     b, h, q_len, d = query.shape
     hkv, skv = key.shape[1], key.shape[2]
-    q, k, v = (t if _rows_addressable(t) else t.contiguous() for t in (query, key, value))
-    if _steps(k) != _steps(v):
-        k, v = k.contiguous(), v.contiguous()
+    q, k, v, qs, ks = _placed_three(query, key, value)
     out = torch.empty((b, q_len, h, d), dtype=query.dtype, device=query.device)
     scale = float(scaling) if scaling is not None else d ** -0.5
     dtype = _lib.DTYPE_F16 if query.dtype == torch.float16 else _lib.DTYPE_BF16
     _lib.check(lib.moba_tail_tiles(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), b, h, hkv, q_len, skv, d,
-                                   (ctypes.c_int64 * 6)(*_steps(q), *_steps(k)), scale, dtype,
+                                   (ctypes.c_int64 * 6)(*qs, *ks), scale, dtype,
                                    torch.cuda.current_stream(query.device).cuda_stream), "moba_tail_tiles")
     return out
 

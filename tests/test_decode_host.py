@@ -1,0 +1,42 @@
+"""How the decode entry points prepare their tensors (no GPU)."""
+
+import torch
+
+
+def _as_strided(shape, strides, offset=0):
+    span = sum((n - 1) * s for n, s in zip(shape, strides)) + 1
+    return torch.arange(span + offset, dtype=torch.float32).to(torch.bfloat16).as_strided(shape, strides, offset)
+
+
+def test_tensors_read_in_place_and_copied():
+    from moba_amd.decode import _placed, _placed_three
+    cases = [  # shape, strides, offset of the address in elements, key rows next to each other asked for, read in place
+        ((2, 4, 10, 128), (5120, 1280, 128, 1), 0, True, True),
+        ((2, 4, 10, 128), (8192, 2048, 128, 1), 0, True, True),       # a slice of a longer cache
+        ((2, 4, 1, 128), (1024, 128, 1, 1), 0, True, True),           # one token: its stride says nothing
+        ((1, 4, 10, 128), (3, 1280, 128, 1), 0, True, True),          # one sequence
+        ((2, 1, 10, 128), (1280, 5, 128, 1), 0, True, True),          # one head
+        ((2, 4, 10, 128), (5120, 128, 512, 1), 0, False, True),       # heads beside heads
+        ((2, 4, 10, 128), (5120, 128, 512, 1), 0, True, False),
+        ((2, 4, 10, 128), (0, 1280, 128, 1), 0, True, True),          # one cache under every sequence
+        ((2, 4, 10, 128), (512, 128, 0, 1), 0, True, False),          # one row under every token
+        ((2, 4, 10, 128), (5120, 1280, 128, 1), 1, True, False),      # an odd address
+        ((2, 4, 10, 128), (5124, 1280, 128, 1), 0, True, False),      # an odd batch stride
+        ((2, 4, 10, 128), (10240, 2560, 256, 2), 0, False, False),    # elements apart
+    ]
+    for shape, strides, offset, rows, kept in cases:
+        t = _as_strided(shape, strides, offset)
+        assert offset or t.data_ptr() % 16 == 0
+        got, steps = _placed(t, 128 if rows else 0)
+        assert (got.data_ptr() == t.data_ptr()) == kept, (shape, strides, offset)
+        assert torch.equal(got, t) and got.data_ptr() % 16 == 0 and got.stride(3) == 1
+        for step, s, n in zip(steps, got.stride(), shape):
+            assert step == (s if n > 1 else 0) and step % 8 == 0
+    # strides that differ only where they say nothing: no copies; others: both packed
+    k = _as_strided((1, 4, 10, 128), (8, 2048, 128, 1))
+    v = _as_strided((1, 4, 10, 128), (8192, 2048, 128, 1))
+    q, k2, v2, qs, ks = _placed_three(k, k, v, 128)
+    assert (q.data_ptr(), k2.data_ptr(), v2.data_ptr()) == (k.data_ptr(), k.data_ptr(), v.data_ptr()) and ks == (0, 2048, 128)
+    v = _as_strided((1, 4, 10, 128), (8192, 1280, 128, 1))
+    q, k2, v2, qs, ks = _placed_three(k, k, v, 128)
+    assert ks == (0, 1280, 128) and qs == (0, 2048, 128) and torch.equal(k2, k) and torch.equal(v2, v)

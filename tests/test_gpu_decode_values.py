@@ -144,3 +144,51 @@ def test_scores_far_below_zero():
     v = _randn(g, 1, 4, 100, 128).to(torch.bfloat16)
     out = decode_attention(q, k, v, 1.0)
     assert _close(out, v.double().mean(2)[:, None], torch.bfloat16)
+
+
+def _odd(t, where):
+    """The same values at other places: strides of one-entry dimensions that are no multiple of 8, or an address that is
+    no multiple of 16."""
+    b, h, n, d = t.shape
+    if where == "address":
+        flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:]
+        return flat.view(t.shape).copy_(t)
+    strides = list(t.contiguous().stride())
+    for i in range(3):
+        if t.shape[i] == 1:
+            strides[i] = 3
+    return torch.empty(t.numel() + 8, dtype=t.dtype, device=t.device).as_strided(t.shape, strides).copy_(t)
+
+
+@pytest.mark.parametrize("B,H,Hkv,Skv,q_len", [
+    (2, 8, 4, 300, 1), (1, 8, 2, 300, 1), (1, 1, 1, 300, 1), (1, 4, 1, 50, 3), (1, 2, 2, 77, 20), (1, 1, 1, 1, 1)])
+@pytest.mark.parametrize("where", ["strides", "address"])
+def test_strides_that_say_nothing_and_odd_addresses(B, H, Hkv, Skv, q_len, where):
+    import moba_amd.decode as D
+    _note("odd layout", B, H, Hkv, Skv, q_len, where)
+    g = torch.Generator(device="cuda").manual_seed(Skv)
+    q, k, v = (_randn(g, B, h, n, 128).to(torch.bfloat16) for h, n in ((H, q_len), (Hkv, Skv), (Hkv, Skv)))
+    for change in ((1, 0, 0), (0, 1, 0), (0, 0, 1), (1, 1, 1)):
+        args = [_odd(t, where) if c else t for t, c in zip((q, k, v), change)]
+        for f in (D.chunk_decode_attention, D._tail_tiles) + ((D.decode_attention,) if q_len == 1 else ()):
+            got = f(*args, None) if f is D._tail_tiles else f(*args)
+            want = f(q, k, v, None) if f is D._tail_tiles else f(q, k, v)
+            assert torch.equal(got, want), (f.__name__, change)
+    # [B, H, D, 1] transposed: the token dimension of one entry has a stride of one element
+    if q_len == 1:
+        assert torch.equal(D.decode_attention(q.transpose(2, 3).contiguous().transpose(2, 3), k, v),
+                           D.decode_attention(q, k, v))
+
+
+def test_a_cache_is_not_copied_for_strides_that_say_nothing():
+    from moba_amd.decode import decode_attention
+    q = torch.zeros((1, 4, 1, 128), device="cuda", dtype=torch.bfloat16)
+    cache = torch.zeros((1, 4, 16384, 128), device="cuda", dtype=torch.bfloat16)
+    k = cache[:, :, :16000]
+    v = torch.zeros_like(cache).as_strided(k.shape, (8, *k.stride()[1:]))
+    decode_attention(q, k, k)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    decode_attention(q, k, v)
+    assert torch.cuda.max_memory_allocated() - before < k.numel()      # (half of one tensor's bytes)
