@@ -66,8 +66,11 @@ def _placed_three(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, r
     return q, k, v, qs, ks
 
 
+MOST_SEQUENCES = 65535  # that a launch of the decode kernel takes: its grid's third dimension
+
+
 def _tail(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, scaling: Optional[float]) -> torch.Tensor:
-    """[B,H,q_len,D] against [B,Hkv,Skv,D] -> [B,q_len,H,D] on the decode kernel: the cache is read once for all
+    """[B,H,q_len,D] against [B,Hkv,Skv,D] -> [B,q_len,H,D] on the decode kernel: the cache is read once for up to 32
     query rows of a key/value head."""
     lib = _lib.load()
     b, h, q_len, d = query.shape
@@ -75,14 +78,19 @@ def _tail(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, scaling: 
     q, k, v, qs, ks = _placed_three(query, key, value, d)
     dev = query.device
     out = torch.empty((b, q_len, h, d), dtype=query.dtype, device=dev)
-    rows = b * q_len * h * lib.moba_tail_splits(b, hkv, h // hkv, q_len, skv)
+    pieces = [(i, min(b - i, MOST_SEQUENCES)) for i in range(0, b or 1, MOST_SEQUENCES)]   # one, but for very many
+    rows = q_len * h * max(n * lib.moba_tail_splits(n, hkv, h // hkv, q_len, skv) for _, n in pieces)
     part = torch.empty(rows * (d + 1), dtype=torch.float32, device=dev)   # partial outputs, then their log-sum-exps
     part_o = part.data_ptr()
     scale = float(scaling) if scaling is not None else d ** -0.5
     dtype = _lib.DTYPE_F16 if query.dtype == torch.float16 else _lib.DTYPE_BF16
-    _lib.check(lib.moba_tail(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), part_o, part_o + rows * d * 4, b, h,
-                             hkv, q_len, skv, d, (ctypes.c_int64 * 5)(*qs, ks[0], ks[1]), scale, dtype,
-                             torch.cuda.current_stream(dev).cuda_stream), "moba_tail")
+    strides = (ctypes.c_int64 * 5)(*qs, ks[0], ks[1])
+    stream = torch.cuda.current_stream(dev).cuda_stream
+    qp, kp, vp, op = q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr()
+    for i, n in pieces:
+        _lib.check(lib.moba_tail(qp + 2 * i * qs[0], kp + 2 * i * ks[0], vp + 2 * i * ks[0], op + 2 * i * q_len * h * d,
+                                 part_o, part_o + rows * d * 4, n, h, hkv, q_len, skv, d, strides, scale, dtype, stream),
+                   "moba_tail")
     return out
 
 

@@ -192,3 +192,17 @@ def test_a_cache_is_not_copied_for_strides_that_say_nothing():
     torch.cuda.reset_peak_memory_stats()
     decode_attention(q, k, v)
     assert torch.cuda.max_memory_allocated() - before < k.numel()      # (half of one tensor's bytes)
+
+
+@pytest.mark.parametrize("q_len,scale", [(1, None), (5, None), (17, -0.1), (3, 0.0)])
+def test_more_sequences_than_one_grid(q_len, scale):
+    """66000 sequences, whatever the number of tokens and the scale."""
+    import moba_amd.decode as D
+    _note("many sequences", q_len, scale)
+    g = torch.Generator(device="cuda").manual_seed(q_len)
+    q, k, v = (_randn(g, 66000, 1, n, 128).to(torch.bfloat16) for n in (q_len, 18, 18))
+    out = D.chunk_decode_attention(q, k, v, scale)
+    some = [0, 1, 32767, 65534, 65535, 65536, 65999]
+    assert _close(out[some], _exact(q[some], k[some], v[some], 128 ** -0.5 if scale is None else scale), torch.bfloat16)
+    if q_len == 1:
+        assert torch.equal(out, D.decode_attention(q, k, v, scale))
