@@ -168,6 +168,8 @@ def chunk_decode_attention(query: torch.Tensor, key: torch.Tensor, value: torch.
                          "keys and a whole number of query heads per key/value head")
     b, h, q_len, d = query.shape
     hkv, kv_len = key.shape[1], key.shape[2]
+    if b == 0:
+        return torch.empty((b, q_len, h, d), dtype=query.dtype, device=query.device)
     if not _takes_tiles(b, h, hkv, q_len) or (scaling is not None and not scaling > 0):
         return _tail(query, key, value, scaling)
     if h * (q_len // 256) < RESIDENT_TILES:

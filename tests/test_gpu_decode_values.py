@@ -194,6 +194,13 @@ def test_a_cache_is_not_copied_for_strides_that_say_nothing():
     assert torch.cuda.max_memory_allocated() - before < k.numel()      # (half of one tensor's bytes)
 
 
+@pytest.mark.parametrize("q_len", [40, 2000])
+def test_no_sequences_at_all(q_len):
+    from moba_amd.decode import chunk_decode_attention
+    q, k = (torch.empty((0, 4, n, 128), device="cuda", dtype=torch.bfloat16) for n in (q_len, 3000))
+    assert chunk_decode_attention(q, k, k).shape == (0, q_len, 4, 128)
+
+
 @pytest.mark.parametrize("q_len,scale", [(1, None), (5, None), (17, -0.1), (3, 0.0)])
 def test_more_sequences_than_one_grid(q_len, scale):
     """66000 sequences, whatever the number of tokens and the scale."""
