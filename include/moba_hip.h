@@ -331,14 +331,14 @@ int moba_bwd(const void* dout, const void* q, const void* k, const void* v, cons
 
 /* Decode: the last nq tokens of every sequence against its key/value cache.  Replaces the
  * flash_attn_func call of the adapter's decode branch, moba/wrapper.py:76-82 (grouped-query heads, bottom-right
- * aligned causal mask: token j of the nq sees the keys up to position Skv - nq + j).  The cache is read once for all
- * the query rows of a key/value head.
- *   q [B,H,nq,D], k, v [B,Hkv,Skv,D]; D contiguous, key rows D apart
+ * aligned causal mask: token j of the nq sees the keys up to position Skv - nq + j).  The cache is read once for up to
+ * 32 query rows (nq * H / Hkv) of a key/value head; from HBM once for up to 128, and once more for every 128 beyond.
+ *   q [B,H,nq,D], k, v [B,Hkv,Skv,D]; D contiguous, key rows D apart; 16-byte aligned
  *   strides: {q batch, q head, q token, k/v batch, k/v head} in elements, multiples of 8
  *   out [B,nq,H,D] elem, contiguous
  *   part_o [B*nq*H*splits, D] fp32 and part_lse [B*nq*H*splits] fp32 scratch,
- *   splits = moba_tail_splits(B, Hkv, H / Hkv, nq, Skv)
- * scale = softmax scale. */
+ *   splits = moba_tail_splits(B, Hkv, H / Hkv, nq, Skv); out and the scratch at any address their elements can have
+ * scale = softmax scale.  B at most 65535. */
 int moba_tail_splits(int B, int Hkv, int rep, int nq, int Skv);
 int moba_tail(const void* q, const void* k, const void* v, void* out, float* part_o, float* part_lse, int B, int H,
               int Hkv, int nq, int Skv, int D, const int64_t* strides, float scale, int dtype, void* stream);

@@ -47,6 +47,11 @@ static_assert(kTailRedStats + 2 * 4 * 32 * 4 <= kTailLds, "the waves' sums fit t
 constexpr int kTailMaxSplits = 128;
 constexpr int kTailExactTokens = 16;  // up to so many new tokens the probabilities keep their 24 bits
 
+// the results and the scratch may lie wherever their elements can
+typedef u32x2 u32x2_any __attribute__((aligned(2)));
+typedef f32x4 f32x4_any __attribute__((aligned(4)));
+typedef float f32x2_any __attribute__((ext_vector_type(2), aligned(4)));
+
 template <class E>
 struct TailParams {
   const typename E::elem* q;
@@ -312,10 +317,11 @@ __global__ __launch_bounds__(256, 1) void tail_partial_kernel(const TailParams<E
       u32x2 w;
       w[0] = pack2<E>(oo[0] * inv, oo[1] * inv);
       w[1] = pack2<E>(oo[2] * inv, oo[3] * inv);
-      *reinterpret_cast<u32x2*>(p.out + orow * kHeadDim + d) = w;
+      *reinterpret_cast<u32x2_any*>(p.out + orow * kHeadDim + d) = w;
     } else {
       const int64_t prow = orow * p.nsplit + split;
-      *reinterpret_cast<f32x4*>(p.part_o + prow * kHeadDim + d) = f32x4{oo[0] * inv, oo[1] * inv, oo[2] * inv, oo[3] * inv};
+      *reinterpret_cast<f32x4_any*>(p.part_o + prow * kHeadDim + d) =
+          f32x4{oo[0] * inv, oo[1] * inv, oo[2] * inv, oo[3] * inv};
       if (d == 0) p.part_lse[prow] = ll > 0.f ? mm - TailShift<E>::value + fast_log2(ll) : -INFINITY;
     }
   }
@@ -341,7 +347,7 @@ __global__ __launch_bounds__(256) void tail_merge_kernel(const float* __restrict
   const float* po = part_o + row * nsplit * kHeadDim + 2 * lane;
   for (int i = wave; i < nsplit; i += 4) {
     const float w = fast_exp2(pl[i] - mm);
-    const float2 x = *reinterpret_cast<const float2*>(po + (int64_t)i * kHeadDim);
+    const f32x2_any x = *reinterpret_cast<const f32x2_any*>(po + (int64_t)i * kHeadDim);
     ll += w;
     o0 += w * x.x;
     o1 += w * x.y;
@@ -435,9 +441,7 @@ extern "C" int moba_tail(const void* q, const void* k, const void* v, void* out,
   if (!q || !k || !v || !out || !part_o || !part_lse || !strides) return MOBA_ERR_ARG;
   if (B <= 0 || H <= 0 || Hkv <= 0 || Skv <= 0 || nq <= 0 || nq > Skv || H % Hkv != 0 || B > 65535) return MOBA_ERR_ARG;
   if (D != kHeadDim || (dtype != MOBA_DTYPE_BF16 && dtype != MOBA_DTYPE_F16)) return MOBA_ERR_UNSUPPORTED;
-  if (((uintptr_t)q & 15) || ((uintptr_t)k & 15) || ((uintptr_t)v & 15) || ((uintptr_t)out & 15) ||
-      ((uintptr_t)part_o & 15))
-    return MOBA_ERR_ARG;
+  if (((uintptr_t)q & 15) || ((uintptr_t)k & 15) || ((uintptr_t)v & 15)) return MOBA_ERR_ARG;
   for (int i = 0; i < 5; ++i)
     if (strides[i] & 7) return MOBA_ERR_ARG;  // 16-byte loads
   const int rep = H / Hkv;

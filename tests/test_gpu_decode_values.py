@@ -213,3 +213,24 @@ def test_more_sequences_than_one_grid(q_len, scale):
     assert _close(out[some], _exact(q[some], k[some], v[some], 128 ** -0.5 if scale is None else scale), torch.bfloat16)
     if q_len == 1:
         assert torch.equal(out, D.decode_attention(q, k, v, scale))
+
+
+def test_the_c_entry_takes_results_at_any_address():
+    """moba_decode writes out and its scratch wherever their elements can lie."""
+    from moba_amd import _lib
+    lib = _lib.load()
+    g = torch.Generator(device="cuda").manual_seed(9)
+    for skv in (60, 3000):                                             # one split, several
+        q, k, v = (_randn(g, 2, h, n, 128).to(torch.bfloat16) for h, n in ((8, 1), (4, skv), (4, skv)))
+        splits = lib.moba_decode_splits(2, 4, skv)
+        got = []
+        for shift in (0, 1):
+            out = torch.zeros(2 * 8 * 128 + 1, dtype=torch.bfloat16, device="cuda")[shift:][:2 * 8 * 128]
+            part_o = torch.zeros(2 * 8 * splits * 128 + 1, dtype=torch.float32, device="cuda")[shift:]
+            part_lse = torch.zeros(2 * 8 * splits + 1, dtype=torch.float32, device="cuda")[shift:]
+            _lib.check(lib.moba_decode(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), part_o.data_ptr(),
+                                       part_lse.data_ptr(), 2, 8, 4, skv, 128, 1024, 128, 4 * skv * 128, skv * 128,
+                                       128 ** -0.5, _lib.DTYPE_BF16, torch.cuda.current_stream().cuda_stream),
+                       "moba_decode")
+            got.append(out.clone())
+        assert torch.equal(*got)
