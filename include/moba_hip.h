@@ -58,7 +58,7 @@ extern "C" {
 
 enum { MOBA_DTYPE_BF16 = 0, MOBA_DTYPE_F16 = 1 };
 
-#define MOBA_ABI_VERSION 116 /* the signatures below; moba_version() returns the number the library was built with */
+#define MOBA_ABI_VERSION 117 /* the signatures below; moba_version() returns the number the library was built with */
 int moba_version(void);
 const char* moba_strerror(int code);
 
@@ -231,14 +231,14 @@ int moba_tile_tables(const int32_t* seg_off, int32_t* tile_off, int32_t* tile_se
  *   queues [8] int32 scratch: the tile counters of the forward kernel, whose workgroups (one per CU) stay
  *              resident and draw tiles from one queue per XCD; the call zeroes them with a kernel of its own.
  *              Calls that overlap in time need their own eight counters each.
- *   redo   [1 + hist_bound + self_tiles * H] int32 scratch, or NULL.  With it, problems large enough for the
- *              resident-workgroup kernel take each tile's softmax relative to one fixed reference per row (the row
- *              maximum of the tile's first 32 keys) instead of a running maximum; a tile in which a row leaves the
- *              range that is safe -- scores that rise more than 96 powers of two above that reference (bf16) or 16
- *              (fp16: a probability beyond the type's range), or accumulators that leave fp32 (products with |v| of
- *              2^31 and more) -- is entered in this list and computed again by the kernel that tracks the maximum
- *              (redo[0] = number of such tiles after the call, normally 0).  The result is within rounding of the
- *              other path's either way.  NULL and small problems: running maximum only.
+ *   redo   [1 + hist_bound + self_tiles * H] int32 scratch, or NULL.  With it each tile's softmax is taken relative to
+ *              one fixed reference per row (the row maximum of the tile's first 32 keys) instead of a running maximum; a
+ *              tile in which a row leaves the range that is safe -- scores that rise more than 96 powers of two above
+ *              that reference (bf16) or 16 (fp16: a probability beyond the type's range), or accumulators that leave
+ *              fp32 (products with |v| of 2^31 and more) -- is computed again with a running maximum.  Problems large
+ *              enough for the resident-workgroup kernel enter such tiles in this list first (redo[0] = number of such
+ *              tiles after the call, normally 0); smaller ones compute them again on the spot and leave the list
+ *              alone.  The result is within rounding of the other form's either way.  NULL: running maximum only.
  *   softmax_scale: the factor on q k^T; 0 (or less) stands for D^-0.5, the reference's only choice
  *              (moba/moba_efficient.py:86).  A caller whose heads are narrower than D pads them with zeros
  *              and passes its own head_dim^-0.5.
@@ -264,7 +264,9 @@ int moba_fwd_partials(const void* q, const void* k, const void* v, void* part_o,
  * (as moba_chunk_mean, moba_gate_topk and moba_fwd_merge do; strides must then be given).  queues is then not used;
  * redo, if given, has redo[0] zeroed by the caller and receives the tiles that were computed again with a running
  * maximum, for information: redo[0] counts every part of a tile cut by key_split, and parts beyond the array's
- * hist_bound + self_tiles * H entries are counted without an entry. */
+ * hist_bound + self_tiles * H entries are counted without an entry.  Those tiles take the fixed reference without a
+ * list too: running_max != 0 asks for the running maximum from the start (and for redo to be left alone), whatever the
+ * tiles. */
 int moba_fwd_partials_rows(const void* q, const void* k, const void* v, void* part_o, float* part_lse,
                            const int32_t* seg_off, const int32_t* tile_off, const int32_t* seg_dest,
                            const int32_t* fchunk_tok, const int32_t* chunk_tok, const int32_t* self_tile_prefix,
@@ -272,7 +274,7 @@ int moba_fwd_partials_rows(const void* q, const void* k, const void* v, void* pa
                            float* lse, int64_t S, int H, int Hkv, int D, int K, int F, int N, int B, int64_t hist_bound,
                            int64_t self_tiles, int key_split, const int64_t* strides, int32_t* queues, int32_t* redo,
                            float softmax_scale, int dtype, int self_tile_skip, int64_t q_tok_shift, int tile_rows,
-                           void* stream);
+                           int running_max, void* stream);
 int moba_fwd_merge(const void* part_o, const float* part_lse, const int32_t* sel, void* out, float* lse, int64_t S,
                    int H, int D, int K, int key_split, const int32_t* mrg_start, const int32_t* mrg_prefix, int nranges,
                    int64_t merge_tokens, int dtype, void* stream);
@@ -344,9 +346,9 @@ int moba_tail(const void* q, const void* k, const void* v, void* out, float* par
               int Hkv, int nq, int Skv, int D, const int64_t* strides, float scale, int dtype, void* stream);
 /* The same for many tokens per head, on the forward kernel's causal tiles: no scratch, probabilities rounded to the
  * element type.  strides, in elements, multiples of 8: {q batch, q head, q token, k/v batch, k/v head, k/v token}, the
- * last at most 2^23; scale > 0. */
+ * last at most 2^23; scale > 0.  running_max: as for moba_fwd_partials_rows. */
 int moba_tail_tiles(const void* q, const void* k, const void* v, void* out, int B, int H, int Hkv, int nq, int Skv,
-                    int D, const int64_t* strides, float scale, int dtype, void* stream);
+                    int D, const int64_t* strides, float scale, int dtype, int running_max, void* stream);
 /* One token by moba_tail (q [B,H,D]; H/Hkv at most 32; splits = moba_decode_splits()). */
 int moba_decode_splits(int B, int Hkv, int Skv);
 int moba_decode(const void* q, const void* k, const void* v, void* out, float* part_o, float* part_lse, int B, int H,

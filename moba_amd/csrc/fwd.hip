@@ -837,7 +837,7 @@ extern "C" int moba_fwd_key_split(int64_t S, int H, int K, int B, int64_t hist_b
 template <class E>
 static int launch_partials(const void* q, const void* k, const void* v, void* part_o, float* part_lse, void* out,
                            float* lse, const TileTables& t, int D, float softmax_scale, int64_t grid, int tile_rows,
-                           int* queues, int* redo, hipStream_t st) {
+                           int* queues, int* redo, int running_max, hipStream_t st) {
   LaunchCheck launch_check;
   FwdParams<E> p;
   p.q = (const typename E::elem*)q; p.k = (const typename E::elem*)k; p.v = (const typename E::elem*)v;
@@ -847,7 +847,9 @@ static int launch_partials(const void* q, const void* k, const void* v, void* pa
   p.scale_log2 = softmax_scale > 0.f ? (float)(1.4426950408889634 * (double)softmax_scale)
                                      : (float)(1.4426950408889634 / sqrt((double)D));
   p.queues = queues;
+  if (running_max) redo = nullptr;
   p.redo = redo;
+  p.running_max = running_max;
   static bool allowed[3][kMaxDevices];  // one set of arrays per element type
   if (grid > 0) {  // resident workgroups drawing from the queues
     hipLaunchKernelGGL(zero_queues_kernel, dim3(1), dim3(8), 0, st, queues, redo);  // a kernel, not a memset: graph safe
@@ -881,7 +883,8 @@ extern "C" int moba_fwd_partials_rows(const void* q, const void* k, const void* 
                                  int64_t S, int H, int Hkv, int D, int K, int F,
                                  int N, int B, int64_t hist_bound, int64_t self_tiles, int key_split,
                                  const int64_t* strides, int32_t* queues, int32_t* redo, float softmax_scale,
-                                 int dtype, int self_tile_skip, int64_t q_tok_shift, int tile_rows, void* stream) {
+                                 int dtype, int self_tile_skip, int64_t q_tok_shift, int tile_rows, int running_max,
+                                 void* stream) {
   if (tile_rows != kFwdTileRows && tile_rows != TM) return MOBA_ERR_ARG;
   if (!q || !k || !v || !part_o || !part_lse || !chunk_tok || !self_tile_prefix || !self_tile_chunk || !queues)
     return MOBA_ERR_ARG;
@@ -931,8 +934,10 @@ extern "C" int moba_fwd_partials_rows(const void* q, const void* k, const void* 
   t.self_skip = self_tile_skip; t.q_shift = (int)q_tok_shift;
   hipStream_t st = (hipStream_t)stream;
   return dtype == MOBA_DTYPE_F16
-             ? launch_partials<F16>(q, k, v, part_o, part_lse, out, lse, t, D, softmax_scale, grid, tile_rows, queues, redo, st)
-             : launch_partials<Bf16>(q, k, v, part_o, part_lse, out, lse, t, D, softmax_scale, grid, tile_rows, queues, redo, st);
+             ? launch_partials<F16>(q, k, v, part_o, part_lse, out, lse, t, D, softmax_scale, grid, tile_rows, queues, redo,
+                                    running_max != 0, st)
+             : launch_partials<Bf16>(q, k, v, part_o, part_lse, out, lse, t, D, softmax_scale, grid, tile_rows, queues, redo,
+                                    running_max != 0, st);
 }
 
 extern "C" int moba_fwd_partials(const void* q, const void* k, const void* v, void* part_o, float* part_lse,
@@ -947,7 +952,7 @@ extern "C" int moba_fwd_partials(const void* q, const void* k, const void* v, vo
   return moba_fwd_partials_rows(q, k, v, part_o, part_lse, seg_off, tile_off, seg_dest, fchunk_tok, chunk_tok,
                                 self_tile_prefix, tile_seg, self_tile_chunk, chunk_direct, out, lse, S, H, Hkv, D, K, F, N,
                                 B, hist_bound, self_tiles, key_split, strides, queues, redo, softmax_scale, dtype,
-                                self_tile_skip, q_tok_shift, kFwdTileRows, stream);
+                                self_tile_skip, q_tok_shift, kFwdTileRows, redo == nullptr, stream);
 }
 
 // mrg_start [nranges], mrg_prefix [nranges + 1], merge_tokens = mrg_prefix[nranges]: the tokens to merge, for a

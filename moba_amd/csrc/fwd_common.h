@@ -17,6 +17,7 @@ struct FwdParams {
   float scale_log2;  // D^-0.5 * log2(e)
   int* queues;       // [8] tile counters, one per XCD, zero when the kernel starts
   int* redo;         // [1 + tiles] count and ids of the tiles to be computed again (see kFixedRef); count zero at the start
+  int running_max;   // one workgroup per tile: track the maximum from the start
 };
 
 // Fixed-reference softmax: a row's sum of exponentials (relative to the row maximum of the tile's first key

@@ -21,7 +21,8 @@
 // to 128, 205 us here; 131072 tokens, chunk 4096, 12 chunks: 64.8 -> 43.6 ms.
 //
 // Softmax: relative to the row maximum of the tile's first 32 keys (see fwd.hip); a tile in which a row leaves the
-// range that is safe is computed again on the spot with a running maximum, by the same workgroup.
+// range that is safe is computed again on the spot with a running maximum, by the same workgroup.  (FwdParams::running_max:
+// with a running maximum from the start.)
 #include <cstddef>
 #include <type_traits>
 #include "fwd_common.h"
@@ -373,18 +374,20 @@ __global__ __launch_bounds__(NW * 64, (FwdTileShape<D, NW>::kWavesPerSimd)) void
   };
 #undef MOBA_PIN
 
-  all_keys(std::true_type{});
-  float l_tot = sum_xhalf(l_run);
-  {
+  float l_tot = 0.f;
+  int again = p.running_max;
+  if (!again) {
+    all_keys(std::true_type{});
+    l_tot = sum_xhalf(l_run);
     const bool bad = row_valid && (beyond_fixed_range(l_tot) || any_not_finite(oacc));
     volatile int* flags = reinterpret_cast<volatile int*>(smem + Shape::kFlags);
     const bool any_bad = __any(bad);
     if (lane == 0) flags[wave] = any_bad ? 1 : 0;
     __syncthreads();
-    int again = 0;
 #pragma unroll
     for (int w = 0; w < NW; ++w) again |= flags[w];
-    if (__builtin_amdgcn_readfirstlane(again)) {
+    again = __builtin_amdgcn_readfirstlane(again);
+    if (again) {
       __syncthreads();  // (every wave has read the flags)
       // back to stage 0: nkt tiles moved K by nkt stages, V by nkt
       const uint32_t dk = (uint32_t)((nkt % 3) * kStage), dv = (uint32_t)((nkt & 1) * kStage);
@@ -396,14 +399,16 @@ __global__ __launch_bounds__(NW * 64, (FwdTileShape<D, NW>::kWavesPerSimd)) void
         voffB[db] -= dv;
       }
       first_copies();
-      all_keys(std::false_type{});
-      l_tot = sum_xhalf(l_run);
       if (p.redo && tid == 0) {  // (listed for a caller that asks which tiles these were)
         const int at = __hip_atomic_fetch_add(p.redo, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         // (every part of a cut tile counts: more of them than the array has entries are counted only)
         if (at < p.t.hist_bound + p.t.self_total) p.redo[1 + at] = t.id;
       }
     }
+  }
+  if (again) {
+    all_keys(std::false_type{});
+    l_tot = sum_xhalf(l_run);
   }
 
   // ---- normalise, write: through 4 KiB of LDS per wave, half a row at a time, so that the rows leave as 128-byte
@@ -480,13 +485,14 @@ static int tail_tile_rows(int64_t blocks, int64_t tall, int cus) {
 
 template <class E>
 static int launch_tail_tiles(const void* q, const void* k, const void* v, void* out, const TileTables& t, float scale,
-                             int64_t workgroups, int tile_rows, hipStream_t st) {
+                             int running_max, int64_t workgroups, int tile_rows, hipStream_t st) {
   LaunchCheck launch_check;
   FwdParams<E> p = {};
   p.q = (const typename E::elem*)q; p.k = (const typename E::elem*)k; p.v = (const typename E::elem*)v;
   p.out = (typename E::elem*)out;
   p.t = t;
   p.scale_log2 = scale * 1.4426950408889634f;
+  p.running_max = running_max;
   const int rc = tile_rows == 128 ? launch<E, 128, 4, true>(p, workgroups, st) : launch<E, 128, 8, true>(p, workgroups, st);
   return rc != MOBA_OK ? rc : launch_check.result();
 }
@@ -501,7 +507,8 @@ using namespace moba;
 // 4 sequences x 1024 tokens, 8 heads, 9000 keys: 836 -> 166 us; 4 x 2048, 32 heads, 9000 keys: 1771 -> 993 us; one of 2048
 // tokens, 32 heads, 34816 keys: 1018 -> 961 us (bound by the products: 1.18 PFLOP/s).
 extern "C" int moba_tail_tiles(const void* q, const void* k, const void* v, void* out, int B, int H, int Hkv, int nq,
-                               int Skv, int D, const int64_t* strides, float scale, int dtype, void* stream) {
+                               int Skv, int D, const int64_t* strides, float scale, int dtype, int running_max,
+                               void* stream) {
   if (!q || !k || !v || !out || !strides) return MOBA_ERR_ARG;
   if (B <= 0 || H <= 0 || Hkv <= 0 || nq <= 0 || nq > Skv || H % Hkv != 0 || !(scale > 0.f)) return MOBA_ERR_ARG;
   if (D != kHeadDim || (dtype != MOBA_DTYPE_BF16 && dtype != MOBA_DTYPE_F16)) return MOBA_ERR_UNSUPPORTED;
@@ -523,6 +530,9 @@ extern "C" int moba_tail_tiles(const void* q, const void* k, const void* v, void
   t.xcd_block_log2 = tile_xcd_block_log2(total);
   const int64_t run = 8LL << t.xcd_block_log2, workgroups = (total + run - 1) / run * run;
   if (workgroups >= 0x7fffffffLL) return MOBA_ERR_LIMIT;
-  return dtype == MOBA_DTYPE_F16 ? launch_tail_tiles<F16>(q, k, v, out, t, scale, workgroups, tile_rows, (hipStream_t)stream)
-                                 : launch_tail_tiles<Bf16>(q, k, v, out, t, scale, workgroups, tile_rows, (hipStream_t)stream);
+  hipStream_t st = (hipStream_t)stream;
+  running_max = running_max != 0;
+  return dtype == MOBA_DTYPE_F16
+             ? launch_tail_tiles<F16>(q, k, v, out, t, scale, running_max, workgroups, tile_rows, st)
+             : launch_tail_tiles<Bf16>(q, k, v, out, t, scale, running_max, workgroups, tile_rows, st);
 }

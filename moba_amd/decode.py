@@ -12,6 +12,7 @@ from typing import Optional
 import torch
 
 from . import _lib
+from . import moba_efficient as E
 from .moba_efficient import _aligned
 
 SUPPORTED_GROUP_SIZES = (1, 2, 4, 8)
@@ -114,7 +115,7 @@ def _tail_tiles(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, sca
     scale = float(scaling) if scaling is not None else d ** -0.5
     dtype = _lib.DTYPE_F16 if query.dtype == torch.float16 else _lib.DTYPE_BF16
     _lib.check(lib.moba_tail_tiles(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), b, h, hkv, q_len, skv, d,
-                                   (ctypes.c_int64 * 6)(*qs, *ks), scale, dtype,
+                                   (ctypes.c_int64 * 6)(*qs, *ks), scale, dtype, 0 if E.FIXED_REFERENCE else 1,
                                    torch.cuda.current_stream(query.device).cuda_stream), "moba_tail_tiles")
     return out
 
@@ -174,7 +175,6 @@ def chunk_decode_attention(query: torch.Tensor, key: torch.Tensor, value: torch.
         return _tail(query, key, value, scaling)
     if h * (q_len // 256) < RESIDENT_TILES:
         return _tail_tiles(query, key, value, scaling)
-    from . import moba_efficient as E
     lib = _lib.load()
     dev = query.device
     tile_rows = lib.moba_fwd_tile_rows()
@@ -202,6 +202,7 @@ def chunk_decode_attention(query: torch.Tensor, key: torch.Tensor, value: torch.
             E._ptr(q_rows), E._ptr(k_rows), E._ptr(v_rows), E._ptr(out_rows), E._ptr(lse_rows), null, null, null, null,
             at(0), at(2), null, at(4), at(4 + m), E._ptr(out_rows), E._ptr(lse_rows), kv_len, h, hkv, d, 0, 0, 1, kv_len,
             0, m, 1, E._strides(q_rows, k_rows), ctypes.c_void_p(scratch.data_ptr()),
-            ctypes.c_void_p(scratch.data_ptr() + 32), scale, code, skip, q_shift, stream), "moba_fwd_partials")
+            ctypes.c_void_p(scratch.data_ptr() + 32) if E.FIXED_REFERENCE else null, scale, code, skip, q_shift, stream),
+            "moba_fwd_partials")
         out[i] = out_rows[pad:]
     return out

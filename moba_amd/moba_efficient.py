@@ -24,8 +24,8 @@ from .plan import FWD_TILE_ROWS, MobaPlan, TILE_ROWS, make_plan
 
 HEAD_DIM = 128
 NARROW_HEAD_DIM = 64   # the forward's kernels also take heads of this width as they are
-# MOBA_FIXED_REFERENCE=0 keeps the forward kernel on its running-maximum softmax for every problem (the
-# fixed-reference form, with its redo list, is otherwise used where the C ABI's `redo` argument says)
+# MOBA_FIXED_REFERENCE=0 keeps the forward kernels on their running-maximum softmax for every problem (they otherwise
+# start from a fixed reference per row and compute a tile again where that fails, see the C ABI's `redo` argument)
 FIXED_REFERENCE = os.environ.get("MOBA_FIXED_REFERENCE", "1") != "0"
 # Dense prefixes (see MobaPlan.dense_local): None = where they pay (problems large enough for the kernels whose
 # workgroups stay resident), True / False (MOBA_DENSE_PREFIX=1 / 0) = always / never.
@@ -451,7 +451,8 @@ def _run_forward(q, k, v, plan: MobaPlan, timer: Optional[StageTimer] = None, sc
                                               tile_segp, tp[g.self_names[1]], tp["achunk_direct"] if DIRECT_ROWS else null,
                                               _ptr(out), _ptr(lse), S, H, Hkv, D, K, plan.F, plan.NA,
                                               plan.chunk_size, g.bound, g.self_tiles, g.split, strides, queuesp,
-                                              redop, scale, code, 0, 0, g.rows_per_tile, stream), "moba_fwd_partials_rows")
+                                              redop, scale, code, 0, 0, g.rows_per_tile, 0 if FIXED_REFERENCE else 1, stream),
+                   "moba_fwd_partials_rows")
     if not DIRECT_ROWS:
         with span("fwd_merge"):
             _lib.check(lib.moba_fwd_merge(part_op, part_lsep, selp, _ptr(out), _ptr(lse), S, H, D, K, g.split,

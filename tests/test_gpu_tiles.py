@@ -180,3 +180,49 @@ def test_list_of_tiles_computed_again_is_bounded(tile_rows, monkeypatch):
     assert redo[0] > entries, (redo[0].item(), entries)
     assert redo[1:].min() >= 0 and redo[1:].max() < g.bound + g.self_tiles * H
     assert (whole[g.ws_bytes - guard:g.ws_bytes] == 255).all()
+
+
+@pytest.mark.parametrize("lens,heads,D,B,topk,rows", [
+    ([3000], 2, 128, 192, 3, 128), ([3000], 2, 128, 192, 3, 256), ([700, 2333], 3, 64, 256, 4, 128),
+    ([4096], 1, 128, 2048, 3, 128),                  # history tiles cut along their keys
+    ([8155, 7777, 8192, 6013, 8000, 8492], 4, 128, 512, 4, 256),    # resident workgroups
+])
+def test_running_maximum_from_the_start(lens, heads, D, B, topk, rows, tile_rows, monkeypatch):
+    """The switch for the running maximum reaches every form of the forward.  Scores rise by up to 2^40 above a row's first
+    32 keys: inside the fixed reference's range, so that no tile is computed again, but beyond the 2^8 by which the running
+    maximum may lag, so that its probabilities are rounded elsewhere: the two agree as far as roundings go (probabilities, partial
+    result and result, to half a step at values of up to about 4.5 each), and not bit for bit."""
+    from moba_amd import moba_efficient as E
+    cu = [0] + np.cumsum(lens).tolist()
+    print("switch case", lens, heads, D, B, topk, rows, flush=True)
+    tile_rows(rows)
+    g = torch.Generator().manual_seed(cu[-1])
+    q, k, v = (torch.randn((cu[-1], heads, D), generator=g) * s for s in (3.0, 2.0, 1.0))
+    q, k, v = (x.to(torch.bfloat16).cuda() for x in (q, k, v))
+    cu_t = torch.tensor(cu, dtype=torch.int32, device="cuda")
+    outs = []
+    for fixed in (True, False):
+        monkeypatch.setattr(E, "FIXED_REFERENCE", fixed)
+        outs.append(E.moba_attn_varlen_with_lse(q, k, v, cu_t, max(lens), B, topk))
+    (out_f, lse_f), (out_r, lse_r) = outs
+    err = (out_f.float() - out_r.float()).abs()
+    assert not torch.equal(out_f, out_r) and err.max() < 2 * 3 * 4.5 * 2.0 ** -9 and err.mean() < 2 * 3 * 0.8 * 2.0 ** -10
+    assert (lse_f - lse_r).abs().max() < 1e-3
+
+
+@pytest.mark.parametrize("q_len,resident", [(600, 1 << 30), (600, 0), (300, 1 << 30)])
+def test_running_maximum_of_new_tokens(q_len, resident, monkeypatch):
+    """The same for new tokens against a cache, on both routes of the causal tiles."""
+    from moba_amd import moba_efficient as E
+    import moba_amd.decode as D
+    g = torch.Generator().manual_seed(q_len)
+    q, k, v = (torch.randn((1, 16, n, 128), generator=g) * s for n, s in ((q_len, 3.0), (1000, 2.0), (1000, 1.0)))
+    q, k, v = (x.to(torch.bfloat16).cuda() for x in (q, k, v))
+    monkeypatch.setattr(D, "RESIDENT_TILES", resident)
+    monkeypatch.setattr(D, "_takes_tiles", lambda *a: True)
+    outs = []
+    for fixed in (True, False):
+        monkeypatch.setattr(E, "FIXED_REFERENCE", fixed)
+        outs.append(D.chunk_decode_attention(q, k, v).float())
+    err = (outs[0] - outs[1]).abs()
+    assert err.max() > 0 and err.max() < 2 * 3 * 4.5 * 2.0 ** -9 and err.mean() < 2 * 3 * 0.8 * 2.0 ** -10
