@@ -75,8 +75,10 @@ constexpr float kTailMaxLag = 8.f;
 constexpr float kTailNoMax = -3e38f;  // before the first visible key (finite: exp2(m - m_new) stays defined)
 
 // kOnce: one workgroup and one wave reads a key's rows (up to 32 query rows per key/value head): they pass the caches by
+// (Held to 256 registers, though its LDS lets one wave per SIMD run: with all 512 the compiler keeps the sums in accumulation
+// registers and moves all of them for every rescale and for the end; partial kernel at 4097 keys: 9.4 us so, 8.9 held.)
 template <class E, bool kOnce>
-__global__ __launch_bounds__(256, 1) void tail_partial_kernel(const TailParams<E> p) {
+__global__ __launch_bounds__(256, 2) void tail_partial_kernel(const TailParams<E> p) {
   MOBA_ELEM_TYPES(E)
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -235,7 +237,7 @@ __global__ __launch_bounds__(256, 1) void tail_partial_kernel(const TailParams<E
       issue(it + 2, it & 1);
     }
   }
-  if (__any(any_not_finite(oacc))) {  // (never for values of ordinary size)
+  if (__builtin_expect(__any(any_not_finite(oacc)), 0)) {  // (never for values of ordinary size)
     auto each_key = [&](auto use) __attribute__((always_inline)) {
       for (int it = 0; it < mine; ++it) {
         const int key0 = key_lo + (wk + it * wk_n) * kTailKeys, key1 = min(key0 + kTailKeys, key_hi);

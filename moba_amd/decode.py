@@ -79,8 +79,11 @@ def _tail(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, scaling: 
     q, k, v, qs, ks = _placed_three(query, key, value, d)
     dev = query.device
     out = torch.empty((b, q_len, h, d), dtype=query.dtype, device=dev)
-    pieces = [(i, min(b - i, MOST_SEQUENCES)) for i in range(0, b or 1, MOST_SEQUENCES)]   # one, but for very many
-    rows = q_len * h * max(n * lib.moba_tail_splits(n, hkv, h // hkv, q_len, skv) for _, n in pieces)
+    most = min(b, MOST_SEQUENCES)
+    rows = q_len * h * most * lib.moba_tail_splits(most, hkv, h // hkv, q_len, skv)
+    if b > most and b % most:    # (the last piece: fewer sequences, perhaps more splits)
+        rest = b % most
+        rows = max(rows, q_len * h * rest * lib.moba_tail_splits(rest, hkv, h // hkv, q_len, skv))
     part = torch.empty(rows * (d + 1), dtype=torch.float32, device=dev)   # partial outputs, then their log-sum-exps
     part_o = part.data_ptr()
     scale = float(scaling) if scaling is not None else d ** -0.5
@@ -88,10 +91,12 @@ def _tail(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, scaling: 
     strides = (ctypes.c_int64 * 5)(*qs, ks[0], ks[1])
     stream = torch.cuda.current_stream(dev).cuda_stream
     qp, kp, vp, op = q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr()
-    for i, n in pieces:
-        _lib.check(lib.moba_tail(qp + 2 * i * qs[0], kp + 2 * i * ks[0], vp + 2 * i * ks[0], op + 2 * i * q_len * h * d,
-                                 part_o, part_o + rows * d * 4, n, h, hkv, q_len, skv, d, strides, scale, dtype, stream),
-                   "moba_tail")
+    for i in range(0, b or 1, MOST_SEQUENCES):   # (one piece, but for very many sequences)
+        if i:
+            qp, kp, vp = (x + 2 * MOST_SEQUENCES * step for x, step in ((qp, qs[0]), (kp, ks[0]), (vp, ks[0])))
+            op += 2 * MOST_SEQUENCES * q_len * h * d
+        _lib.check(lib.moba_tail(qp, kp, vp, op, part_o, part_o + rows * d * 4, min(b - i, MOST_SEQUENCES), h, hkv, q_len,
+                                 skv, d, strides, scale, dtype, stream), "moba_tail")
     return out
 
 
