@@ -261,8 +261,8 @@ int moba_fwd_partials(const void* q, const void* k, const void* v, void* part_o,
 /* The same on tile tables (self_tile_prefix, self_tile_chunk, tile_off, tile_seg, hist_bound, self_tiles) for tiles of
  * tile_rows rows: moba_fwd_tile_rows(), or moba_bwd_tile_rows(), whose tiles run one workgroup each, two side by side
  * on a compute unit, for problems of short chunks or few tiles.  Those of moba_bwd_tile_rows() rows also take D = 64
- * (as moba_chunk_mean, moba_gate_topk and moba_fwd_merge do; strides must then be given).  queues is then not used;
- * redo, if given, has redo[0] zeroed by the caller and receives the tiles that were computed again with a running
+ * (as moba_chunk_mean, moba_gate_topk and moba_fwd_merge do; strides must then be given).  queues is then not used
+ * and may be NULL; redo, if given, has redo[0] zeroed by the caller and receives the tiles that were computed again with a running
  * maximum, for information: redo[0] counts every part of a tile cut by key_split, and parts beyond the array's
  * hist_bound + self_tiles * H entries are counted without an entry.  Those tiles take the fixed reference without a
  * list too: running_max != 0 asks for the running maximum from the start (and for redo to be left alone), whatever the

@@ -886,7 +886,8 @@ extern "C" int moba_fwd_partials_rows(const void* q, const void* k, const void* 
                                  int dtype, int self_tile_skip, int64_t q_tok_shift, int tile_rows, int running_max,
                                  void* stream) {
   if (tile_rows != kFwdTileRows && tile_rows != TM) return MOBA_ERR_ARG;
-  if (!q || !k || !v || !part_o || !part_lse || !chunk_tok || !self_tile_prefix || !self_tile_chunk || !queues)
+  if (!q || !k || !v || !part_o || !part_lse || !chunk_tok || !self_tile_prefix || !self_tile_chunk ||
+      (!queues && tile_rows == kFwdTileRows))
     return MOBA_ERR_ARG;
   if (chunk_direct && (!out || !lse || ((uintptr_t)out & 15))) return MOBA_ERR_ARG;
   // queries that are the tail of their sequence: plain causal attention whose rows all go straight to the outputs

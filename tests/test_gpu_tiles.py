@@ -226,3 +226,24 @@ def test_running_maximum_of_new_tokens(q_len, resident, monkeypatch):
         outs.append(D.chunk_decode_attention(q, k, v).float())
     err = (outs[0] - outs[1]).abs()
     assert err.max() > 0 and err.max() < 2 * 3 * 4.5 * 2.0 ** -9 and err.mean() < 2 * 3 * 0.8 * 2.0 ** -10
+
+
+def test_short_tiles_need_no_queues(tile_rows, monkeypatch):
+    """The tiles with a workgroup each draw nothing from queues: the C entry takes none."""
+    from moba_amd import _lib
+    from moba_amd import moba_efficient as E
+    lib = _lib.load()
+
+    class WithoutQueues:
+        def __getattr__(self, name):
+            if name != "moba_fwd_partials_rows":
+                return getattr(lib, name)
+            return lambda *a: lib.moba_fwd_partials_rows(*a[:28], None, *a[29:])
+
+    g = torch.Generator().manual_seed(2)
+    q, k, v = (torch.randn((900, 2, 128), generator=g).to(torch.bfloat16).cuda() for _ in range(3))
+    cu_t = torch.tensor([0, 900], dtype=torch.int32, device="cuda")
+    tile_rows(128)
+    want = E.moba_attn_varlen(q, k, v, cu_t, 900, 128, 3)
+    monkeypatch.setattr(_lib, "load", lambda: WithoutQueues())
+    assert torch.equal(E.moba_attn_varlen(q, k, v, cu_t, 900, 128, 3), want)
