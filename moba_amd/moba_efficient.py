@@ -645,8 +645,9 @@ class _MobaAttentionInGroups(torch.autograd.Function):
 def _attend(q, k, v, plan, timer=None, scale=0.0):
     """(out, lse): through autograd when a gradient may be asked for, straight to the kernels otherwise."""
     S, H, D = _dims(q)
-    groups = _head_groups(plan, H, _dims(k)[1], D, q.element_size())
     grad = torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad)
+    # (the backward's partials are those of heads of 128 elements, whatever the forward's)
+    groups = _head_groups(plan, H, _dims(k)[1], HEAD_DIM if grad else D, q.element_size())
     if len(groups) > 1:
         if grad:
             return _MobaAttentionInGroups.apply(q, k, v, plan, groups, timer, scale)

@@ -717,3 +717,38 @@ def test_heads_in_groups(heads, kv_heads, batched, monkeypatch):
         q, k, v = (hf_to_fa(x).contiguous() for x in (query, key, value))
         out, lse = E.moba_attn_varlen_with_lse(q, k, v, cu, s, B, topk, gqa=True)
     assert torch.equal(out, whole[0])
+
+
+def test_narrow_heads_in_training_keep_to_the_scratch_limit(monkeypatch):
+    """The backward pads 64-element heads to 128: a call whose partials fit the limit at 64 and not at 128 goes in
+    groups of heads when a gradient will be asked for, with the results of one go, bit for bit."""
+    from moba_amd import moba_efficient as E
+    S, H, Hkv, B, topk = 3000, 8, 4, 256, 3
+    g = torch.Generator().manual_seed(12)
+    q, k, v, do = (torch.randn((S, h, 64), generator=g).to(torch.bfloat16).cuda() for h in (H, Hkv, Hkv, H))
+    for t in (q, k, v):
+        t.requires_grad_(True)
+    cu_t = torch.tensor([0, 1111, S], dtype=torch.int32, device="cuda")
+    plan = E.make_plan(cu_t, B, topk)
+    bytes_64, bytes_128 = (S * H * (plan.K + 1) * (d * 2 + 4) for d in (64, 128))
+    heads, inner = [], E._backward
+
+    def seen(dout, q, *rest):
+        heads.append((q.shape[1], q.shape[2]))
+        return inner(dout, q, *rest)
+
+    monkeypatch.setattr(E, "_backward", seen)
+    runs = []
+    for limit in (bytes_128, (bytes_64 + bytes_128) // 2):
+        monkeypatch.setattr(E, "SCRATCH_LIMIT_BYTES", limit)
+        q.grad = k.grad = v.grad = None
+        heads.clear()
+        out = E.moba_attn_varlen_gqa(q, k, v, cu_t, S, B, topk)
+        out.backward(do)
+        wide = [h for h, d in heads if d == 128]
+        assert wide and all(S * h * (plan.K + 1) * 260 <= limit for h in wide)
+        runs.append((out.detach(), q.grad, k.grad, v.grad))
+    assert len(wide) > 1 and all(torch.equal(a, b) for a, b in zip(*runs))
+    with torch.no_grad():   # (without gradients the call still goes in one go)
+        monkeypatch.setattr(E, "_forward_in_groups", None)
+        assert torch.equal(E.moba_attn_varlen_gqa(q, k, v, cu_t, S, B, topk), runs[0][0])
