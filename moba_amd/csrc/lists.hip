@@ -237,7 +237,7 @@ __global__ __launch_bounds__(1024) void scan_kernel(int* __restrict__ a, int n) 
 // in about 2.5 us): 9.4 million counts -- 196608 tokens, 32 heads, chunks of 256 -- took it 5.8 ms of a call of 14 ms.
 __global__ __launch_bounds__(1024) void scan_sums_kernel(const int* __restrict__ a, int n, int per, int* __restrict__ sums) {
   __shared__ int wsum[16];
-  const int lo = blockIdx.x * per, hi = min(n, lo + per);
+  const int lo = blockIdx.x * per, hi = lo + min(n - lo, per);
   int s = 0;
   for (int i = lo + threadIdx.x; i < hi; i += 1024) s += a[i];
 #pragma unroll
@@ -260,7 +260,7 @@ __global__ __launch_bounds__(1024) void scan_apply_kernel(int* __restrict__ a, i
   int carry = 0;
 #pragma unroll
   for (int w = 0; w < 16; ++w) carry += wsum[w];
-  const int lo = blockIdx.x * per, hi = min(n, lo + per);
+  const int lo = blockIdx.x * per, hi = lo + min(n - lo, per);
   const int total = scan_range(a, lo, hi, carry);
   if (blockIdx.x + 1 == gridDim.x && threadIdx.x == 0) a[n] = total;
 }
@@ -501,7 +501,8 @@ extern "C" int moba_build_lists(const int32_t* sel, const int32_t* chunk_tok, co
     return MOBA_ERR_ARG;
   if (S <= 0 || H <= 0 || K <= 0 || N <= 0 || F <= 0 || P <= 0 || cmax <= 0 || tile_rows <= 0) return MOBA_ERR_ARG;
   if (dense_local < 0 || dense_local > K) return MOBA_ERR_ARG;
-  if ((int64_t)S * H * (K + 1) >= 0x7fffffffLL || (int64_t)P * H >= 0x7fffffffLL) return MOBA_ERR_LIMIT;
+  if ((int64_t)S * H * (K + 1) >= 0x7fffffffLL || (int64_t)P * H > 0x7fffffffLL - 4096) return MOBA_ERR_LIMIT;
+  // (the scan's steps of 4096 counts stay within an int)
   if (H > 65535 || (size_t)cmax * 12 > 160 * 1024) return MOBA_ERR_LIMIT;
   hipStream_t st = (hipStream_t)stream;
   dim3 grid(N, H);

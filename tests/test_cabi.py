@@ -81,3 +81,14 @@ def test_binding_signatures_match_header():
                 assert p.startswith("int "), (name, p)
                 want = (ctypes.c_int,)
             assert a in want, (name, p, a)
+
+
+def test_list_counts_beyond_an_int_are_refused(lib):
+    """The scan of the list counts steps through them 4096 at a time in 32 bits: a number of counts whose last step would
+    pass 2^31 is refused before anything is launched."""
+    from moba_amd import _lib
+    bound = _lib.load()
+    some = ctypes.c_void_p(256)   # (never read)
+    for P, H in ((0x7fffffff - 4095, 1), (0x7ffffffe, 1), ((0x7fffffff - 100) // 2, 2)):
+        rc = bound.moba_build_lists(*[some] * 10, 4096, H, 1, 16, 64, P, 10, 128, 1024, 1, 0, None, None, 0, 0, None)
+        assert rc == -4, (P, H, rc)
