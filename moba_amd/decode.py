@@ -142,10 +142,13 @@ def _takes_tiles(b: int, h: int, hkv: int, q_len: int) -> bool:
     return q_len > 16 and blocks > max(288, tiles * 3 // 2)
 
 
-# A single sequence of at least this many tiles of 256 rows goes to the forward kernel with resident workgroups, which
-# reads its tiles' tables: 32768 tokens, 32 heads, 131072 keys: 50.7 ms there, 51.2 on _tail_tiles; with 2048 tiles (8192
-# tokens, 64 heads) 13.72 and 13.74 ms at 65536 keys, 3.10 and 2.83 ms at 16384.
-RESIDENT_TILES = 4096
+# The causal tiles of all sequences in one launch number their rows in 32 bits.  Calls of more rows (this many tiles of
+# 256) go one sequence at a time to the forward kernel with resident workgroups, which reads its tiles' tables and
+# wants q, the result and the log-sum-exps as copies.  It is the slower of the two at every size measured, resident
+# workgroups / tiles, heads on key/value heads, new tokens, keys: 32 on 8, 32768, 32769: 8.3 / 7.4 ms; 65536: 22.9 / 21.7;
+# 131072: 51.3 / 50.1; 64 on 8, 16384, 16385: 4.6 / 3.8; 65536, 262144: 402 / 398; 128 on 16, 65536, 131072: 347 / 341; 8 on
+# 1, 262144, 300000: 149 / 146; four sequences of 32768 on 40000: 46.7 / 41.9.
+RESIDENT_TILES = (1 << 31) // 256
 
 
 _TAIL_TABLES = {}  # (kv_len, row tiles skipped, device) -> int32 tables of the causal tiles of a sequence's tail
@@ -178,7 +181,7 @@ def chunk_decode_attention(query: torch.Tensor, key: torch.Tensor, value: torch.
         return torch.empty((b, q_len, h, d), dtype=query.dtype, device=query.device)
     if not _takes_tiles(b, h, hkv, q_len) or (scaling is not None and not scaling > 0):
         return _tail(query, key, value, scaling)
-    if h * (q_len // 256) < RESIDENT_TILES:
+    if b * h * q_len // 256 < RESIDENT_TILES:
         return _tail_tiles(query, key, value, scaling)
     lib = _lib.load()
     dev = query.device

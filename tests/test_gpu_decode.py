@@ -228,3 +228,19 @@ def test_routes_of_new_tokens(monkeypatch):
     assert torch.equal(tiles, D._tail_tiles(q, k, v, None))
     monkeypatch.setattr(D, "RESIDENT_TILES", 0)
     assert torch.equal(tiles, D.chunk_decode_attention(q, k, v))
+
+
+def test_long_pieces_of_a_prompt_take_the_tiles(monkeypatch):
+    """Very many new tokens of one sequence: the causal tiles, read in place (the other route copies q and the result)."""
+    import moba_amd.decode as D
+    calls, real = [], D._tail_tiles
+    monkeypatch.setattr(D, "_tail_tiles", lambda *a: (calls.append(1), real(*a))[1])
+    g = torch.Generator(device="cuda").manual_seed(6)
+    q = torch.randn((1, 128, 8200, 128), generator=g, device="cuda", dtype=torch.bfloat16)
+    k, v = (torch.randn((1, 2, 8300, 128), generator=g, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    out = D.chunk_decode_attention(q, k, v)
+    assert calls == [1]
+    rows = [0, 1, 127, 128, 4097, 8199]
+    for j in rows:
+        want = _ref(q[:, :, j:j + 1], k[:, :, :101 + j], v[:, :, :101 + j], 128 ** -0.5)
+        assert (out[:, j:j + 1].float() - want).abs().max() < 2e-2
