@@ -232,14 +232,21 @@ extern "C" size_t moba_chunk_mean_workspace_bytes(int H, int D, int F, int B) {
 }
 
 // Whether one workgroup per (chunk, head) will do: where there are enough of them to keep the memory busy, or so little
-// to read for each that a second launch would take longer.  Not for very many chunks of at most eight tokens per lane:
-// whole rows of all heads, in the order they lie, then read faster than they add up (65536 tokens, 32 heads, chunk 128:
-// 104 us in two stages, 114 in one; 8 heads: 28 and 22).
+// to read for each that a second launch would take longer.  One workgroup reads its 256 KiB in 9 us, 512 KiB in 15, 1 MiB in
+// 25, alone or not; the two stages take 8 and what the bytes of all take, and more for rows of many heads.  One workgroup
+// each / two stages in us, 128-element heads (heads x chunks, tokens a chunk): 1 x 31, 1024: 9.3 / 8.6; 1 x 64: 9.8 / 10.2;
+// 1 x 15, 2048: 14.1 / 9.9; 1 x 64: 15.8 / 14.5; 2 x 16: 15.5 / 14.8; 2 x 32: 16.8 / 18.2; 4 x 8: 15.9 / 12.2; 4 x 16: 17.1 / 14.3;
+// 8 x 4: 15.9 / 16.6; 1 x 31, 4096: 25.3 / 18.2; 4 x 31: 35.2 / 42.8; 8 x 31: 48.6 / 72.1; 64-element heads: 1 x 31, 2048: 9.5 /
+// 9.2; 4 x 8: 10.2 / 12.9; 1 x 31, 4096: 15.3 / 12.7; 4 x 7: 16.5 / 21.0.
+// Not for very many chunks of at most eight tokens per lane: whole rows of all heads, in the order they lie, then read
+// faster than they add up (65536 tokens, 32 heads, chunk 128: 104 us in two stages, 114 in one; 8 heads: 28 and 22).
 static bool whole_chunks(int H, int D, int F, int B) {
   const int d8 = D / 8;
   if (d8 > 16 || (d8 & (d8 - 1)) || H > 65535) return false;
-  if (B * d8 <= 256 * 8 && (int64_t)F * H > 8192) return false;
-  return (int64_t)F * H >= 128 || (int64_t)B * D <= 2048 * 128;
+  const int64_t groups = (int64_t)F * H, elems = (int64_t)B * D;
+  if (B * d8 <= 256 * 8 && groups > 8192) return false;
+  if (groups >= 128 || elems <= 1024 * 128) return true;
+  return elems <= 2048 * 128 && (groups >= 64 || H * 32 > D);
 }
 
 static int launch_chunk_mean(const void* k, const int32_t* fchunk_tok, void* kbar, double* partial, int H, int D,

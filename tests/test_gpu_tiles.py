@@ -247,3 +247,16 @@ def test_short_tiles_need_no_queues(tile_rows, monkeypatch):
     want = E.moba_attn_varlen(q, k, v, cu_t, 900, 128, 3)
     monkeypatch.setattr(_lib, "load", lambda: WithoutQueues())
     assert torch.equal(E.moba_attn_varlen(q, k, v, cu_t, 900, 128, 3), want)
+
+
+@pytest.mark.parametrize("S,H,B,D", [
+    (6200, 1, 2048, 128), (6200, 4, 2048, 128), (6200, 5, 2048, 128), (3200, 1, 1025, 128), (3200, 1, 1024, 128),
+    (9000, 1, 2049, 64), (9000, 3, 2900, 64), (134000, 1, 2050, 128)])
+def test_chunk_mean_at_the_line_between_its_forms(S, H, B, D):
+    """Few chunks on either side of the line between one workgroup each and two stages: the rounded exact mean."""
+    from moba_amd import moba_efficient as E
+    print("mean line", S, H, B, D, flush=True)
+    k = torch.randn((S, H, D), generator=torch.Generator().manual_seed(S + H)).to(torch.bfloat16)
+    want = O.chunk_mean(k, [0, S], B)
+    got = E.chunk_mean(k.cuda(), E.make_plan([0, S], B, 3, device="cuda"))
+    assert torch.equal(got.cpu().view(torch.int16), want.view(torch.int16))
