@@ -12,7 +12,8 @@
 // A wave copies its own K and V blocks of 32 keys global -> LDS (two stages of 16 KiB, no barrier: the wait for a
 // block counts the wave's own copies) while it computes the block before: 64 to 128 KiB per compute unit in flight,
 // where about 40 KiB cover the latency at the full rate.  One workgroup per compute unit (128 KiB of LDS); the
-// splits are chosen so that the workgroups come out just below a multiple of the units.
+// splits are chosen so that the workgroups come out just below a multiple of the units.  Where the sequences alone are more than
+// the units, short caches take workgroups of two waves or one, two or five to a unit (tail_split).
 // Keys that one wave reads alone (up to 32 rows) are copied past the caches: 1 x 65536 keys, 64 heads: 368 us without, 314
 // with (6.8 TB/s); keys that several waves or workgroups read are not: 40000 keys, 128 rows: 69.4 us without, 75.6 with.
 //
@@ -40,10 +41,9 @@ namespace moba {
 constexpr int kTailKeys = 32;                                 // keys a wave handles per step
 constexpr int kTailTile = kTailKeys * kHeadDim * 2;           // bytes of its K (or V) block
 constexpr int kTailWaveLds = 4 * kTailTile;                   // two stages of K and V
-constexpr int kTailLds = 4 * kTailWaveLds;
 constexpr int kTailRedRow = kHeadDim + 4;                     // floats per row when the waves' sums meet in LDS
-constexpr int kTailRedStats = 4 * 32 * kTailRedRow * 4;       // byte offset of [4 waves][32 rows] maxima, then sums
-static_assert(kTailRedStats + 2 * 4 * 32 * 4 <= kTailLds, "the waves' sums fit the stages");
+constexpr int kTailRedStats = 32 * kTailRedRow * 4;           // times the waves: byte offset of their 32 maxima each, then sums
+static_assert(kTailRedStats + 2 * 32 * 4 <= kTailWaveLds, "the waves' sums fit the stages");
 constexpr int kTailMaxSplits = 128;
 constexpr int kTailExactTokens = 16;  // up to so many new tokens the probabilities keep their 24 bits
 
@@ -77,8 +77,9 @@ constexpr float kTailNoMax = -3e38f;  // before the first visible key (finite: e
 // kOnce: one workgroup and one wave reads a key's rows (up to 32 query rows per key/value head): they pass the caches by
 // (Held to 256 registers, though its LDS lets one wave per SIMD run: with all 512 the compiler keeps the sums in accumulation
 // registers and moves all of them for every rescale and for the end; partial kernel at 4097 keys: 9.4 us so, 8.9 held.)
-template <class E, bool kOnce>
-__global__ __launch_bounds__(256, 2) void tail_partial_kernel(const TailParams<E> p) {
+// NW: waves of a workgroup; fewer than four go with kOnce
+template <class E, bool kOnce, int NW>
+__global__ __launch_bounds__(64 * NW, 2) void tail_partial_kernel(const TailParams<E> p) {
   MOBA_ELEM_TYPES(E)
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -86,7 +87,7 @@ __global__ __launch_bounds__(256, 2) void tail_partial_kernel(const TailParams<E
   const int n = lane & 31, hh = lane >> 5;
   const int split = blockIdx.x, b = blockIdx.z;
   const int group = blockIdx.y / p.Hkv, hkv = blockIdx.y - group * p.Hkv;
-  const int wr_n = 1 << p.wr_log2, wk_n = 4 >> p.wr_log2;
+  const int wr_n = 1 << p.wr_log2, wk_n = NW >> p.wr_log2;
   const int wr = wave & (wr_n - 1), wk = wave >> p.wr_log2;
   const int rows = p.nq * p.rep;
   const int row0 = (group * wr_n + wr) * 32;
@@ -281,8 +282,8 @@ __global__ __launch_bounds__(256, 2) void tail_partial_kernel(const TailParams<E
   // The waves that hold the same rows meet in LDS.  Element e of lane (n, hh) is O[row n][32*db + 8*(e/4) + 4*hh + e%4].
   __syncthreads();  // every wave has read its last fragments
   float* red = reinterpret_cast<float*>(smem);
-  float* red_m = reinterpret_cast<float*>(smem + kTailRedStats);
-  float* red_l = red_m + 4 * 32;
+  float* red_m = reinterpret_cast<float*>(smem + NW * kTailRedStats);
+  float* red_l = red_m + NW * 32;
 #pragma unroll
   for (int db = 0; db < 4; ++db)
 #pragma unroll
@@ -295,7 +296,7 @@ __global__ __launch_bounds__(256, 2) void tail_partial_kernel(const TailParams<E
   }
   __syncthreads();
   const int rows_here = min(32 * wr_n, rows - group * wr_n * 32);
-  for (int i = tid; i < rows_here * 32; i += 256) {
+  for (int i = tid; i < rows_here * 32; i += 64 * NW) {
     const int rr = i >> 5, d = (i & 31) * 4;      // row of the workgroup, dimension
     const int w0 = rr >> 5, nn = rr & 31;         // its row block (= its first wave), its row in there
     float mm = red_m[w0 * 32 + nn];
@@ -371,30 +372,56 @@ using namespace moba;
 
 struct TailSplit {
   int wr_log2, groups, keys_per_split, nsplit;  // groups: workgroups per (sequence, key/value head, split)
+  int waves;                                    // of a workgroup: 4 or 1
 };
 
-// How the work is cut: row blocks over the waves of a workgroup, then the keys over workgroups.  A workgroup's time
-// is its steps (kTailKeys keys per wave that splits the keys) plus about one more for start and end, and a compute
-// unit holds one workgroup: the number of splits is the one that gives the shortest rounds * steps.
+// How the work is cut: row blocks over the waves of a workgroup, then the keys over workgroups.
+//
+// Up to 32 rows a workgroup of four, two or one waves would do, of which a compute unit holds one, two or five: small ones
+// run their starts (first copies) and ends (sums through LDS) under the copies of the others, where there are
+// sequences enough to fill the chip with them, and few large ones leave least to merge where there are not.  A
+// step (kTailKeys keys per wave) takes what the waves beside it on the unit leave it of latency, or of the chip's
+// bandwidth if that is longer, and every round of workgroups a start and an end; the cut is the one that comes out shortest.  The
+// numbers, hundredths of a microsecond up to a common factor, rank 25 cuts at 230 sizes to within 1 % of the best one on
+// average.  Four waves each whatever the size / so, key/value heads of all sequences x keys: 2000 x 8, 64: 239 / 84 us; 1024, 300:
+// 41 / 29; 8192, 128: 155 / 86; 1024, 600: 60 / 52; 320, 1000: 41 / 34; 200, 2500: 55 / 44.  Beyond 4096 keys a start and an
+// end weigh little and four waves keep pace better (1300 x 6000: 591 us, 611 with two).
 static TailSplit tail_split(int B, int Hkv, int rows, int Skv) {
   TailSplit t;
   t.wr_log2 = rows <= 32 ? 0 : (rows <= 64 ? 1 : 2);
   t.groups = (rows + (32 << t.wr_log2) - 1) / (32 << t.wr_log2);
-  const int unit = kTailKeys * (4 >> t.wr_log2);
-  const int steps = (Skv + unit - 1) / unit;
+  const bool once = t.wr_log2 == 0;
   const int64_t wgs = (int64_t)B * Hkv * t.groups;
   int cus = compute_units();
   if (cus <= 0) cus = 256;
-  int64_t best = 0;
-  t.nsplit = 1;
-  t.keys_per_split = steps * unit;
-  for (int ns = 1; ns <= steps && ns <= kTailMaxSplits; ++ns) {
-    const int per = (steps + ns - 1) / ns, n = (steps + per - 1) / per;  // (no empty split)
-    const int64_t cost = ((wgs * n + cus - 1) / cus) * (per + 1);
-    if (ns == 1 || cost < best) {
-      best = cost;
-      t.nsplit = n;
-      t.keys_per_split = per * unit;
+  const bool many = once && wgs > cus && Skv <= 4096;
+  // (one round, and what rounds the last one of several off: more splits are starts and ends for nothing)
+  const int most = once ? (int)(cus / wgs) + 8 : kTailMaxSplits;
+  int64_t best = -1;
+  for (int waves = 4; waves >= (many ? 1 : 4); waves >>= 1) {
+    const int unit = kTailKeys * (waves >> t.wr_log2);
+    const int steps = (Skv + unit - 1) / unit;
+    const int64_t slots = (int64_t)cus * (waves == 1 ? 5 : 4 / waves);
+    for (int ns = 1; ns <= steps && ns <= kTailMaxSplits && ns <= most; ++ns) {
+      const int per = (steps + ns - 1) / ns, n = (steps + per - 1) / per;  // (no empty split)
+      int64_t cost;
+      if (once) {
+        auto round = [&](int64_t workgroups) {
+          const int64_t latency = 92 + 8 * waves * ((workgroups + cus - 1) / cus), bandwidth = 47 * waves * workgroups / cus;
+          return per * (latency > bandwidth ? latency : bandwidth) + 224;
+        };
+        const int64_t rounds = wgs * n / slots, rest = wgs * n - rounds * slots;
+        cost = (rounds ? rounds * round(slots) : 0) + (rest ? round(rest) : 0);
+        if (n > 1) cost += 227 + 47 * wgs * n * rows / (16 * cus);  // (the merge; the partial results out and in)
+      } else {  // (bound by the products: whole rounds, each its steps and about one more)
+        cost = (wgs * n + slots - 1) / slots * (per + 1);
+      }
+      if (best < 0 || cost < best) {
+        best = cost;
+        t.waves = waves;
+        t.nsplit = n;
+        t.keys_per_split = per * unit;
+      }
     }
   }
   return t;
@@ -423,11 +450,15 @@ static int launch_tail(const void* q, const void* k, const void* v, void* out, f
   p.Hkv = Hkv; p.rep = rep; p.Skv = Skv; p.nq = nq;
   p.wr_log2 = ts.wr_log2; p.keys_per_split = ts.keys_per_split; p.nsplit = ts.nsplit;
   p.scale_log2 = scale * 1.4426950408889634f;
-  static bool allowed[2][kMaxDevices];  // one set per element type
-  const bool once = ts.wr_log2 == 0 && ts.groups == 1;
-  const auto kernel = once ? tail_partial_kernel<E, true> : tail_partial_kernel<E, false>;
-  if (!allow_dynamic_lds((const void*)kernel, kTailLds, allowed[once])) return MOBA_ERR_LAUNCH;
-  hipLaunchKernelGGL(kernel, dim3(ts.nsplit, Hkv * ts.groups, B), dim3(256), kTailLds, st, p);
+  static bool allowed[4][kMaxDevices];  // one set per element type
+  typedef void (*Kernel)(TailParams<E>);
+  static const Kernel kernels[4] = {tail_partial_kernel<E, false, 4>, tail_partial_kernel<E, true, 4>,
+                                    tail_partial_kernel<E, true, 2>, tail_partial_kernel<E, true, 1>};
+  const int form = ts.wr_log2 > 0 ? 0 : (ts.waves == 4 ? 1 : (ts.waves == 2 ? 2 : 3));
+  const Kernel kernel = kernels[form];
+  const int lds = ts.waves * kTailWaveLds;
+  if (!allow_dynamic_lds((const void*)kernel, lds, allowed[form])) return MOBA_ERR_LAUNCH;
+  hipLaunchKernelGGL(kernel, dim3(ts.nsplit, Hkv * ts.groups, B), dim3(64 * ts.waves), lds, st, p);
   if (ts.nsplit > 1)
     hipLaunchKernelGGL(tail_merge_kernel<E>, dim3((unsigned)((int64_t)B * nq * Hkv * rep)), dim3(256), 0, st,
                        (const float*)part_o, (const float*)part_lse, (elem*)out, ts.nsplit);

@@ -215,6 +215,32 @@ def test_more_sequences_than_one_grid(q_len, scale):
         assert torch.equal(out, D.decode_attention(q, k, v, scale))
 
 
+@pytest.mark.parametrize("B,H,Hkv,q_len", [
+    (163, 8, 8, 1), (75, 8, 4, 1), (321, 1, 1, 7), (90, 32, 8, 8), (257, 5, 1, 4), (130, 16, 8, 3), (1300, 33, 1, 1)])
+@pytest.mark.parametrize("Skv", [8, 31, 33, 64, 129, 300, 777, 1500, 4096, 4097])
+def test_many_sequences_of_short_caches(B, H, Hkv, q_len, Skv):
+    """More key/value heads than compute units: workgroups of one, two and four waves, with and without splits, on caches
+    that end within, at and behind a wave's and a workgroup's step; the last case has a row more than they take.  The
+    same sequences alone (four waves, more splits) agree to a rounding each."""
+    import moba_amd.decode as D
+    _note("short caches", B, H, Hkv, q_len, Skv)
+    dtype = torch.float16 if Skv % 2 else torch.bfloat16
+    g = torch.Generator(device="cuda").manual_seed(Skv)
+    q, k, v = (torch.randn((B, h, n, 128), generator=g, device="cuda", dtype=dtype)
+               for h, n in ((H, q_len), (Hkv, Skv), (Hkv, Skv)))
+    out = D._tail(q, k, v, None)
+    some = sorted({0, 1, B // 2, B - 2, B - 1})
+    assert _close(out[some], _exact(q[some], k[some], v[some], 128 ** -0.5), dtype)
+    few = torch.cat([D._tail(q[i:i + 1], k[i:i + 1], v[i:i + 1], None) for i in range(B)])
+    assert (out.float() - few.float()).abs().max() < 2 * 5.0 * 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    # a value that is not finite stays with the tokens that see it, in these forms too
+    v[:, :, -1, 3] = float("inf")
+    hit = D._tail(q, k, v, None)
+    assert (hit[:, -1, :, 3] == float("inf")).all() and torch.isfinite(hit[..., 4:].float()).all()
+    if q_len > 1:
+        assert _close(hit[some][:, :-1], _exact(q[some][:, :, :-1], k[some][:, :, :-1], v[some][:, :, :-1], 128 ** -0.5), dtype)
+
+
 def test_the_c_entry_takes_results_at_any_address():
     """moba_decode writes out and its scratch wherever their elements can lie."""
     from moba_amd import _lib
