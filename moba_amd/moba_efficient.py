@@ -465,14 +465,44 @@ def _run_forward(q, k, v, plan: MobaPlan, timer: Optional[StageTimer] = None, sc
     return out, lse, sel, seg_off, tile_off, seg_dest, tile_seg
 
 
+def _widened(tensors, width: int):
+    """The tensors with heads of `width` elements, zeros behind narrower ones, which share one buffer (cleared at once:
+    clearing and copying tensor by tensor is what a small call would spend most of its time on)."""
+    narrow = [t for t in tensors if t.shape[-1] != width]
+    if not narrow:
+        return tuple(tensors)
+    rows = [t.numel() // t.shape[-1] for t in narrow]
+    parts = iter(torch.zeros((sum(rows), width), dtype=narrow[0].dtype, device=narrow[0].device).split(rows))
+    res = []
+    for t in tensors:
+        if t.shape[-1] != width:
+            wide = next(parts).view(*t.shape[:-1], width)
+            wide[..., :t.shape[-1]].copy_(t)
+            t = wide
+        res.append(t)
+    return tuple(res)
+
+
+def _for_training(*tensors: torch.Tensor):
+    """(what the backward will read, what the forward reads) of q, k, v: heads of 64 and of 128 elements as they are,
+    others widened once, to the backward's 128, of which the forward reads 64 where they fit."""
+    width = tensors[0].shape[-1]
+    if width in (NARROW_HEAD_DIM, HEAD_DIM):
+        return tensors, tensors
+    wide = _widened(tensors, HEAD_DIM)
+    return wide, tuple(t[..., :NARROW_HEAD_DIM] for t in wide) if width < NARROW_HEAD_DIM else wide
+
+
 def _backward(dout, q, k, v, out, lse, sel, seg_off, seg_dest, plan: MobaPlan, scale: float = 0.0, tables=None):
-    """tables: the backward kernels' (tile_off, tile_seg) if the forward made them (made here otherwise)."""
+    """tables: the backward kernels' (tile_off, tile_seg) if the forward made them (made here otherwise).
+    The gradients' heads have dout's width."""
     lib = _lib.load()
     S, H, D = _dims(q)
-    if D < HEAD_DIM:   # (the backward's kernels take heads of 128 elements)
-        dout, q, k, v, out = (torch.nn.functional.pad(x, (0, HEAD_DIM - D)) for x in (dout, q, k, v, out))
-        grads = _backward(dout, q, k, v, out, lse, sel, seg_off, seg_dest, plan, scale or D ** -0.5, tables)
-        return tuple(x[..., :D].contiguous() for x in grads)
+    width = dout.shape[-1]
+    if width < HEAD_DIM:   # (the backward's kernels take heads of 128 elements)
+        grads = _backward(*_widened((dout, q, k, v, out), HEAD_DIM), lse, sel, seg_off, seg_dest, plan,
+                          scale or width ** -0.5, tables)
+        return tuple(x[..., :width].contiguous() for x in grads)
     Hkv = _dims(k)[1]
     dev = q.device
     K = plan.K
@@ -526,15 +556,18 @@ class _MobaAttention(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, v, plan, timer=None, scale=0.0):
+        # (narrow heads are widened and cut in here: autograd would do both once more on the way back)
+        width = q.shape[-1]
+        kept, (q, k, v) = _for_training(q, k, v)
         tables = []  # the backward's tile tables, made by the forward's list stage
         out, lse, sel, seg_off, _, seg_dest, _ = _run_forward(q, k, v, plan, timer, scale, bwd_tables=tables)
         ctx.plan = plan
         ctx.scale = scale
         ctx.aux = (sel, seg_off, seg_dest, tables)
-        ctx.save_for_backward(q, k, v, out, lse)
+        ctx.save_for_backward(*kept, out, lse)
         ctx.mark_non_differentiable(lse)
         ctx.set_materialize_grads(False)  # no zero-filled gradient for lse on the way back
-        return out, lse
+        return (out if out.shape[-1] == width else out[..., :width].contiguous()), lse
 
     @staticmethod
     def backward(ctx, dout, _dlse):
@@ -610,21 +643,22 @@ class _MobaAttentionInGroups(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, v, plan, groups, timer=None, scale=0.0):
-        keep = []
+        keep, width = [], q.shape[-1]
+        kept, (q, k, v) = _for_training(q, k, v)
         out, lse = _forward_in_groups(q, k, v, plan, groups, timer, scale, keep)
         ctx.groups, ctx.keep, ctx.scale = groups, keep, scale
-        ctx.save_for_backward(q, k, v, out, lse)
+        ctx.save_for_backward(*kept, out, lse)
         ctx.mark_non_differentiable(lse)
         ctx.set_materialize_grads(False)
-        return out, lse
+        return (out if out.shape[-1] == width else out[..., :width].contiguous()), lse
 
     @staticmethod
     def backward(ctx, dout, _dlse):
         q, k, v, out, lse = ctx.saved_tensors
         if dout is None:
             return None, None, None, None, None, None, None
-        S, H, D = _dims(q)
-        Hkv = _dims(k)[1]
+        S, H, _ = _dims(q)
+        Hkv, D = _dims(k)[1], dout.shape[-1]
         rep = H // Hkv
         dout = dout.to(q.dtype)
         dq = torch.empty((S, H, D), dtype=q.dtype, device=q.device)
@@ -644,18 +678,21 @@ class _MobaAttentionInGroups(torch.autograd.Function):
 
 def _attend(q, k, v, plan, timer=None, scale=0.0):
     """(out, lse): through autograd when a gradient may be asked for, straight to the kernels otherwise."""
-    S, H, D = _dims(q)
+    S, H, width = _dims(q)
+    D = NARROW_HEAD_DIM if width <= NARROW_HEAD_DIM else HEAD_DIM
     grad = torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad)
     # (the backward's partials are those of heads of 128 elements, whatever the forward's)
     groups = _head_groups(plan, H, _dims(k)[1], HEAD_DIM if grad else D, q.element_size())
-    if len(groups) > 1:
-        if grad:
-            return _MobaAttentionInGroups.apply(q, k, v, plan, groups, timer, scale)
-        return _forward_in_groups(q, k, v, plan, groups, timer, scale, None)
-    plan = _choose_plan(plan, H)
     if grad:
-        return _MobaAttention.apply(q, k, v, plan, timer, scale)
-    return _run_forward(q, k, v, plan, timer, scale)[:2]
+        if len(groups) > 1:
+            return _MobaAttentionInGroups.apply(q, k, v, plan, groups, timer, scale)
+        return _MobaAttention.apply(q, k, v, _choose_plan(plan, H), timer, scale)
+    q, k, v = _widened((q, k, v), D)
+    if len(groups) > 1:
+        out, lse = _forward_in_groups(q, k, v, plan, groups, timer, scale, None)
+    else:
+        out, lse = _run_forward(q, k, v, _choose_plan(plan, H), timer, scale)[:2]
+    return (out if width == D else out[..., :width].contiguous()), lse
 
 
 def moba_attn_varlen(
@@ -735,9 +772,6 @@ def moba_attn_varlen_with_lse(q, k, v, cu_seqlens, max_seqlen, moba_chunk_size, 
         raise ValueError(f"cu_seqlens ends at {plan.S} but q has {q.shape[0]} tokens")
     head_dim = q.shape[2]
     if head_dim not in (HEAD_DIM, NARROW_HEAD_DIM):
-        pad = (0, (NARROW_HEAD_DIM if head_dim < NARROW_HEAD_DIM else HEAD_DIM) - head_dim)
-        q, k, v = (torch.nn.functional.pad(x, pad) for x in (q, k, v))
-        out, lse = _attend(q, k, v, plan, timer, head_dim ** -0.5)
-        return out[..., :head_dim].contiguous(), lse
+        return _attend(q, k, v, plan, timer, head_dim ** -0.5)
     q, k, v = _in_place(q, k, v)
     return _attend(q, k, v, plan, timer)

@@ -524,6 +524,33 @@ def test_narrow_heads_are_padded(head_dim, dtype):
     check_selection(sel, O.select_topk(gate, plan.K), gate)
 
 
+@pytest.mark.parametrize("head_dim,groups", [(32, 1), (1, 1), (63, 2), (65, 1), (96, 2), (127, 1)])
+def test_narrow_heads_in_training_equal_padded_ones(head_dim, groups, monkeypatch):
+    """Gradients of narrow heads, of inputs and of an output gradient that lie strided, are those of heads that the caller
+    pads to 64 or 128, bit for bit, with their own width and contiguous; so with all heads at once and in groups."""
+    from moba_amd import moba_efficient as E
+    S, H, Hkv, B, topk = 1500, 4, 2, 128, 3
+    g = torch.Generator().manual_seed(head_dim)
+    wide = 64 if head_dim < 64 else 128
+    q, k, v, do = (torch.randn((S, h, 2 * head_dim), generator=g).to(torch.bfloat16).cuda()[..., :head_dim] for h in (H, Hkv, Hkv, H))
+    cu_t = torch.tensor([0, 700, S], dtype=torch.int32, device="cuda")
+    plan = E.make_plan(cu_t, B, topk)
+    if groups > 1:
+        monkeypatch.setattr(E, "SCRATCH_LIMIT_BYTES", S * H // groups * (plan.K + 1) * (128 * 2 + 4))
+        assert len(E._head_groups(plan, H, Hkv, 128, 2)) == groups
+    narrow = [x.clone().requires_grad_(True) for x in (q, k, v)]
+    out = E.moba_attn_varlen_gqa(*narrow, cu_t, 800, B, topk)
+    out.backward(do)
+    padded = [torch.nn.functional.pad(x, (0, wide - head_dim)).requires_grad_(True) for x in (q, k, v)]
+    ref = E._attend(*padded, plan, None, head_dim ** -0.5)[0]
+    ref.backward(torch.nn.functional.pad(do, (0, wide - head_dim)))
+    with torch.no_grad():
+        assert torch.equal(out, E.moba_attn_varlen_gqa(*narrow, cu_t, 800, B, topk))
+    assert out.is_contiguous() and torch.equal(out, ref[..., :head_dim])
+    for a, b in zip(narrow, padded):
+        assert a.grad.shape == a.shape and torch.equal(a.grad, b.grad[..., :head_dim])
+
+
 def test_heads_wider_than_128_are_refused():
     from moba_amd import moba_attn_varlen
     q, k, v, _, cu, mx = make_case(1, 256, 1, head_dim=192, seed=3)
