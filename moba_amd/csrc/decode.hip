@@ -401,20 +401,23 @@ static TailSplit tail_split(int B, int Hkv, int rows, int Skv) {
   for (int waves = 4; waves >= (many ? 1 : 4); waves >>= 1) {
     const int unit = kTailKeys * (waves >> t.wr_log2);
     const int steps = (Skv + unit - 1) / unit;
-    const int64_t slots = (int64_t)cus * (waves == 1 ? 5 : 4 / waves);
-    for (int ns = 1; ns <= steps && ns <= kTailMaxSplits && ns <= most; ++ns) {
-      const int per = (steps + ns - 1) / ns, n = (steps + per - 1) / per;  // (no empty split)
+    const int slots = cus * (waves == 1 ? 5 : 4 / waves);
+    auto step_time = [&](int workgroups) {  // with so many of them on the chip
+      const int latency = 92 + 8 * waves * ((workgroups + cus - 1) / cus), bandwidth = 47 * waves * workgroups / cus;
+      return latency > bandwidth ? latency : bandwidth;
+    };
+    const int64_t full = step_time(slots);
+    // (only the numbers of splits that shorten the longest one; none is empty then)
+    for (int n = 1, per; n <= kTailMaxSplits && n <= most; n = (steps - 1) / (per - 1) + 1) {
+      per = (steps + n - 1) / n;
+      const int64_t total = wgs * n, rounds = total / slots;
+      const int rest = (int)(total - rounds * slots);
       int64_t cost;
       if (once) {
-        auto round = [&](int64_t workgroups) {
-          const int64_t latency = 92 + 8 * waves * ((workgroups + cus - 1) / cus), bandwidth = 47 * waves * workgroups / cus;
-          return per * (latency > bandwidth ? latency : bandwidth) + 224;
-        };
-        const int64_t rounds = wgs * n / slots, rest = wgs * n - rounds * slots;
-        cost = (rounds ? rounds * round(slots) : 0) + (rest ? round(rest) : 0);
-        if (n > 1) cost += 227 + 47 * wgs * n * rows / (16 * cus);  // (the merge; the partial results out and in)
+        cost = rounds * (per * full + 224) + (rest ? (int64_t)per * step_time(rest) + 224 : 0);
+        if (n > 1) cost += 227 + 47 * total * rows / (16 * cus);  // (the merge; the partial results out and in)
       } else {  // (bound by the products: whole rounds, each its steps and about one more)
-        cost = (wgs * n + slots - 1) / slots * (per + 1);
+        cost = (rounds + (rest > 0)) * (per + 1);
       }
       if (best < 0 || cost < best) {
         best = cost;
@@ -422,6 +425,7 @@ static TailSplit tail_split(int B, int Hkv, int rows, int Skv) {
         t.nsplit = n;
         t.keys_per_split = per * unit;
       }
+      if (per == 1) break;
     }
   }
   return t;
