@@ -466,11 +466,9 @@ def _run_forward(q, k, v, plan: MobaPlan, timer: Optional[StageTimer] = None, sc
 
 
 def _widened(tensors, width: int):
-    """The tensors with heads of `width` elements, zeros behind narrower ones, which share one buffer (cleared at once:
-    clearing and copying tensor by tensor is what a small call would spend most of its time on)."""
+    """The tensors, some of them with narrower heads, with heads of `width` elements: zeros behind the narrower ones, which
+    share one buffer (cleared at once: clearing tensor by tensor doubles the launches, which bound a small call)."""
     narrow = [t for t in tensors if t.shape[-1] != width]
-    if not narrow:
-        return tuple(tensors)
     rows = [t.numel() // t.shape[-1] for t in narrow]
     parts = iter(torch.zeros((sum(rows), width), dtype=narrow[0].dtype, device=narrow[0].device).split(rows))
     res = []
@@ -687,7 +685,8 @@ def _attend(q, k, v, plan, timer=None, scale=0.0):
         if len(groups) > 1:
             return _MobaAttentionInGroups.apply(q, k, v, plan, groups, timer, scale)
         return _MobaAttention.apply(q, k, v, _choose_plan(plan, H), timer, scale)
-    q, k, v = _widened((q, k, v), D)
+    if width != D:
+        q, k, v = _widened((q, k, v), D)
     if len(groups) > 1:
         out, lse = _forward_in_groups(q, k, v, plan, groups, timer, scale, None)
     else:
