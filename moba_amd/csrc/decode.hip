@@ -17,7 +17,7 @@
 // Keys that one wave reads alone (up to 32 rows) are copied past the caches: 1 x 65536 keys, 64 heads: 368 us without, 314
 // with (6.8 TB/s); keys that several waves or workgroups read are not: 40000 keys, 128 rows: 69.4 us without, 75.6 with.
 //
-// Measured (32 query heads on 8): 131072 keys, one token: 86 us a call = 6.2 TB/s (108 with a vector-unit kernel of 128
+// Measured (32 query heads on 8): 131072 keys, one token: 84 us a call = 6.4 TB/s (108 with a vector-unit kernel of 128
 // splits); 16 x 8191 keys: 84 us = 6.4 TB/s (102); 4 x 20000 keys, 5 tokens: 60 us (348, once per token).
 // Beyond 128 rows per key/value head it is bound by its own instruction chain (one wave per SIMD), 0.45 PFLOP/s.
 //

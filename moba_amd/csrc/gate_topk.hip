@@ -195,7 +195,7 @@ __global__ __launch_bounds__(256, KMAX <= 4 ? 3 : (KMAX <= 16 ? 2 : 1)) void gat
   // lanes on consecutive ints (a lane storing its own K ints touches a cache line for 4K bytes of it).
   __syncthreads();  // (the score tile is read out)
   int* stage = reinterpret_cast<int*>(&sc[0][0][0]);  // [64 tokens][4 heads][K]
-  if (4 * 64 * K <= (int)(sizeof(sc) / sizeof(int))) {  // (uniform; K <= 33)
+  if (4 * 64 * K <= (int)(sizeof(sc) / sizeof(int))) {  // (uniform; K <= 34)
 #pragma unroll
     for (int j = 0; j < KMAX; ++j)
       if (j < K) stage[(lane * 4 + wave) * K + j] = top.idx[j];

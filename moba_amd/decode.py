@@ -1,8 +1,8 @@
 """Decode attention on MI355X: new query tokens against the key/value cache (the adapter's decode
 branch, moba/wrapper.py:76-82, which calls flash_attn_func in the reference: every cached key is
 visible to a new token up to its own position).  One token or a few: the HIP decode kernel reads K and V of
-the cache once, in place, for all query rows of a key/value head.  Many tokens (chunked prefill against a cache):
-the forward attention kernel's causal tiles on the tail of the sequences."""
+the cache in place, once for up to 32 query rows of a key/value head.  Many tokens (chunked prefill against a
+cache): the forward attention kernel's causal tiles on the tail of the sequences."""
 
 from __future__ import annotations
 
@@ -128,8 +128,8 @@ def _tail_tiles(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, sca
 def _takes_tiles(b: int, h: int, hkv: int, q_len: int) -> bool:
     """Whether the causal tiles beat the decode kernel, by the number of 32-row blocks that one walks (rows of a key/value
     head packed together, whole workgroups of 32, 64 or 128 rows) and of 128-row tiles of the other, both times the keys.
-    At 40000 keys a block takes 1.5 us; tiles take 540 us up to about one per compute unit and 2.25 us each in the long
-    run.  Decode kernel / tiles in us: 512 tokens, 32 heads on 8: 681 / 542; 256 tokens: 367 / 540; 4 sequences of 40
+    At 40000 keys a block takes 1.5 us; tiles take 540 us up to about one per compute unit (of 256: as long as 288 blocks
+    and a margin) and 2.25 us each, as long as one and a half blocks, in the long run.  Decode kernel / tiles in us: 512 tokens, 32 heads on 8: 681 / 542; 256 tokens: 367 / 540; 4 sequences of 40
     tokens: 405 / 584; of 100: 787 / 585; 4 x 4096 tokens, 1 head: 741 / 549; 4 x 2048: 402 / 551.  (Up to 16 tokens it is
     always the decode kernel, whose probabilities are not rounded to the element type.)"""
     rows = h // hkv * q_len

@@ -583,8 +583,12 @@ class _MobaAttention(torch.autograd.Function):
 
 def _choose_plan(plan: MobaPlan, H: int) -> MobaPlan:
     """The plan the kernels run: the batch's own, or its form with dense prefixes (MobaPlan.dense_local) where that
-    pays -- when the forward kernel would still keep its workgroups resident, i.e. for problems of many tiles; on
-    a problem of a few hundred tiles the long causal tiles of a dense prefix would run alone at the end."""
+    pays: for problems of many tiles; on a problem of a few hundred tiles the long causal tiles of a dense prefix would run
+    alone at the end.  The measure is whether tiles of FWD_TILE_ROWS rows would be enough for resident workgroups, whichever
+    form the forward takes (forward_tile_rows).  Shorter tiles, one workgroup each, forward / with backward in ms, without and
+    with dense prefixes: 98304 tokens in twelve sequences, 32 heads, chunk 512: 4.69 / 16.6 and 4.39 / 15.9; 65536 tokens,
+    chunk 512, top-k 12: 9.38 / 33.7 and 9.20 / 33.3; 196608 tokens, chunk 256: 7.62 / 22.1 both ways; 64-element heads, 98304
+    tokens, chunk 1024: 2.98 / 17.4 and 2.80 / 17.1; 131072 tokens, chunk 4096, 16 heads: 15.9 / 96.9 and 15.7 / 96.9."""
     if plan.fallback or plan.dense_local:
         return plan
     key = ("dense", H, DENSE_PREFIX)
@@ -715,8 +719,7 @@ def moba_attn_varlen(
 
     The kernels are built for head_dim 128, and those of the forward for 64 too.  Other heads are padded with zeros to
     the next of the two, and for the backward to 128 (the scores, the gate and the softmax scale head_dim ** -0.5 are
-    those of the narrow heads; the padding costs the work
-    and memory of 128); wider heads are refused.
+    those of the narrow heads; the padding costs the work and memory of the wider ones); heads wider than 128 are refused.
     """
     return moba_attn_varlen_with_lse(q, k, v, cu_seqlens, max_seqlen, moba_chunk_size, moba_topk)[0]
 
