@@ -89,7 +89,7 @@ def _tail(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, scaling: 
     scale = float(scaling) if scaling is not None else d ** -0.5
     dtype = _lib.DTYPE_F16 if query.dtype == torch.float16 else _lib.DTYPE_BF16
     strides = (ctypes.c_int64 * 5)(*qs, ks[0], ks[1])
-    stream = torch.cuda.current_stream(dev).cuda_stream
+    stream = E._stream(dev)
     qp, kp, vp, op = q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr()
     for i in range(0, b or 1, MOST_SEQUENCES):   # (one piece, but for very many sequences)
         if i:
@@ -121,7 +121,7 @@ def _tail_tiles(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, sca
     dtype = _lib.DTYPE_F16 if query.dtype == torch.float16 else _lib.DTYPE_BF16
     _lib.check(lib.moba_tail_tiles(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), b, h, hkv, q_len, skv, d,
                                    (ctypes.c_int64 * 6)(*qs, *ks), scale, dtype, 0 if E.FIXED_REFERENCE else 1,
-                                   torch.cuda.current_stream(query.device).cuda_stream), "moba_tail_tiles")
+                                   E._stream(query.device)), "moba_tail_tiles")
     return out
 
 
