@@ -116,6 +116,24 @@ def load():
     return lib
 
 
+_host = None
+
+
+def host():
+    """The extension module of csrc/host.cpp, bound to the library's entry points: built with it, and as little optional."""
+    global _host
+    if _host is None:
+        lib = load()
+        try:
+            from . import _host as module
+        except ImportError as e:
+            raise RuntimeError(f"{os.path.join(_HERE, '_host.so')} cannot be loaded ({e}): build it with "
+                               "`python -m moba_amd.build`") from e
+        module.bind(*(ctypes.cast(f, c_void_p).value for f in (lib.moba_tail_splits, lib.moba_tail, lib.moba_strerror)))
+        _host = module
+    return _host
+
+
 def exported_symbols():
     return list(_SIGNATURES)
 

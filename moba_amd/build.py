@@ -1,4 +1,5 @@
-"""Builds the HIP kernels into ``moba_amd/libmoba_hip.so`` with hipcc for gfx950.
+"""Builds the HIP kernels into ``moba_amd/libmoba_hip.so`` with hipcc for gfx950, and the extension module
+``moba_amd/_host.so`` (csrc/host.cpp, host code) with g++.
 
 Run as ``python -m moba_amd.build``.  hipcc cross-compiles without a GPU.
 """
@@ -8,12 +9,14 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(CSRC, "build")
 LIB = os.path.join(HERE, "libmoba_hip.so")
+HOST = os.path.join(HERE, "_host.so")   # extension module, see csrc/host.cpp
 SOURCES = ["chunk_mean.hip", "gate_topk.hip", "lists.hip", "fwd.hip", "fwd_tile.hip", "bwd.hip", "decode.hip", "plan.hip", "probe.hip", "capi.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -47,11 +50,31 @@ def _compile(src: str, force: bool) -> str:
     return obj
 
 
+def _host_module(force: bool) -> None:
+    """csrc/host.cpp against the installed PyTorch (host code only)."""
+    import torch
+    src = os.path.join(CSRC, "host.cpp")
+    deps = [src, os.path.abspath(__file__)]
+    if not force and os.path.exists(HOST) and all(os.path.getmtime(HOST) > os.path.getmtime(d) for d in deps):
+        return
+    root = os.path.dirname(torch.__file__)
+    include = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
+               os.path.join(os.path.dirname(os.path.dirname(HIPCC)), "include"), sysconfig.get_paths()["include"]]
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *("-I" + d for d in include), src, "-o", HOST,
+           "-L" + os.path.join(root, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed for host.cpp:\n{r.stderr[-8000:]}")
+
+
 def build(force: bool = True, verbose: bool = True) -> str:
     os.makedirs(OBJ, exist_ok=True)
     srcs = [s for s in SOURCES if os.path.exists(os.path.join(CSRC, s))]
-    with ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:
+    with ThreadPoolExecutor(max_workers=min(8, len(srcs) + 1)) as ex:
+        host = ex.submit(_host_module, force)
         objs = list(ex.map(lambda s: _compile(s, force), srcs))
+        host.result()
     # the hand-issued MFMAs of the dK/dV kernel: nothing touches their results too early in the generated code
     from . import asm_check
     report = asm_check.check_dkv_kernel(asm_check.device_assembly(HIPCC, FLAGS, os.path.join(CSRC, "bwd.hip")))

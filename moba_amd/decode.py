@@ -20,22 +20,12 @@ SUPPORTED_GROUP_SIZES = (1, 2, 4, 8)
 
 def supported(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor) -> bool:
     """True when decode_attention can take these tensors ([B,H,1,D] and [B,Hkv,Skv,D])."""
-    return (chunk_supported(query, key, value) and query.shape[2] == 1
-            and query.shape[1] // key.shape[1] in SUPPORTED_GROUP_SIZES)
+    return query.is_cuda and _lib.host().supported(query, key, value, False)
 
 
 def chunk_supported(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor) -> bool:
     """True when chunk_decode_attention can take these tensors ([B,H,q_len,D] and [B,Hkv,Skv,D], q_len <= Skv)."""
-    if not (query.is_cuda and key.is_cuda and value.is_cuda):
-        return False
-    if query.dtype not in (torch.bfloat16, torch.float16) or key.dtype != query.dtype or value.dtype != query.dtype:
-        return False
-    if query.dim() != 4 or key.dim() != 4 or key.shape != value.shape:
-        return False
-    b, h, q_len, d = query.shape
-    if d != 128 or key.shape[0] != b or key.shape[3] != d or not 0 < q_len <= key.shape[2]:
-        return False
-    return key.shape[1] > 0 and h % key.shape[1] == 0
+    return query.is_cuda and _lib.host().supported(query, key, value, True)
 
 
 def _packed(t: torch.Tensor):
@@ -73,6 +63,10 @@ MOST_SEQUENCES = 65535  # that a launch of the decode kernel takes: its grid's t
 def _tail(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, scaling: Optional[float]) -> torch.Tensor:
     """[B,H,q_len,D] against [B,Hkv,Skv,D] -> [B,q_len,H,D] on the decode kernel: the cache is read once for up to 32
     query rows of a key/value head."""
+    out = _lib.host().tail(query, key, value, scaling)
+    if out is not None:
+        return out
+    # tensors that have to be copied first, very many sequences, none at all
     lib = _lib.load()
     b, h, q_len, d = query.shape
     hkv, skv = key.shape[1], key.shape[2]

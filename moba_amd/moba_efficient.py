@@ -51,11 +51,11 @@ def _ptr(t: Optional[torch.Tensor]):
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
-def _stream(device) -> ctypes.c_void_p:
+def _stream(device) -> int:
     if _raw_stream is None:
-        return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+        return torch.cuda.current_stream(device).cuda_stream
     index = device.index
-    return ctypes.c_void_p(_raw_stream(torch.cuda.current_device() if index is None else index))
+    return _raw_stream(torch.cuda.current_device() if index is None else index)
 
 
 def _dtype_code(t: torch.Tensor) -> int:
@@ -303,8 +303,7 @@ class _Geometry:
         tall = self.rows_per_tile == FWD_TILE_ROWS
         self.self_tiles = plan.fwd_self_tiles if tall else plan.self_tiles
         self.self_names = (("fwd_" if tall else "") + "self_tile_prefix", ("fwd_" if tall else "") + "self_tile_chunk")
-        self.tptr = {name: _ptr(t) for name, t in plan.tables.items()}
-        self.null = ctypes.c_void_p(0)
+        self.tptr = {name: t.data_ptr() for name, t in plan.tables.items()}
         self.bound = plan.hist_tile_bound(H, self.rows_per_tile)
         if plan.fallback:
             self.split = 1
@@ -338,7 +337,7 @@ class _Geometry:
         self.part_o_bytes = rows * D * esize
         self.scratch_ints = 8 + 1 + self.bound + self.self_tiles * H
         self.ws_bytes = self.part_o_bytes + rows * 4 + self.scratch_ints * 4
-        self.mean_ws = {}  # kv heads -> fp64 elements of the chunk mean's workspace
+        self.mean = {}     # kv heads -> bytes of the chunk representatives and of the chunk mean's workspace
         self.bwd = {}      # kv heads -> sizes of the backward's scratch
 
 
@@ -379,50 +378,67 @@ def _forward(q, k, v, plan: MobaPlan, timer: Optional[StageTimer] = None, scale:
     return out, lse, sel, seg_off, tile_off, seg_dest, tile_seg
 
 
-def _run_forward(q, k, v, plan: MobaPlan, timer: Optional[StageTimer] = None, scale: float = 0.0, bwd_tables=None):
+def _run_forward(q, k, v, plan: MobaPlan, timer: Optional[StageTimer] = None, scale: float = 0.0, bwd_tables=None,
+                 lists_too=True):
     """q, k, v: [tokens, heads, 128], or batched [batch, heads, tokens, 128] (read in place, see _dims), already
-    addressable (_in_place).  Returns (out, lse, sel, seg_off, tile_off, seg_dest, tile_seg).
+    addressable (_in_place).  Returns (out, lse, sel, seg_off, tile_off, seg_dest, tile_seg), or (out, lse) without
+    lists_too.
     bwd_tables: a list that receives the backward kernels' (tile_off, tile_seg), made on the way.
     The stages are those of chunk_mean(), gate_topk(), build_lists() above, called on precomputed sizes and
-    addresses: at small shapes a forward is bound by the host's time per call."""
+    addresses, in two allocations of scratch (what a backward reads again, and what it does not) and one of each result, and
+    with addresses as plain numbers: at small shapes a forward is bound by the host's time per call (4096 tokens, 4
+    heads: 58 us with an allocation per buffer, a ctypes object per address and a view per list, 44 so)."""
     lib = _lib.load()
     S, H, D = _dims(q)
     Hkv = _dims(k)[1]
     dev = q.device
     K = plan.K
     g = _geometry(plan, lib, H, D, q.element_size())
-    tp, null = g.tptr, g.null
+    tp = g.tptr
     span = (lambda name: timer.span(name, dev)) if timer is not None else (lambda name: _NO_SPAN)
     stream, code, strides = _stream(dev), _dtype_code(q), _strides(q, k)
-    qp, kp, vp = _ptr(q), _ptr(k), _ptr(v)
+    qp, kp, vp = q.data_ptr(), k.data_ptr(), v.data_ptr()
+    out = torch.empty((S, H, D), dtype=q.dtype, device=dev)
+    lse = torch.empty((S, H), dtype=torch.float32, device=dev)
+    outp, lsep = out.data_ptr(), lse.data_ptr()
+    scratch_bytes = g.ws_bytes
+    if not plan.fallback:
+        mean = g.mean.get(Hkv)
+        if mean is None:
+            mean = g.mean[Hkv] = ((plan.F * Hkv * D * q.element_size() + 15) // 16 * 16,
+                                  lib.moba_chunk_mean_workspace_bytes(Hkv, D, plan.F, plan.chunk_size))
+        kbar_at = (g.ws_bytes + 15) // 16 * 16
+        scratch_bytes = kbar_at + mean[0] + mean[1]
+    # the attention's scratch, then the chunk representatives and the chunk mean's workspace
+    ws2 = torch.empty(scratch_bytes, dtype=torch.uint8, device=dev)
+    ws = ws2.data_ptr()
+    part_lsep = ws + g.part_o_bytes
+    queuesp = part_lsep + g.rows * 4
+    sel = seg_off = tile_off = seg_dest = tile_seg = None
     if plan.fallback:
-        sel = seg_off = tile_off = seg_dest = tile_seg = None
-        selp = seg_offp = tile_offp = seg_destp = tile_segp = null
+        selp = seg_offp = tile_offp = seg_destp = tile_segp = None
     else:
-        mean_ws = g.mean_ws.get(Hkv)
-        if mean_ws is None:
-            mean_ws = g.mean_ws[Hkv] = lib.moba_chunk_mean_workspace_bytes(Hkv, D, plan.F, plan.chunk_size) // 8
-        kbar = torch.empty((plan.F, Hkv, D), dtype=q.dtype, device=dev)
-        ws = torch.empty(mean_ws, dtype=torch.float64, device=dev)
-        sel = torch.empty((S, H, K), dtype=torch.int32, device=dev)
-        lists = torch.empty(g.list_starts[-1] if bwd_tables is None else g.list_ints_with_bwd, dtype=torch.int32,
-                            device=dev)
+        # the lists, then the picks
+        sel_at = g.list_starts[-1] if bwd_tables is None else (g.list_ints_with_bwd + 3) // 4 * 4
+        lists = torch.empty(sel_at + S * H * K, dtype=torch.int32, device=dev)
         base = lists.data_ptr()
-        bwd_args = (0, null, null, 0)
+        bwd_args = (0, None, None, 0)
         if bwd_tables is not None:
             b0, b1 = g.bwd_starts
             bwd_tables += [lists[b0:b0 + plan.F * H + 1], lists[b1:b1 + g.bwd_bound]]
-        if bwd_tables is not None and g.rows_per_tile != TILE_ROWS:
-            bwd_args = (TILE_ROWS, ctypes.c_void_p(base + 4 * b0), ctypes.c_void_p(base + 4 * b1), g.bwd_bound)
-        cntp, seg_offp, tile_offp, seg_destp, tile_segp = (ctypes.c_void_p(base + 4 * a) for a in g.list_starts[:5])
-        seg_off, tile_off, seg_dest, tile_seg = (lists[a:a + n] for a, n in zip(g.list_starts[1:5], g.list_sizes[1:]))
-        selp, kbarp = _ptr(sel), _ptr(kbar)
+            if g.rows_per_tile != TILE_ROWS:
+                bwd_args = (TILE_ROWS, base + 4 * b0, base + 4 * b1, g.bwd_bound)
+        cntp, seg_offp, tile_offp, seg_destp, tile_segp = (base + 4 * a for a in g.list_starts[:5])
+        selp, kbarp = base + 4 * sel_at, ws + kbar_at
+        if lists_too:
+            sel = lists[sel_at:].view(S, H, K)
+            seg_off, tile_off, seg_dest, tile_seg = (lists[a:a + n] for a, n in zip(g.list_starts[1:5], g.list_sizes[1:]))
         # the lists' counts are a by-product of the gate: the chunk mean clears the array, the gate adds to it
         with span("chunk_mean"):
-            _lib.check(lib.moba_chunk_mean(kp, tp["fchunk_tok"], kbarp, _ptr(ws), S, Hkv, D, plan.F, plan.chunk_size,
+            _lib.check(lib.moba_chunk_mean(kp, tp["fchunk_tok"], kbarp, kbarp + mean[0], S, Hkv, D, plan.F, plan.chunk_size,
                                            strides, code, cntp, g.list_sizes[0], stream), "moba_chunk_mean")
         with span("gate_topk"):
-            _lib.check(lib.moba_gate_topk(qp, kbarp, tp["cu_seqlens"], tp["seq_fbase"], selp, null, tp["pair_off"],
+            _lib.check(lib.moba_gate_topk(qp, kbarp, tp["cu_seqlens"], tp["seq_fbase"], selp, None, tp["pair_off"],
                                           cntp, S, H, Hkv, D, plan.nseq, plan.F, plan.chunk_size, K, plan.dense_local,
                                           strides, code, stream), "moba_gate_topk")
         with span("build_lists"):
@@ -430,38 +446,33 @@ def _run_forward(q, k, v, plan: MobaPlan, timer: Optional[StageTimer] = None, sc
                                             cntp, seg_offp, tile_offp, seg_destp, tile_segp, S, H, K, plan.N, plan.F,
                                             plan.P, plan.cmax, g.rows_per_tile, g.bound, 1, *bwd_args, plan.dense_local,
                                             stream), "moba_build_lists")
-    out = torch.empty((S, H, D), dtype=q.dtype, device=dev)
-    lse = torch.empty((S, H), dtype=torch.float32, device=dev)
-    ws2 = torch.empty(g.ws_bytes, dtype=torch.uint8, device=dev)
-    base = ws2.data_ptr()
-    part_op = ctypes.c_void_p(base)
-    part_lsep = ctypes.c_void_p(base + g.part_o_bytes)
-    queuesp = ctypes.c_void_p(base + g.part_o_bytes + g.rows * 4)
-    redop = ctypes.c_void_p(base + g.part_o_bytes + g.rows * 4 + 32) if FIXED_REFERENCE else null
+    redop = queuesp + 32 if FIXED_REFERENCE else None
     if g.rows_per_tile == TILE_ROWS and not KEEP_SCRATCH:
-        redop = null    # (these tiles need no list: their workgroups compute them again themselves)
+        redop = None    # (these tiles need no list: their workgroups compute them again themselves)
     if KEEP_SCRATCH:
         at = g.part_o_bytes + g.rows * 4 + 32
         redo = last_scratch["redo"] = ws2[at:at + 4 * (g.scratch_ints - 8)].view(torch.int32) if FIXED_REFERENCE else None
         if redo is not None:
             redo[0] = 0
     with span("fwd_partials"):
-        _lib.check(lib.moba_fwd_partials_rows(qp, kp, vp, part_op, part_lsep, seg_offp, tile_offp, seg_destp,
-                                              tp.get("fchunk_tok", null), tp["achunk_tok"], tp[g.self_names[0]],
-                                              tile_segp, tp[g.self_names[1]], tp["achunk_direct"] if DIRECT_ROWS else null,
-                                              _ptr(out), _ptr(lse), S, H, Hkv, D, K, plan.F, plan.NA,
+        _lib.check(lib.moba_fwd_partials_rows(qp, kp, vp, ws, part_lsep, seg_offp, tile_offp, seg_destp,
+                                              tp.get("fchunk_tok"), tp["achunk_tok"], tp[g.self_names[0]],
+                                              tile_segp, tp[g.self_names[1]], tp["achunk_direct"] if DIRECT_ROWS else None,
+                                              outp, lsep, S, H, Hkv, D, K, plan.F, plan.NA,
                                               plan.chunk_size, g.bound, g.self_tiles, g.split, strides, queuesp,
                                               redop, scale, code, 0, 0, g.rows_per_tile, 0 if FIXED_REFERENCE else 1, stream),
                    "moba_fwd_partials_rows")
     if not DIRECT_ROWS:
         with span("fwd_merge"):
-            _lib.check(lib.moba_fwd_merge(part_op, part_lsep, selp, _ptr(out), _ptr(lse), S, H, D, K, g.split,
-                                          null, null, 0, S, code, stream), "moba_fwd_merge")
+            _lib.check(lib.moba_fwd_merge(ws, part_lsep, selp, outp, lsep, S, H, D, K, g.split,
+                                          None, None, 0, S, code, stream), "moba_fwd_merge")
     elif plan.merge_tokens:   # (the rows of every sequence's first attention chunk are written by the kernel above)
         with span("fwd_merge"):
-            _lib.check(lib.moba_fwd_merge(part_op, part_lsep, selp, _ptr(out), _ptr(lse), S, H, D, K, g.split,
+            _lib.check(lib.moba_fwd_merge(ws, part_lsep, selp, outp, lsep, S, H, D, K, g.split,
                                           tp["mrg_start"], tp["mrg_prefix"], plan.nseq, plan.merge_tokens, code,
                                           stream), "moba_fwd_merge")
+    if not lists_too:
+        return out, lse
     return out, lse, sel, seg_off, tile_off, seg_dest, tile_seg
 
 
@@ -505,7 +516,7 @@ def _backward(dout, q, k, v, out, lse, sel, seg_off, seg_dest, plan: MobaPlan, s
     dev = q.device
     K = plan.K
     g = _geometry(plan, lib, H, D, q.element_size())
-    tp, null = g.tptr, g.null
+    tp = g.tptr
     stream = _stream(dev)
     # One allocation for the call's scratch, every part a multiple of 16 bytes: the per-slot partial dQ, delta and
     # the log2 lse, the 16 tile counters of the two kernels (zeroed by the call), the backward kernels' own tile
@@ -526,9 +537,9 @@ def _backward(dout, q, k, v, out, lse, sel, seg_off, seg_dest, plan: MobaPlan, s
     bound, kv_bytes, starts, split = b
     ws = torch.empty(starts[-1], dtype=torch.uint8, device=dev)
     base = ws.data_ptr()
-    part_dqp, deltap, queuesp, tile_offp, tile_segp, kvp = (ctypes.c_void_p(base + a) for a in starts[:6])
+    part_dqp, deltap, queuesp, tile_offp, tile_segp, kvp = (base + a for a in starts[:6])
     if plan.fallback:
-        tile_offp = tile_segp = null
+        tile_offp = tile_segp = None
     elif tables:
         tile_offp, tile_segp = _ptr(tables[0]), _ptr(tables[1])
     else:
@@ -538,14 +549,14 @@ def _backward(dout, q, k, v, out, lse, sel, seg_off, seg_dest, plan: MobaPlan, s
     dk = torch.empty((S, Hkv, D), dtype=k.dtype, device=dev)
     dv = torch.empty((S, Hkv, D), dtype=v.dtype, device=dev)
     _lib.check(lib.moba_bwd(_ptr(dout), _ptr(q), _ptr(k), _ptr(v), _ptr(out), _ptr(lse), _ptr(sel), _ptr(seg_off),
-                            tile_offp, _ptr(seg_dest), tp.get("fchunk_tok", null), tp["achunk_tok"],
-                            tp["self_tile_prefix"], tile_segp, tp["self_tile_chunk"], tp.get("chunk_fid", null),
+                            tile_offp, _ptr(seg_dest), tp.get("fchunk_tok"), tp["achunk_tok"],
+                            tp["self_tile_prefix"], tile_segp, tp["self_tile_chunk"], tp.get("chunk_fid"),
                             tp["chunk_tok"], tp["kv_tile_prefix"], tp["kv_tile_chunk"], tp["chunk_self_end"],
                             *((tp["achunk_direct"], tp["mrg_start"], tp["mrg_prefix"], plan.nseq, plan.merge_tokens)
-                              if DIRECT_ROWS else (null, null, null, 0, S)),
+                              if DIRECT_ROWS else (None, None, None, 0, S)),
                             deltap, part_dqp, _ptr(dq), _ptr(dk), _ptr(dv), S, H, Hkv, D, K, plan.F, plan.NA,
                             plan.chunk_size, bound, plan.self_tiles, plan.kv_tiles, split, _strides(q, k), queuesp,
-                            kvp if kv_bytes else null, kv_bytes, scale, _dtype_code(q), stream), "moba_bwd")
+                            kvp if kv_bytes else None, kv_bytes, scale, _dtype_code(q), stream), "moba_bwd")
     return dq, dk, dv
 
 
@@ -631,7 +642,7 @@ def _forward_in_groups(q, k, v, plan, groups, timer, scale, keep):
         group_plan = _choose_plan(plan, h1 - h0)
         tables = [] if keep is not None else None
         res = _run_forward(q[:, h0:h1], k[:, h0 // rep:h1 // rep], v[:, h0 // rep:h1 // rep], group_plan, timer,
-                           scale, bwd_tables=tables)
+                           scale, bwd_tables=tables, lists_too=keep is not None)
         out[:, h0:h1] = res[0]
         lse[:, h0:h1] = res[1]
         if keep is not None:
@@ -694,7 +705,7 @@ def _attend(q, k, v, plan, timer=None, scale=0.0):
     if len(groups) > 1:
         out, lse = _forward_in_groups(q, k, v, plan, groups, timer, scale, None)
     else:
-        out, lse = _run_forward(q, k, v, _choose_plan(plan, H), timer, scale)[:2]
+        out, lse = _run_forward(q, k, v, _choose_plan(plan, H), timer, scale, lists_too=False)
     return (out if width == D else out[..., :width].contiguous()), lse
 
 

@@ -13,6 +13,7 @@ from typing import Callable, Optional, Tuple
 import torch
 import torch.nn.functional as F
 
+from . import decode
 from .config import MoBAConfig
 
 
@@ -41,8 +42,7 @@ def _hip_decode(moba_impl, query, key, value, several=False) -> bool:
     anything else decodes with PyTorch's scaled_dot_product_attention."""
     if not getattr(moba_impl, "takes_host_lengths", False):
         return False
-    from .decode import chunk_supported, supported
-    return chunk_supported(query, key, value) if several else supported(query, key, value)
+    return decode.chunk_supported(query, key, value) if several else decode.supported(query, key, value)
 
 
 def hf_to_fa(x: torch.Tensor) -> torch.Tensor:
@@ -123,12 +123,10 @@ def moba_layer(
         )
     elif q_len == 1 and dropout == 0.0 and _hip_decode(moba_impl, query, key, value):
         # one new token against the cache: the HIP decode kernel reads K and V once, in place
-        from .decode import decode_attention
-        out = decode_attention(query, key, value, scaling)
+        out = decode.decode_attention(query, key, value, scaling)
     elif q_len < kv_len and dropout == 0.0 and _hip_decode(moba_impl, query, key, value, several=True):
         # several new tokens against the cache: the decode kernel, or the forward kernel's causal tiles
-        from .decode import chunk_decode_attention
-        out = chunk_decode_attention(query, key, value, scaling)
+        out = decode.chunk_decode_attention(query, key, value, scaling)
     else:
         # decode: every cached key is visible to the new queries (bottom-right aligned causal mask)
         mask = None

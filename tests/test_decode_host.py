@@ -40,3 +40,29 @@ def test_tensors_read_in_place_and_copied():
     v = _as_strided((1, 4, 10, 128), (8192, 1280, 128, 1))
     q, k2, v2, qs, ks = _placed_three(k, k, v, 128)
     assert ks == (0, 1280, 128) and qs == (0, 2048, 128) and torch.equal(k2, k) and torch.equal(v2, v)
+
+
+def test_the_extension_reads_in_place_what_the_general_path_does():
+    """csrc/host.cpp decides on strides and addresses as _placed does, over layouts of every kind."""
+    import random
+    from moba_amd import _lib
+    from moba_amd.decode import _placed
+    host, rng, kept = _lib.host(), random.Random(1), 0
+    for _ in range(3000):
+        shape = tuple(rng.choice((1, 1, 2, 3)) for _ in range(3)) + (128,)
+        strides = tuple(rng.choice((0, 3, 8, 100, 128, 256, 1024, 1 << 23, (1 << 23) + 8)) for _ in range(3)) + (rng.choice((1, 1, 1, 2)),)
+        span = sum((n - 1) * s for n, s in zip(shape, strides)) + 1
+        if span > 1 << 22:
+            continue     # (memory)
+        base = torch.empty(span + 8, dtype=torch.bfloat16)
+        t = base.as_strided(shape, strides, rng.choice((0, 0, 0, 1, 8)))     # (also odd addresses)
+        step = rng.choice((0, 128))
+        got, steps = _placed(t, step)
+        same = got.data_ptr() == t.data_ptr() and got.stride() == t.stride()
+        native = host.in_place(t, step)
+        if native is not None:
+            kept += 1
+            assert same and native == steps, (shape, strides, step)
+        else:
+            assert not same or t.is_contiguous(), (shape, strides, step)
+    assert kept > 200
