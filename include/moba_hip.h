@@ -58,7 +58,7 @@ extern "C" {
 
 enum { MOBA_DTYPE_BF16 = 0, MOBA_DTYPE_F16 = 1 };
 
-#define MOBA_ABI_VERSION 117 /* the signatures below; moba_version() returns the number the library was built with */
+#define MOBA_ABI_VERSION 118 /* the signatures below; moba_version() returns the number the library was built with */
 int moba_version(void);
 const char* moba_strerror(int code);
 
@@ -312,11 +312,14 @@ int moba_fwd(const void* q, const void* k, const void* v, void* part_o, float* p
  *              of 64 * dq_key_split (MOBA_ERR_ARG otherwise).
  *   dq, dk, dv: out; dk and dv of a key/value head sum over its query heads
  *   queues [16] int32 scratch: tile counters of the dQ and dK/dV kernels (as in moba_fwd_partials)
- *   dkv_scratch: moba_bwd_dkv_scratch_bytes(S, Hkv, kv_tiles) bytes, 16-byte aligned, or null.  With few key tiles
- *              (fewer than two per compute unit, S >= 4096) the dK/dV kernel cuts each into up to 4 parts that run
- *              side by side and leave fp32 sums there, added up in a fixed order (deterministic all the same);
- *              without the scratch, or when the query returns 0, every tile is one piece.
+ *   dkv_shares, dkv_scratch: with few key tiles (fewer than two per compute unit) the dK/dV kernel walks the work of all
+ *              key tiles of a head in dkv_shares = moba_bwd_dkv_shares() equal shares; the fp32 sums of the tiles that
+ *              several shares have parts of go through dkv_scratch, moba_bwd_dkv_scratch_bytes(S, Hkv, kv_tiles) bytes,
+ *              16-byte aligned, and are added up in a fixed order (deterministic all the same).  Without the scratch (null, or
+ *              too small) or with dkv_shares = 0, every tile is one piece.  A call for some of the heads gives what a call
+ *              for all would, bit for bit, with that call's dkv_shares.
  *   softmax_scale: as in the forward call */
+int moba_bwd_dkv_shares(int64_t S, int Hkv, int64_t kv_tiles);
 size_t moba_bwd_dkv_scratch_bytes(int64_t S, int Hkv, int64_t kv_tiles);
 int moba_bwd_dq_key_split(int64_t S, int H, int K, int B, int64_t hist_bound, int64_t self_tiles);
 int moba_bwd(const void* dout, const void* q, const void* k, const void* v, const void* out, const float* lse,
@@ -329,7 +332,7 @@ int moba_bwd(const void* dout, const void* q, const void* k, const void* v, cons
              void* dk, void* dv, int64_t S, int H,
              int Hkv, int D, int K, int F, int N, int B, int64_t hist_bound, int64_t self_tiles, int64_t kv_tiles,
              int dq_key_split, const int64_t* strides, int32_t* queues, void* dkv_scratch, int64_t dkv_scratch_bytes,
-             float softmax_scale, int dtype, void* stream);
+             int dkv_shares, float softmax_scale, int dtype, void* stream);
 
 /* Decode: the last nq tokens of every sequence against its key/value cache.  Replaces the
  * flash_attn_func call of the adapter's decode branch, moba/wrapper.py:76-82 (grouped-query heads, bottom-right

@@ -60,17 +60,31 @@ struct BwdParams {
   TileTables t;
   float scale_log2;
   float scale;
-  uint32_t hk_magic;  // n / (H*K1) == (n * hk_magic) >> hk_shift for every n < 2^31
+  uint32_t hk_magic;  // n / (H*K1) == (n * hk_magic) >> hk_shift for every n < 2^31 (H*K1 >= 2)
   uint32_t hk_shift;
   int* queues;        // [16] tile counters, one per XCD, of the dQ kernel and of the dK/dV kernel; zero at the start
-  // Small problems: every key tile of the dK/dV kernel is cut into dkv_split parts (its heads' stages in equal
-  // shares) that run as tiles of their own and leave fp32 sums in part_dkv [tiles * dkv_split][2][128][128],
-  // which bwd_dkv_reduce_kernel adds up in a fixed order.  dkv_split = 1: whole tiles, dk and dv written directly.
+  // Problems of few key tiles: the stages of all key tiles of a key/value head, one tile's behind the other's, are cut into equal
+  // shares (bwd_dkv_tiles).  share_tiles [Hkv * kv_tiles + 1]: the tiles, head by head, worked out by bwd_delta_kernel; part_dkv:
+  // the fp32 sums of the tiles that several shares have parts of, which bwd_dkv_reduce_kernel adds up in the
+  // order of the shares: those of tile j and share i of head h are number h * (kv_tiles + dkv_shares) + i + j.
   float* part_dkv;
-  int dkv_split;
+  struct ShareTile* share_tiles;
+  int kv_tiles;    // of a head
+  int dkv_shares;  // the most there are of a head; 0: whole tiles, drawn from the queues
+  uint32_t k1_magic, k1_shift, h_magic, h_shift;  // as hk_magic, for divisions by K1 and by H
   // 3: eight queues, one per XCD (tiles that share rows or keys run behind one L2); 0: one queue for all, for a
   // problem of few tiles per workgroup, whose ids come longest tile first: whoever is free takes the longest left
   int queues_log2;
+};
+
+// A key tile where the query heads' rows are walked in one go: those that attend its keys causally, head by head, then the
+// gather lists of all heads, which lie one behind the other.
+struct alignas(32) ShareTile {
+  int begin;                // its first place (share_count)
+  int tok0, keys;           // first token, keys of the chunk from there on
+  int self_rows;            // rows per head that attend its keys causally: tokens tok0 .. tok0 + self_rows - 1
+  int list_base, list_rows;
+  int unused[2];
 };
 
 // which 128-key tile of which key/value head: the forward's self-tile enumeration over the chunks and Hkv heads
@@ -93,17 +107,71 @@ __device__ __forceinline__ KvTile decode_kv_tile(const BwdParams<E>& p, int st) 
   return t;
 }
 
+// The shares of a head, equal in places: its stages have one each, of about 2 us, and every tile begins with kTileStart empty
+// ones, for what its start costs (its lookups, keys, first copies and products: 9 to 12 us).  A share should have at
+// least kMinShare.  (Nothing of another head goes into this: a call for some of the heads gives the same sums.)
+constexpr int kTileStart = 5, kMinShare = 16;
+__device__ __forceinline__ int share_count(int places, int most) { return max(1, min(most, places / kMinShare)); }
+__device__ __forceinline__ int share_begin(int places, int shares, int i) { return (int)((int64_t)places * i / shares); }
+// the share that holds place x
+__device__ __forceinline__ int share_of(int places, int shares, int x) { return (int)((((int64_t)x + 1) * shares - 1) / places); }
+
+// tile number `at`, head by head; `places` receives its number of places
+template <class E>
+__device__ __forceinline__ ShareTile share_tile(const BwdParams<E>& p, int at, int& places) {
+  const int hkv = at / p.kv_tiles, j = at - hkv * p.kv_tiles, c = p.kv_tile_chunk[j], key0 = (j - p.kv_tile_prefix[c]) * TM;
+  ShareTile t = {};
+  t.tok0 = p.kv_chunk_tok[c] + key0;
+  t.keys = p.kv_chunk_tok[c + 1] - t.tok0;
+  t.self_rows = p.chunk_self_end[c] - t.tok0;
+  const int fid = (p.chunk_fid && p.t.K1 > 1) ? p.chunk_fid[c] : -1;
+  if (fid >= 0) {
+    const int* off = p.t.seg_off + fid * p.t.H + hkv * p.t.rep;
+    t.list_base = off[0];
+    t.list_rows = off[p.t.rep] - t.list_base;
+  }
+  places = kTileStart + (t.self_rows + TQ - 1) / TQ * p.t.rep + (t.list_rows + TQ - 1) / TQ;
+  return t;
+}
 template <class E>
 __global__ __launch_bounds__(256) void bwd_delta_kernel(const typename E::elem* __restrict__ dout,
                                                         const typename E::elem* __restrict__ out,
                                                         const float* __restrict__ lse, float* __restrict__ delta,
                                                         float* __restrict__ lse2, int64_t rows,
-                                                        int* __restrict__ queues) {
+                                                        int* __restrict__ queues, const BwdParams<E> p) {
   MOBA_ELEM_TYPES(E)
+  const int extra = p.dkv_shares ? 1 : 0;
+  if (extra && blockIdx.x == 0) {  // the key tiles' first places: a thread adds up some tiles in a row
+    __shared__ int sums[4];
+    const int per = (p.kv_total + 255) / 256, t0 = min((int)threadIdx.x * per, p.kv_total), t1 = min(t0 + per, p.kv_total);
+    int sum = 0, places;
+    for (int t = t0; t < t1; ++t) {
+      share_tile(p, t, places);
+      sum += places;
+    }
+    int inc = sum;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int x = __shfl_up(inc, o, 64);
+      if ((int)(threadIdx.x & 63) >= o) inc += x;
+    }
+    if ((threadIdx.x & 63) == 63) sums[threadIdx.x >> 6] = inc;
+    __syncthreads();
+    int at = inc - sum;
+    for (int w = 0; w < (int)(threadIdx.x >> 6); ++w) at += sums[w];
+    for (int t = t0; t < t1; ++t) {
+      ShareTile x = share_tile(p, t, places);
+      x.begin = at;
+      p.share_tiles[t] = x;
+      at += places;
+    }
+    if (threadIdx.x == 255) p.share_tiles[p.kv_total].begin = at;
+    return;
+  }
   // the 16 tile counters of the two kernels that follow start at zero (here: one launch less than a kernel of its
   // own, and, unlike a memset, safe to record into a graph)
-  if (blockIdx.x == 0 && threadIdx.x < 16) queues[threadIdx.x] = 0;
-  const int64_t row = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
+  if (blockIdx.x == extra && threadIdx.x < 16) queues[threadIdx.x] = 0;
+  const int64_t row = (int64_t)(blockIdx.x - extra) * 16 + (threadIdx.x >> 4);
   const int c8 = threadIdx.x & 15;
   float acc = 0.f;
   if (row < rows) {
@@ -518,8 +586,16 @@ __global__ __launch_bounds__(256) void bwd_dq_reduce_kernel(const typename E::el
 // ------------------------------------------------------------------------------------ dK, dV
 // kBatched: q is a batched layout (rows of different batch entries are not an affine function of the token);
 // the common case has no division and no branch in the address of a gathered Q row.
-// kParts: tiles cut into dkv_split parts (a form of its own: the other has no scalar registers to
-// spare, 302060 tokens, 32 heads, forward and backward: 104.8 ms with both in one, 104.3 before, and no slower apart).
+// kParts: the stages of all key tiles in equal shares, drawn from a queue (a form of its own: the other has no scalar
+// registers to spare).  Of a tile all query heads' rows are walked in one pipeline: their lists lie one behind the other,
+// and a row is known by its number token * H + head alone.  (kBatched then stands for any layout of q but the packed one,
+// whose rows lie in the order of their numbers.)
+// With few tiles the time is that of the workgroup with the most to do, and what a tile costs beside its stages of 2.2 us: 9 to
+// 12 us for lookups, keys, first copies and products.  One share per workgroup leaves the ends within 5 % and two starts
+// each.  Forward and backward, tiles in four parts each and every head a pipeline of its own / shares: 32768 tokens, one
+// head, chunk 2048: 485 / 470 us; 20480 tokens in five sequences, 8 heads on 2, chunk 512: 666 / 647; 7900 tokens, 8
+// heads on one: 375 / 296.  Whole tiles / shares below 4096 tokens: 3900 tokens, 16 heads on 4, chunk 1024: 506 / 324; 3000 tokens, 4
+// heads on one: 308 / 148.
 template <class E, bool kBatched, bool kParts>
 __device__ __forceinline__ void bwd_dkv_tiles(const BwdParams<E>& p) {
   MOBA_ELEM_TYPES(E)
@@ -535,7 +611,50 @@ __device__ __forceinline__ void bwd_dkv_tiles(const BwdParams<E>& p) {
   // finish together.  A tile runs for about a millisecond: the draw (one atomic, two barriers) is free.
   const int ql = p.queues_log2, qmask = (1 << ql) - 1;
   int queue = blockIdx.x & qmask, empty_queues = 0;
+  int place = 0, share_end = 0, share_tile = 0, share = 0;  // kParts: next place of the share, its end, its tile, its number in its head
   while (true) {
+  ShareTile st = {};
+  int unit = 0, q_first = 0, q_last = 0x7fffffff, slot = -1;  // kParts: the tile's stages q_first .. q_last - 1, and where their sums go
+  if constexpr (kParts) {
+    int* const word = reinterpret_cast<int*>(smem + kDkvIdSlot);
+    if (place >= share_end) {  // the next share
+      __syncthreads();
+      if (tid == 0) word[0] = __hip_atomic_fetch_add(p.queues + 8, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __syncthreads();
+      // whose it is: a lane per head
+      const int drawn = __builtin_amdgcn_readfirstlane(word[0]), hl = min(lane, Hkv - 1);
+      const int b = p.share_tiles[hl * p.kv_tiles].begin, n = p.share_tiles[(hl + 1) * p.kv_tiles].begin - b;
+      const int mine = lane < Hkv ? share_count(n, p.dkv_shares) : 0;
+      int inc = mine;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int x = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += x;
+      }
+      const uint64_t after = __ballot(drawn < inc);
+      if (!after) break;  // no share left
+      const int hkv = __builtin_ctzll(after), shares = __builtin_amdgcn_readlane(mine, hkv);
+      const int begin = __builtin_amdgcn_readlane(b, hkv), places = __builtin_amdgcn_readlane(n, hkv);
+      share = drawn - (__builtin_amdgcn_readlane(inc, hkv) - shares);
+      place = begin + share_begin(places, shares, share);
+      share_end = begin + share_begin(places, shares, share + 1);
+      for (int t = hkv * p.kv_tiles + tid; t < (hkv + 1) * p.kv_tiles; t += 256)
+        if (p.share_tiles[t].begin <= place && place < p.share_tiles[t + 1].begin) word[1] = t;
+      __syncthreads();
+      share_tile = __builtin_amdgcn_readfirstlane(word[1]);
+    }
+    unit = share_tile++;
+    st = table_load(p.share_tiles + unit);
+    const int begin = st.begin + kTileStart, end = table_load(&p.share_tiles[unit + 1].begin);
+    q_first = max(place - begin, 0);
+    q_last = min(share_end, end) - begin;
+    place = min(share_end, end);
+    if (q_last <= q_first) continue;  // (nothing but of its start)
+    if (q_first > 0 || end > share_end) {
+      const int hkv = unit / p.kv_tiles;
+      slot = hkv * p.dkv_shares + unit + share;  // (= hkv * (kv_tiles + dkv_shares) + tile of the head + share)
+    }
+  } else {
   __syncthreads();  // every wave is done with the LDS of the previous tile and has read the previous draw
   if (tid == 0)
     *reinterpret_cast<int*>(smem + kDkvIdSlot) =
@@ -543,25 +662,34 @@ __device__ __forceinline__ void bwd_dkv_tiles(const BwdParams<E>& p) {
   __syncthreads();
   const int drawn = __builtin_amdgcn_readfirstlane(*reinterpret_cast<const int*>(smem + kDkvIdSlot));
   const int64_t id = (((int64_t)(drawn / kXcdBlock) << ql) + queue) * kXcdBlock + (drawn % kXcdBlock);
-  const int split = kParts ? p.dkv_split : 1;
-  if (id >= (int64_t)p.kv_total * split) {
+  if (id >= (int64_t)p.kv_total) {
     queue = (queue + 1) & qmask;
     if (++empty_queues > qmask) break;
     continue;
   }
   empty_queues = 0;
-  // ---- which part of which 128-key tile (consecutive ids: the parts of one tile) ----
-  const int unit = (int)id;
-  const int part = unit % split;
-  const KvTile kt = decode_kv_tile(p, unit / split);
+  unit = (int)id;
+  }
+  KvTile kt;
+  if constexpr (kParts) kt = {-1, unit / p.kv_tiles, 0, st.tok0, st.keys, st.self_rows};
+  else kt = decode_kv_tile(p, unit);
   const int c = kt.c, hkv = kt.hkv, c0 = kt.c0, len = kt.len, key0 = kt.key0;
   const int mykey = key0 + wave * 32 + n;        // position inside the chunk
   const bool key_valid = mykey < len;
 
   // ---- the rows that attend these keys: the causal rows (of the chunk, or of its dense prefix), then the gather list ----
   const int self_rows = kt.self_len - key0;      // chunk positions key0 .. self_len-1
-  const int nself = (self_rows + TQ - 1) / TQ;
-  const int fid = (p.chunk_fid && K1 > 1) ? p.chunk_fid[c] : -1;
+  int nself = (self_rows + TQ - 1) / TQ;
+  const int fid = !kParts && p.chunk_fid && K1 > 1 ? p.chunk_fid[c] : -1;
+  const int nself1 = nself;  // (kParts: of one head; nself counts those of all)
+  const uint32_t nself_magic = (uint32_t)(0xffffffffu / (uint32_t)nself1) + 1;  // qi / nself1 = high word of the product, for qi * nself1 < 2^32
+  // kParts: head and first position of a causal stage
+  auto self_stage = [&](int qi, int& head) __attribute__((always_inline)) {
+    int g = 0;
+    if (nself != nself1) g = nself1 == 1 ? qi : (int)__umulhi((uint32_t)qi, nself_magic);  // (nself == nself1: one head)
+    head = hkv * rep + g;
+    return (qi - g * nself1) * TQ;
+  };
   // the query heads of this key/value head are walked one after the other; per head:
   int h = hkv * rep, list_base = 0, list_rows = 0, ntile = nself;
   auto select_head = [&](int hq) __attribute__((always_inline)) {
@@ -574,6 +702,12 @@ __device__ __forceinline__ void bwd_dkv_tiles(const BwdParams<E>& p) {
     }
     ntile = nself + (list_rows + TQ - 1) / TQ;
   };
+  if constexpr (kParts) {
+    nself *= rep;
+    list_base = st.list_base;
+    list_rows = st.list_rows;
+    ntile = q_last;
+  }
 
   // ---- K^T and V^T operands of this lane's key: [16*ks + 8*hh .. +7] ----
   elem8 bk[8], bv[8];
@@ -604,15 +738,25 @@ __device__ __forceinline__ void bwd_dkv_tiles(const BwdParams<E>& p) {
   uint64_t q_lane_base = 0, do_lane_base = 0;  // this lane's 16 bytes in token 0's row of q and dO, head h
   auto set_lane_bases = [&]() __attribute__((always_inline)) {
     const int c16 = ld_pc ^ (ld_rin << 2) ^ (wave_u & 3);  // sw_col16(4*slab + ld_rin, ld_pc) for slab = 4*i + wave
-    q_lane_base = (uint64_t)p.q + (uint64_t)((int64_t)h * p.t.q_head_b + c16 * 16);
-    do_lane_base = (uint64_t)p.dout + (uint64_t)(h * (kHeadDim * 2) + c16 * 16);
+    q_lane_base = (uint64_t)p.q + (uint64_t)((kParts ? 0 : (int64_t)h * p.t.q_head_b) + c16 * 16);
+    do_lane_base = (uint64_t)p.dout + (uint64_t)((kParts ? 0 : h * (kHeadDim * 2)) + c16 * 16);
   };
-  int toks[5];  // tokens of the rows of the stage whose copies are being issued
+  int toks[5];  // tokens (kParts: numbers) of the rows of the stage whose copies are being issued
   auto prepare_stage = [&](int qi) __attribute__((always_inline)) {
     // (a list entry is (token*H + h)*K1 + 1 + slot with H*K1 >= 2: the quotient by H*K1 is the high word of the
     // product with the magic number, shifted; exact for entries below 2^31)
-    toks[4] = qi < nself ? c0 + key0 + min(qi * TQ + lane, self_rows - 1)
-                         : (int)(__umulhi((uint32_t)raw, p.hk_magic) >> (p.hk_shift - 32));
+    if constexpr (kParts) {
+      if (qi < nself) {
+        int head;
+        const int pos0 = self_stage(qi, head);
+        toks[4] = (c0 + key0 + min(pos0 + lane, self_rows - 1)) * H + head;
+      } else {
+        toks[4] = (int)(__umulhi((uint32_t)raw, p.k1_magic) >> (p.k1_shift - 32));
+      }
+    } else {
+      toks[4] = qi < nself ? c0 + key0 + min(qi * TQ + lane, self_rows - 1)
+                           : (int)(__umulhi((uint32_t)raw, p.hk_magic) >> (p.hk_shift - 32));
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) toks[i] = __builtin_amdgcn_ds_bpermute(row_src_lane4 + 64 * i, toks[4]);
   };
@@ -627,7 +771,20 @@ __device__ __forceinline__ void bwd_dkv_tiles(const BwdParams<E>& p) {
     const uint32_t qdst = lds_base + buf * kQStage;
     const int i = g >> 1;
     const int slab = 4 * i + wave_u;
-    if ((g & 1) == 0) {
+    if constexpr (kParts) {
+      if ((g & 1) == 0) {
+        uint64_t src = q_lane_base;
+        if constexpr (kBatched) {
+          const int tok = H == 1 ? toks[i] : (int)(__umulhi((uint32_t)toks[i], p.h_magic) >> (p.h_shift - 32));
+          src += (uint64_t)(q_tok_bytes(p.t, tok) + (int64_t)(toks[i] - tok * H) * p.t.q_head_b);
+        } else {
+          src += (uint64_t)(uint32_t)toks[i] * (kHeadDim * 2);
+        }
+        async_copy16((const char*)src, qdst + slab * 1024);
+      } else {
+        async_copy16((const char*)(do_lane_base + (uint64_t)(uint32_t)toks[i] * (kHeadDim * 2)), qdst + TQ * kHeadDim * 2 + slab * 1024);
+      }
+    } else if ((g & 1) == 0) {
       if constexpr (kBatched)
         async_copy16((const char*)q_lane_base + q_tok_bytes(p.t, toks[i]), qdst + slab * 1024);
       else
@@ -637,7 +794,7 @@ __device__ __forceinline__ void bwd_dkv_tiles(const BwdParams<E>& p) {
                    qdst + TQ * kHeadDim * 2 + slab * 1024);
     }
     if (g == 7 && wave_u < 2) {
-      const float* src = (wave_u == 0 ? p.lse2 : p.delta) + ((int64_t)toks[4] * H + h);
+      const float* src = (wave_u == 0 ? p.lse2 : p.delta) + (kParts ? (int64_t)toks[4] : (int64_t)toks[4] * H + h);
       async_copy4(src, qdst + 2 * TQ * kHeadDim * 2 + wave_u * (TQ * 4));
     }
   };
@@ -801,37 +958,9 @@ __device__ __forceinline__ void bwd_dkv_tiles(const BwdParams<E>& p) {
     }
   };
 
-  // This part's share of the stages of all heads, one head's behind the other's: a head costs a part the start of a
-  // pipeline (lookups, first copies, first products: 3 us, two stages' time), so a part should meet few of them.  (A
-  // share of every head's stages instead: 271 us where this takes 253, 20480 tokens in five sequences, 8 heads on 2, chunk 512.)
-  int skip = 0, left = 0x7fffffff;  // stages before the part's first one, and how many it has
-  if constexpr (kParts) {
-    int total = nself * rep;
-    if (fid >= 0) {
-      const int* ends = p.t.seg_off + fid * H + hkv * rep;
-      int before = table_load(ends);
-      for (int i = 1; i <= rep; ++i) {
-        const int end = table_load(ends + i);
-        total += (end - before + TQ - 1) / TQ;
-        before = end;
-      }
-    }
-    skip = (int)((int64_t)total * part / split);
-    left = (int)((int64_t)total * (part + 1) / split) - skip;
-    // (vector registers, of which there are some left, hold the two across the stage loop: scalar ones are short there)
-    asm volatile("" : "+v"(skip));
-    asm volatile("" : "+v"(left));
-  }
-  for (int hq = hkv * rep; hq < (hkv + 1) * rep; ++hq) {
-  select_head(hq);
-  int q_first = 0, q_end = ntile;
-  if constexpr (kParts) {
-    q_first = min(__builtin_amdgcn_readfirstlane(skip), ntile);
-    q_end = q_first + min(__builtin_amdgcn_readfirstlane(left), ntile - q_first);
-    skip -= q_first;
-    left -= q_end - q_first;
-  }
-  if (q_end == q_first) continue;  // (uniform)
+  for (int hq = hkv * rep; hq < (kParts ? hkv * rep + 1 : (hkv + 1) * rep); ++hq) {
+  if constexpr (!kParts) select_head(hq);
+  const int q_end = ntile;
   set_lane_bases();
   __syncthreads();  // every wave is done with the LDS stages of the previous head
   raw = 0;
@@ -864,8 +993,10 @@ __device__ __forceinline__ void bwd_dkv_tiles(const BwdParams<E>& p) {
     const bool has_next = qi + 1 < q_end;
     const bool is_self = qi < nself;
     // number of real rows in this stage, and for self stages the chunk position of row 0
-    const int rows_here = is_self ? min(TQ, self_rows - qi * TQ) : min(TQ, list_rows - (qi - nself) * TQ);
-    const int qpos0 = key0 + qi * TQ;  // only meaningful for self stages
+    int pos0 = qi * TQ, head;
+    if constexpr (kParts) pos0 = self_stage(qi, head);
+    const int rows_here = is_self ? min(TQ, self_rows - pos0) : min(TQ, list_rows - (qi - nself) * TQ);
+    const int qpos0 = key0 + pos0;  // only meaningful for self stages
     // causal masking can only bite while the stage's first row is before the wave's last key
     const bool masked = (rows_here < TQ) || (is_self && qpos0 < key0 + wave * 32 + 31);
     // the block after the last one is the last one again: its S is computed and dropped
@@ -896,9 +1027,9 @@ __device__ __forceinline__ void bwd_dkv_tiles(const BwdParams<E>& p) {
   wait_vmem();  // (the copies past the last stage: nothing may be on its way into LDS when the workgroup ends)
   }  // query heads
 
-  if constexpr (kParts) {
+  if (kParts && slot >= 0) {
     // this part's sums, unscaled, in fp32: [dk, dv][key of the tile][128]
-    float* dst = p.part_dkv + (int64_t)unit * (2 * TM * kHeadDim) + (wave * 32 + n) * kHeadDim + 4 * hh;
+    float* dst = p.part_dkv + (int64_t)slot * (2 * TM * kHeadDim) + (wave * 32 + n) * kHeadDim + 4 * hh;
 #pragma unroll
     for (int db = 0; db < 4; ++db)
 #pragma unroll
@@ -936,25 +1067,29 @@ __global__ __launch_bounds__(256, 1) void bwd_dkv_parts_kernel(const BwdParams<E
   bwd_dkv_tiles<E, kBatched, true>(p);
 }
 
-// dk, dv of the 128-key tiles from the fp32 sums of their parts, added in the order of the parts.
-// Sixteen workgroups per tile; a thread owns four consecutive elements of one key (coalesced 16-byte loads).
+// dk, dv of the 128-key tiles that several shares have parts of, from the fp32 sums of the parts, added in the order of the
+// shares.  Sixteen workgroups per tile; a thread owns four consecutive elements of one key (coalesced 16-byte loads).
 template <class E>
 __global__ __launch_bounds__(256) void bwd_dkv_reduce_kernel(const BwdParams<E> p) {
   MOBA_ELEM_TYPES(E)
-  const int tile = blockIdx.x >> 4;
-  const KvTile kt = decode_kv_tile(p, tile);
+  const int tile = blockIdx.x >> 4, hkv = tile / p.kv_tiles;
+  const int head = table_load(&p.share_tiles[hkv * p.kv_tiles].begin);
+  const int places = table_load(&p.share_tiles[(hkv + 1) * p.kv_tiles].begin) - head, shares = share_count(places, p.dkv_shares);
+  const ShareTile st = table_load(p.share_tiles + tile);
+  const int begin = st.begin - head + kTileStart, end = table_load(&p.share_tiles[tile + 1].begin) - head;
+  const int first = share_of(places, shares, begin), last = share_of(places, shares, end - 1);
+  if (first == last) return;  // (one workgroup had the whole tile and wrote dk and dv itself)
   const int in_tile = (blockIdx.x & 15) * 256 + threadIdx.x;  // 128 keys x 32 groups of four elements
   const int key = in_tile >> 5, d = (in_tile & 31) * 4;
-  if (kt.key0 + key >= kt.len) return;
-  const int split = p.dkv_split;
-  const float* src = p.part_dkv + (int64_t)tile * split * (2 * TM * kHeadDim) + key * kHeadDim + d;
+  if (key >= st.keys) return;
+  const float* src = p.part_dkv + (int64_t)(hkv * p.dkv_shares + tile) * (2 * TM * kHeadDim) + key * kHeadDim + d;
   f32x4 sk = {0.f, 0.f, 0.f, 0.f}, sv = sk;
-  for (int r = 0; r < split; ++r) {
+  for (int r = first; r <= last; ++r) {
     const float* s = src + (int64_t)r * (2 * TM * kHeadDim);
     sk += *reinterpret_cast<const f32x4*>(s);
     sv += *reinterpret_cast<const f32x4*>(s + TM * kHeadDim);
   }
-  const int64_t off = ((int64_t)(kt.c0 + kt.key0 + key) * p.t.Hkv + kt.hkv) * kHeadDim + d;
+  const int64_t off = ((int64_t)(st.tok0 + key) * p.t.Hkv + hkv) * kHeadDim + d;
   u32x2 wk, wv;
   wk[0] = pack2<E>(sk[0] * p.scale, sk[1] * p.scale);
   wk[1] = pack2<E>(sk[2] * p.scale, sk[3] * p.scale);
@@ -974,7 +1109,7 @@ static int launch_bwd(const void* dout, const void* q, const void* k, const void
                       const int32_t* kv_tile_prefix, const int32_t* kv_tile_chunk, const int32_t* chunk_self_end,
                       int kv_total, const int32_t* mrg_start, const int32_t* mrg_prefix, int nranges,
                       int64_t merge_tokens, float* delta, void* part_dq, void* dq, void* dk, void* dv, const TileTables& t, int64_t S, int H, int D, int K, float softmax_scale, int64_t grid_q,
-                      int64_t grid_kv, int* queues, float* part_dkv, int dkv_split, hipStream_t st) {
+                      int64_t grid_kv, int* queues, float* part_dkv, int dkv_shares, hipStream_t st) {
   LaunchCheck launch_check;
   typedef typename E::elem elem;
   BwdParams<E> p;
@@ -986,7 +1121,9 @@ static int launch_bwd(const void* dout, const void* q, const void* k, const void
   p.chunk_self_end = chunk_self_end; p.kv_total = kv_total;
   p.queues = queues;
   p.part_dkv = part_dkv;
-  p.dkv_split = dkv_split;
+  p.dkv_shares = dkv_shares;
+  p.kv_tiles = kv_total / t.Hkv;
+  p.share_tiles = (ShareTile*)(part_dkv + ((int64_t)kv_total + (int64_t)t.Hkv * dkv_shares) * (2 * TM * kHeadDim));
   p.queues_log2 = t.self_first ? 0 : 3;
   p.t = t;
   p.scale = softmax_scale > 0.f ? softmax_scale : (float)(1.0 / sqrt((double)D));
@@ -994,24 +1131,28 @@ static int launch_bwd(const void* dout, const void* q, const void* k, const void
                                      : (float)(1.4426950408889634 / sqrt((double)D));
   // division by H*K1 as a multiplication: with s = 31 + ceil(log2 d) and m = floor(2^s / d) + 1 the
   // error m*d - 2^s is at most d <= 2^(s-31), so n*m >> s is the exact quotient for n < 2^31; m < 2^32
-  const uint64_t hk = (uint64_t)H * (K + 1);
-  uint32_t lg = 1;  // (at least 1: the kernels take the product's high word and shift by hk_shift - 32; a list entry
-                    // exists only with K >= 1, hence H*K1 >= 2)
-  while ((1ull << lg) < hk) ++lg;
-  p.hk_shift = 31 + lg;
-  p.hk_magic = (uint32_t)((1ull << p.hk_shift) / hk + 1);
+  auto magic = [](uint64_t d, uint32_t& m, uint32_t& shift) {
+    uint32_t lg = 1;  // (at least 1: the kernels take the product's high word and shift by shift - 32; for d >= 2)
+    while ((1ull << lg) < d) ++lg;
+    shift = 31 + lg;
+    m = (uint32_t)((1ull << shift) / d + 1);
+  };
+  magic((uint64_t)H * (K + 1), p.hk_magic, p.hk_shift);  // (a list entry exists only with K >= 1, hence H*K1 >= 2)
+  magic((uint64_t)K + 1, p.k1_magic, p.k1_shift);
+  magic((uint64_t)H, p.h_magic, p.h_shift);              // (not used with one head)
 
   static bool allowed_dq[kMaxDevices], allowed_dkv[4][kMaxDevices];  // one set per element type
   typedef void (*DkvKernel)(const BwdParams<E>);
   static const DkvKernel dkv_kernels[4] = {bwd_dkv_kernel<E, false>, bwd_dkv_parts_kernel<E, false>,
                                            bwd_dkv_kernel<E, true>, bwd_dkv_parts_kernel<E, true>};
-  const int form = (t.batch_rows != 0 ? 2 : 0) + (dkv_split > 1 ? 1 : 0);
+  const bool packed = t.batch_rows == 0 && t.q_head_b == kHeadDim * 2 && t.q_tok_b == (int64_t)H * kHeadDim * 2;
+  const int form = dkv_shares ? (packed ? 1 : 3) : (t.batch_rows != 0 ? 2 : 0);
   if (!allow_dynamic_lds((const void*)bwd_dq_kernel<E>, kBwdDqLds, allowed_dq) ||
       !allow_dynamic_lds((const void*)dkv_kernels[form], kBwdDkvLds, allowed_dkv[form]))
     return MOBA_ERR_LAUNCH;
   const int64_t rows = S * H;
-  hipLaunchKernelGGL(bwd_delta_kernel<E>, dim3((unsigned)((rows + 15) / 16)), dim3(256), 0, st, (const elem*)dout,
-                     (const elem*)out, lse, delta, delta + S * H, rows, queues);
+  hipLaunchKernelGGL(bwd_delta_kernel<E>, dim3((unsigned)((rows + 15) / 16 + (dkv_shares ? 1 : 0))), dim3(256), 0, st,
+                     (const elem*)dout, (const elem*)out, lse, delta, delta + S * H, rows, queues, p);
   hipLaunchKernelGGL(bwd_dq_kernel<E>, dim3((unsigned)grid_q), dim3(256), kBwdDqLds, st, p);
   if (merge_tokens > 0) {  // (0: the dQ kernel wrote every row itself)
     const int64_t sum_rows = merge_tokens * H;
@@ -1020,29 +1161,32 @@ static int launch_bwd(const void* dout, const void* q, const void* k, const void
                        mrg_prefix, nranges, H);
   }
   hipLaunchKernelGGL(dkv_kernels[form], dim3((unsigned)grid_kv), dim3(256), kBwdDkvLds, st, p);
-  if (dkv_split > 1)
+  if (dkv_shares)
     hipLaunchKernelGGL(bwd_dkv_reduce_kernel<E>, dim3((unsigned)p.kv_total * 16), dim3(256), 0, st, p);
   return launch_check.result();
 }
 
 extern "C" int moba_bwd_tile_rows(void) { return TM; }
 
-// Parts per key tile of the dK/dV kernel.  With fewer tiles than two per compute unit the tiles of the first
-// chunks of a sequence, whose gather lists are the longest, set the kernel's time while most of the chip is
-// idle: they are cut into parts then (at most 4: every part leaves 128 KiB of fp32 sums to be added up).
-// Problems below 4096 tokens are too short for the parts' extra traffic to pay.
-static int dkv_split_for(int64_t S, int64_t tiles) {
+// Into how many shares the places of a head's key tiles are cut (share_count: fewer where they would be short): one per
+// compute unit over all heads; or 0 for whole tiles drawn from queues.  Those take over at two tiles per unit: a share walks
+// tiles far from those of its neighbours, whose rows the caches of an XCD then no longer share, and their starts are no
+// fewer.  Whole tiles / shares in us, forward and backward: 15 heads of 4096 tokens, chunk 512 (480 tiles): 310 / 315; 4 of 16384
+// (512): 352 / 346; 8 of 16384, chunk 1024 (1024): 866 / 895; 32 heads on 8, 32768 tokens, chunk 2048 (2048): 14907 / 15890.
+// Below 1024 tokens there is nothing to cut (8 tiles of a head then, so no more than 64 heads: a lane each in the kernel).
+extern "C" int moba_bwd_dkv_shares(int64_t S, int Hkv, int64_t kv_tiles) {
   const int cus = resident_compute_units();
-  if (cus <= 0 || tiles <= 0 || tiles >= 2 * (int64_t)cus || S < 4096) return 1;
-  const int64_t r = (3 * (int64_t)cus + tiles - 1) / tiles;
-  return (int)(r < 1 ? 1 : (r > 4 ? 4 : r));
+  if (cus <= 0 || Hkv <= 0 || kv_tiles <= 0 || kv_tiles * Hkv >= 2 * (int64_t)cus || S < 1024 || Hkv > 64) return 0;
+  return Hkv < cus ? cus / Hkv : 1;
 }
 
+// dkv_shares: of a head
+static size_t dkv_scratch_bytes(int Hkv, int64_t kv_tiles, int dkv_shares) {
+  return (size_t)Hkv * (kv_tiles + dkv_shares) * (2 * TM * kHeadDim) * sizeof(float) + (Hkv * kv_tiles + 1) * sizeof(ShareTile);
+}
 extern "C" size_t moba_bwd_dkv_scratch_bytes(int64_t S, int Hkv, int64_t kv_tiles) {
-  if (S <= 0 || Hkv <= 0 || kv_tiles <= 0) return 0;
-  const int64_t tiles = kv_tiles * Hkv;
-  const int split = dkv_split_for(S, tiles);
-  return split > 1 ? (size_t)tiles * split * (2 * TM * kHeadDim) * sizeof(float) : 0;
+  const int shares = moba_bwd_dkv_shares(S, Hkv, kv_tiles);
+  return shares ? dkv_scratch_bytes(Hkv, kv_tiles, shares) : 0;
 }
 
 // Parts per history tile of the dQ kernel (a power of two).  With fewer tiles than workgroup slots to fill a few
@@ -1069,8 +1213,8 @@ extern "C" int moba_bwd(const void* dout, const void* q, const void* k, const vo
                         float* delta, void* part_dq,
                         void* dq, void* dk, void* dv, int64_t S, int H, int Hkv, int D, int K, int F, int N, int B,
                         int64_t hist_bound, int64_t self_tiles, int64_t kv_tiles, int dq_key_split, const int64_t* strides,
-                        int32_t* queues, void* dkv_scratch, int64_t dkv_scratch_bytes, float softmax_scale, int dtype,
-                        void* stream) {
+                        int32_t* queues, void* dkv_scratch, int64_t dkv_scratch_bytes, int dkv_shares, float softmax_scale,
+                        int dtype, void* stream) {
   if (!dout || !q || !k || !v || !out || !lse || !chunk_tok || !self_tile_prefix || !self_tile_chunk || !delta ||
       !part_dq || !dq || !dk || !dv || !queues || !kv_chunk_tok || !kv_tile_prefix || !kv_tile_chunk || !chunk_self_end)
     return MOBA_ERR_ARG;
@@ -1111,21 +1255,21 @@ extern "C" int moba_bwd(const void* dout, const void* q, const void* k, const vo
   while ((1 << t.key_split_log2) < dq_key_split) ++t.key_split_log2;
   t.part_stride = (int)(S * H * (K + 1));
   t.chunk_direct = chunk_direct;
-  // the key tiles are cut into parts only if the caller brought the scratch for their sums
+  // the stages of the key tiles are dealt in shares only if the caller brought the scratch for their sums
   const int64_t kv_total = kv_tiles * Hkv;
-  int dkv_split = dkv_split_for(S, kv_total);
-  if (dkv_split > 1 && (!dkv_scratch || ((uintptr_t)dkv_scratch & 15) ||
-                        dkv_scratch_bytes < (int64_t)(kv_total * dkv_split * (2 * TM * kHeadDim) * sizeof(float))))
-    dkv_split = 1;
-  if (kv_total * dkv_split >= 0x7fffffffLL) return MOBA_ERR_LIMIT;
+  if (kv_total >= 0x7fffffffLL) return MOBA_ERR_LIMIT;
+  if (dkv_shares < 0 || (dkv_shares > 0 && Hkv > 64)) return MOBA_ERR_ARG;
+  if (dkv_shares && (!dkv_scratch || ((uintptr_t)dkv_scratch & 15) ||
+                     dkv_scratch_bytes < (int64_t)::dkv_scratch_bytes(Hkv, kv_tiles, dkv_shares)))
+    dkv_shares = 0;
   hipStream_t st = (hipStream_t)stream;
   return dtype == MOBA_DTYPE_F16
              ? launch_bwd<F16>(dout, q, k, v, out, lse, sel, chunk_fid, kv_chunk_tok, kv_tile_prefix, kv_tile_chunk,
                                chunk_self_end, (int)kv_total, mrg_start, mrg_prefix, nranges, merge_tokens, delta, part_dq, dq, dk, dv,
                                 t, S, H, D, K,
-                               softmax_scale, grid_q, grid_kv, queues, (float*)dkv_scratch, dkv_split, st)
+                               softmax_scale, grid_q, grid_kv, queues, (float*)dkv_scratch, dkv_shares, st)
              : launch_bwd<Bf16>(dout, q, k, v, out, lse, sel, chunk_fid, kv_chunk_tok, kv_tile_prefix, kv_tile_chunk,
                                 chunk_self_end, (int)kv_total, mrg_start, mrg_prefix, nranges, merge_tokens, delta, part_dq, dq, dk, dv,
                                 t, S, H, D, K,
-                                softmax_scale, grid_q, grid_kv, queues, (float*)dkv_scratch, dkv_split, st);
+                                softmax_scale, grid_q, grid_kv, queues, (float*)dkv_scratch, dkv_shares, st);
 }

@@ -502,15 +502,17 @@ def _for_training(*tensors: torch.Tensor):
     return wide, tuple(t[..., :NARROW_HEAD_DIM] for t in wide) if width < NARROW_HEAD_DIM else wide
 
 
-def _backward(dout, q, k, v, out, lse, sel, seg_off, seg_dest, plan: MobaPlan, scale: float = 0.0, tables=None):
-    """tables: the backward kernels' (tile_off, tile_seg) if the forward made them (made here otherwise).
+def _backward(dout, q, k, v, out, lse, sel, seg_off, seg_dest, plan: MobaPlan, scale: float = 0.0, tables=None,
+              all_kv_heads: int = 0):
+    """tables: the backward kernels' (tile_off, tile_seg) if the forward made them (made here otherwise).  all_kv_heads:
+    the key/value heads of the call of which this is a part (0: it is not).
     The gradients' heads have dout's width."""
     lib = _lib.load()
     S, H, D = _dims(q)
     width = dout.shape[-1]
     if width < HEAD_DIM:   # (the backward's kernels take heads of 128 elements)
         grads = _backward(*_widened((dout, q, k, v, out), HEAD_DIM), lse, sel, seg_off, seg_dest, plan,
-                          scale or width ** -0.5, tables)
+                          scale or width ** -0.5, tables, all_kv_heads)
         return tuple(x[..., :width].contiguous() for x in grads)
     Hkv = _dims(k)[1]
     dev = q.device
@@ -521,11 +523,12 @@ def _backward(dout, q, k, v, out, lse, sel, seg_off, seg_dest, plan: MobaPlan, s
     # One allocation for the call's scratch, every part a multiple of 16 bytes: the per-slot partial dQ, delta and
     # the log2 lse, the 16 tile counters of the two kernels (zeroed by the call), the backward kernels' own tile
     # tables (they cut the gather lists into tiles of their own height) and, for small problems, the fp32 sums of
-    # the parts the dK/dV kernel cuts its key tiles into (0 bytes otherwise)
-    b = g.bwd.get(Hkv)
+    # the key tiles that several workgroups of the dK/dV kernel have parts of (0 bytes otherwise)
+    b = g.bwd.get((Hkv, all_kv_heads))
     if b is None:
         bound = plan.hist_tile_bound(H, TILE_ROWS)
-        kv_bytes = int(lib.moba_bwd_dkv_scratch_bytes(S, Hkv, plan.kv_tiles))
+        kv_shares = lib.moba_bwd_dkv_shares(S, all_kv_heads or Hkv, plan.kv_tiles)
+        kv_bytes = int(lib.moba_bwd_dkv_scratch_bytes(S, Hkv, plan.kv_tiles)) if kv_shares else 0
         # small problems: the keys of every history tile of the dQ kernel in `split` parts with slots of their own
         split = 1 if plan.fallback else int(lib.moba_bwd_dq_key_split(S, H, K, plan.chunk_size, bound, plan.self_tiles))
         sizes = [split * S * H * (K + 1) * D * q.element_size(), 2 * S * H * 4, 64,
@@ -533,8 +536,8 @@ def _backward(dout, q, k, v, out, lse, sel, seg_off, seg_dest, plan: MobaPlan, s
         starts = [0]
         for n in sizes:
             starts.append(starts[-1] + (n + 15) // 16 * 16)
-        b = g.bwd[Hkv] = (bound, kv_bytes, starts, split)
-    bound, kv_bytes, starts, split = b
+        b = g.bwd[Hkv, all_kv_heads] = (bound, kv_bytes, kv_shares, starts, split)
+    bound, kv_bytes, kv_shares, starts, split = b
     ws = torch.empty(starts[-1], dtype=torch.uint8, device=dev)
     base = ws.data_ptr()
     part_dqp, deltap, queuesp, tile_offp, tile_segp, kvp = (base + a for a in starts[:6])
@@ -556,7 +559,7 @@ def _backward(dout, q, k, v, out, lse, sel, seg_off, seg_dest, plan: MobaPlan, s
                               if DIRECT_ROWS else (None, None, None, 0, S)),
                             deltap, part_dqp, _ptr(dq), _ptr(dk), _ptr(dv), S, H, Hkv, D, K, plan.F, plan.NA,
                             plan.chunk_size, bound, plan.self_tiles, plan.kv_tiles, split, _strides(q, k), queuesp,
-                            kvp if kv_bytes else None, kv_bytes, scale, _dtype_code(q), stream), "moba_bwd")
+                            kvp if kv_bytes else None, kv_bytes, kv_shares, scale, _dtype_code(q), stream), "moba_bwd")
     return dq, dk, dv
 
 
@@ -680,7 +683,7 @@ class _MobaAttentionInGroups(torch.autograd.Function):
         for (h0, h1), (group_plan, sel, seg_off, seg_dest, tables) in zip(ctx.groups, ctx.keep):
             g0, g1 = h0 // rep, h1 // rep
             got = _backward(_aligned(dout[:, h0:h1]), q[:, h0:h1], k[:, g0:g1], v[:, g0:g1], out[:, h0:h1].contiguous(),
-                            lse[:, h0:h1].contiguous(), sel, seg_off, seg_dest, group_plan, ctx.scale, tables)
+                            lse[:, h0:h1].contiguous(), sel, seg_off, seg_dest, group_plan, ctx.scale, tables, Hkv)
             dq[:, h0:h1], dk[:, g0:g1], dv[:, g0:g1] = got
             del got
         if q.dim() == 4:
