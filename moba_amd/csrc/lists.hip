@@ -305,11 +305,12 @@ __global__ __launch_bounds__(256) void lists_tile_seg_kernel(const int* __restri
 // seg_off is given), the scan of the tile counts and lists_tile_seg_kernel do, in one workgroup with the counts
 // in LDS -- three dependent launches of a few microseconds each are most of the list stage of a small problem.
 constexpr int kTailMaxSegments = 4096, kTailMaxTiles = 16384;
-// (off: kTailMaxSegments + 1 ints of LDS, wsum: 16; `base` may point into LDS)
-__device__ __forceinline__ void lists_tail_body(const int* base, const int* __restrict__ pair_off,
-                                                int* __restrict__ seg_off, int* __restrict__ tile_off,
-                                                int* __restrict__ tile_seg, int F, int H, int tile_rows, int bound,
-                                                int* off, int* wsum) {
+__global__ __launch_bounds__(1024) void lists_tail_kernel(const int* __restrict__ base, const int* __restrict__ pair_off,
+                                                          int* __restrict__ seg_off, int* __restrict__ tile_off,
+                                                          int* __restrict__ tile_seg, int F, int H, int tile_rows,
+                                                          int bound) {
+  __shared__ int off[kTailMaxSegments + 1];
+  __shared__ int wsum[16];
   const int FH = F * H, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // this thread's four consecutive segments: list starts (written out when they come from the counts), tile counts
   int v[4];
@@ -380,74 +381,147 @@ __device__ __forceinline__ void lists_tail_body(const int* base, const int* __re
   }
 }
 
-__global__ __launch_bounds__(1024) void lists_tail_kernel(const int* __restrict__ base, const int* __restrict__ pair_off,
-                                                          int* __restrict__ seg_off, int* __restrict__ tile_off,
-                                                          int* __restrict__ tile_seg, int F, int H, int tile_rows,
-                                                          int bound) {
-  __shared__ int off[kTailMaxSegments + 1];
-  __shared__ int wsum[16];
-  lists_tail_body(base, pair_off, seg_off, tile_off, tile_seg, F, H, tile_rows, bound, off, wsum);
-}
-
-// Small problems (few counts, few segments, few tiles, few workgroups): the scan, the fill and the tail in one
-// launch.  Every workgroup scans the whole count array for itself into LDS (cheaper than a launch that does it
-// once); workgroups (cq < N, h) fill their part of the lists with 16 waves, workgroup (N, 0) writes the segment and
-// tile tables, which depend on the scanned counts only.
-constexpr int kFusedMaxCounts = 4096, kFusedMaxCand = 128;
-template <int KC>
-__global__ __launch_bounds__(1024) void lists_fill_tail_kernel(
+// Small problems: the scan, the fill and the tables in one launch.  Every workgroup scans the whole count array for itself
+// into LDS (cheaper than a launch that does it once); workgroups (cq < N, h) fill their part of the lists, workgroups
+// (N, h) write an H-th of the tables each, which depend on the scanned counts only.
+// NW waves as in lists_fill_kernel: 16 for long chunks, 4 otherwise -- workgroups of 16 waves start one after the other, 22 ns
+// apart, and a chunk of 512 tokens is half a batch for each.  Measured: 8191 tokens, 32 heads, chunk 512 (16 waves each
+// and one of them for all tables before): 19.0 -> 15.9 us; 3 x 2001 tokens, 32 heads, chunk 256 (scan, fill and tables as
+// three launches before): 17.3 -> 10.4 us; 20480 tokens, 8 heads, chunk 512: 11.8 -> 9.0.
+constexpr int kFusedMaxCounts = 8192, kFusedMaxCand = 128;
+constexpr int64_t kFusedMaxWork = 1 << 22;
+template <int KC, int NW>
+__global__ __launch_bounds__(NW * 64) void lists_fill_tail_kernel(
     const int* __restrict__ sel, const int* __restrict__ chunk_tok, const int* __restrict__ chunk_fb,
     const int* __restrict__ chunk_local, const int* __restrict__ pair_off, const int* __restrict__ cnt,
     int* __restrict__ seg_dest, int* __restrict__ seg_off, int* __restrict__ tile_off, int* __restrict__ tile_seg,
     int N, int H, int K, int F, int PH, int tile_rows, int bound, int tile_rows_b, int* __restrict__ tile_off_b,
     int* __restrict__ tile_seg_b, int bound_b, int dense_local) {
-  __shared__ int sbase[kFusedMaxCounts + 1];
-  // the tail's tile starts, or the fill's positions and lane masks: 16 waves x 3 ints per candidate chunk
-  __shared__ int off[kFusedMaxCand * 48 > kTailMaxSegments + 1 ? kFusedMaxCand * 48 : kTailMaxSegments + 1];
-  __shared__ int wsum[16];
-  if (blockIdx.x == N && blockIdx.y != 0) return;
-  auto scanned_counts = [&]() -> const int* {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int i0 = tid * 4;
-    int v[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = (i0 + e < PH) ? cnt[i0 + e] : 0;
-    const int tsum = v[0] + v[1] + v[2] + v[3];
-    int inc = tsum;
+  constexpr int NT = NW * 64, kSteps = kFusedMaxCounts / (4 * NT);
+  // the scanned counts [PH + 1]; the tables' tile starts [F*H + 1], or the fill's positions and lane masks: NW x 3 ints per
+  // candidate chunk
+  extern __shared__ int lds[];
+  __shared__ int wsum[kSteps][NW];
+  int* const sbase = lds;
+  int* const off = lds + PH + 1;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // inclusive sum over the workgroup's lanes up to this one within its wave
+  auto wave_scan = [&](int x) {
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
-      const int t = __shfl_up(inc, o, 64);
-      if (lane >= o) inc += t;
+      const int t = __shfl_up(x, o, 64);
+      if (lane >= o) x += t;
     }
-    if (lane == 63) wsum[wave] = inc;
+    return x;
+  };
+  // (asked for ahead of everything else: the fill's lookups and picks travel meanwhile)
+  int v[kSteps][4];
+#pragma unroll
+  for (int st = 0; st < kSteps; ++st) {
+    const int i0 = (st * NT + tid) * 4;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[st][e] = i0 + e < PH ? cnt[i0 + e] : 0;
+  }
+  auto scanned_counts = [&]() -> const int* {
+    int inc[kSteps], sum[kSteps];
+#pragma unroll
+    for (int st = 0; st < kSteps; ++st) {
+      if (st * NT * 4 >= PH) break;  // (uniform)
+      sum[st] = v[st][0] + v[st][1] + v[st][2] + v[st][3];
+      inc[st] = wave_scan(sum[st]);
+      if (lane == 63) wsum[st][wave] = inc[st];
+    }
     __syncthreads();
-    int woff = 0, total = 0;
+    int carry = 0;
 #pragma unroll
-    for (int w = 0; w < 16; ++w) {
-      const int x = wsum[w];
-      if (w < wave) woff += x;
-      total += x;
-    }
-    int run = woff + inc - tsum;
+    for (int st = 0; st < kSteps; ++st) {
+      if (st * NT * 4 >= PH) break;
+      int woff = 0, total = 0;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      if (i0 + e < PH) sbase[i0 + e] = run;
-      run += v[e];
+      for (int w = 0; w < NW; ++w) {
+        const int x = wsum[st][w];
+        if (w < wave) woff += x;
+        total += x;
+      }
+      int run = carry + woff + inc[st] - sum[st];
+      const int i0 = (st * NT + tid) * 4;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (i0 + e < PH) sbase[i0 + e] = run;
+        run += v[st][e];
+      }
+      carry += total;
     }
-    if (tid == 0) sbase[PH] = total;
+    if (tid == 0) sbase[PH] = carry;
     __syncthreads();
     return sbase;
   };
-  if (blockIdx.x == N) {
-    const int* base = scanned_counts();
-    lists_tail_body(base, pair_off, seg_off, tile_off, tile_seg, F, H, tile_rows, bound, off, wsum);
-    if (tile_off_b) {  // the same lists cut into tiles of another height (the backward kernels')
+  if (blockIdx.x < N) {
+    lists_fill_body<KC, NW>(sel, chunk_tok, chunk_fb, chunk_local, pair_off, scanned_counts, seg_dest, H, K, dense_local, off);
+    return;
+  }
+  // the tables: this workgroup's share of the segments and of the tiles
+  const int FH = F * H, part = blockIdx.y;
+  const int* base = scanned_counts();
+  auto tables = [&](int rows, int* toff, int* tseg, int nbound, bool starts) {
+    int carry = 0;
+    for (int f0 = 0; f0 < FH; f0 += NT) {
+      const int fh = f0 + tid;
+      int start = 0, n = 0;
+      if (fh < FH) {
+        const int f = fh / H, h = fh - f * H;
+        const int p0 = pair_off[f], nq = pair_off[f + 1] - p0;
+        start = base[p0 * H + h * nq];
+        n = (base[p0 * H + (h + 1) * nq] - start + rows - 1) / rows;
+      }
+      const int inc = wave_scan(n);
+      if (lane == 63) wsum[0][wave] = inc;
       __syncthreads();
-      lists_tail_body(base, pair_off, seg_off, tile_off_b, tile_seg_b, F, H, tile_rows_b, bound_b, off, wsum);
+      int woff = 0, total = 0;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        const int x = wsum[0][w];
+        if (w < wave) woff += x;
+        total += x;
+      }
+      const int at = carry + woff + inc - n;
+      if (fh < FH) {
+        off[fh] = at;
+        if (fh % H == part) {
+          toff[fh] = at;
+          if (starts) seg_off[fh] = start;
+        }
+      }
+      carry += total;
+      __syncthreads();  // (the sums are read)
     }
-  } else
-    lists_fill_body<KC, 16>(sel, chunk_tok, chunk_fb, chunk_local, pair_off, scanned_counts, seg_dest, H, K,
-                            dense_local, off);
+    if (tid == 0) {
+      off[FH] = carry;
+      if (part == 0) {
+        toff[FH] = carry;
+        if (starts) seg_off[FH] = base[PH];
+      }
+    }
+    __syncthreads();
+    const int t1 = (int)((int64_t)nbound * (part + 1) / H);
+    for (int t = (int)((int64_t)nbound * part / H) + tid; t < t1; t += NT) {
+      int seg = -1;
+      if (t < carry) {
+        int lo = 0, hi = FH;  // off[lo] <= t < off[hi]
+        while (hi - lo > 1) {
+          const int mid = (lo + hi) >> 1;
+          if (off[mid] <= t) lo = mid; else hi = mid;
+        }
+        seg = lo;
+      }
+      tseg[t] = seg;
+    }
+  };
+  tables(tile_rows, tile_off, tile_seg, bound, true);
+  if (tile_off_b) {  // the same lists cut into tiles of another height (the backward kernels')
+    __syncthreads();
+    tables(tile_rows_b, tile_off_b, tile_seg_b, bound_b, false);
+  }
 }
 
 }  // namespace moba
@@ -507,18 +581,27 @@ extern "C" int moba_build_lists(const int32_t* sel, const int32_t* chunk_tok, co
   hipStream_t st = (hipStream_t)stream;
   dim3 grid(N, H);
   const bool small_tail = (int64_t)F * H < kTailMaxSegments && hist_bound <= kTailMaxTiles;
-  if (small_tail && (int64_t)P * H <= kFusedMaxCounts && cmax <= kFusedMaxCand && (int64_t)N * H <= 512 && K <= 16 &&
+  // One launch for all: its workgroups scan all counts each, so it is for few counts times workgroups; of 16 waves where a
+  // chunk has batches of 64 tokens for so many and the workgroups are few.
+  const int64_t counts = (int64_t)P * H, groups = (int64_t)N * H;
+  const bool many_waves = S / N >= 1024 && groups <= 512;
+  if (small_tail && counts <= kFusedMaxCounts && cmax <= kFusedMaxCand && groups * counts <= kFusedMaxWork && K <= 16 &&
       (!tile_off_b || hist_bound_b <= kTailMaxTiles)) {
     if (!counted)
-      hipLaunchKernelGGL(lists_count_kernel<1024>, grid, dim3(1024), (size_t)cmax * 4, st, sel, chunk_tok, chunk_fb,
+      hipLaunchKernelGGL(lists_count_kernel<256>, grid, dim3(256), (size_t)cmax * 4, st, sel, chunk_tok, chunk_fb,
                          chunk_local, pair_off, cnt, H, K, dense_local);
-#define MOBA_FILL_TAIL(KC)                                                                                       \
-  hipLaunchKernelGGL(lists_fill_tail_kernel<KC>, dim3(N + 1, H), dim3(1024), 0, st, sel, chunk_tok, chunk_fb,    \
-                     chunk_local, pair_off, (const int*)cnt, seg_dest, seg_off, tile_off, tile_seg, N, H, K, F,  \
-                     P * H, tile_rows, (int)hist_bound, tile_rows_b, tile_off_b, tile_seg_b, (int)hist_bound_b,     \
+    const int nw = many_waves ? 16 : 4, tables = F * H + 1, fill = nw * 3 * cmax;
+    const size_t lds = ((size_t)counts + 1 + (tables > fill ? tables : fill)) * 4;  // (at most 56 KiB)
+#define MOBA_FILL_TAIL(KC, NW)                                                                                       \
+  hipLaunchKernelGGL((lists_fill_tail_kernel<KC, NW>), dim3(N + 1, H), dim3(NW * 64), lds, st, sel, chunk_tok, chunk_fb, \
+                     chunk_local, pair_off, (const int*)cnt, seg_dest, seg_off, tile_off, tile_seg, N, H, K, F,      \
+                     P * H, tile_rows, (int)hist_bound, tile_rows_b, tile_off_b, tile_seg_b, (int)hist_bound_b,      \
                      dense_local)
-    if (K <= 4) MOBA_FILL_TAIL(4);
-    else MOBA_FILL_TAIL(16);
+    if (K <= 4) {
+      if (many_waves) MOBA_FILL_TAIL(4, 16); else MOBA_FILL_TAIL(4, 4);
+    } else {
+      if (many_waves) MOBA_FILL_TAIL(16, 16); else MOBA_FILL_TAIL(16, 4);
+    }
 #undef MOBA_FILL_TAIL
     return launch_check.result();
   }
