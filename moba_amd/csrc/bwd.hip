@@ -189,6 +189,11 @@ __global__ __launch_bounds__(256) void bwd_delta_kernel(const typename E::elem* 
 }
 
 // ------------------------------------------------------------------------------------ dQ
+// Bound by the matrix products at long chunks (and by the chip's power, like the forward); at short ones by what a tile costs
+// beside its key tiles of 2.2 us: the draw, three dependent lookups, the rows, and the result.  So the next tile is drawn
+// under the last key tile, its first keys are fetched while its rows' lookups run, and the result leaves from the
+// registers instead of through LDS: 14 to 16 us a tile -> 10 to 11.  20480 tokens, 8 heads on 2, chunk 512: 200 to 208 us -> 182;
+// 32768 tokens, one head, chunk 2048: 139 to 144 us -> 138; forward and backward together 641 -> 628 and 468 -> 461 us.
 template <class E>
 __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(const BwdParams<E> p) {
   MOBA_ELEM_TYPES(E)
@@ -201,36 +206,38 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(const BwdParams<E> p) {
   // hands out the ids (8i + x) * kXcdBlock + j in order, so that the tiles in flight on an XCD are
   // consecutive ids (tiles that share a K/V chunk behind one L2), and a workgroup whose queue is empty
   // goes on with the next XCD's: the XCDs differ in speed by a few percent and finish together this way.
-  // The draw for the next tile is in flight while the current one is computed.
   const int ql = p.queues_log2, qmask = (1 << ql) - 1;  // eight queues, or one for a problem of few tiles
   int queue = blockIdx.x & qmask, empty_queues = 0;
-  int drawn_next = 0;  // thread 0: the counter value drawn for the next tile
-  // (With few tiles per workgroup a tile drawn ahead is a tile that waits for its holder while other workgroups
-  // run out of work: the draw is made when the tile is due then, two microseconds that nothing hides.)
-  const bool draw_ahead = !p.t.self_first;
-  if (tid == 0 && draw_ahead)
-    drawn_next = __hip_atomic_fetch_add(p.queues + queue, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  while (true) {
-  __syncthreads();  // the previous tile is done with LDS, and every wave has read the previous draw
-  if (tid == 0) {
-    if (!draw_ahead)
-      drawn_next = __hip_atomic_fetch_add(p.queues + queue, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    *reinterpret_cast<int*>(smem + kDqIdSlot) = drawn_next;
-  }
-  __syncthreads();
-  const int drawn = __builtin_amdgcn_readfirstlane(*reinterpret_cast<const int*>(smem + kDqIdSlot));
-  const int64_t id = (((int64_t)(drawn / kXcdBlock) << ql) + queue) * kXcdBlock + (drawn % kXcdBlock);
+  int drawn = 0;  // thread 0: the counter value drawn for the next tile
+  // (With few tiles per workgroup a tile drawn early is a tile that waits for its holder while other workgroups run
+  // out of work: the draw is made in the tile's last key tile then, otherwise in its first.)
+  const bool draw_early = !p.t.self_first;
   const int ks = p.t.key_split_log2;
-  const bool past_end = id >= ((int64_t)p.t.hist_bound << ks) + p.t.self_total;
-  if (past_end) {
+  const int hist_tiles = p.t.hist_bound == 0 ? 0 : table_load(p.t.tile_off + p.t.F * p.t.H) << ks;  // parts of history tiles
+  int* const id_word = reinterpret_cast<int*>(smem + kDqIdSlot);
+  auto draw = [&]() __attribute__((always_inline)) {
+    if (tid == 0) drawn = __hip_atomic_fetch_add(p.queues + queue, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  // the id behind the value that thread 0 left in id_word, -1 past the last tile of this queue
+  auto id_of = [&](int x) __attribute__((always_inline)) {
+    const int64_t id = (((int64_t)(x / kXcdBlock) << ql) + queue) * kXcdBlock + (x % kXcdBlock);
+    return id < (int64_t)hist_tiles + p.t.self_total ? (int)id : -1;
+  };
+  draw();
+  if (tid == 0) *id_word = drawn;
+  __syncthreads();
+  int id = id_of(__builtin_amdgcn_readfirstlane(*id_word));
+  while (true) {
+  while (id < 0) {  // this queue is empty: the next one (a few draws in the open, at the end of the kernel)
     queue = (queue + 1) & qmask;
-    if (++empty_queues > qmask) break;
-  } else {
-    empty_queues = 0;
+    if (++empty_queues > qmask) return;
+    draw();
+    __syncthreads();  // (every wave has read the last value)
+    if (tid == 0) *id_word = drawn;
+    __syncthreads();
+    id = id_of(__builtin_amdgcn_readfirstlane(*id_word));
   }
-  if (tid == 0 && draw_ahead)
-    drawn_next = __hip_atomic_fetch_add(p.queues + queue, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  if (past_end) continue;
+  empty_queues = 0;
 
   Tile t;
   const int r = wave * 32 + n;
@@ -238,39 +245,16 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(const BwdParams<E> p) {
   // long as a history tile, and drawn last they would run alone at the end -- and the keys of a history tile
   // are cut into 1 << ks parts that are tiles of their own, each with slot rows of its own for its partial dQ
   // (part g of a slot row lies g * part_stride rows behind part 0; bwd_dq_reduce_kernel adds them up).
-  int logical = (int)id, key_part = 0;
-  if (p.t.self_first) {
-    if (logical < p.t.self_total) {
-      logical += p.t.hist_bound;
-    } else {
-      logical -= p.t.self_total;
-      key_part = logical & ((1 << ks) - 1);
-      logical >>= ks;
-    }
-  }
-  if (!decode_tile_head(p.t, logical, t)) continue;  // an unused id below hist_bound
+  const int hist = p.t.self_first ? id - p.t.self_total : (id < hist_tiles ? id : -1);
+  const int logical = hist >= 0 ? hist >> ks : p.t.hist_bound + (p.t.self_first ? id : id - hist_tiles);
+  const int key_part = hist >= 0 ? hist & ((1 << ks) - 1) : 0;
+  decode_tile_head(p.t, logical, t);
   if (t.base >= 0) {
     t.nkeys >>= ks;
     t.kv_tok0 += key_part * t.nkeys;
   }
-  decode_tile_rows(p.t, wave, r, t);
-  t.dest += key_part * p.t.part_stride;
-  const int h = t.h, nkeys = t.nkeys, kv_tok0 = t.kv_tok0, limit = t.limit;
-  const bool row_valid = r < t.row_count;
-
-  elem8 bq[8], bdo[8];
-  {
-    const int64_t off = ((int64_t)t.tok * H + h) * kHeadDim + 8 * hh;
-    const elem* qsrc = reinterpret_cast<const elem*>((const char*)p.q + q_tok_bytes(p.t, t.tok) + h * p.t.q_head_b) + 8 * hh;
-#pragma unroll
-    for (int ks = 0; ks < 8; ++ks) {
-      bq[ks] = *reinterpret_cast<const elem8*>(qsrc + 16 * ks);
-      bdo[ks] = *reinterpret_cast<const elem8*>(p.dout + off + 16 * ks);
-    }
-  }
-  const float lse2 = p.lse[(int64_t)t.tok * H + h] * kLog2e;
-  const float dl = p.delta[(int64_t)t.tok * H + h];
-
+  const int entry = decode_tile_row_entry(p.t, r, t);  // (asked for ahead of the first copies)
+  const int h = t.h, nkeys = t.nkeys, kv_tok0 = t.kv_tok0;
   const int hkv = h / p.t.rep;                                // key/value head of this query head
   const int64_t row_bytes = p.t.kv_tok_b;                     // from one K or V token to the next
   const uint32_t lds_base = lds_addr(smem);
@@ -334,6 +318,25 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(const BwdParams<E> p) {
   const int rot = t.rot % nkt;
   auto key_tile = [&](int it) __attribute__((always_inline)) { const int x = it + rot; return x >= nkt ? x - nkt : x; };
   issue_tile(key_tile(0), 0);
+
+  decode_tile_rows(p.t, wave, r, entry, t);
+  t.dest += key_part * p.t.part_stride;
+  const int limit = t.limit;
+  const bool row_valid = r < t.row_count;
+
+  elem8 bq[8], bdo[8];
+  {
+    const int64_t off = ((int64_t)t.tok * H + h) * kHeadDim + 8 * hh;
+    const elem* qsrc = reinterpret_cast<const elem*>((const char*)p.q + q_tok_bytes(p.t, t.tok) + h * p.t.q_head_b) + 8 * hh;
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) {
+      bq[ks] = *reinterpret_cast<const elem8*>(qsrc + 16 * ks);
+      bdo[ks] = *reinterpret_cast<const elem8*>(p.dout + off + 16 * ks);
+    }
+  }
+  const float lse2 = p.lse[(int64_t)t.tok * H + h] * kLog2e;
+  const float dl = p.delta[(int64_t)t.tok * H + h];
+
   wait_vmem();
   scrub_tile(key_tile(0), 0);
   __syncthreads();
@@ -376,6 +379,7 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(const BwdParams<E> p) {
     const int kt = key_tile(it);
     const bool has_next = it + 1 < nkt;
     if (has_next) issue_tile(key_tile(it + 1), buf ^ 1);
+    if (draw_early ? it == 0 : !has_next) draw();
 
     if (kt * TN <= t.wave_max_limit) {
       constexpr uint32_t ks = buf * kTileBytes;         // K stage, relative to stage 0
@@ -447,6 +451,8 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(const BwdParams<E> p) {
     if (has_next) {
       wait_vmem();
       scrub_tile(key_tile(it + 1), buf ^ 1);
+    } else if (tid == 0) {
+      *id_word = drawn;
     }
     __syncthreads();
   };
@@ -459,34 +465,30 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(const BwdParams<E> p) {
     if (it < nkt) key_tile_body(it, std::integral_constant<int, 0>{});
   }
 
-  // The accumulators hold dQ^T (a lane owns 4-element pieces of one row).  The partial is rounded to the
-  // element type, as the per-chunk dQ that flash-attn returns to the reference is, and goes through this
-  // wave's 8 KiB of LDS (free since the barrier that ended the last key tile) so that it leaves as whole
-  // 256-byte rows, four per store instruction.
+  id = id_of(__builtin_amdgcn_readfirstlane(*id_word));
+  // The accumulators hold dQ^T: element e of lane (n, hh) is dQ[row n][32*db + 8*(e/4) + 4*hh + e%4].  The partial is rounded to
+  // the element type, as the per-chunk dQ that flash-attn returns to the reference is; the two lanes of a row exchange
+  // halves, and each stores 16 bytes, 32 bytes of a row side by side.
   {
-    char* stage = smem + wave_u * 8192;
-    char* wrow = stage + n * 256 + 8 * hh;
+    u32x4 w[8];
 #pragma unroll
     for (int db = 0; db < 4; ++db)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        u32x2 w;
-        // (scaled before the rounding: a partial then overflows fp16 only where dQ itself would)
-        w[0] = pack2<E>(dqacc[db][4 * g + 0] * p.scale, dqacc[db][4 * g + 1] * p.scale);
-        w[1] = pack2<E>(dqacc[db][4 * g + 2] * p.scale, dqacc[db][4 * g + 3] * p.scale);
-        // elements 32*db + 8*g + 4*hh .. +3 of row n: 16-byte column 4*db + g, swizzled by the row
-        *reinterpret_cast<u32x2*>(wrow + (((4 * db + g) ^ (n & 15)) << 4)) = w;
-      }
-    const int c16 = lane & 15;
-    const int rows_here = t.row_count - wave_u * 32;  // rows of this wave that exist
-    // (a tile of a chunk without history slots holds the whole dQ of its rows: nothing to add it to)
-    elem* const dq_base = t.direct ? p.dq : p.part_dq;
+      for (int pair = 0; pair < 2; ++pair)
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int row = 4 * i + (lane >> 4);
-      const int dest = __shfl(t.dest, row, 64);
-      const u32x4 x = *reinterpret_cast<const u32x4*>(stage + row * 256 + ((c16 ^ (row & 15)) << 4));
-      if (row < rows_here) *reinterpret_cast<u32x4*>(dq_base + (int64_t)dest * kHeadDim + c16 * 8) = x;
+        for (int i = 0; i < 2; ++i) {
+          const int e = 8 * pair + 2 * i;
+          // (scaled before the rounding: a partial then overflows fp16 only where dQ itself would)
+          const auto x = __builtin_amdgcn_permlane32_swap(pack2<E>(dqacc[db][e] * p.scale, dqacc[db][e + 1] * p.scale),
+                                                          pack2<E>(dqacc[db][e + 4] * p.scale, dqacc[db][e + 5] * p.scale), false, false);
+          w[2 * db + pair][i] = x[0];
+          w[2 * db + pair][2 + i] = x[1];
+        }
+    // (a tile of a chunk without history slots holds the whole dQ of its rows: nothing to add it to)
+    elem* const row = (t.direct ? p.dq : p.part_dq) + (int64_t)t.dest * kHeadDim + 8 * hh;
+    if (row_valid) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) *reinterpret_cast<u32x4*>(row + 16 * i) = w[i];
     }
   }
   }  // tiles
