@@ -868,16 +868,19 @@ __device__ __forceinline__ void bwd_dkv_tiles(const BwdParams<E>& p) {
         if (u == 0) mfma32_into_vgprs(s_next, qa[s8], bk[s8], s8 == 0);
         else        mfma32_into_vgprs(dp_next, oa[s8], bv[s8], s8 == 0);
         const int e = k + u, g = e >> 2, rr = e & 3;
-        // (the inputs of an element are taken up one slot before the element's own: without the pins the
+        // (the inputs of an element are taken up two slots before the element's own: without the pins the
         // scale-and-subtract of all sixteen elements runs ahead of the first MFMA of the phase, with the matrix
-        // pipe idle meanwhile; a pin right in front of its use costs a wait state)
+        // pipe idle meanwhile.  The compiler puts the pins of a slot behind its vector instructions, and a wait state between a
+        // pin and a use that follows it at once: with one slot ahead those were 24 of a stage's 479 instructions.)
         if (e == 0) {
           sx[0] = s_cur[0];
           MOBA_PIN(sx[0]);
+          sx[1] = s_cur[1];
+          MOBA_PIN(sx[1]);
         }
-        if (e + 1 < 16) {
-          sx[e + 1] = s_cur[e + 1];
-          MOBA_PIN(sx[e + 1]);
+        if (e + 2 < 16) {
+          sx[e + 2] = s_cur[e + 2];
+          MOBA_PIN(sx[e + 2]);
         }
         dx[e] = dp_cur[e];
         MOBA_PIN(dx[e]);
