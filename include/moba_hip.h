@@ -58,7 +58,7 @@ extern "C" {
 
 enum { MOBA_DTYPE_BF16 = 0, MOBA_DTYPE_F16 = 1 };
 
-#define MOBA_ABI_VERSION 118 /* the signatures below; moba_version() returns the number the library was built with */
+#define MOBA_ABI_VERSION 119 /* the signatures below; moba_version() returns the number the library was built with */
 int moba_version(void);
 const char* moba_strerror(int code);
 
@@ -195,6 +195,15 @@ int moba_build_lists(const int32_t* sel, const int32_t* chunk_tok, const int32_t
                      int64_t hist_bound, int counted, int tile_rows_b, int32_t* tile_off_b, int32_t* tile_seg_b,
                      int64_t hist_bound_b, int dense_local, void* stream);
 
+/* The same with tile tables that cut the lists of list_heads heads (1, or all those of a key/value head, whose lists lie one
+ * behind the other) into tiles together: tile_off [F*H/list_heads+1], tile_seg names segment f*H/list_heads + h/list_heads,
+ * hist_bound e.g. M / tile_rows + F * H / list_heads; list_heads_b for the second pair. */
+int moba_build_lists_grouped(const int32_t* sel, const int32_t* chunk_tok, const int32_t* chunk_fb, const int32_t* chunk_local,
+                             const int32_t* pair_off, int32_t* cnt, int32_t* seg_off, int32_t* tile_off, int32_t* seg_dest,
+                             int32_t* tile_seg, int64_t S, int H, int K, int N, int F, int P, int cmax, int tile_rows,
+                             int64_t hist_bound, int counted, int tile_rows_b, int32_t* tile_off_b, int32_t* tile_seg_b,
+                             int64_t hist_bound_b, int dense_local, int list_heads, int list_heads_b, void* stream);
+
 /* The tile tables of moba_build_lists alone, for another tile height: the forward and the backward kernels cut
  * the same gather lists into tiles of moba_fwd_tile_rows() and moba_bwd_tile_rows() rows.  No counterpart in the
  * reference (flash-attn tiles its varlen batches internally).
@@ -265,7 +274,8 @@ int moba_fwd_partials(const void* q, const void* k, const void* v, void* part_o,
  * and may be NULL; redo, if given, has redo[0] zeroed by the caller and receives the tiles that were computed again with a running
  * maximum, for information: redo[0] counts every part of a tile cut by key_split, and parts beyond the array's
  * hist_bound + self_tiles * H entries are counted without an entry.  Those tiles take the fixed reference without a
- * list too: running_max != 0 asks for the running maximum from the start (and for redo to be left alone), whatever the
+ * list too (list_heads: of the tile tables, see moba_build_lists_grouped; 1 for tiles of moba_fwd_tile_rows() rows);
+ * running_max != 0 asks for the running maximum from the start (and for redo to be left alone), whatever the
  * tiles. */
 int moba_fwd_partials_rows(const void* q, const void* k, const void* v, void* part_o, float* part_lse,
                            const int32_t* seg_off, const int32_t* tile_off, const int32_t* seg_dest,
@@ -274,7 +284,7 @@ int moba_fwd_partials_rows(const void* q, const void* k, const void* v, void* pa
                            float* lse, int64_t S, int H, int Hkv, int D, int K, int F, int N, int B, int64_t hist_bound,
                            int64_t self_tiles, int key_split, const int64_t* strides, int32_t* queues, int32_t* redo,
                            float softmax_scale, int dtype, int self_tile_skip, int64_t q_tok_shift, int tile_rows,
-                           int running_max, void* stream);
+                           int running_max, int list_heads, void* stream);
 int moba_fwd_merge(const void* part_o, const float* part_lse, const int32_t* sel, void* out, float* lse, int64_t S,
                    int H, int D, int K, int key_split, const int32_t* mrg_start, const int32_t* mrg_prefix, int nranges,
                    int64_t merge_tokens, int dtype, void* stream);
@@ -318,6 +328,7 @@ int moba_fwd(const void* q, const void* k, const void* v, void* part_o, float* p
  *              16-byte aligned, and are added up in a fixed order (deterministic all the same).  Without the scratch (null, or
  *              too small) or with dkv_shares = 0, every tile is one piece.  A call for some of the heads gives what a call
  *              for all would, bit for bit, with that call's dkv_shares.
+ *   list_heads: of tile_off and tile_seg, see moba_build_lists_grouped
  *   softmax_scale: as in the forward call */
 int moba_bwd_dkv_shares(int64_t S, int Hkv, int64_t kv_tiles);
 size_t moba_bwd_dkv_scratch_bytes(int64_t S, int Hkv, int64_t kv_tiles);
@@ -332,7 +343,7 @@ int moba_bwd(const void* dout, const void* q, const void* k, const void* v, cons
              void* dk, void* dv, int64_t S, int H,
              int Hkv, int D, int K, int F, int N, int B, int64_t hist_bound, int64_t self_tiles, int64_t kv_tiles,
              int dq_key_split, const int64_t* strides, int32_t* queues, void* dkv_scratch, int64_t dkv_scratch_bytes,
-             int dkv_shares, float softmax_scale, int dtype, void* stream);
+             int dkv_shares, int list_heads, float softmax_scale, int dtype, void* stream);
 
 /* Decode: the last nq tokens of every sequence against its key/value cache.  Replaces the
  * flash_attn_func call of the adapter's decode branch, moba/wrapper.py:76-82 (grouped-query heads, bottom-right

@@ -36,6 +36,8 @@ _SIGNATURES = {
     "moba_topk_from_scores": (c_int, [c_void_p, c_void_p, c_int64, c_int, c_int, c_int, c_void_p]),
     "moba_build_lists": (c_int, [c_void_p] * 10 + [c_int64] + [c_int] * 7 + [c_int64, c_int, c_int, c_void_p, c_void_p,
                                                                              c_int64, c_int, c_void_p]),
+    "moba_build_lists_grouped": (c_int, [c_void_p] * 10 + [c_int64] + [c_int] * 7 + [c_int64, c_int, c_int, c_void_p, c_void_p,
+                                                                                     c_int64, c_int, c_int, c_int, c_void_p]),
     "moba_tile_tables": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int64, c_void_p]),
     "moba_fwd_tile_rows": (c_int, []),
     "moba_bwd_tile_rows": (c_int, []),
@@ -44,7 +46,7 @@ _SIGNATURES = {
                                                    c_int, c_int64, c_void_p]),
     "moba_fwd_partials_rows": (c_int, [c_void_p] * 16 + [c_int64, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
                                                         c_int64, c_int64, c_int, c_strides, c_void_p, c_void_p, c_float,
-                                                        c_int, c_int, c_int64, c_int, c_int, c_void_p]),
+                                                        c_int, c_int, c_int64, c_int, c_int, c_int, c_void_p]),
     "moba_fwd_merge": (c_int, [c_void_p] * 5 + [c_int64, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_int, c_int64,
                                                c_int, c_void_p]),
     "moba_fwd_key_split": (c_int, [c_int64, c_int, c_int, c_int, c_int64, c_int64]),
@@ -56,7 +58,7 @@ _SIGNATURES = {
     "moba_bwd_dkv_shares": (c_int, [c_int64, c_int, c_int64]),
     "moba_bwd_dq_key_split": (c_int, [c_int64, c_int, c_int, c_int, c_int64, c_int64]),
     "moba_bwd": (c_int, [c_void_p] * 23 + [c_int, c_int64] + [c_void_p] * 5 + [c_int64, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int64, c_int64,
-                                          c_int64, c_int, c_strides, c_void_p, c_void_p, c_int64, c_int, c_float, c_int, c_void_p]),
+                                          c_int64, c_int, c_strides, c_void_p, c_void_p, c_int64, c_int, c_int, c_float, c_int, c_void_p]),
     "moba_mfma_probe": (c_int, [c_void_p, c_void_p, c_int, c_int, c_void_p]),
     "moba_tail_splits": (c_int, [c_int] * 5),
     "moba_tail": (c_int, [c_void_p] * 6 + [c_int] * 6 + [c_strides, c_float, c_int, c_void_p]),
@@ -86,7 +88,7 @@ class SizesStruct(ctypes.Structure):
     _fields_ = [(n, c_int64) for n in ("kbar_elems", "chunk_mean_workspace_bytes", "sel_ints", "cnt_ints", "seg_off_ints",
                                        "seg_dest_ints", "fwd_hist_bound", "bwd_hist_bound", "part_rows", "redo_ints",
                                        "lse_floats", "delta_floats")]
-ABI_VERSION = 118  # MOBA_ABI_VERSION of include/moba_hip.h, the signatures above
+ABI_VERSION = 119  # MOBA_ABI_VERSION of include/moba_hip.h, the signatures above
 DTYPE_BF16, DTYPE_F16 = 0, 1
 
 

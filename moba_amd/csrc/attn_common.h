@@ -19,18 +19,21 @@ constexpr int kQueueRun = 256;
 // Index tables that define the tiles of one call.
 struct TileTables {
   const int* seg_off;           // [F*H+1] list start of segment (f, h)
-  const int* tile_off;          // [F*H+1] prefix sum of row tiles per segment
+  // The gather lists of seg_heads heads of a key/value head (1, or all of them) lie one behind the other and are cut into
+  // tiles together; such a segment is number f * seg_groups + its first head / seg_heads, seg_groups = H / seg_heads.
+  const int* tile_off;          // [F*seg_groups+1] prefix sum of row tiles per segment
   const int* seg_dest;          // [M] (token*H + h)*K1 + 1 + slot
   const int* fchunk_tok;        // [F] first token of filtered chunk f
   const int* chunk_tok;         // [N+1] first token of every chunk
   const int* self_tile_prefix;  // [N+1] prefix sum of row tiles per chunk
-  const int* tile_seg;          // [hist_bound] segment (f*H + h) of every history tile, -1 past the last one
+  const int* tile_seg;          // [hist_bound] segment of every history tile, -1 past the last one
   const int* self_tile_chunk;   // [self_tile_prefix[N]] chunk of every per-head self tile
   // [N] or null: 1 for a chunk whose rows have no history slots at all (the first attention chunk of a sequence).
   // The forward kernel writes the result of such a chunk's self tiles straight into the operator's outputs: there
   // is nothing to merge it with.  Null (the backward): every tile writes its slot row.
   const int* chunk_direct;
   int S, H, K1, F, N, B;
+  int seg_heads, seg_groups;
   int Hkv, rep;                 // key/value heads and query heads per key/value head (H = Hkv * rep)
   int hist_bound;               // logical tile ids below it are history tiles
   int self_total;               // self_tile_prefix[N] * H
@@ -76,6 +79,7 @@ inline bool set_layout(TileTables& t, const int64_t* strides) {
   t.chunk_direct = nullptr;
   t.key_split_log2 = 0; t.part_stride = 0; t.xcd_block_log2 = 6; t.self_first = 0;
   t.self_skip = 0; t.q_shift = 0;
+  t.seg_heads = 1; t.seg_groups = t.H;
   if (!strides) {
     t.q_tok_b = (int64_t)t.H * kHeadDim * 2; t.q_head_b = kHeadDim * 2;
     t.kv_tok_b = (int64_t)t.Hkv * kHeadDim * 2; t.kv_head_b = kHeadDim * 2;
@@ -97,7 +101,8 @@ inline bool set_layout(TileTables& t, const int64_t* strides) {
 // One tile of up to TM query rows of one head, as seen by a lane.
 struct Tile {
   int id;         // logical tile id
-  int h;          // head
+  int h;          // head (history tile: the first of its lists)
+  int rh;         // this lane's row: head
   int kv_tok0;    // token of key 0
   int nkeys;      // keys the tile attends (before masking)
   int row_count;  // valid rows
@@ -171,14 +176,16 @@ struct TileHeadEntries {
                    // self tile: self_tile_prefix[c], self_tile_prefix[c+1], chunk_tok[c], chunk_tok[c+1]
   int e;           // self tile: chunk_direct[c] (0 without that table)
 };
+// kGrouped: the kernel takes segments of more than one head (TileTables::seg_heads)
+template <bool kGrouped = false>
 __device__ __forceinline__ TileHeadEntries tile_head_entries(const TileTables& p, int logical, int code) {
   TileHeadEntries e = {0, 0, 0, 0, 0};
   if (code < 0) return e;
   if (logical < p.hist_bound) {
     e.a = table_load(p.tile_off + code);
-    e.b = table_load(p.seg_off + code);
-    e.c = table_load(p.seg_off + code + 1);
-    e.d = table_load(p.fchunk_tok + code / p.H);
+    e.b = table_load(p.seg_off + (kGrouped ? code * p.seg_heads : code));
+    e.c = table_load(p.seg_off + (kGrouped ? (code + 1) * p.seg_heads : code + 1));
+    e.d = table_load(p.fchunk_tok + code / (kGrouped ? p.seg_groups : p.H));
   } else {
     e.a = table_load(p.self_tile_prefix + code);
     e.b = table_load(p.self_tile_prefix + code + 1);
@@ -188,6 +195,7 @@ __device__ __forceinline__ TileHeadEntries tile_head_entries(const TileTables& p
   }
   return e;
 }
+template <bool kGrouped = false>
 __device__ __forceinline__ bool decode_tile_head(const TileTables& p, int logical, int code, const TileHeadEntries& e,
                                                  Tile& t, int tm = TM) {
   const int H = p.H;
@@ -199,8 +207,9 @@ __device__ __forceinline__ bool decode_tile_head(const TileTables& p, int logica
   if (logical < p.hist_bound) {
     const int seg = code;
     const int tile = logical - e.a;
-    const int f = seg / H;
-    t.h = seg - f * H;
+    const int groups = kGrouped ? p.seg_groups : H, f = seg / groups;
+    t.h = seg - f * groups;
+    if constexpr (kGrouped) t.h *= p.seg_heads;
     t.base = e.b + tile * tm;
     t.row_count = min(tm, e.c - t.base);
     t.kv_tok0 = e.d;
@@ -223,27 +232,38 @@ __device__ __forceinline__ bool decode_tile_head(const TileTables& p, int logica
   t.direct = e.e;
   return true;
 }
+template <bool kGrouped = false>
 __device__ __forceinline__ bool decode_tile_head(const TileTables& p, int logical, int code, Tile& t, int tm = TM) {
-  return decode_tile_head(p, logical, code, tile_head_entries(p, logical, code), t, tm);
+  return decode_tile_head<kGrouped>(p, logical, code, tile_head_entries<kGrouped>(p, logical, code), t, tm);
 }
+template <bool kGrouped = false>
 __device__ __forceinline__ bool decode_tile_head(const TileTables& p, int logical, Tile& t, int tm = TM) {
-  return decode_tile_head(p, logical, decode_tile_code(p, logical), t, tm);
+  return decode_tile_head<kGrouped>(p, logical, decode_tile_code(p, logical), t, tm);
 }
 // Step 2a, per row: the gather-list entry of row r (history tiles; self tiles need no lookup).
 __device__ __forceinline__ int decode_tile_row_entry(const TileTables& p, int r, const Tile& t) {
   return (t.row_count > 0 && t.base >= 0) ? p.seg_dest[t.base + min(r, t.row_count - 1)] : 0;
 }
 // Step 2b, per row: everything else from that entry.  r = row of this lane inside the tile (wave*32 + lane%32).
+template <bool kGrouped = false>
 __device__ __forceinline__ void decode_tile_rows(const TileTables& p, int wave, int r, int entry, Tile& t) {
   const int H = p.H;
   if (t.base >= 0) {
     t.dest = entry;
-    t.tok = t.dest / (H * p.K1);
+    if (kGrouped && p.seg_heads > 1) {
+      const int row = entry / p.K1;
+      t.tok = row / H;
+      t.rh = row - t.tok * H;
+    } else {
+      t.tok = t.dest / (H * p.K1);
+      t.rh = t.h;
+    }
     t.limit = t.nkeys - 1;
     t.wave_min_limit = t.limit;
     t.wave_max_limit = t.limit;
   } else {
     const int r0 = -1 - t.base;
+    t.rh = t.h;
     t.tok = t.kv_tok0 + r0 + min(r, t.row_count - 1);
     t.dest = t.direct ? (t.tok - p.q_shift) * H + t.h : (t.tok * H + t.h) * p.K1;
     t.limit = r0 + min(r, t.row_count - 1);
@@ -251,15 +271,6 @@ __device__ __forceinline__ void decode_tile_rows(const TileTables& p, int wave, 
     t.wave_max_limit = r0 + min(wave * 32 + 31, t.row_count - 1);
   }
 }
-__device__ __forceinline__ void decode_tile_rows(const TileTables& p, int wave, int r, Tile& t) {
-  decode_tile_rows(p, wave, r, decode_tile_row_entry(p, r, t), t);
-}
-__device__ __forceinline__ bool decode_tile(const TileTables& p, int logical, int wave, int r, Tile& t) {
-  if (!decode_tile_head(p, logical, t)) return false;
-  decode_tile_rows(p, wave, r, t);
-  return true;
-}
-
 // max over the two halves of the wave (lane l and lane l^32), without LDS traffic
 __device__ __forceinline__ float max_xhalf(float x) {
   const uint32_t u = __builtin_bit_cast(uint32_t, x);

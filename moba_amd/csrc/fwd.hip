@@ -884,8 +884,9 @@ extern "C" int moba_fwd_partials_rows(const void* q, const void* k, const void* 
                                  int N, int B, int64_t hist_bound, int64_t self_tiles, int key_split,
                                  const int64_t* strides, int32_t* queues, int32_t* redo, float softmax_scale,
                                  int dtype, int self_tile_skip, int64_t q_tok_shift, int tile_rows, int running_max,
-                                 void* stream) {
+                                 int list_heads, void* stream) {
   if (tile_rows != kFwdTileRows && tile_rows != TM) return MOBA_ERR_ARG;
+  if (list_heads != 1 && (Hkv <= 0 || list_heads != H / Hkv || tile_rows != TM)) return MOBA_ERR_ARG;
   if (!q || !k || !v || !part_o || !part_lse || !chunk_tok || !self_tile_prefix || !self_tile_chunk ||
       (!queues && tile_rows == kFwdTileRows))
     return MOBA_ERR_ARG;
@@ -924,6 +925,7 @@ extern "C" int moba_fwd_partials_rows(const void* q, const void* k, const void* 
   t.self_total = (int)(self_tiles * H);
   if (!strides && D != kHeadDim) return MOBA_ERR_ARG;  // (packed is said for 128 only)
   if (!set_layout(t, strides)) return MOBA_ERR_ARG;
+  t.seg_heads = list_heads; t.seg_groups = H / list_heads;
   t.key_split_log2 = key_split_log2;
   t.part_stride = (int)(S * H * (K + 1));
   t.xcd_block_log2 = tile_xcd_block_log2(total);
@@ -953,7 +955,7 @@ extern "C" int moba_fwd_partials(const void* q, const void* k, const void* v, vo
   return moba_fwd_partials_rows(q, k, v, part_o, part_lse, seg_off, tile_off, seg_dest, fchunk_tok, chunk_tok,
                                 self_tile_prefix, tile_seg, self_tile_chunk, chunk_direct, out, lse, S, H, Hkv, D, K, F, N,
                                 B, hist_bound, self_tiles, key_split, strides, queues, redo, softmax_scale, dtype,
-                                self_tile_skip, q_tok_shift, kFwdTileRows, redo == nullptr, stream);
+                                self_tile_skip, q_tok_shift, kFwdTileRows, redo == nullptr, 1, stream);
 }
 
 // mrg_start [nranges], mrg_prefix [nranges + 1], merge_tokens = mrg_prefix[nranges]: the tokens to merge, for a

@@ -93,7 +93,7 @@ __global__ __launch_bounds__(NW * 64, (FwdTileShape<D, NW>::kWavesPerSimd)) void
     } else {
       logical = p.t.hist_bound + (p.t.self_first ? logical : logical - parts_end);
     }
-    if (!decode_tile_head(p.t, logical, t, kRows)) return;
+    if (!decode_tile_head<true>(p.t, logical, t, kRows)) return;
     if (t.base >= 0) {  // this part's share of the chunk's keys
       t.nkeys >>= ks;
       t.kv_tok0 += key_part * t.nkeys;
@@ -159,12 +159,13 @@ __global__ __launch_bounds__(NW * 64, (FwdTileShape<D, NW>::kWavesPerSimd)) void
   const char* q_row;
   if constexpr (kTail) {
     const int row = row0 + min(r, t.row_count - 1);
+    t.rh = h;
     t.dest = (seq * p.t.S + row) * p.t.H + h;
     t.limit = p.t.q_shift + row;
     t.wave_min_limit = p.t.q_shift + row0 + min(wave * 32, t.row_count - 1);
     q_row = (const char*)p.q + seq * p.t.q_batch_b + row * p.t.q_tok_b;
   } else {
-    decode_tile_rows(p.t, wave, r, decode_tile_row_entry(p.t, r, t), t);
+    decode_tile_rows<true>(p.t, wave, r, decode_tile_row_entry(p.t, r, t), t);
     q_row = (const char*)p.q + q_tok_bytes(p.t, t.tok);
   }
   const int dest = t.dest + key_part * p.t.part_stride;  // (part 0 for a self tile)
@@ -173,7 +174,7 @@ __global__ __launch_bounds__(NW * 64, (FwdTileShape<D, NW>::kWavesPerSimd)) void
   const bool row_valid = r < t.row_count;
   elem8 bq[kKs];
   {
-    const elem* src = reinterpret_cast<const elem*>(q_row + h * p.t.q_head_b) + 8 * hh;
+    const elem* src = reinterpret_cast<const elem*>(q_row + t.rh * p.t.q_head_b) + 8 * hh;
 #pragma unroll
     for (int s8 = 0; s8 < kKs; ++s8) bq[s8] = *reinterpret_cast<const elem8*>(src + 16 * s8);
   }

@@ -265,31 +265,35 @@ __global__ __launch_bounds__(1024) void scan_apply_kernel(int* __restrict__ a, i
   if (blockIdx.x + 1 == gridDim.x && threadIdx.x == 0) a[n] = total;
 }
 
-// per (f, h): list start and number of row tiles
+// List of (f, heads h .. h + n - 1) from the scanned counts: start and length.
+__device__ __forceinline__ int2 list_range(const int* base, const int* __restrict__ pair_off, int fh, int H, int n) {
+  const int f = fh / H, h = fh - f * H;
+  const int p0 = pair_off[f], nq = pair_off[f + 1] - p0;
+  const int start = base[p0 * H + h * nq];
+  return make_int2(start, base[p0 * H + (h + n) * nq] - start);
+}
+
+// per (f, h): list start; per segment, the lists of G heads (1, or those of a key/value head): number of row tiles
 __global__ __launch_bounds__(256) void lists_segments_kernel(const int* __restrict__ base,
                                                              const int* __restrict__ pair_off,
                                                              int* __restrict__ seg_off, int* __restrict__ tile_off,
-                                                             int F, int H, int tile_rows) {
+                                                             int F, int H, int G, int tile_rows) {
   const int fh = blockIdx.x * 256 + threadIdx.x;
   if (fh > F * H) return;
   if (fh == F * H) {
     seg_off[fh] = base[pair_off[F] * H];
     return;
   }
-  const int f = fh / H, h = fh % H;
-  const int p0 = pair_off[f];
-  const int nq = pair_off[f + 1] - p0;
-  const int start = base[p0 * H + h * nq];
-  const int end = base[p0 * H + (h + 1) * nq];
-  seg_off[fh] = start;
-  tile_off[fh] = (end - start + tile_rows - 1) / tile_rows;
+  const int2 list = list_range(base, pair_off, fh, H, fh % G == 0 ? G : 1);
+  seg_off[fh] = list.x;
+  if (fh % G == 0) tile_off[fh / G] = (list.y + tile_rows - 1) / tile_rows;
 }
 
-// number of row tiles per (f, h) from the list starts
+// number of row tiles per segment of G heads from the list starts
 __global__ __launch_bounds__(256) void lists_tile_counts_kernel(const int* __restrict__ seg_off,
-                                                                int* __restrict__ tile_off, int FH, int tile_rows) {
-  const int fh = blockIdx.x * 256 + threadIdx.x;
-  if (fh < FH) tile_off[fh] = (seg_off[fh + 1] - seg_off[fh] + tile_rows - 1) / tile_rows;
+                                                                int* __restrict__ tile_off, int segments, int G, int tile_rows) {
+  const int s = blockIdx.x * 256 + threadIdx.x;
+  if (s < segments) tile_off[s] = (seg_off[(s + 1) * G] - seg_off[s * G] + tile_rows - 1) / tile_rows;
 }
 
 // segment of every history tile id below `bound` (-1 past the last tile): the attention
@@ -307,34 +311,22 @@ __global__ __launch_bounds__(256) void lists_tile_seg_kernel(const int* __restri
 constexpr int kTailMaxSegments = 4096, kTailMaxTiles = 16384;
 __global__ __launch_bounds__(1024) void lists_tail_kernel(const int* __restrict__ base, const int* __restrict__ pair_off,
                                                           int* __restrict__ seg_off, int* __restrict__ tile_off,
-                                                          int* __restrict__ tile_seg, int F, int H, int tile_rows,
+                                                          int* __restrict__ tile_seg, int F, int H, int G, int tile_rows,
                                                           int bound) {
   __shared__ int off[kTailMaxSegments + 1];
   __shared__ int wsum[16];
-  const int FH = F * H, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  // this thread's four consecutive segments: list starts (written out when they come from the counts), tile counts
+  const int FH = F * H / G, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;  // (FH: segments)
+  if (base) {  // the list starts
+    for (int fh = tid; fh <= F * H; fh += 1024)
+      seg_off[fh] = fh == F * H ? base[pair_off[F] * H] : list_range(base, pair_off, fh, H, 1).x;
+  }
+  // this thread's four consecutive segments: tile counts
   int v[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    const int fh = tid * 4 + e;
+    const int s = tid * 4 + e;
     v[e] = 0;
-    if (fh < FH) {
-      int start, end;
-      if (base) {
-        const int f = fh / H, h = fh % H;
-        const int p0 = pair_off[f];
-        const int nq = pair_off[f + 1] - p0;
-        start = base[p0 * H + h * nq];
-        end = base[p0 * H + (h + 1) * nq];
-        seg_off[fh] = start;
-      } else {
-        start = seg_off[fh];
-        end = seg_off[fh + 1];
-      }
-      v[e] = (end - start + tile_rows - 1) / tile_rows;
-    } else if (fh == FH && base) {
-      seg_off[fh] = base[pair_off[F] * H];
-    }
+    if (s < FH) v[e] = ((base ? list_range(base, pair_off, s * G, H, G).y : seg_off[(s + 1) * G] - seg_off[s * G]) + tile_rows - 1) / tile_rows;
   }
   const int tsum = v[0] + v[1] + v[2] + v[3];
   int inc = tsum;  // inclusive scan across the wave, then across the waves
@@ -395,8 +387,8 @@ __global__ __launch_bounds__(NW * 64) void lists_fill_tail_kernel(
     const int* __restrict__ sel, const int* __restrict__ chunk_tok, const int* __restrict__ chunk_fb,
     const int* __restrict__ chunk_local, const int* __restrict__ pair_off, const int* __restrict__ cnt,
     int* __restrict__ seg_dest, int* __restrict__ seg_off, int* __restrict__ tile_off, int* __restrict__ tile_seg,
-    int N, int H, int K, int F, int PH, int tile_rows, int bound, int tile_rows_b, int* __restrict__ tile_off_b,
-    int* __restrict__ tile_seg_b, int bound_b, int dense_local) {
+    int N, int H, int K, int F, int PH, int G, int tile_rows, int bound, int Gb, int tile_rows_b,
+    int* __restrict__ tile_off_b, int* __restrict__ tile_seg_b, int bound_b, int dense_local) {
   constexpr int NT = NW * 64, kSteps = kFusedMaxCounts / (4 * NT);
   // the scanned counts [PH + 1]; the tables' tile starts [F*H + 1], or the fill's positions and lane masks: NW x 3 ints per
   // candidate chunk
@@ -461,19 +453,16 @@ __global__ __launch_bounds__(NW * 64) void lists_fill_tail_kernel(
     return;
   }
   // the tables: this workgroup's share of the segments and of the tiles
-  const int FH = F * H, part = blockIdx.y;
+  const int part = blockIdx.y;
   const int* base = scanned_counts();
-  auto tables = [&](int rows, int* toff, int* tseg, int nbound, bool starts) {
+  for (int fh = part * NT + tid; fh <= F * H; fh += H * NT)
+    seg_off[fh] = fh == F * H ? base[PH] : list_range(base, pair_off, fh, H, 1).x;
+  auto tables = [&](int G, int rows, int* toff, int* tseg, int nbound) {
+    const int segments = F * H / G;
     int carry = 0;
-    for (int f0 = 0; f0 < FH; f0 += NT) {
-      const int fh = f0 + tid;
-      int start = 0, n = 0;
-      if (fh < FH) {
-        const int f = fh / H, h = fh - f * H;
-        const int p0 = pair_off[f], nq = pair_off[f + 1] - p0;
-        start = base[p0 * H + h * nq];
-        n = (base[p0 * H + (h + 1) * nq] - start + rows - 1) / rows;
-      }
+    for (int s0 = 0; s0 < segments; s0 += NT) {
+      const int s = s0 + tid;
+      const int n = s < segments ? (list_range(base, pair_off, s * G, H, G).y + rows - 1) / rows : 0;
       const int inc = wave_scan(n);
       if (lane == 63) wsum[0][wave] = inc;
       __syncthreads();
@@ -485,29 +474,23 @@ __global__ __launch_bounds__(NW * 64) void lists_fill_tail_kernel(
         total += x;
       }
       const int at = carry + woff + inc - n;
-      if (fh < FH) {
-        off[fh] = at;
-        if (fh % H == part) {
-          toff[fh] = at;
-          if (starts) seg_off[fh] = start;
-        }
+      if (s < segments) {
+        off[s] = at;
+        if (s % H == part) toff[s] = at;
       }
       carry += total;
       __syncthreads();  // (the sums are read)
     }
     if (tid == 0) {
-      off[FH] = carry;
-      if (part == 0) {
-        toff[FH] = carry;
-        if (starts) seg_off[FH] = base[PH];
-      }
+      off[segments] = carry;
+      if (part == 0) toff[segments] = carry;
     }
     __syncthreads();
     const int t1 = (int)((int64_t)nbound * (part + 1) / H);
     for (int t = (int)((int64_t)nbound * part / H) + tid; t < t1; t += NT) {
       int seg = -1;
       if (t < carry) {
-        int lo = 0, hi = FH;  // off[lo] <= t < off[hi]
+        int lo = 0, hi = segments;  // off[lo] <= t < off[hi]
         while (hi - lo > 1) {
           const int mid = (lo + hi) >> 1;
           if (off[mid] <= t) lo = mid; else hi = mid;
@@ -517,10 +500,10 @@ __global__ __launch_bounds__(NW * 64) void lists_fill_tail_kernel(
       tseg[t] = seg;
     }
   };
-  tables(tile_rows, tile_off, tile_seg, bound, true);
+  tables(G, tile_rows, tile_off, tile_seg, bound);
   if (tile_off_b) {  // the same lists cut into tiles of another height (the backward kernels')
     __syncthreads();
-    tables(tile_rows_b, tile_off_b, tile_seg_b, bound_b, false);
+    tables(Gb, tile_rows_b, tile_off_b, tile_seg_b, bound_b);
   }
 }
 
@@ -544,28 +527,30 @@ static void launch_scan(int* a, int n, int* scratch, int64_t scratch_ints, hipSt
   hipLaunchKernelGGL(scan_apply_kernel, grid, dim3(1024), 0, st, a, n, per, (const int*)scratch);
 }
 
-static void launch_tile_tables(const int32_t* seg_off, int32_t* tile_off, int32_t* tile_seg, int H, int F,
+static void launch_tile_tables(const int32_t* seg_off, int32_t* tile_off, int32_t* tile_seg, int H, int F, int G,
                                int tile_rows, int64_t hist_bound, hipStream_t st) {
-  if ((int64_t)F * H < kTailMaxSegments && hist_bound <= kTailMaxTiles) {
+  const int segments = F * H / G;
+  if (segments < kTailMaxSegments && hist_bound <= kTailMaxTiles) {
     hipLaunchKernelGGL(lists_tail_kernel, dim3(1), dim3(1024), 0, st, (const int*)nullptr, (const int*)nullptr,
-                       const_cast<int*>(seg_off), tile_off, tile_seg, F, H, tile_rows, (int)hist_bound);
+                       const_cast<int*>(seg_off), tile_off, tile_seg, F, H, G, tile_rows, (int)hist_bound);
     return;
   }
-  hipLaunchKernelGGL(lists_tile_counts_kernel, dim3((F * H + 255) / 256), dim3(256), 0, st, seg_off, tile_off, F * H,
+  hipLaunchKernelGGL(lists_tile_counts_kernel, dim3((segments + 255) / 256), dim3(256), 0, st, seg_off, tile_off, segments, G,
                      tile_rows);
-  launch_scan(tile_off, F * H, tile_seg, hist_bound, st);
+  launch_scan(tile_off, segments, tile_seg, hist_bound, st);
   hipLaunchKernelGGL(lists_tile_seg_kernel, dim3((unsigned)((hist_bound + 255) / 256)), dim3(256), 0, st,
-                     (const int*)tile_off, tile_seg, F * H, (int)hist_bound);
+                     (const int*)tile_off, tile_seg, segments, (int)hist_bound);
 }
 
 // Limits: chunks per sequence minus one (cmax) is bounded by the LDS the fill pass
 // needs, 12 bytes per wave and candidate chunk (4 waves up to 3413 chunks, one wave up to 13653).
-extern "C" int moba_build_lists(const int32_t* sel, const int32_t* chunk_tok, const int32_t* chunk_fb,
+extern "C" int moba_build_lists_grouped(const int32_t* sel, const int32_t* chunk_tok, const int32_t* chunk_fb,
                                 const int32_t* chunk_local, const int32_t* pair_off, int32_t* cnt,
                                 int32_t* seg_off, int32_t* tile_off, int32_t* seg_dest, int32_t* tile_seg,
                                 int64_t S, int H, int K, int N, int F, int P, int cmax, int tile_rows,
                                 int64_t hist_bound, int counted, int tile_rows_b, int32_t* tile_off_b,
-                                int32_t* tile_seg_b, int64_t hist_bound_b, int dense_local, void* stream) {
+                                int32_t* tile_seg_b, int64_t hist_bound_b, int dense_local, int list_heads,
+                                int list_heads_b, void* stream) {
   LaunchCheck launch_check;
   if (!sel || !chunk_tok || !chunk_fb || !chunk_local || !pair_off || !cnt || !seg_off || !tile_off || !seg_dest ||
       !tile_seg)
@@ -575,6 +560,7 @@ extern "C" int moba_build_lists(const int32_t* sel, const int32_t* chunk_tok, co
     return MOBA_ERR_ARG;
   if (S <= 0 || H <= 0 || K <= 0 || N <= 0 || F <= 0 || P <= 0 || cmax <= 0 || tile_rows <= 0) return MOBA_ERR_ARG;
   if (dense_local < 0 || dense_local > K) return MOBA_ERR_ARG;
+  if (list_heads <= 0 || H % list_heads != 0 || list_heads_b <= 0 || H % list_heads_b != 0) return MOBA_ERR_ARG;
   if ((int64_t)S * H * (K + 1) >= 0x7fffffffLL || (int64_t)P * H > 0x7fffffffLL - 4096) return MOBA_ERR_LIMIT;
   // (the scan's steps of 4096 counts stay within an int)
   if (H > 65535 || (size_t)cmax * 12 > 160 * 1024) return MOBA_ERR_LIMIT;
@@ -595,7 +581,7 @@ extern "C" int moba_build_lists(const int32_t* sel, const int32_t* chunk_tok, co
 #define MOBA_FILL_TAIL(KC, NW)                                                                                       \
   hipLaunchKernelGGL((lists_fill_tail_kernel<KC, NW>), dim3(N + 1, H), dim3(NW * 64), lds, st, sel, chunk_tok, chunk_fb, \
                      chunk_local, pair_off, (const int*)cnt, seg_dest, seg_off, tile_off, tile_seg, N, H, K, F,      \
-                     P * H, tile_rows, (int)hist_bound, tile_rows_b, tile_off_b, tile_seg_b, (int)hist_bound_b,      \
+                     P * H, list_heads, tile_rows, (int)hist_bound, list_heads_b, tile_rows_b, tile_off_b, tile_seg_b, (int)hist_bound_b,      \
                      dense_local)
     if (K <= 4) {
       if (many_waves) MOBA_FILL_TAIL(4, 16); else MOBA_FILL_TAIL(4, 4);
@@ -639,16 +625,27 @@ extern "C" int moba_build_lists(const int32_t* sel, const int32_t* chunk_tok, co
 #undef MOBA_FILL
   if (small_tail) {
     hipLaunchKernelGGL(lists_tail_kernel, dim3(1), dim3(1024), 0, st, (const int*)cnt, pair_off, seg_off, tile_off,
-                       tile_seg, F, H, tile_rows, (int)hist_bound);
+                       tile_seg, F, H, list_heads, tile_rows, (int)hist_bound);
   } else {
     hipLaunchKernelGGL(lists_segments_kernel, dim3((F * H + 1 + 255) / 256), dim3(256), 0, st, (const int*)cnt,
-                       pair_off, seg_off, tile_off, F, H, tile_rows);
-    launch_scan(tile_off, F * H, tile_seg, hist_bound, st);
+                       pair_off, seg_off, tile_off, F, H, list_heads, tile_rows);
+    launch_scan(tile_off, F * H / list_heads, tile_seg, hist_bound, st);
     hipLaunchKernelGGL(lists_tile_seg_kernel, dim3((unsigned)((hist_bound + 255) / 256)), dim3(256), 0, st,
-                       (const int*)tile_off, tile_seg, F * H, (int)hist_bound);
+                       (const int*)tile_off, tile_seg, F * H / list_heads, (int)hist_bound);
   }
-  if (tile_off_b) launch_tile_tables(seg_off, tile_off_b, tile_seg_b, H, F, tile_rows_b, hist_bound_b, st);
+  if (tile_off_b) launch_tile_tables(seg_off, tile_off_b, tile_seg_b, H, F, list_heads_b, tile_rows_b, hist_bound_b, st);
   return launch_check.result();
+}
+
+extern "C" int moba_build_lists(const int32_t* sel, const int32_t* chunk_tok, const int32_t* chunk_fb,
+                                const int32_t* chunk_local, const int32_t* pair_off, int32_t* cnt,
+                                int32_t* seg_off, int32_t* tile_off, int32_t* seg_dest, int32_t* tile_seg,
+                                int64_t S, int H, int K, int N, int F, int P, int cmax, int tile_rows,
+                                int64_t hist_bound, int counted, int tile_rows_b, int32_t* tile_off_b,
+                                int32_t* tile_seg_b, int64_t hist_bound_b, int dense_local, void* stream) {
+  return moba_build_lists_grouped(sel, chunk_tok, chunk_fb, chunk_local, pair_off, cnt, seg_off, tile_off, seg_dest, tile_seg,
+                                  S, H, K, N, F, P, cmax, tile_rows, hist_bound, counted, tile_rows_b, tile_off_b, tile_seg_b,
+                                  hist_bound_b, dense_local, 1, 1, stream);
 }
 
 // The tile tables alone, for another number of rows per tile, from the list starts moba_build_lists wrote
@@ -659,6 +656,6 @@ extern "C" int moba_tile_tables(const int32_t* seg_off, int32_t* tile_off, int32
   if (!seg_off || !tile_off || !tile_seg) return MOBA_ERR_ARG;
   if (H <= 0 || F <= 0 || tile_rows <= 0 || hist_bound <= 0 || hist_bound >= 0x7fffffffLL) return MOBA_ERR_ARG;
   if ((int64_t)F * H >= 0x7fffffffLL) return MOBA_ERR_LIMIT;
-  launch_tile_tables(seg_off, tile_off, tile_seg, H, F, tile_rows, hist_bound, (hipStream_t)stream);
+  launch_tile_tables(seg_off, tile_off, tile_seg, H, F, 1, tile_rows, hist_bound, (hipStream_t)stream);
   return launch_check.result();
 }

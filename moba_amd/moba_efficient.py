@@ -296,7 +296,7 @@ class _Geometry:
     """What a forward call needs besides its tensors, worked out once per (plan, heads, head_dim, element size):
     buffer sizes, the carving of the two scratch allocations, the key split and the tables' addresses."""
 
-    def __init__(self, plan: MobaPlan, lib, H: int, D: int, esize: int):
+    def __init__(self, plan: MobaPlan, lib, H: int, Hkv: int, D: int, esize: int):
         S, K = plan.S, plan.K
         # rows per tile of the forward (forward_tile_rows); tiles of the backward's height share its tables
         self.rows_per_tile = forward_tile_rows(plan, H, D)
@@ -304,15 +304,24 @@ class _Geometry:
         self.self_tiles = plan.fwd_self_tiles if tall else plan.self_tiles
         self.self_names = (("fwd_" if tall else "") + "self_tile_prefix", ("fwd_" if tall else "") + "self_tile_chunk")
         self.tptr = {name: t.data_ptr() for name, t in plan.tables.items()}
-        self.bound = plan.hist_tile_bound(H, self.rows_per_tile)
+        # Heads whose lists are cut into tiles together: those of a key/value head, whose lists lie one behind the other and
+        # attend the same keys, so that only the last of their tiles is part empty.  Worth the more, the fewer tiles a list
+        # has (32 heads over 8, 3 x 2001 tokens, chunk 256: 155 -> 152 us; 8191 tokens, chunk 512: 217 -> 213 us; a training
+        # step of 17301 packed tokens, 8 heads over 2: 644 -> 631 us) and never a loss; not for the forward's tall tiles,
+        # which long chunks have and whose kernel has no registers left.
+        self.list_heads = 1 if tall else H // Hkv
+        self.bwd_list_heads = H // Hkv
+        self.bound = plan.hist_tile_bound(H, self.rows_per_tile, self.list_heads)
         if plan.fallback:
             self.split = 1
         else:
             # (two of the short tiles share a compute unit: they count half.  16384 tokens, 2 heads, chunk 4096 in two parts:
             # 149 -> 130 us; 8192 tokens, 4 heads, chunk 1024: 57 -> 49 us; with twice as many tiles the merge of the
             # parts takes what they gain)
+            # (the number of parts does not depend on the heads that are cut together: it is part of the result's rounding)
             n = 1 if tall else 2
-            self.split = int(lib.moba_fwd_key_split(S, H, K, plan.chunk_size, -(-self.bound // n), -(-self.self_tiles // n)))
+            bound = plan.hist_tile_bound(H, self.rows_per_tile)
+            self.split = int(lib.moba_fwd_key_split(S, H, K, plan.chunk_size, -(-bound // n), -(-self.self_tiles // n)))
         # lists: cnt, seg_off, tile_off, seg_dest, tile_seg (int32, each start a multiple of 4 ints)
         sizes = [plan.P * H + 1, plan.F * H + 1, plan.F * H + 1, max(plan.pairs_per_head * H, 1), self.bound]
         self.list_sizes = sizes
@@ -322,7 +331,7 @@ class _Geometry:
         self.list_starts = starts
         # ... and, for a call that a backward will follow, the backward kernels' tile tables behind them, unless the
         # forward's tiles have the same height
-        self.bwd_bound = plan.hist_tile_bound(H, TILE_ROWS)
+        self.bwd_bound = plan.hist_tile_bound(H, TILE_ROWS, self.bwd_list_heads)
         if tall:
             self.bwd_starts = [starts[-1], starts[-1] + (plan.F * H + 1 + 3) // 4 * 4]
             self.list_ints_with_bwd = self.bwd_starts[1] + self.bwd_bound
@@ -338,7 +347,7 @@ class _Geometry:
         self.scratch_ints = 8 + 1 + self.bound + self.self_tiles * H
         self.ws_bytes = self.part_o_bytes + rows * 4 + self.scratch_ints * 4
         self.mean = {}     # kv heads -> bytes of the chunk representatives and of the chunk mean's workspace
-        self.bwd = {}      # kv heads -> sizes of the backward's scratch
+        self.bwd = {}      # (heads cut together, kv heads of the whole call) -> sizes of the backward's scratch
 
 
 # Which of its two forms the forward attention kernel takes: tiles of TILE_ROWS rows, one workgroup each, two side by side
@@ -359,11 +368,11 @@ def forward_tile_rows(plan: MobaPlan, H: int, D: int = HEAD_DIM) -> int:
     return TILE_ROWS if short_chunks or plan.flops_per_head * HEAD_DIM * H <= SHORT_TILES_FLOPS else FWD_TILE_ROWS
 
 
-def _geometry(plan: MobaPlan, lib, H: int, D: int, esize: int) -> _Geometry:
-    key = (H, D, esize)
+def _geometry(plan: MobaPlan, lib, H: int, D: int, esize: int, Hkv: int = 0) -> _Geometry:
+    key = (H, Hkv or H, D, esize)
     g = plan.memo.get(key)
     if g is None:
-        g = plan.memo[key] = _Geometry(plan, lib, H, D, esize)
+        g = plan.memo[key] = _Geometry(plan, lib, H, Hkv or H, D, esize)
     return g
 
 
@@ -393,7 +402,7 @@ def _run_forward(q, k, v, plan: MobaPlan, timer: Optional[StageTimer] = None, sc
     Hkv = _dims(k)[1]
     dev = q.device
     K = plan.K
-    g = _geometry(plan, lib, H, D, q.element_size())
+    g = _geometry(plan, lib, H, D, q.element_size(), Hkv)
     tp = g.tptr
     span = (lambda name: timer.span(name, dev)) if timer is not None else (lambda name: _NO_SPAN)
     stream, code, strides = _stream(dev), _dtype_code(q), _strides(q, k)
@@ -425,7 +434,7 @@ def _run_forward(q, k, v, plan: MobaPlan, timer: Optional[StageTimer] = None, sc
         bwd_args = (0, None, None, 0)
         if bwd_tables is not None:
             b0, b1 = g.bwd_starts
-            bwd_tables += [lists[b0:b0 + plan.F * H + 1], lists[b1:b1 + g.bwd_bound]]
+            bwd_tables += [lists[b0:b0 + plan.F * H + 1], lists[b1:b1 + g.bwd_bound], g.bwd_list_heads]
             if g.rows_per_tile != TILE_ROWS:
                 bwd_args = (TILE_ROWS, base + 4 * b0, base + 4 * b1, g.bwd_bound)
         cntp, seg_offp, tile_offp, seg_destp, tile_segp = (base + 4 * a for a in g.list_starts[:5])
@@ -442,10 +451,11 @@ def _run_forward(q, k, v, plan: MobaPlan, timer: Optional[StageTimer] = None, sc
                                           cntp, S, H, Hkv, D, plan.nseq, plan.F, plan.chunk_size, K, plan.dense_local,
                                           strides, code, stream), "moba_gate_topk")
         with span("build_lists"):
-            _lib.check(lib.moba_build_lists(selp, tp["chunk_tok"], tp["chunk_fb"], tp["chunk_local"], tp["pair_off"],
-                                            cntp, seg_offp, tile_offp, seg_destp, tile_segp, S, H, K, plan.N, plan.F,
-                                            plan.P, plan.cmax, g.rows_per_tile, g.bound, 1, *bwd_args, plan.dense_local,
-                                            stream), "moba_build_lists")
+            _lib.check(lib.moba_build_lists_grouped(selp, tp["chunk_tok"], tp["chunk_fb"], tp["chunk_local"],
+                                                    tp["pair_off"], cntp, seg_offp, tile_offp, seg_destp, tile_segp, S, H,
+                                                    K, plan.N, plan.F, plan.P, plan.cmax, g.rows_per_tile, g.bound, 1,
+                                                    *bwd_args, plan.dense_local, g.list_heads, g.bwd_list_heads, stream),
+                       "moba_build_lists_grouped")
     redop = queuesp + 32 if FIXED_REFERENCE else None
     if g.rows_per_tile == TILE_ROWS and not KEEP_SCRATCH:
         redop = None    # (these tiles need no list: their workgroups compute them again themselves)
@@ -460,7 +470,8 @@ def _run_forward(q, k, v, plan: MobaPlan, timer: Optional[StageTimer] = None, sc
                                               tile_segp, tp[g.self_names[1]], tp["achunk_direct"] if DIRECT_ROWS else None,
                                               outp, lsep, S, H, Hkv, D, K, plan.F, plan.NA,
                                               plan.chunk_size, g.bound, g.self_tiles, g.split, strides, queuesp,
-                                              redop, scale, code, 0, 0, g.rows_per_tile, 0 if FIXED_REFERENCE else 1, stream),
+                                              redop, scale, code, 0, 0, g.rows_per_tile, 0 if FIXED_REFERENCE else 1,
+                                              g.list_heads, stream),
                    "moba_fwd_partials_rows")
     if not DIRECT_ROWS:
         with span("fwd_merge"):
@@ -504,8 +515,8 @@ def _for_training(*tensors: torch.Tensor):
 
 def _backward(dout, q, k, v, out, lse, sel, seg_off, seg_dest, plan: MobaPlan, scale: float = 0.0, tables=None,
               all_kv_heads: int = 0):
-    """tables: the backward kernels' (tile_off, tile_seg) if the forward made them (made here otherwise).  all_kv_heads:
-    the key/value heads of the call of which this is a part (0: it is not).
+    """tables: the backward kernels' tile_off, tile_seg and heads cut together if the forward made them (made here, for
+    single heads, otherwise).  all_kv_heads: the key/value heads of the call of which this is a part (0: it is not).
     The gradients' heads have dout's width."""
     lib = _lib.load()
     S, H, D = _dims(q)
@@ -517,26 +528,29 @@ def _backward(dout, q, k, v, out, lse, sel, seg_off, seg_dest, plan: MobaPlan, s
     Hkv = _dims(k)[1]
     dev = q.device
     K = plan.K
-    g = _geometry(plan, lib, H, D, q.element_size())
+    g = _geometry(plan, lib, H, D, q.element_size(), Hkv)
     tp = g.tptr
     stream = _stream(dev)
     # One allocation for the call's scratch, every part a multiple of 16 bytes: the per-slot partial dQ, delta and
     # the log2 lse, the 16 tile counters of the two kernels (zeroed by the call), the backward kernels' own tile
     # tables (they cut the gather lists into tiles of their own height) and, for small problems, the fp32 sums of
     # the key tiles that several workgroups of the dK/dV kernel have parts of (0 bytes otherwise)
-    b = g.bwd.get((Hkv, all_kv_heads))
+    list_heads = tables[2] if tables else 1
+    b = g.bwd.get((list_heads, all_kv_heads))
     if b is None:
-        bound = plan.hist_tile_bound(H, TILE_ROWS)
+        bound = plan.hist_tile_bound(H, TILE_ROWS, list_heads)
         kv_shares = lib.moba_bwd_dkv_shares(S, all_kv_heads or Hkv, plan.kv_tiles)
         kv_bytes = int(lib.moba_bwd_dkv_scratch_bytes(S, Hkv, plan.kv_tiles)) if kv_shares else 0
         # small problems: the keys of every history tile of the dQ kernel in `split` parts with slots of their own
-        split = 1 if plan.fallback else int(lib.moba_bwd_dq_key_split(S, H, K, plan.chunk_size, bound, plan.self_tiles))
+        # (of whatever heads are cut together: the parts are part of the result's rounding)
+        split = 1 if plan.fallback else int(lib.moba_bwd_dq_key_split(S, H, K, plan.chunk_size, plan.hist_tile_bound(H, TILE_ROWS),
+                                                                      plan.self_tiles))
         sizes = [split * S * H * (K + 1) * D * q.element_size(), 2 * S * H * 4, 64,
                  0 if plan.fallback else (plan.F * H + 1) * 4, 0 if plan.fallback else bound * 4, kv_bytes]
         starts = [0]
         for n in sizes:
             starts.append(starts[-1] + (n + 15) // 16 * 16)
-        b = g.bwd[Hkv, all_kv_heads] = (bound, kv_bytes, kv_shares, starts, split)
+        b = g.bwd[list_heads, all_kv_heads] = (bound, kv_bytes, kv_shares, starts, split)
     bound, kv_bytes, kv_shares, starts, split = b
     ws = torch.empty(starts[-1], dtype=torch.uint8, device=dev)
     base = ws.data_ptr()
@@ -559,7 +573,8 @@ def _backward(dout, q, k, v, out, lse, sel, seg_off, seg_dest, plan: MobaPlan, s
                               if DIRECT_ROWS else (None, None, None, 0, S)),
                             deltap, part_dqp, _ptr(dq), _ptr(dk), _ptr(dv), S, H, Hkv, D, K, plan.F, plan.NA,
                             plan.chunk_size, bound, plan.self_tiles, plan.kv_tiles, split, _strides(q, k), queuesp,
-                            kvp if kv_bytes else None, kv_bytes, kv_shares, scale, _dtype_code(q), stream), "moba_bwd")
+                            kvp if kv_bytes else None, kv_bytes, kv_shares, list_heads, scale, _dtype_code(q), stream),
+               "moba_bwd")
     return dq, dk, dv
 
 

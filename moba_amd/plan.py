@@ -54,9 +54,10 @@ class MobaPlan:
     memo: Dict[tuple, object] = field(default_factory=dict)  # what callers derive once per plan (sizes, pointers)
     device: object = None
 
-    def hist_tile_bound(self, H: int, rows: int = TILE_ROWS) -> int:
-        """Upper bound on the number of history tiles of `rows` rows (every segment may end in a partial tile)."""
-        return (self.pairs_per_head * H) // rows + self.F * H
+    def hist_tile_bound(self, H: int, rows: int = TILE_ROWS, list_heads: int = 1) -> int:
+        """Upper bound on the number of history tiles of `rows` rows (every segment may end in a partial tile).
+        list_heads: heads whose lists are cut into tiles together."""
+        return (self.pairs_per_head * H) // rows + self.F * (H // list_heads)
 
     def with_dense_prefix(self) -> "MobaPlan":
         """The plan of the same batch with the first K + 1 chunks of every sequence as one attention chunk."""

@@ -21,3 +21,44 @@ def test_lists_in_one_launch(batch, seqlen, heads, B, topk, counted, dense):
     if dense and seqlen <= topk * B:
         pytest.skip("every token lies in a dense prefix")
     check_lists(batch, seqlen, heads, B, topk, counted, dense)
+
+
+@pytest.mark.parametrize("seqlen,heads,group,B,topk", [
+    (1500, 6, 3, 100, 4),        # one launch
+    (5000, 4, 4, 1024, 3),       # ... of 16 waves
+    (129 * 66, 2, 2, 66, 3),     # separate launches, one workgroup for the tables
+    (60007, 4, 2, 16, 3),        # ... and many
+])
+def test_tiles_of_several_heads(seqlen, heads, group, B, topk):
+    """Tile tables that cut the lists of the heads of a key/value head together: lists as ever, tiles of all their rows."""
+    import numpy as np
+    import torch
+    from moba_amd import _lib
+    from moba_amd import moba_efficient as E
+    lib = _lib.load()
+    print("tiles of heads", seqlen, heads, group, B, topk, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(heads)
+    plan = E.make_plan(torch.tensor([0, seqlen], dtype=torch.int32, device="cuda"), B, topk)
+    q = torch.randn((seqlen, heads, 128), generator=g, device="cuda").to(torch.bfloat16)
+    sel = E.gate_topk(q, E.chunk_mean(q, plan), plan)
+    want_off, _, want_dest, _ = E.build_lists(sel, plan)
+    segments, t = plan.F * heads // group, plan.tables
+    bounds = [plan.hist_tile_bound(heads, rows, n) for rows, n in ((256, 1), (128, group))]
+    dev = dict(dtype=torch.int32, device="cuda")
+    cnt, seg_off = torch.empty(plan.P * heads + 1, **dev), torch.empty(plan.F * heads + 1, **dev)
+    seg_dest = torch.empty_like(want_dest)
+    off_a, seg_a = torch.empty(plan.F * heads + 1, **dev), torch.full((bounds[0],), -7, **dev)
+    off_b, seg_b = torch.empty(segments + 1, **dev), torch.full((bounds[1],), -7, **dev)
+    p = lambda x: x.data_ptr()
+    _lib.check(lib.moba_build_lists_grouped(
+        p(sel), p(t["chunk_tok"]), p(t["chunk_fb"]), p(t["chunk_local"]), p(t["pair_off"]), p(cnt), p(seg_off), p(off_a),
+        p(seg_dest), p(seg_a), seqlen, heads, plan.K, plan.N, plan.F, plan.P, plan.cmax, 256, bounds[0], 0, 128, p(off_b),
+        p(seg_b), bounds[1], 0, 1, group, torch.cuda.current_stream().cuda_stream), "moba_build_lists_grouped")
+    assert torch.equal(seg_off, want_off) and torch.equal(seg_dest, want_dest)
+    counts = np.diff(want_off.cpu().numpy())
+    for n, rows, off, seg in ((1, 256, off_a, seg_a), (group, 128, off_b, seg_b)):
+        tiles = -(-counts.reshape(-1, n).sum(1) // rows)
+        assert np.array_equal(off.cpu().numpy(), np.concatenate([[0], np.cumsum(tiles)]))
+        names = np.repeat(np.arange(tiles.size), tiles)
+        got = seg.cpu().numpy()
+        assert names.size <= got.size and np.array_equal(got[:names.size], names) and (got[names.size:] == -1).all()
