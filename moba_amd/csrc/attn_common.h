@@ -250,14 +250,8 @@ __device__ __forceinline__ void decode_tile_rows(const TileTables& p, int wave, 
   const int H = p.H;
   if (t.base >= 0) {
     t.dest = entry;
-    if (kGrouped && p.seg_heads > 1) {
-      const int row = entry / p.K1;
-      t.tok = row / H;
-      t.rh = row - t.tok * H;
-    } else {
-      t.tok = t.dest / (H * p.K1);
-      t.rh = t.h;
-    }
+    t.tok = t.dest / (H * p.K1);
+    t.rh = kGrouped ? (entry - t.tok * (H * p.K1)) / p.K1 : t.h;
     t.limit = t.nkeys - 1;
     t.wave_min_limit = t.limit;
     t.wave_max_limit = t.limit;
