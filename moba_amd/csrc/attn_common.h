@@ -110,7 +110,6 @@ struct Tile {
   int tok;        // this lane's row: token
   int limit;      // this lane's row attends keys <= limit
   int wave_min_limit, wave_max_limit;  // over the wave's 32 rows
-  int rot;        // history tiles may visit their key tiles in any order: start offset
   int base;       // history tile: index of row 0 in seg_dest; self tile: -(row 0 inside the chunk) - 1
   int direct;     // self tile of a chunk without history slots: dest is the output row token*H + h
 };
@@ -214,7 +213,6 @@ __device__ __forceinline__ bool decode_tile_head(const TileTables& p, int logica
     t.row_count = min(tm, e.c - t.base);
     t.kv_tok0 = e.d;
     t.nkeys = p.B;
-    t.rot = tile;
     return true;
   }
   const int st = logical - p.hist_bound;
@@ -228,7 +226,6 @@ __device__ __forceinline__ bool decode_tile_head(const TileTables& p, int logica
   t.row_count = min(tm, len - tin * tm);
   t.kv_tok0 = c0;
   t.nkeys = min(len, tin * tm + tm);
-  t.rot = 0;
   t.direct = e.e;
   return true;
 }

@@ -315,7 +315,7 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(const BwdParams<E> p) {
   const int nkt = (nkeys + TN - 1) / TN;
   // (every tile goes through its keys from the first on: a row's dQ does not depend on the tile that its list puts it in.
   // Tiles of a chunk that start at different keys, so as not to ask for the same lines at once, gained nothing: 105.3 against
-  // 104.9 ms for a training step of 524288 tokens in 8 sequences)
+  // 104.9 ms for a training step of 302060 tokens in 8 sequences)
   issue_tile(0, 0);
 
   decode_tile_rows<true>(p.t, wave, r, entry, t);
