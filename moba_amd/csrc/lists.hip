@@ -594,7 +594,9 @@ extern "C" int moba_build_lists_grouped(const int32_t* sel, const int32_t* chunk
   if (!counted)
     hipLaunchKernelGGL(lists_count_kernel<256>, grid, dim3(256), (size_t)cmax * 4, st, sel, chunk_tok, chunk_fb,
                        chunk_local, pair_off, cnt, H, K, dense_local);
-  launch_scan(cnt, P * H, tile_off, (int64_t)F * H, st);
+  // (scratch: the list starts, F*H+1 ints that the launches behind the scan write.  The tile tables are shorter where heads
+  // are cut together, and the sums -- one per 4096 counts -- can be more than they hold.)
+  launch_scan(cnt, P * H, seg_off, (int64_t)F * H, st);
   // more than 64 KiB of dynamic LDS has to be asked for explicitly
   // (LDS: 12 bytes per wave and candidate chunk)
   const bool wide = S / N >= 1024 && (size_t)cmax * 192 <= 64 * 1024;  // long chunks: 16 waves per (chunk, head)

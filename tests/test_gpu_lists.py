@@ -62,3 +62,41 @@ def test_tiles_of_several_heads(seqlen, heads, group, B, topk):
         names = np.repeat(np.arange(tiles.size), tiles)
         got = seg.cpu().numpy()
         assert names.size <= got.size and np.array_equal(got[:names.size], names) and (got[names.size:] == -1).all()
+
+
+def test_first_tables_of_several_heads():
+    """Both pairs of tile tables for all heads of a key/value head, in arrays of just their size: 511 segments, while the scan of
+    the 4.2 million counts works on 1021 sums, more than the tables hold.  What lies behind the arrays stays as it was."""
+    import numpy as np
+    import torch
+    from moba_amd import _lib
+    from moba_amd import moba_efficient as E
+    lib = _lib.load()
+    seqlen, heads, B, topk = 512 * 16, 32, 16, 3
+    plan = E.make_plan(torch.tensor([0, seqlen], dtype=torch.int32, device="cuda"), B, topk)
+    segments, t = plan.F, plan.tables      # (one segment per chunk: 32 heads on one)
+    assert -(-plan.P * heads // 4096) > segments + 1
+    print("tables of all heads", plan.P * heads, segments, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    q = torch.randn((seqlen, heads, 128), generator=g, device="cuda").to(torch.bfloat16)
+    sel = E.gate_topk(q, E.chunk_mean(q, plan), plan)
+    want_off, _, want_dest, _ = E.build_lists(sel, plan)
+    dev, guard, p = dict(dtype=torch.int32, device="cuda"), 4096, lambda x: x.data_ptr()
+    cnt, seg_off = torch.empty(plan.P * heads + 1, **dev), torch.empty(plan.F * heads + 1, **dev)
+    seg_dest = torch.empty_like(want_dest)
+    bounds = [plan.hist_tile_bound(heads, rows, heads) for rows in (256, 128)]
+    offs = [torch.full((segments + 1 + guard,), -7, **dev) for _ in bounds]
+    segs = [torch.full((n + guard,), -7, **dev) for n in bounds]
+    _lib.check(lib.moba_build_lists_grouped(
+        p(sel), p(t["chunk_tok"]), p(t["chunk_fb"]), p(t["chunk_local"]), p(t["pair_off"]), p(cnt), p(seg_off), p(offs[0]),
+        p(seg_dest), p(segs[0]), seqlen, heads, plan.K, plan.N, plan.F, plan.P, plan.cmax, 256, bounds[0], 0, 128, p(offs[1]),
+        p(segs[1]), bounds[1], 0, heads, heads, torch.cuda.current_stream().cuda_stream), "moba_build_lists_grouped")
+    assert torch.equal(seg_off, want_off) and torch.equal(seg_dest, want_dest)
+    counts = np.diff(want_off.cpu().numpy()).reshape(-1, heads).sum(1)
+    for rows, off, seg, bound in zip((256, 128), offs, segs, bounds):
+        tiles = -(-counts // rows)
+        off, seg = off.cpu().numpy(), seg.cpu().numpy()
+        assert np.array_equal(off[:segments + 1], np.concatenate([[0], np.cumsum(tiles)])) and (off[segments + 1:] == -7).all()
+        names = np.repeat(np.arange(tiles.size), tiles)
+        assert np.array_equal(seg[:names.size], names)
+        assert (seg[names.size:bound] == -1).all() and (seg[bound:] == -7).all()
