@@ -77,15 +77,18 @@ struct BwdParams {
   int queues_log2;
 };
 
+constexpr int kDkvScratchAlign = 16;  // of the scratch that holds the sums and, whole 128 KiB behind its start, the table of ShareTile
 // A key tile where the query heads' rows are walked in one go: those that attend its keys causally, head by head, then the
 // gather lists of all heads, which lie one behind the other.
-struct alignas(32) ShareTile {
+struct alignas(16) ShareTile {
   int begin;                // its first place (share_count)
   int tok0, keys;           // first token, keys of the chunk from there on
   int self_rows;            // rows per head that attend its keys causally: tokens tok0 .. tok0 + self_rows - 1
   int list_base, list_rows;
   int unused[2];
 };
+static_assert(alignof(ShareTile) <= kDkvScratchAlign && (2 * TM * kHeadDim * sizeof(float)) % alignof(ShareTile) == 0,
+              "the table lies where the caller's scratch puts it");
 
 // which 128-key tile of which key/value head: the forward's self-tile enumeration over the chunks and Hkv heads
 struct KvTile {
@@ -1263,7 +1266,7 @@ extern "C" int moba_bwd(const void* dout, const void* q, const void* k, const vo
   const int64_t kv_total = kv_tiles * Hkv;
   if (kv_total >= 0x7fffffffLL) return MOBA_ERR_LIMIT;
   if (dkv_shares < 0 || (dkv_shares > 0 && Hkv > 64)) return MOBA_ERR_ARG;
-  if (dkv_shares && (!dkv_scratch || ((uintptr_t)dkv_scratch & 15) ||
+  if (dkv_shares && (!dkv_scratch || ((uintptr_t)dkv_scratch & (kDkvScratchAlign - 1)) ||
                      dkv_scratch_bytes < (int64_t)::dkv_scratch_bytes(Hkv, kv_tiles, dkv_shares)))
     dkv_shares = 0;
   hipStream_t st = (hipStream_t)stream;
