@@ -58,7 +58,7 @@ extern "C" {
 
 enum { MOBA_DTYPE_BF16 = 0, MOBA_DTYPE_F16 = 1 };
 
-#define MOBA_ABI_VERSION 119 /* the signatures below; moba_version() returns the number the library was built with */
+#define MOBA_ABI_VERSION 120 /* the signatures below; moba_version() returns the number the library was built with */
 int moba_version(void);
 const char* moba_strerror(int code);
 
@@ -326,11 +326,12 @@ int moba_fwd(const void* q, const void* k, const void* v, void* part_o, float* p
  *              key tiles of a head in dkv_shares = moba_bwd_dkv_shares() equal shares; the fp32 sums of the tiles that
  *              several shares have parts of go through dkv_scratch, moba_bwd_dkv_scratch_bytes(S, Hkv, kv_tiles) bytes,
  *              16-byte aligned, and are added up in a fixed order (deterministic all the same).  Without the scratch (null, or
- *              too small) or with dkv_shares = 0, every tile is one piece.  A call for some of the heads gives what a call
+ *              too small) or with dkv_shares = 0, every tile is one piece.  Shares of more stages than 32-bit numbers hold
+ *              are refused (-4); moba_bwd_dkv_shares() gives 0 for such sizes.  A call for some of the heads gives what a call
  *              for all would, bit for bit, with that call's dkv_shares.
  *   list_heads: of tile_off and tile_seg, see moba_build_lists_grouped
  *   softmax_scale: as in the forward call */
-int moba_bwd_dkv_shares(int64_t S, int Hkv, int64_t kv_tiles);
+int moba_bwd_dkv_shares(int64_t S, int H, int Hkv, int64_t kv_tiles);
 size_t moba_bwd_dkv_scratch_bytes(int64_t S, int Hkv, int64_t kv_tiles);
 int moba_bwd_dq_key_split(int64_t S, int H, int K, int B, int64_t hist_bound, int64_t self_tiles);
 int moba_bwd(const void* dout, const void* q, const void* k, const void* v, const void* out, const float* lse,

@@ -1180,10 +1180,22 @@ extern "C" int moba_bwd_tile_rows(void) { return TM; }
 // fewer.  Whole tiles / shares in us, forward and backward: 15 heads of 4096 tokens, chunk 512 (480 tiles): 310 / 315; 4 of 16384
 // (512): 352 / 346; 8 of 16384, chunk 1024 (1024): 866 / 895; 32 heads on 8, 32768 tokens, chunk 2048 (2048): 14907 / 15890.
 // Below 1024 tokens there is nothing to cut (8 tiles of a head then, so no more than 64 heads: a lane each in the kernel).
-extern "C" int moba_bwd_dkv_shares(int64_t S, int Hkv, int64_t kv_tiles) {
+static int most_dkv_shares(int64_t S, int Hkv, int64_t kv_tiles) {
   const int cus = resident_compute_units();
   if (cus <= 0 || Hkv <= 0 || kv_tiles <= 0 || kv_tiles * Hkv >= 2 * (int64_t)cus || S < 1024 || Hkv > 64) return 0;
   return Hkv < cus ? cus / Hkv : 1;
+}
+// Whether the kernel's 32-bit numbers hold the shares' stages: of a key tile's causal ones, `stages` per head, the number times
+// `stages` (self_stage divides by a multiplication that is exact up to 2^32), and the places of all tiles, each with
+// no more list stages than causal ones.
+static bool shares_fit(int64_t S, int64_t rep, int64_t kv_tiles, int64_t Hkv) {
+  if (S >= 0x7fffffffLL || rep >= 0x7fffffffLL || kv_tiles >= 0x7fffffffLL) return false;
+  const int64_t stages = (S + TQ - 1) / TQ;
+  return stages * rep <= (1LL << 32) / stages && kv_tiles * Hkv <= 0x7fffffffLL / (kTileStart + 2 * stages * rep);
+}
+extern "C" int moba_bwd_dkv_shares(int64_t S, int H, int Hkv, int64_t kv_tiles) {
+  if (H <= 0 || Hkv <= 0 || H % Hkv != 0 || kv_tiles <= 0 || S <= 0 || !shares_fit(S, H / Hkv, kv_tiles, Hkv)) return 0;
+  return most_dkv_shares(S, Hkv, kv_tiles);
 }
 
 // dkv_shares: of a head
@@ -1191,7 +1203,7 @@ static size_t dkv_scratch_bytes(int Hkv, int64_t kv_tiles, int dkv_shares) {
   return (size_t)Hkv * (kv_tiles + dkv_shares) * (2 * TM * kHeadDim) * sizeof(float) + (Hkv * kv_tiles + 1) * sizeof(ShareTile);
 }
 extern "C" size_t moba_bwd_dkv_scratch_bytes(int64_t S, int Hkv, int64_t kv_tiles) {
-  const int shares = moba_bwd_dkv_shares(S, Hkv, kv_tiles);
+  const int shares = most_dkv_shares(S, Hkv, kv_tiles);
   return shares ? dkv_scratch_bytes(Hkv, kv_tiles, shares) : 0;
 }
 
@@ -1240,6 +1252,14 @@ extern "C" int moba_bwd(const void* dout, const void* q, const void* k, const vo
   if (dq_key_split < 1 || dq_key_split > 8 || (dq_key_split & (dq_key_split - 1))) return MOBA_ERR_ARG;
   if (dq_key_split > 1 && (K == 0 || B % (64 * dq_key_split) != 0)) return MOBA_ERR_ARG;
   if ((int64_t)S * H * (K + 1) * dq_key_split >= 0x7fffffffLL) return MOBA_ERR_LIMIT;
+  const int64_t kv_total = kv_tiles * Hkv;
+  if (kv_total >= 0x7fffffffLL) return MOBA_ERR_LIMIT;
+  // the stages of the key tiles are dealt in shares only if the caller brought the scratch for their sums
+  if (dkv_shares < 0 || (dkv_shares > 0 && Hkv > 64)) return MOBA_ERR_ARG;
+  if (dkv_shares && (!dkv_scratch || ((uintptr_t)dkv_scratch & (kDkvScratchAlign - 1)) ||
+                     dkv_scratch_bytes < (int64_t)::dkv_scratch_bytes(Hkv, kv_tiles, dkv_shares)))
+    dkv_shares = 0;
+  if (dkv_shares && !shares_fit(S, H / Hkv, kv_tiles, Hkv)) return MOBA_ERR_LIMIT;
   const int64_t total_q = (K > 0 ? hist_bound * dq_key_split : 0) + self_tiles * H;
   // the dK/dV kernel: one workgroup per CU, resident, drawing its tiles from the queues
   const int cus = resident_compute_units();
@@ -1262,13 +1282,6 @@ extern "C" int moba_bwd(const void* dout, const void* q, const void* k, const vo
   while ((1 << t.key_split_log2) < dq_key_split) ++t.key_split_log2;
   t.part_stride = (int)(S * H * (K + 1));
   t.chunk_direct = chunk_direct;
-  // the stages of the key tiles are dealt in shares only if the caller brought the scratch for their sums
-  const int64_t kv_total = kv_tiles * Hkv;
-  if (kv_total >= 0x7fffffffLL) return MOBA_ERR_LIMIT;
-  if (dkv_shares < 0 || (dkv_shares > 0 && Hkv > 64)) return MOBA_ERR_ARG;
-  if (dkv_shares && (!dkv_scratch || ((uintptr_t)dkv_scratch & (kDkvScratchAlign - 1)) ||
-                     dkv_scratch_bytes < (int64_t)::dkv_scratch_bytes(Hkv, kv_tiles, dkv_shares)))
-    dkv_shares = 0;
   hipStream_t st = (hipStream_t)stream;
   return dtype == MOBA_DTYPE_F16
              ? launch_bwd<F16>(dout, q, k, v, out, lse, sel, chunk_fid, kv_chunk_tok, kv_tile_prefix, kv_tile_chunk,

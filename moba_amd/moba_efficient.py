@@ -539,7 +539,8 @@ def _backward(dout, q, k, v, out, lse, sel, seg_off, seg_dest, plan: MobaPlan, s
     b = g.bwd.get((list_heads, all_kv_heads))
     if b is None:
         bound = plan.hist_tile_bound(H, TILE_ROWS, list_heads)
-        kv_shares = lib.moba_bwd_dkv_shares(S, all_kv_heads or Hkv, plan.kv_tiles)
+        of_call = all_kv_heads or Hkv
+        kv_shares = lib.moba_bwd_dkv_shares(S, H // Hkv * of_call, of_call, plan.kv_tiles)
         kv_bytes = int(lib.moba_bwd_dkv_scratch_bytes(S, Hkv, plan.kv_tiles)) if kv_shares else 0
         # small problems: the keys of every history tile of the dQ kernel in `split` parts with slots of their own
         # (of whatever heads are cut together: the parts are part of the result's rounding)

@@ -92,3 +92,24 @@ def test_list_counts_beyond_an_int_are_refused(lib):
     for P, H in ((0x7fffffff - 4095, 1), (0x7ffffffe, 1), ((0x7fffffff - 100) // 2, 2)):
         rc = bound.moba_build_lists(*[some] * 10, 4096, H, 1, 16, 64, P, 10, 128, 1024, 1, 0, None, None, 0, 0, None)
         assert rc == -4, (P, H, rc)
+
+
+def test_shares_beyond_32_bits_are_refused(lib):
+    """moba_bwd with shares of a key/value head's work: more stages than the kernel's numbers hold are refused before anything is
+    launched; without the scratch for the shares, which leaves whole tiles, they are no matter."""
+    from moba_amd import _lib
+    bound = _lib.load()
+    some = 256   # (never read: the odd strides end every call that gets that far)
+    odd = (ctypes.c_int64 * 7)(*[1] * 7)
+
+    def call(S, H, Hkv, kv_tiles, shares, scratch=some, size=1 << 62):
+        return bound.moba_bwd(*[some] * 20, None, None, None, 0, S, *[some] * 5, S, H, Hkv, 128, 0, 0, 1, 64, 0, 1, kv_tiles, 1, odd,
+                              some, scratch, size, shares, 1, 0.0, 0, None)
+
+    refused = [(1 << 19, 64 * 2, 2, 4096),        # 8192 causal stages a head, 64 heads: 2^32 exactly, but too many places
+               ((1 << 19) + 64, 64, 1, 1),        # one stage a head more than the division takes
+               (1 << 16, 1 << 14, 4, 512)]        # 2^31 places
+    for sizes in refused:
+        assert call(*sizes, 4) == -4, sizes
+        assert call(*sizes, 0) != -4 and call(*sizes, 4, None) != -4 and call(*sizes, 4, some, 4096) != -4, sizes
+    assert call(1 << 19, 64, 1, 1, 4) != -4

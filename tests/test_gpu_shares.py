@@ -52,3 +52,12 @@ def test_shares_of_key_tiles(lens, heads, kv_heads, B, topk, dtype, monkeypatch)
         a, b = a.float(), b.float()
         assert torch.isfinite(a).all()
         assert (a - b).norm() < step / 2 * b.norm() and (a - b).abs().max() <= 2 * step * b.abs().max()
+
+
+def test_no_shares_beyond_32_bits():
+    """What moba_bwd would refuse for its number of stages gets no shares in the first place."""
+    from moba_amd import _lib
+    lib = _lib.load()
+    assert lib.moba_bwd_dkv_shares(65280, 8, 1, 510) > 0
+    assert lib.moba_bwd_dkv_shares(65280, 4200, 1, 510) == 0
+    assert lib.moba_bwd_dkv_shares(65280, 4200, 4200, 510) == 0 and lib.moba_bwd_dkv_shares(65280, 7, 2, 100) == 0
