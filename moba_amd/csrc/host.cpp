@@ -66,6 +66,13 @@ PyObject* py_supported(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// The allocations may have to free memory and the launches wait for room in the queue, where a callback may in turn wait for
+// Python: other threads go on meanwhile, as they do under PyTorch's own calls and under ctypes.
+struct NoGil {
+  PyThreadState* const state = PyEval_SaveThread();
+  ~NoGil() { PyEval_RestoreThread(state); }
+};
+
 // tail(query, key, value, scaling or None): [B,q_len,H,D] on the decode kernel, or None where that needs copies or pieces
 PyObject* py_tail(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
@@ -87,15 +94,22 @@ PyObject* py_tail(PyObject*, PyObject* const* args, Py_ssize_t n) {
     Py_RETURN_NONE;
   const int splits = tail_splits((int)b, (int)hkv, (int)(h / hkv), (int)q_len, (int)skv);
   const int64_t rows = b * q_len * h * splits;
-  at::Tensor out = at::empty({b, q_len, h, kHeadDim}, at::TensorOptions().dtype(q.scalar_type()).device(q.device()));
-  // partial outputs, then their log-sum-exps (neither is touched with one split)
-  at::Tensor part = at::empty({splits > 1 ? rows * (kHeadDim + 1) : 4}, at::TensorOptions().dtype(at::kFloat).device(q.device()));
-  float* const part_o = part.mutable_data_ptr<float>();
+  const void *const qp = q.const_data_ptr(), *const kp = k.const_data_ptr(), *const vp = v.const_data_ptr();
+  const auto type = q.scalar_type();
+  const auto device = q.device();
   const int64_t strides[5] = {qs[0], qs[1], qs[2], ks[0], ks[1]};
-  const int rc = tail_call(q.const_data_ptr(), k.const_data_ptr(), v.const_data_ptr(), out.mutable_data_ptr(), part_o,
-                           splits > 1 ? part_o + rows * kHeadDim : part_o, (int)b, (int)h, (int)hkv, (int)q_len, (int)skv,
-                           (int)kHeadDim, strides, (float)scale, q.scalar_type() == at::kHalf ? 1 : 0,
-                           c10::hip::getCurrentHIPStream(q.device().index()).stream());
+  at::Tensor out;
+  int rc;
+  {
+    const NoGil no_gil;
+    out = at::empty({b, q_len, h, kHeadDim}, at::TensorOptions().dtype(type).device(device));
+    // partial outputs, then their log-sum-exps (neither is touched with one split)
+    at::Tensor part = at::empty({splits > 1 ? rows * (kHeadDim + 1) : 4}, at::TensorOptions().dtype(at::kFloat).device(device));
+    float* const part_o = part.mutable_data_ptr<float>();
+    rc = tail_call(qp, kp, vp, out.mutable_data_ptr(), part_o, splits > 1 ? part_o + rows * kHeadDim : part_o, (int)b, (int)h,
+                   (int)hkv, (int)q_len, (int)skv, (int)kHeadDim, strides, (float)scale, type == at::kHalf ? 1 : 0,
+                   c10::hip::getCurrentHIPStream(device.index()).stream());
+  }
   if (rc != 0) {
     PyErr_Format(PyExc_RuntimeError, "moba_tail failed with code %d: %s", rc, str_error(rc));
     return nullptr;

@@ -244,3 +244,19 @@ def test_long_pieces_of_a_prompt_take_the_tiles(monkeypatch):
     for j in rows:
         want = _ref(q[:, :, j:j + 1], k[:, :, :101 + j], v[:, :, :101 + j], 128 ** -0.5)
         assert (out[:, j:j + 1].float() - want).abs().max() < 2e-2
+
+
+def test_a_call_lets_other_python_threads_run():
+    """The native call holds no interpreter lock while it allocates and launches: in the place of moba_tail stands CPython's own
+    PyGILState_Check, whose answer -- 1 with the lock -- would be taken for an error code."""
+    import ctypes
+    from moba_amd import _lib
+    host, lib = _lib.host(), _lib.load()
+    at = lambda f: ctypes.cast(f, ctypes.c_void_p).value
+    q, k = torch.zeros((1, 8, 1, 128), device="cuda", dtype=torch.bfloat16), torch.zeros((1, 2, 64, 128), device="cuda", dtype=torch.bfloat16)
+    try:
+        host.bind(at(lib.moba_tail_splits), at(ctypes.pythonapi.PyGILState_Check), at(lib.moba_strerror))
+        assert host.tail(q, k, k, None).shape == (1, 1, 8, 128)
+    finally:
+        host.bind(at(lib.moba_tail_splits), at(lib.moba_tail), at(lib.moba_strerror))
+    assert host.tail(q, k, k, None).abs().max() == 0
