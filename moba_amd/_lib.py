@@ -123,18 +123,29 @@ _host = None
 
 
 def host():
-    """The extension module of csrc/host.cpp, bound to the library's entry points: built with it, and as little optional."""
+    """The extension module of csrc/host.cpp, bound to the library's entry points: built with it, and as little optional.  One that
+    was built for another PyTorch or another version of the C ABI is refused."""
     global _host
     if _host is None:
+        import torch
         lib = load()
         try:
             from . import _host as module
         except ImportError as e:
-            raise RuntimeError(f"{os.path.join(_HERE, '_host.so')} cannot be loaded ({e}): build it with "
-                               "`python -m moba_amd.build`") from e
-        module.bind(*(ctypes.cast(f, c_void_p).value for f in (lib.moba_tail_splits, lib.moba_tail, lib.moba_strerror)))
+            raise RuntimeError(f"moba_amd._host cannot be loaded ({e}): build it with `python -m moba_amd.build`") from e
+        built_for = getattr(module, "torch_version", "an unknown version")
+        if built_for != torch.__version__:
+            raise RuntimeError(f"{module.__file__} was built for PyTorch {built_for}, this is {torch.__version__}: rebuild it with "
+                               "`python -m moba_amd.build`")
+        bind(module, lib.moba_tail)
         _host = module
     return _host
+
+
+def bind(module, tail):
+    """Give the extension module the library's entry points, with `tail` for moba_tail."""
+    lib = load()
+    module.bind(*(ctypes.cast(f, c_void_p).value for f in (lib.moba_version, lib.moba_tail_splits, tail, lib.moba_strerror)))
 
 
 def exported_symbols():

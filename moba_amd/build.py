@@ -1,5 +1,5 @@
 """Builds the HIP kernels into ``moba_amd/libmoba_hip.so`` with hipcc for gfx950, and the extension module
-``moba_amd/_host.so`` (csrc/host.cpp, host code) with g++.
+``moba_amd._host`` (csrc/host.cpp, host code) with g++.
 
 Run as ``python -m moba_amd.build``.  hipcc cross-compiles without a GPU.
 """
@@ -16,7 +16,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(CSRC, "build")
 LIB = os.path.join(HERE, "libmoba_hip.so")
-HOST = os.path.join(HERE, "_host.so")   # extension module, see csrc/host.cpp
+HOST = os.path.join(HERE, "_host" + sysconfig.get_config_var("EXT_SUFFIX"))   # extension module, see csrc/host.cpp
 SOURCES = ["chunk_mean.hip", "gate_topk.hip", "lists.hip", "fwd.hip", "fwd_tile.hip", "bwd.hip", "decode.hip", "plan.hip", "probe.hip", "capi.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -54,18 +54,26 @@ def _host_module(force: bool) -> None:
     """csrc/host.cpp against the installed PyTorch (host code only)."""
     import torch
     src = os.path.join(CSRC, "host.cpp")
-    deps = [src, os.path.abspath(__file__)]
-    if not force and os.path.exists(HOST) and all(os.path.getmtime(HOST) > os.path.getmtime(d) for d in deps):
-        return
+    deps = [src, os.path.abspath(__file__), os.path.join(os.path.dirname(HERE), "include", "moba_hip.h")]
     root = os.path.dirname(torch.__file__)
     include = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
                os.path.join(os.path.dirname(os.path.dirname(HIPCC)), "include"), sysconfig.get_paths()["include"]]
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f'-DMOBA_TORCH_VERSION="{torch.__version__}"',
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *("-I" + d for d in include), src, "-o", HOST,
            "-L" + os.path.join(root, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
+    stamp = os.path.join(OBJ, "host.cmd")   # the command the module was built with: PyTorch's version and place are in it
+    same = os.path.exists(stamp) and open(stamp).read() == "\n".join(cmd)
+    if not force and same and os.path.exists(HOST) and all(os.path.getmtime(HOST) > os.path.getmtime(d) for d in deps):
+        return
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"g++ failed for host.cpp:\n{r.stderr[-8000:]}")
+    with open(stamp, "w") as f:
+        f.write("\n".join(cmd))
+    former = os.path.join(HERE, "_host.so")   # the name without the interpreter's tag that it once had
+    if os.path.exists(former):
+        os.remove(former)
 
 
 def build(force: bool = True, verbose: bool = True) -> str:

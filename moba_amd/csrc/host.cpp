@@ -7,7 +7,9 @@
 // takes.  (Putting the splits together in the first launch, by its last workgroup, would spare the host the second and
 // costs the device more than that: 11.4 us.)
 //
-// Nothing is kept between calls but the addresses of the library's entry points (bind).  What these functions do not
+// Nothing is kept between calls but the addresses of the library's entry points (bind): types by the library's header, whose
+// version the library has to have.  The module itself is tied to one interpreter and one PyTorch: its file name says the
+// first, `torch_version` the second, and _lib.host() refuses it for another.  What these functions do not
 // take -- tensors that have to be copied first, more sequences than a launch takes -- they leave to the caller.
 #include <ATen/ATen.h>
 #include <Python.h>
@@ -15,15 +17,13 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include "../../include/moba_hip.h"
+
 namespace {
 
-using TailSplits = int (*)(int, int, int, int, int);
-using Tail = int (*)(const void*, const void*, const void*, void*, float*, float*, int, int, int, int, int, int, const int64_t*,
-                     float, int, void*);
-using StrError = const char* (*)(int);
-TailSplits tail_splits = nullptr;
-Tail tail_call = nullptr;
-StrError str_error = nullptr;
+decltype(&moba_tail_splits) tail_splits = nullptr;
+decltype(&moba_tail) tail_call = nullptr;
+decltype(&moba_strerror) str_error = nullptr;
 
 constexpr int64_t kHeadDim = 128, kMostSequences = 65535;
 
@@ -131,18 +131,21 @@ PyObject* py_in_place(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// bind(moba_tail_splits, moba_tail, moba_strerror): the addresses of the library's entry points
+// bind(moba_version, moba_tail_splits, moba_tail, moba_strerror): the addresses of the library's entry points
 PyObject* py_bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  TORCH_CHECK_TYPE(n == 3, "bind takes three addresses");
-  void* at[3];
-  for (int i = 0; i < 3; ++i) {
+  TORCH_CHECK_TYPE(n == 4, "bind takes four addresses");
+  void* at[4];
+  for (int i = 0; i < 4; ++i) {
     at[i] = PyLong_AsVoidPtr(args[i]);
     if (PyErr_Occurred()) return nullptr;
   }
-  tail_splits = reinterpret_cast<TailSplits>(at[0]);
-  tail_call = reinterpret_cast<Tail>(at[1]);
-  str_error = reinterpret_cast<StrError>(at[2]);
+  const int version = reinterpret_cast<decltype(&moba_version)>(at[0])();
+  TORCH_CHECK(version == MOBA_ABI_VERSION, "this module was built for version ", MOBA_ABI_VERSION, " of the C ABI, the library has ",
+              version);
+  tail_splits = reinterpret_cast<decltype(tail_splits)>(at[1]);
+  tail_call = reinterpret_cast<decltype(tail_call)>(at[2]);
+  str_error = reinterpret_cast<decltype(str_error)>(at[3]);
   Py_RETURN_NONE;
   END_HANDLE_TH_ERRORS
 }
@@ -157,4 +160,11 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods, null
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__host() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__host() {
+  PyObject* const m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "torch_version", MOBA_TORCH_VERSION) != 0) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

@@ -66,3 +66,27 @@ def test_the_extension_reads_in_place_what_the_general_path_does():
         else:
             assert not same or t.is_contiguous(), (shape, strides, step)
     assert kept > 200
+
+
+def test_an_extension_built_for_something_else_is_refused_and_built_again(monkeypatch):
+    """Another PyTorch's tensors, another version of the C ABI: neither may meet code compiled for the former one."""
+    import ctypes
+    import pytest
+    from moba_amd import _lib, build
+    host, lib = _lib.host(), _lib.load()
+    assert host.torch_version == torch.__version__
+    with pytest.raises(RuntimeError, match="of the C ABI"):
+        other = ctypes.CFUNCTYPE(ctypes.c_int)(lambda: _lib.ABI_VERSION + 1)
+        host.bind(*(ctypes.cast(f, ctypes.c_void_p).value for f in (other, lib.moba_tail_splits, lib.moba_tail, lib.moba_strerror)))
+    build._host_module(force=False)
+    ran = []
+    monkeypatch.setattr(build.subprocess, "run", lambda cmd, **kw: ran.append(cmd) or (_ for _ in ()).throw(InterruptedError))
+    build._host_module(force=False)
+    assert not ran     # (nothing changed: nothing to build)
+    monkeypatch.setattr(torch, "__version__", "2.0.0")
+    with pytest.raises(InterruptedError):
+        build._host_module(force=False)
+    assert '-DMOBA_TORCH_VERSION="2.0.0"' in ran[0]
+    monkeypatch.setattr(_lib, "_host", None)
+    with pytest.raises(RuntimeError, match="was built for PyTorch"):
+        _lib.host()

@@ -252,11 +252,10 @@ def test_a_call_lets_other_python_threads_run():
     import ctypes
     from moba_amd import _lib
     host, lib = _lib.host(), _lib.load()
-    at = lambda f: ctypes.cast(f, ctypes.c_void_p).value
     q, k = torch.zeros((1, 8, 1, 128), device="cuda", dtype=torch.bfloat16), torch.zeros((1, 2, 64, 128), device="cuda", dtype=torch.bfloat16)
     try:
-        host.bind(at(lib.moba_tail_splits), at(ctypes.pythonapi.PyGILState_Check), at(lib.moba_strerror))
+        _lib.bind(host, ctypes.pythonapi.PyGILState_Check)
         assert host.tail(q, k, k, None).shape == (1, 1, 8, 128)
     finally:
-        host.bind(at(lib.moba_tail_splits), at(lib.moba_tail), at(lib.moba_strerror))
+        _lib.bind(host, lib.moba_tail)
     assert host.tail(q, k, k, None).abs().max() == 0
