@@ -379,7 +379,9 @@ __global__ __launch_bounds__(1024) void lists_tail_kernel(const int* __restrict_
 // NW waves as in lists_fill_kernel: 16 for long chunks, 4 otherwise -- workgroups of 16 waves start one after the other, 22 ns
 // apart, and a chunk of 512 tokens is half a batch for each.  Measured: 8191 tokens, 32 heads, chunk 512 (16 waves each
 // and one of them for all tables before): 19.0 -> 15.9 us; 3 x 2001 tokens, 32 heads, chunk 256 (scan, fill and tables as
-// three launches before): 17.3 -> 10.4 us; 20480 tokens, 8 heads, chunk 512: 11.8 -> 9.0.
+// three launches before): 17.3 -> 10.4 us; 20480 tokens, 8 heads, chunk 512: 11.8 -> 9.0; 4096 tokens, 4 heads, chunk
+// 512: 6.4 -> 5.6.  The form of 16 waves is as fast as its forerunner, within 0.3 us, but for 256 workgroups of 1024
+// tokens, where the tables' workgroups are a second round: 9.4 -> 10.4 us.
 constexpr int kFusedMaxCounts = 8192, kFusedMaxCand = 128;
 constexpr int64_t kFusedMaxWork = 1 << 22;
 template <int KC, int NW>
@@ -410,6 +412,8 @@ __global__ __launch_bounds__(NW * 64) void lists_fill_tail_kernel(
   int v[kSteps][4];
 #pragma unroll
   for (int st = 0; st < kSteps; ++st) {
+    if (st * NT * 4 >= PH) break;  // (uniform; without it the loads of the empty steps, which return nothing, cost
+                                   // 0.8 us of 6.4 at 8 chunks of 512, 4 heads, and 0.2 of 9.0 in the form of 16 waves)
     const int i0 = (st * NT + tid) * 4;
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[st][e] = i0 + e < PH ? cnt[i0 + e] : 0;
@@ -568,9 +572,12 @@ extern "C" int moba_build_lists_grouped(const int32_t* sel, const int32_t* chunk
   dim3 grid(N, H);
   const bool small_tail = (int64_t)F * H < kTailMaxSegments && hist_bound <= kTailMaxTiles;
   // One launch for all: its workgroups scan all counts each, so it is for few counts times workgroups; of 16 waves where a
-  // chunk has batches of 64 tokens for so many and the workgroups are few.
+  // chunk has batches of 64 tokens for so many and the workgroups are few: from 1024 tokens on, or from 512 with more than
+  // four picks a token, whose batches are longer, and few workgroups.  4 waves / 16 waves in us, 16 chunks of one head: 512
+  // tokens, 3 picks: 5.1 / 5.8, 12 picks: 12.0 / 11.1; 1024 tokens, 3 picks: 8.3 / 6.6; 512 tokens, 12 picks, 64 workgroups:
+  // 13.2 / 12.9, 128 workgroups: 12.7 / 14.0.
   const int64_t counts = (int64_t)P * H, groups = (int64_t)N * H;
-  const bool many_waves = S / N >= 1024 && groups <= 512;
+  const bool many_waves = groups <= 512 && (S / N >= 1024 || (S / N >= 512 && K > 4 && groups <= 64));
   if (small_tail && counts <= kFusedMaxCounts && cmax <= kFusedMaxCand && groups * counts <= kFusedMaxWork && K <= 16 &&
       (!tile_off_b || hist_bound_b <= kTailMaxTiles)) {
     if (!counted)

@@ -23,6 +23,19 @@ def test_lists_in_one_launch(batch, seqlen, heads, B, topk, counted, dense):
     check_lists(batch, seqlen, heads, B, topk, counted, dense)
 
 
+@pytest.mark.parametrize("counted", [False, True])
+@pytest.mark.parametrize("batch,seqlen,heads,B,topk", [
+    (1, 16 * 512, 4, 512, 13),   # 64 workgroups of 16 waves for chunks of 512 and more than 4 picks
+    (1, 16 * 512, 5, 512, 13),   # ... one more head: 4 waves
+    (1, 45 * 64, 1, 64, 3),      # 990 counts: one step of 4 waves
+    (1, 46 * 64, 1, 64, 3),      # 1035: two
+    (1, 91 * 1024, 1, 1024, 3),  # 4095 counts: one step of 16 waves
+    (1, 92 * 1024, 1, 1024, 3),  # 4186: two
+])
+def test_steps_of_the_scan(batch, seqlen, heads, B, topk, counted):
+    check_lists(batch, seqlen, heads, B, topk, counted, False)
+
+
 @pytest.mark.parametrize("seqlen,heads,group,B,topk", [
     (1500, 6, 3, 100, 4),        # one launch
     (5000, 4, 4, 1024, 3),       # ... of 16 waves
