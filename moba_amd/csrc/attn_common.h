@@ -16,6 +16,18 @@ constexpr int kXcdBlock = 64;  // consecutive logical tiles that share an XCD (o
 // span about two of its 64 slots' worth; with runs of 256 they still mostly belong to one K/V chunk.
 constexpr int kQueueRun = 256;
 
+// Division by a number d >= 2 as a multiplication: with s = 31 + ceil(log2 d) and m = floor(2^s / d) + 1 the error
+// m*d - 2^s is at most d <= 2^(s-31), so n*m >> s is the exact quotient for 0 <= n < 2^31; m < 2^32, s >= 32.
+struct Divisor {
+  uint32_t magic, shift;  // shift: s - 32
+};
+inline Divisor divisor(uint64_t d) {
+  uint32_t lg = 1;
+  while ((1ull << lg) < d) ++lg;
+  return {(uint32_t)((1ull << (31 + lg)) / d + 1), lg - 1};
+}
+__device__ __forceinline__ int quotient(int n, Divisor d) { return (int)(__umulhi((uint32_t)n, d.magic) >> d.shift); }
+
 // Index tables that define the tiles of one call.
 struct TileTables {
   const int* seg_off;           // [F*H+1] list start of segment (f, h)
@@ -34,6 +46,7 @@ struct TileTables {
   const int* chunk_direct;
   int S, H, K1, F, N, B;
   int seg_heads, seg_groups;
+  Divisor by_hk1, by_k1;        // H*K1 and K1, for the entries of the lists (which exist only with K1 >= 2)
   int Hkv, rep;                 // key/value heads and query heads per key/value head (H = Hkv * rep)
   int hist_bound;               // logical tile ids below it are history tiles
   int self_total;               // self_tile_prefix[N] * H
@@ -80,6 +93,7 @@ inline bool set_layout(TileTables& t, const int64_t* strides) {
   t.key_split_log2 = 0; t.part_stride = 0; t.xcd_block_log2 = 6; t.self_first = 0;
   t.self_skip = 0; t.q_shift = 0;
   t.seg_heads = 1; t.seg_groups = t.H;
+  t.by_hk1 = divisor((uint64_t)t.H * t.K1); t.by_k1 = divisor(t.K1);
   if (!strides) {
     t.q_tok_b = (int64_t)t.H * kHeadDim * 2; t.q_head_b = kHeadDim * 2;
     t.kv_tok_b = (int64_t)t.Hkv * kHeadDim * 2; t.kv_head_b = kHeadDim * 2;
@@ -247,8 +261,13 @@ __device__ __forceinline__ void decode_tile_rows(const TileTables& p, int wave, 
   const int H = p.H;
   if (t.base >= 0) {
     t.dest = entry;
-    t.tok = t.dest / (H * p.K1);
-    t.rh = kGrouped ? (entry - t.tok * (H * p.K1)) / p.K1 : t.h;
+    // (Multiplications where the head is asked for too: two divisions, one behind the other before the row can be fetched,
+    // cost calls of short lists and single heads more than tables of several heads saved them.  Forward of six
+    // sequences, 3112 tokens in all, 16 heads on 2, chunk 512: 57.0 -> 55.8 us; of 8191 tokens, 8 heads, chunk 512: 114.5 ->
+    // 113.3; with backward, 20480 tokens in five sequences, 8 heads on 2, chunk 512: 610 -> 606.  The kernel of tall tiles was no shorter for it:
+    // 65536 tokens, 32 heads on 8, chunk 4096: 12.34 ms dividing, 12.39 multiplying)
+    t.tok = kGrouped ? quotient(entry, p.by_hk1) : entry / (H * p.K1);
+    t.rh = kGrouped ? quotient(entry - t.tok * (H * p.K1), p.by_k1) : t.h;
     t.limit = t.nkeys - 1;
     t.wave_min_limit = t.limit;
     t.wave_max_limit = t.limit;

@@ -60,8 +60,6 @@ struct BwdParams {
   TileTables t;
   float scale_log2;
   float scale;
-  uint32_t hk_magic;  // n / (H*K1) == (n * hk_magic) >> hk_shift for every n < 2^31 (H*K1 >= 2)
-  uint32_t hk_shift;
   int* queues;        // [16] tile counters, one per XCD, of the dQ kernel and of the dK/dV kernel; zero at the start
   // Problems of few key tiles: the stages of all key tiles of a key/value head, one tile's behind the other's, are cut into equal
   // shares (bwd_dkv_tiles).  share_tiles [Hkv * kv_tiles + 1]: the tiles, head by head, worked out by bwd_delta_kernel; part_dkv:
@@ -71,7 +69,7 @@ struct BwdParams {
   struct ShareTile* share_tiles;
   int kv_tiles;    // of a head
   int dkv_shares;  // the most there are of a head; 0: whole tiles, drawn from the queues
-  uint32_t k1_magic, k1_shift, h_magic, h_shift;  // as hk_magic, for divisions by K1 and by H
+  Divisor by_h;    // H (not used with one head)
   // 3: eight queues, one per XCD (tiles that share rows or keys run behind one L2); 0: one queue for all, for a
   // problem of few tiles per workgroup, whose ids come longest tile first: whoever is free takes the longest left
   int queues_log2;
@@ -754,11 +752,11 @@ __device__ __forceinline__ void bwd_dkv_tiles(const BwdParams<E>& p) {
         const int pos0 = self_stage(qi, head);
         toks[4] = (c0 + key0 + min(pos0 + lane, self_rows - 1)) * H + head;
       } else {
-        toks[4] = (int)(__umulhi((uint32_t)raw, p.k1_magic) >> (p.k1_shift - 32));
+        toks[4] = quotient(raw, p.t.by_k1);
       }
     } else {
       toks[4] = qi < nself ? c0 + key0 + min(qi * TQ + lane, self_rows - 1)
-                           : (int)(__umulhi((uint32_t)raw, p.hk_magic) >> (p.hk_shift - 32));
+                           : quotient(raw, p.t.by_hk1);
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) toks[i] = __builtin_amdgcn_ds_bpermute(row_src_lane4 + 64 * i, toks[4]);
@@ -778,7 +776,7 @@ __device__ __forceinline__ void bwd_dkv_tiles(const BwdParams<E>& p) {
       if ((g & 1) == 0) {
         uint64_t src = q_lane_base;
         if constexpr (kBatched) {
-          const int tok = H == 1 ? toks[i] : (int)(__umulhi((uint32_t)toks[i], p.h_magic) >> (p.h_shift - 32));
+          const int tok = H == 1 ? toks[i] : quotient(toks[i], p.by_h);
           src += (uint64_t)(q_tok_bytes(p.t, tok) + (int64_t)(toks[i] - tok * H) * p.t.q_head_b);
         } else {
           src += (uint64_t)(uint32_t)toks[i] * (kHeadDim * 2);
@@ -1135,17 +1133,7 @@ static int launch_bwd(const void* dout, const void* q, const void* k, const void
   p.scale = softmax_scale > 0.f ? softmax_scale : (float)(1.0 / sqrt((double)D));
   p.scale_log2 = softmax_scale > 0.f ? (float)(1.4426950408889634 * (double)softmax_scale)
                                      : (float)(1.4426950408889634 / sqrt((double)D));
-  // division by H*K1 as a multiplication: with s = 31 + ceil(log2 d) and m = floor(2^s / d) + 1 the
-  // error m*d - 2^s is at most d <= 2^(s-31), so n*m >> s is the exact quotient for n < 2^31; m < 2^32
-  auto magic = [](uint64_t d, uint32_t& m, uint32_t& shift) {
-    uint32_t lg = 1;  // (at least 1: the kernels take the product's high word and shift by shift - 32; for d >= 2)
-    while ((1ull << lg) < d) ++lg;
-    shift = 31 + lg;
-    m = (uint32_t)((1ull << shift) / d + 1);
-  };
-  magic((uint64_t)H * (K + 1), p.hk_magic, p.hk_shift);  // (a list entry exists only with K >= 1, hence H*K1 >= 2)
-  magic((uint64_t)K + 1, p.k1_magic, p.k1_shift);
-  magic((uint64_t)H, p.h_magic, p.h_shift);              // (not used with one head)
+  p.by_h = divisor(H);
 
   static bool allowed_dq[kMaxDevices], allowed_dkv[4][kMaxDevices];  // one set per element type
   typedef void (*DkvKernel)(const BwdParams<E>);
