@@ -310,13 +310,10 @@ class _Geometry:
         self.self_tiles = plan.fwd_self_tiles if tall else plan.self_tiles
         self.self_names = (("fwd_" if tall else "") + "self_tile_prefix", ("fwd_" if tall else "") + "self_tile_chunk")
         self.tptr = {name: t.data_ptr() for name, t in plan.tables.items()}
-        # Heads whose lists are cut into tiles together: those of a key/value head, whose lists lie one behind the other and
-        # attend the same keys, so that only the last of their tiles is part empty.  Worth the more, the fewer tiles a list
-        # has (32 heads over 8, 3 x 2001 tokens, chunk 256: 155 -> 152 us; 8191 tokens, chunk 512: 217 -> 213 us; a training
-        # step of 17301 packed tokens, 8 heads over 2: 644 -> 631 us) and never a loss; not for the forward's tall tiles,
-        # which long chunks have and whose kernel has no registers left.
-        self.list_heads = 1 if tall else H // Hkv
-        self.bwd_list_heads = H // Hkv
+        # Heads whose lists are cut into tiles together (shares_lists); not for the forward's tall tiles, whose kernel has no
+        # registers left.
+        self.bwd_list_heads = H // Hkv if shares_lists(plan, H // Hkv) else 1
+        self.list_heads = 1 if tall else self.bwd_list_heads
         self.bound = plan.hist_tile_bound(H, self.rows_per_tile, self.list_heads)
         if plan.fallback:
             self.split = 1
@@ -372,6 +369,21 @@ def forward_tile_rows(plan: MobaPlan, H: int, D: int = HEAD_DIM) -> int:
         return TILE_ROWS    # (the only form for such heads)
     short_chunks = not plan.fallback and plan.chunk_size <= SHORT_TILES_CHUNK
     return TILE_ROWS if short_chunks or plan.flops_per_head * HEAD_DIM * H <= SHORT_TILES_FLOPS else FWD_TILE_ROWS
+
+
+# The lists of a key/value head's heads lie one behind the other and attend the same keys.  Cut into tiles together, only the
+# last of their tiles is part empty: worth the more, the fewer tiles a list has, and no more than the tiles' luck in
+# meeting the compute units where each has dozens.  Single heads / together in us, forward: 32 heads on 8, 2 x 3040
+# tokens, chunk 256: 188 / 180; 32 on 4, 6676, chunk 512: 394 / 378; 8 on 4, 13927, chunk 1024: 199.4 / 198.7; 8 on one, 2 x
+# 4242, chunk 2048: 135.5 / 129.6; 8 on 4, 20396, chunk 2048: 322 / 318.  Chunk 4096: 8 on 4, 2 x 8519: 369 / 378; 16 on 8,
+# 6917: 263.0 / 266.5; 8 on one, 2 x 17259: 1203 / 1206; 32 on 4, 11735: 1198 / 1196.  With backward, 2 on one, 32768, chunk 4096:
+# 1645 / 1636; 8 on 2, 142548 in three sequences, chunk 2048: 12754 / 12705; 8 on 2, 20480 in five, chunk 512: 631 together, 644 before.
+SHARED_LISTS_CHUNK = 4096
+
+
+def shares_lists(plan: MobaPlan, rep: int) -> bool:
+    """Whether the lists of the `rep` heads of a key/value head are cut into tiles together."""
+    return rep > 1 and plan.chunk_size < SHARED_LISTS_CHUNK
 
 
 def _geometry(plan: MobaPlan, lib, H: int, D: int, esize: int, Hkv: int = 0) -> _Geometry:

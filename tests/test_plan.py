@@ -219,3 +219,12 @@ def test_c_planner_rejects_bad_input():
         assert lib.moba_plan(arr, len(cu) - 1, 4, 3, 0, ctypes.byref(ps)) == -1
     arr = (ctypes.c_int32 * 2)(0, 8)
     assert lib.moba_plan(arr, 1, 0, 3, 0, ctypes.byref(ps)) == -1 and lib.moba_plan(arr, 1, 4, 0, 1, ctypes.byref(ps)) == -1
+
+
+def test_lists_of_several_heads_where_that_spares_tiles():
+    """Heads of a key/value head are cut into tiles together where their lists are of few tiles."""
+    from moba_amd import moba_efficient as E
+    from moba_amd.plan import make_plan
+    shares = lambda B, rep: E.shares_lists(make_plan([0, 8519, 17038], B, 3), rep)
+    assert shares(256, 4) and shares(2048, 8) and shares(4095, 2)
+    assert not shares(4096, 2) and not shares(8192, 8) and not shares(256, 1)
