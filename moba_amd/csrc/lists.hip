@@ -380,8 +380,8 @@ __global__ __launch_bounds__(1024) void lists_tail_kernel(const int* __restrict_
 // apart, and a chunk of 512 tokens is half a batch for each.  Measured: 8191 tokens, 32 heads, chunk 512 (16 waves each
 // and one of them for all tables before): 19.0 -> 15.9 us; 3 x 2001 tokens, 32 heads, chunk 256 (scan, fill and tables as
 // three launches before): 17.3 -> 10.4 us; 20480 tokens, 8 heads, chunk 512: 11.8 -> 9.0; 4096 tokens, 4 heads, chunk
-// 512: 6.4 -> 5.6.  The form of 16 waves is as fast as its forerunner, within 0.3 us, but for 256 workgroups of 1024
-// tokens, where the tables' workgroups are a second round: 9.4 -> 10.4 us.
+// 512: 6.4 -> 5.6.  The form of 16 waves is as fast as its forerunner, within 0.3 us, but for 256 workgroups and about 4000
+// counts (32 chunks of 1024 tokens, 8 heads): 9.4 -> 10.5 us.
 constexpr int kFusedMaxCounts = 8192, kFusedMaxCand = 128;
 constexpr int64_t kFusedMaxWork = 1 << 22;
 template <int KC, int NW>
@@ -572,12 +572,16 @@ extern "C" int moba_build_lists_grouped(const int32_t* sel, const int32_t* chunk
   dim3 grid(N, H);
   const bool small_tail = (int64_t)F * H < kTailMaxSegments && hist_bound <= kTailMaxTiles;
   // One launch for all: its workgroups scan all counts each, so it is for few counts times workgroups; of 16 waves where a
-  // chunk has batches of 64 tokens for so many and the workgroups are few: from 1024 tokens on, or from 512 with more than
-  // four picks a token, whose batches are longer, and few workgroups.  4 waves / 16 waves in us, 16 chunks of one head: 512
-  // tokens, 3 picks: 5.1 / 5.8, 12 picks: 12.0 / 11.1; 1024 tokens, 3 picks: 8.3 / 6.6; 512 tokens, 12 picks, 64 workgroups:
-  // 13.2 / 12.9, 128 workgroups: 12.7 / 14.0.
-  const int64_t counts = (int64_t)P * H, groups = (int64_t)N * H;
-  const bool many_waves = groups <= 512 && (S / N >= 1024 || (S / N >= 512 && K > 4 && groups <= 64));
+  // chunk's batches of 64 tokens are many for four, the workgroups few.  A chunk's length is not known here but between
+  // S / N and S / F, as only the last chunk of a sequence is shorter: with that one half as long it is 2 S / (N + F).
+  // (The line by S / N >= 1024 missed most sequences that end within a chunk of 1024.)  4 waves / 16 waves in us, up to 64
+  // workgroups: 1 to 4 picks: chunk 512: 5.7 / 6.3; 768: 7.1 / 6.9; 1024: 8.6 / 7.5; 7 and 11 picks: 320: 10.5 / 9.9;
+  // 512: 10.5 / 10.5; 640: 15.0 / 11.4.  256 workgroups: 1 to 4 picks: 768:
+  // 9.7 / 10.2; 896: 11.6 / 11.0; 7 and 11 picks: 512: 16.7 / 18.0; 640: 22.4 / 20.4.  512 workgroups, 2 picks: 1024:
+  // 15.7 / 17.9; 2048: 27.2 / 26.0.
+  const int64_t counts = (int64_t)P * H, groups = (int64_t)N * H, rows = 2 * S / ((int64_t)N + F);
+  const bool many_waves = rows >= (K > 4 ? 576 : 704) ? groups <= (rows >= 1024 ? 512 : 256)
+                                                      : K > 4 && rows >= 288 && groups <= 64;
   if (small_tail && counts <= kFusedMaxCounts && cmax <= kFusedMaxCand && groups * counts <= kFusedMaxWork && K <= 16 &&
       (!tile_off_b || hist_bound_b <= kTailMaxTiles)) {
     if (!counted)

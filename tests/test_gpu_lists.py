@@ -25,8 +25,12 @@ def test_lists_in_one_launch(batch, seqlen, heads, B, topk, counted, dense):
 
 @pytest.mark.parametrize("counted", [False, True])
 @pytest.mark.parametrize("batch,seqlen,heads,B,topk", [
-    (1, 16 * 512, 4, 512, 13),   # 64 workgroups of 16 waves for chunks of 512 and more than 4 picks
+    (1, 16 * 512, 4, 512, 13),   # 64 workgroups of 16 waves for chunks of 512 and 12 picks
     (1, 16 * 512, 5, 512, 13),   # ... one more head: 4 waves
+    (1, 4500, 3, 1024, 3),       # chunks of 1024, the last one short: 16 waves
+    (1, 6 * 704, 2, 704, 9),     # ... of a length between
+    (3, 3000, 3, 300, 6),        # 300 and 5 picks: 16 waves
+    (1, 16 * 512, 8, 512, 4),    # 512 and few picks: 4 waves
     (1, 45 * 64, 1, 64, 3),      # 990 counts: one step of 4 waves
     (1, 46 * 64, 1, 64, 3),      # 1035: two
     (1, 91 * 1024, 1, 1024, 3),  # 4095 counts: one step of 16 waves
