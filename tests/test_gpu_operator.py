@@ -339,6 +339,7 @@ def test_history_tiles_of_dq_cut_into_parts():
     of the oracle for each.  Three sequences with partial last chunks, grouped-query heads."""
     from moba_amd import _lib, moba_attn_varlen_gqa
     from moba_amd import moba_efficient as E
+    from moba_amd import plan as P
     from moba_amd.plan import make_plan
     heads, kv_heads, B, topk = 2, 1, 1024, 3
     q, _, _, do, cu, mx = make_case(3, 16384, heads, seed=23)
@@ -428,6 +429,7 @@ def test_key_tiles_cut_into_parts():
     different summation order, and both lie within the tolerance of the oracle."""
     from moba_amd import _lib, moba_attn_varlen_gqa
     from moba_amd import moba_efficient as E
+    from moba_amd import plan as P
     from moba_amd.plan import make_plan
     heads, kv_heads, B, topk = 2, 1, 1024, 3
     q, _, _, do, cu, mx = make_case(3, 16384, heads, seed=21)
@@ -440,6 +442,8 @@ def test_key_tiles_cut_into_parts():
         pytest.skip("the key tiles are not cut with MOBA_RESIDENT_CUS set")
 
     def run():
+        P._BY_VALUE.clear()   # (a plan keeps the sizes of its scratch: without a new one the same form would run again)
+        P._BY_TENSOR.clear()
         qg, kg, vg = (x.cuda().requires_grad_(True) for x in (q, k, v))
         out = moba_attn_varlen_gqa(qg, kg, vg, cu_t, mx, B, topk)
         out.backward(do.cuda())
@@ -448,13 +452,15 @@ def test_key_tiles_cut_into_parts():
     cut, again = run(), run()
     for a, b in zip(cut, again):
         assert torch.equal(a, b)
-    real = lib.moba_bwd_dkv_scratch_bytes
+    real, asked = lib.moba_bwd_dkv_scratch_bytes, []
     try:
-        lib.moba_bwd_dkv_scratch_bytes = lambda *a: 0   # no scratch: every key tile in one piece
+        lib.moba_bwd_dkv_scratch_bytes = lambda *a: asked.append(real(*a)) or 0   # no scratch: every key tile in one piece
         whole = run()
     finally:
         lib.moba_bwd_dkv_scratch_bytes = real
+    assert len(asked) == 1 and asked[0] > 0
     assert torch.equal(cut[0], whole[0]) and torch.equal(cut[1], whole[1])
+    assert not torch.equal(cut[2], whole[2])      # (sums in another order: the two forms did run)
     for name, a, b in (("dk", cut[2], whole[2]), ("dv", cut[3], whole[3])):
         e = (a.float() - b.float()).abs()
         assert e.max() <= 2.0 ** -7 * b.float().abs().max() and (e > 0).float().mean() < 0.05, (name, e.max().item())
