@@ -197,7 +197,8 @@ int moba_build_lists(const int32_t* sel, const int32_t* chunk_tok, const int32_t
 
 /* The same with tile tables that cut the lists of list_heads heads (1, or all those of a key/value head, whose lists lie one
  * behind the other) into tiles together: tile_off [F*H/list_heads+1], tile_seg names segment f*H/list_heads + h/list_heads,
- * hist_bound e.g. M / tile_rows + F * H / list_heads; list_heads_b for the second pair. */
+ * hist_bound e.g. M / tile_rows + F * H / list_heads; list_heads_b for the second pair.  (Worth it where lists have few
+ * tiles each: chunks below 4096 tokens.) */
 int moba_build_lists_grouped(const int32_t* sel, const int32_t* chunk_tok, const int32_t* chunk_fb, const int32_t* chunk_local,
                              const int32_t* pair_off, int32_t* cnt, int32_t* seg_off, int32_t* tile_off, int32_t* seg_dest,
                              int32_t* tile_seg, int64_t S, int H, int K, int N, int F, int P, int cmax, int tile_rows,
@@ -274,9 +275,9 @@ int moba_fwd_partials(const void* q, const void* k, const void* v, void* part_o,
  * and may be NULL; redo, if given, has redo[0] zeroed by the caller and receives the tiles that were computed again with a running
  * maximum, for information: redo[0] counts every part of a tile cut by key_split, and parts beyond the array's
  * hist_bound + self_tiles * H entries are counted without an entry.  Those tiles take the fixed reference without a
- * list too (list_heads: of the tile tables, see moba_build_lists_grouped; 1 for tiles of moba_fwd_tile_rows() rows);
- * running_max != 0 asks for the running maximum from the start (and for redo to be left alone), whatever the
- * tiles. */
+ * list too; running_max != 0 asks for the running maximum from the start (and for redo to be left alone), whatever the
+ * tiles.  list_heads is that of tile_off and tile_seg (moba_build_lists_grouped): 1 or H / Hkv, and 1 for tiles of
+ * moba_fwd_tile_rows() rows. */
 int moba_fwd_partials_rows(const void* q, const void* k, const void* v, void* part_o, float* part_lse,
                            const int32_t* seg_off, const int32_t* tile_off, const int32_t* seg_dest,
                            const int32_t* fchunk_tok, const int32_t* chunk_tok, const int32_t* self_tile_prefix,

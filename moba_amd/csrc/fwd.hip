@@ -147,11 +147,12 @@ __global__ __launch_bounds__(512, 2) void moba_fwd_kernel(const FwdParams<E> p) 
       if (key0 + key >= nkeys) *reinterpret_cast<u32x4*>(vdst + slab * 1024 + ln * 16) = u32x4{0, 0, 0, 0};
     }
   };
-  // Tiles that run side by side on an XCD work on the same chunk; starting each at a
-  // different key tile spreads their first touches of the chunk over all of it.
-  // (every tile goes through its keys from the first on.  History tiles that start at different keys, so that neighbours do
-  // not ask for the same lines at once, were slower: 131072 tokens, 32 heads, chunk 4096: 71.4 against
-  // 70.9 ms; 8 sequences of 302060 tokens together, chunk 2048: 25.9 against 25.7 ms)
+  // (Every tile goes through its keys from the first on.  History tiles that start at different keys, so that neighbours do
+  // not ask for the same lines at once, were up to 0.8 % slower, twelve runs of each on two boxes: 65536 tokens, 32 heads,
+  // chunk 4096: 12.36 against 12.28 ms; 131072 tokens, chunk 2048: 22.9 against 22.75; 8 sequences of 302060 tokens
+  // together, chunk 2048: 25.85 against 25.7; 131072 tokens, chunk 4096: 71.4 against 71.3, within what runs differ; chunk
+  // 1024: equal.  What is saved are the modulo per tile and the compare and select per key tile: of HBM traffic the fixed
+  // order makes more, 124 against 98 GB in that forward of 131072 tokens, with 66 against 72 % of reads found in L2)
   int nkt = 1;
 
   // ---- fragment addressing: per-lane LDS byte addresses inside a tile (numbers, not pointers into smem:

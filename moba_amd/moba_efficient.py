@@ -410,7 +410,8 @@ def _run_forward(q, k, v, plan: MobaPlan, timer: Optional[StageTimer] = None, sc
     """q, k, v: [tokens, heads, 128], or batched [batch, heads, tokens, 128] (read in place, see _dims), already
     addressable (_in_place).  Returns (out, lse, sel, seg_off, tile_off, seg_dest, tile_seg), or (out, lse) without
     lists_too.
-    bwd_tables: a list that receives the backward kernels' (tile_off, tile_seg), made on the way.
+    bwd_tables: a list that receives the backward kernels' tile_off and tile_seg, made on the way, and the heads that these cut
+    together.
     The stages are those of chunk_mean(), gate_topk(), build_lists() above, called on precomputed sizes and
     addresses, in two allocations of scratch (what a backward reads again, and what it does not) and one of each result, and
     with addresses as plain numbers: at small shapes a forward is bound by the host's time per call (4096 tokens, 4
