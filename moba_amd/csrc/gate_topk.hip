@@ -10,7 +10,8 @@
 // chunks 0..d of every sequence (which would pick every earlier chunk) get no picks
 // at all: the attention kernels serve them through one causal pass over the prefix.
 //
-// One wave handles 64 consecutive tokens of one head: the score tile (32 chunks x 64 tokens) is two 32x32x16 MFMA
+// One wave handles 64 consecutive tokens of one head (a workgroup four heads of them, or 256 tokens of one head: the rule stands
+// at the launch): the score tile (32 chunks x 64 tokens) is two 32x32x16 MFMA
 // accumulators.  Sixteen lane-half swaps leave the 32 scores of token `lane` in lane `lane`; a lane marks those that
 // beat the worst entry of its list (three instructions each, no LDS) and inserts them one per pass, lowest id first, in
 // a top-k held in registers.  Scores never reach HBM (except through the optional debug output).
@@ -18,7 +19,9 @@
 // Bound: Q is read once (HBM) for few candidates; with many the vector instructions per candidate decide.  Measured at
 // 196608 tokens, 32 heads on 8, up to 767 candidates, 2 picks: 2.20 ms with the tile transposed through LDS and a
 // barrier on either side of it, 1.39 ms here; 302060 tokens, up to 147 candidates: 1.12 -> 0.91 ms; 65536 tokens, 16
-// heads, up to 511 candidates, 11 picks: 422 -> 333 us.
+// heads, up to 511 candidates, 11 picks: 422 -> 333 us.  Calls of a few microseconds are a chain of round trips to memory:
+// where the counters of the candidates lie is looked up beside Q, and the first block stops at the last candidate (4096
+// tokens, 4 heads: 9.3 -> 8.6 us; 3 x 2001, 32 heads: 15.7 -> 14.5).
 #include "common.h"
 
 namespace moba {
@@ -66,15 +69,17 @@ __global__ __launch_bounds__(256, KMAX <= 4 ? 3 : (KMAX <= 16 ? 2 : 1)) void gat
     const typename E::elem* __restrict__ q, const typename E::elem* __restrict__ kbar, const int* __restrict__ cu_seqlens,
     const int* __restrict__ seq_fbase, int* __restrict__ sel, float* __restrict__ scores_out,
     int S, int H, int Hkv, int nseq, int F, int B, int K, int64_t q_tok_stride, int64_t q_head_stride,
-    int batch_rows, int64_t q_batch_stride, const int* __restrict__ pair_off, int* __restrict__ cnt, int dense_local) {
+    int batch_rows, int64_t q_batch_stride, const int* __restrict__ pair_off, int* __restrict__ cnt, int dense_local,
+    int one_head) {
   MOBA_ELEM_TYPES(E)
   // a lane's 32 scores, for the passes that take one of them by its number (rows 136 bytes apart: 8-byte writes, and reads of
   // one number by all lanes, spread over the banks); later the staged lists and the histograms
   __shared__ __attribute__((aligned(16))) float sc[4][64][34];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int n = lane & 31, hh = lane >> 5;
-  const int tok0 = blockIdx.x * 64;
-  const int h = blockIdx.y * 4 + wave;
+  const int tile = one_head ? blockIdx.x / H : blockIdx.x;  // (one_head: the heads of the same tokens side by side)
+  const int tok0 = one_head ? tile * 256 + wave * 64 : tile * 64;
+  const int h = one_head ? blockIdx.x - tile * H : blockIdx.y * 4 + wave;
   const bool head_ok = h < H;
   const int hc = head_ok ? h : H - 1;
 
@@ -99,8 +104,14 @@ __global__ __launch_bounds__(256, KMAX <= 4 ? 3 : (KMAX <= 16 ? 2 : 1)) void gat
 
   TopK<KMAX> top;
   top.init();
+  // where the counts of this lane's chunk start (the first 64 of the wave's candidates; looked up ahead, for the end)
+  int2 my_pairs = make_int2(0, 0);
+  if (cnt && fhi > 0) {
+    const int f = min(flo + lane, F - 1);
+    my_pairs = make_int2(pair_off[f], pair_off[f + 1]);
+  }
 
-  if (fhi > 0) {  // wave-uniform (and block-uniform)
+  if (fhi > 0) {  // wave-uniform
     // Q^T operand: lane (n, hh) holds q[token n (+32)][16*ks + 8*hh .. +7]
     elem8 bq[2][D / 16];
 #pragma unroll
@@ -161,6 +172,7 @@ __global__ __launch_bounds__(256, KMAX <= 4 ? 3 : (KMAX <= 16 ? 2 : 1)) void gat
         if constexpr (KMAX <= 16) {
 #pragma unroll
           for (int j = 0; j < 32; ++j) {
+            if ((j & 7) == 0 && f0 + j >= fhi) break;  // (wave-uniform)
             const float x = score(j);
             if (j >= lo && j < hi) top.push(x, f0 + j);
           }
@@ -198,14 +210,22 @@ __global__ __launch_bounds__(256, KMAX <= 4 ? 3 : (KMAX <= 16 ? 2 : 1)) void gat
   if (4 * 64 * K <= (int)(sizeof(sc) / sizeof(int))) {  // (uniform; K <= 34)
 #pragma unroll
     for (int j = 0; j < KMAX; ++j)
-      if (j < K) stage[(lane * 4 + wave) * K + j] = top.idx[j];
+      if (j < K) stage[(one_head ? wave * 64 + lane : lane * 4 + wave) * K + j] = top.idx[j];
     __syncthreads();
-    const int run = 4 * K;                       // ints per token in this workgroup's four heads
-    const int heads_here = min(4, H - blockIdx.y * 4);
-    for (int i = threadIdx.x; i < 64 * run; i += 256) {
-      const int tk = i / run, w = i - tk * run;  // token of the tile, int within its run
-      if (tok0 + tk < S && w < heads_here * K)
-        sel[((int64_t)(tok0 + tk) * H + blockIdx.y * 4) * K + w] = stage[i];
+    if (one_head) {
+      const int first = tile * 256;
+      for (int i = threadIdx.x; i < 256 * K; i += 256) {
+        const int tk = i / K;  // [256 tokens][K]
+        if (first + tk < S) sel[((int64_t)(first + tk) * H + h) * K + i - tk * K] = stage[i];
+      }
+    } else {
+      const int run = 4 * K;                       // ints per token in this workgroup's four heads
+      const int heads_here = min(4, H - blockIdx.y * 4);
+      for (int i = threadIdx.x; i < 64 * run; i += 256) {
+        const int tk = i / run, w = i - tk * run;  // token of the tile, int within its run
+        if (tok0 + tk < S && w < heads_here * K)
+          sel[((int64_t)(tok0 + tk) * H + blockIdx.y * 4) * K + w] = stage[i];
+      }
     }
   } else if (s < S && head_ok) {
     int* dst = sel + ((int64_t)s * H + h) * K;
@@ -217,11 +237,48 @@ __global__ __launch_bounds__(256, KMAX <= 4 ? 3 : (KMAX <= 16 ? 2 : 1)) void gat
   // added into cnt[(chunk, head, query chunk)] (integer sums: the order of the additions does not matter).  A
   // wave's 64 tokens lie in one query chunk, or in a few: one pass per chunk, through a histogram in LDS.
   if (!cnt) return;
-  __syncthreads();  // (the staged lists are stored)
   constexpr int kHist = (int)(sizeof(sc) / sizeof(int)) / 4;
-  int* hist = reinterpret_cast<int*>(&sc[0][0][0]) + wave * kHist;
+  int* const hists = reinterpret_cast<int*>(&sc[0][0][0]);
   const bool counts = head_ok && s < S && c > 0;
   uint64_t todo = __ballot(counts);
+  int* hist = hists + wave * kHist;
+  auto add_up = [&](int* hist, int cfb, int w0, int wn) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < KMAX; ++j) {
+      const int i = (j < K && top.idx[j] >= 0) ? top.idx[j] - cfb - w0 : -1;
+      if ((unsigned)i < (unsigned)wn) atomicAdd(&hist[i], 1);
+    }
+  };
+  auto to_counts = [&](int n, int cc, int cfb, int at) __attribute__((always_inline)) {  // n picks of chunk cfb + at
+    const int f = cfb + at, l = f - flo;
+    int2 pr = my_pairs;
+    if (l != lane) pr = make_int2(pair_off[f], pair_off[f + 1]);
+    if (n) atomicAdd(&cnt[pr.x * H + h * (pr.y - pr.x) + (cc - at - 1)], n);
+  };
+  if (one_head) {
+    // the four waves' tokens, if they lie in one query chunk: one histogram, one addition for each count where the waves on
+    // their own make four (the additions of a call of few heads meet in a few cache lines)
+    __shared__ int4 of_wave[4];
+    const int leader = todo ? __ffsll((unsigned long long)todo) - 1 : 0;
+    const int cc = __shfl(c, leader, 64), cfb = __shfl(fb, leader, 64);
+    const bool same = __ballot(counts && c == cc && fb == cfb) == todo;
+    if (lane == 0) of_wave[wave] = make_int4(todo != 0, cc, cfb, same);
+    __syncthreads();  // (the staged lists are stored)
+    const int4 w0 = of_wave[0];
+    bool joint = w0.x != 0 && w0.y <= 64;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) joint = joint && (of_wave[w].x != 0 && of_wave[w].y == w0.y && of_wave[w].z == w0.z && of_wave[w].w != 0);
+    if (joint) {  // (block-uniform)
+      if (threadIdx.x < 64) hists[threadIdx.x] = 0;
+      __syncthreads();
+      if (counts) add_up(hists, cfb, 0, cc);
+      __syncthreads();
+      if ((int)threadIdx.x < cc) to_counts(hists[threadIdx.x], cc, cfb, threadIdx.x);
+      return;
+    }
+  } else {
+    __syncthreads();  // (the staged lists are stored)
+  }
   while (todo) {  // (wave-uniform)
     const int leader = __ffsll((unsigned long long)todo) - 1;
     const int cc = __shfl(c, leader, 64), cfb = __shfl(fb, leader, 64);
@@ -231,23 +288,10 @@ __global__ __launch_bounds__(256, KMAX <= 4 ? 3 : (KMAX <= 16 ? 2 : 1)) void gat
       for (int i = lane; i < wn; i += 64) hist[i] = 0;
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
-      if (mine) {
-#pragma unroll
-        for (int j = 0; j < KMAX; ++j) {
-          const int i = (j < K && top.idx[j] >= 0) ? top.idx[j] - cfb - w0 : -1;
-          if ((unsigned)i < (unsigned)wn) atomicAdd(&hist[i], 1);
-        }
-      }
+      if (mine) add_up(hist, cfb, w0, wn);
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
-      for (int i = lane; i < wn; i += 64) {
-        const int n = hist[i];
-        if (n) {
-          const int f = cfb + w0 + i;
-          const int q0 = pair_off[f], nq = pair_off[f + 1] - q0;
-          atomicAdd(&cnt[q0 * H + h * nq + (cc - (w0 + i) - 1)], n);
-        }
-      }
+      for (int i = lane; i < wn; i += 64) to_counts(hist[i], cc, cfb, w0 + i);
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
     }
@@ -305,12 +349,21 @@ extern "C" int moba_gate_topk(const void* q, const void* kbar, const int32_t* cu
   const int64_t qbs = strides ? strides[5] : 0;
   if (qts <= 0 || qhs <= 0 || (qts & 7) || (qhs & 7)) return MOBA_ERR_ARG;
   if (qbr < 0 || (qbr > 0 && (qbs <= 0 || (qbs & 7)))) return MOBA_ERR_ARG;
+  // What a workgroup's four waves are: heads of the same 64 tokens, whose picks leave as one run per token, or 256 tokens of a
+  // head, whose counts leave as one addition.  The additions of all workgroups meet in P * H counters, a few cache lines where
+  // there are few heads and chunks, and a short kernel waits for them; beyond that the longer runs count, and below four
+  // heads waves that have no head.  By heads / by tokens, us, with the counts: one head, 32768 tokens, chunk 2048: 14.9 / 8.5,
+  // 262144, chunk 512: 182 / 66; 2 heads, 131072, chunk 512: 68 / 44; 4 heads, 4096 tokens, chunk 512: 8.6 / 7.4, 32768, chunk
+  // 1024: 15.1 / 13.2, 131072, chunk 4096, 11 picks: 65 / 54, 524288: 330 / 335; 8 heads, 8192: 8.6 / 8.5; 32 heads, 2048, chunk
+  // 256: 8.0 / 7.8; 8 heads, 20480 in five sequences, chunk 512: 14.5 / 16.6; 32 heads, 3 x 2001, chunk 256: 14.5 / 16.1.
+  const int one_head = H < 4 || S * H <= (H == 4 ? 1 << 20 : 65536);
   dim3 grid((unsigned)((S + 63) / 64), (unsigned)((H + 3) / 4));
+  if (one_head) grid = dim3((unsigned)((S + 255) / 256 * H));
   hipStream_t st = (hipStream_t)stream;
 #define GATE(EL, KM, DIM)                                                                                             \
   hipLaunchKernelGGL((gate_topk_kernel<EL, KM, DIM>), grid, dim3(256), 0, st, (const EL::elem*)q, (const EL::elem*)kbar, \
                      cu_seqlens, seq_fbase, sel, scores_out, (int)S, H, Hkv, nseq, F, B, K, qts, qhs, qbr, qbs,       \
-                     pair_off, cnt, dense_local)
+                     pair_off, cnt, dense_local, one_head)
 #define CALL(KM)                                                       \
   if (dtype == MOBA_DTYPE_F16) {                                       \
     if (D == 64) GATE(F16, KM, 64); else GATE(F16, KM, 128);           \
