@@ -11,7 +11,7 @@
 //   bwd_dq_kernel        row-tile major, same tiling as the forward: each tile (128
 //                        query rows x the keys of one chunk) writes its partial dQ, scaled
 //                        and rounded to the element type, into the row's slot;
-//                        bwd_dq_reduce_kernel sums the K+1 slots in fp32
+//                        bwd_dq_sum_few_kernel or bwd_dq_reduce_kernel sums the K+1 slots in fp32
 //   bwd_dkv_kernel       key-tile major: a workgroup owns 128 keys of (chunk, head) and
 //                        walks first the causal rows of the same chunk, then the gather
 //                        list of rows that selected the chunk; dK/dV accumulate in
@@ -22,7 +22,7 @@
 // (the recomputation of S and dO V^T in both kernels adds 4*D on top).
 #include <type_traits>
 
-#include "attn_common.h"
+#include "slots.h"
 
 namespace moba {
 
@@ -245,7 +245,7 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(const BwdParams<E> p) {
   // With few tiles per workgroup (self_first) the self tiles take the first ids -- the longest of them are as
   // long as a history tile, and drawn last they would run alone at the end -- and the keys of a history tile
   // are cut into 1 << ks parts that are tiles of their own, each with slot rows of its own for its partial dQ
-  // (part g of a slot row lies g * part_stride rows behind part 0; bwd_dq_reduce_kernel adds them up).
+  // (part g of a slot row lies g * part_stride rows behind part 0; the sum over the slots adds them up).
   const int hist = p.t.self_first ? id - p.t.self_total : (id < hist_tiles ? id : -1);
   const int logical = hist >= 0 ? hist >> ks : p.t.hist_bound + (p.t.self_first ? id : id - hist_tiles);
   const int key_part = hist >= 0 ? hist & ((1 << ks) - 1) : 0;
@@ -493,25 +493,42 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(const BwdParams<E> p) {
   }  // tiles
 }
 
-// dq[row] = sum over the row's valid slots of part_dq (in fp32); 16 lanes per row.  With token ranges (mrg_start /
-// mrg_prefix, as in the forward's merge) only the rows of those tokens, `rows` counting them: the dQ kernel wrote
-// the others itself.
+// dq[row] = sum over the row's valid slots of part_dq (in fp32); 16 lanes per row.  With token ranges (SlotRows, as in the
+// forward's merge) only the rows of those tokens: the dQ kernel wrote the others itself.  For rows of few slots a form with
+// their number as a constant, as the merge has and for the same reason.  General / this, us: 20480 tokens, 8 heads, 3 slots:
+// 26.0 / 23.8; 32768, one head, 2 parts of 3: 11.1 / 10.1; 302060, 32 heads, 3: 1509 / 1381; 16384, 8 heads, 12: 44.4 / 42.5;
+// 32768, 16 heads, 9: 165 / 153.
+template <class E, int NV, bool kParts>
+__global__ __launch_bounds__(256) void bwd_dq_sum_few_kernel(const typename E::elem* __restrict__ part_dq,
+                                                             const int* __restrict__ sel, typename E::elem* __restrict__ dq,
+                                                             int K1, int part_rows, const SlotRows which) {
+  MOBA_ELEM_TYPES(E)
+  const int at = (int)blockIdx.x * 16 + (threadIdx.x >> 4), c8 = threadIdx.x & 15;
+  const int row = slot_row(which, min(at, which.rows - 1));
+  RowSlots<E, kHeadDim, NV, kParts> slots;
+  slots.request(part_dq, row, c8, K1, part_rows);
+  slots.take_picks(sel, row, K1);
+  float acc[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) acc[e] = 0.f;
+#pragma unroll
+  for (int u = 0; u < NV; ++u) slots.add(u, 1.f, acc);
+  if (at >= which.rows) return;
+  elem8 o;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) o[e] = (elem)acc[e];
+  *reinterpret_cast<elem8*>(dq + (int64_t)row * kHeadDim + c8 * 8) = o;
+}
+
 template <class E>
 __global__ __launch_bounds__(256) void bwd_dq_reduce_kernel(const typename E::elem* __restrict__ part_dq,
                                                             const int* __restrict__ sel,
-                                                            typename E::elem* __restrict__ dq, int64_t rows, int K1,
-                                                            int parts, int64_t all_rows,
-                                                            const int* __restrict__ mrg_start,
-                                                            const int* __restrict__ mrg_prefix, int nranges, int H) {
+                                                            typename E::elem* __restrict__ dq, int K1, int parts,
+                                                            int part_rows, const SlotRows which) {
   MOBA_ELEM_TYPES(E)
-  const int64_t row_raw = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
-  const bool row_ok = row_raw < rows;
-  int64_t row = row_ok ? row_raw : rows - 1;  // whole 16-lane groups stay active for the shuffles
-  if (mrg_start) {
-    const int t = (int)(row / H), h = (int)(row - (int64_t)t * H);
-    const int b = upper_row(mrg_prefix, nranges, t);
-    row = (int64_t)(mrg_start[b] + (t - mrg_prefix[b])) * H + h;
-  }
+  const int at_raw = (int)blockIdx.x * 16 + (threadIdx.x >> 4);
+  const bool row_ok = at_raw < which.rows;
+  const int64_t row = slot_row(which, row_ok ? at_raw : which.rows - 1);  // whole 16-lane groups stay active for the shuffles
   const int c8 = threadIdx.x & 15;
   const int K = K1 - 1;
   const int* ps = sel + row * K;
@@ -521,37 +538,9 @@ __global__ __launch_bounds__(256) void bwd_dq_reduce_kernel(const typename E::el
   const elem* src = part_dq + row * K1 * kHeadDim + c8 * 8;
   // lane c8 fetches the presence of slot j0 + c8; absent slots are redirected to slot 0 and
   // multiplied by 0, so the loads of eight slots are unconditional and in flight together.
-  // With parts, slot v of the parts * K1 is slot v % K1 of part v / K1, rows * K1 slot rows behind the part
+  // With parts, slot v of the parts * K1 is slot v % K1 of part v / K1, part_rows slot rows behind the part
   // before (an int: the buffer holds fewer than 2^31 slot rows); the self slot exists in part 0 only.
   const int nvirt = parts * K1;
-  const int part_rows = (int)(all_rows * K1);
-  if (nvirt <= 8) {  // (uniform)
-    // Few slots: all are requested at once, before the picks that say which are present have arrived -- one
-    // round trip instead of two.  (An absent slot's bytes are whatever the buffer holds: dropped by selection.)
-    elem8 a[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int part = parts == 1 ? 0 : u / K1, j = u - part * K1;
-      if (u < nvirt)
-        a[u] = __builtin_nontemporal_load(reinterpret_cast<const elem8*>(src + (int64_t)(part * part_rows + j) * kHeadDim));
-    }
-    const int part = parts == 1 ? 0 : c8 / K1, j = c8 - part * K1;
-    const bool ok = c8 < nvirt && (j == 0 ? part == 0 : ps[j - 1] >= 0);
-    const float present = ok ? 1.f : 0.f;
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      if (u >= nvirt) break;
-      const float w = __shfl(present, u, 16);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) acc[e] += w > 0.f ? (float)a[u][e] : 0.f;
-    }
-    if (!row_ok) return;
-    elem8 o;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) o[e] = (elem)acc[e];
-    *reinterpret_cast<elem8*>(dq + row * kHeadDim + c8 * 8) = o;
-    return;
-  }
   for (int j0 = 0; j0 < nvirt; j0 += 16) {
     const int v = j0 + c8;
     const int part = parts == 1 ? 0 : v / K1, j = v - part * K1;
@@ -1150,9 +1139,16 @@ static int launch_bwd(const void* dout, const void* q, const void* k, const void
   hipLaunchKernelGGL(bwd_dq_kernel<E>, dim3((unsigned)grid_q), dim3(256), kBwdDqLds, st, p);
   if (merge_tokens > 0) {  // (0: the dQ kernel wrote every row itself)
     const int64_t sum_rows = merge_tokens * H;
-    hipLaunchKernelGGL(bwd_dq_reduce_kernel<E>, dim3((unsigned)((sum_rows + 15) / 16)), dim3(256), 0, st,
-                       (const elem*)part_dq, sel, (elem*)dq, sum_rows, K + 1, 1 << t.key_split_log2, rows, mrg_start,
-                       mrg_prefix, nranges, H);
+    const SlotRows which = slot_rows(mrg_start, mrg_prefix, nranges, (int)H, sum_rows);
+    const dim3 grid((unsigned)((sum_rows + 15) / 16));
+    const int K1 = (int)K + 1, parts = 1 << t.key_split_log2, part_rows = (int)(rows * K1);
+    const bool few = for_slots(K1, parts, [&](auto nv, auto several) {
+      hipLaunchKernelGGL((bwd_dq_sum_few_kernel<E, decltype(nv)::value, decltype(several)::value>), grid, dim3(256), 0, st,
+                         (const elem*)part_dq, sel, (elem*)dq, K1, part_rows, which);
+    });
+    if (!few)
+      hipLaunchKernelGGL(bwd_dq_reduce_kernel<E>, grid, dim3(256), 0, st, (const elem*)part_dq, sel, (elem*)dq, K1, parts, part_rows,
+                         which);
   }
   hipLaunchKernelGGL(dkv_kernels[form], dim3((unsigned)grid_kv), dim3(256), kBwdDkvLds, st, p);
   if (dkv_shares)

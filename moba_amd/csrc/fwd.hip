@@ -20,6 +20,7 @@
 #include <cstddef>
 #include <type_traits>
 #include "fwd_common.h"
+#include "slots.h"
 
 namespace moba {
 
@@ -658,55 +659,57 @@ __global__ __launch_bounds__(512, 2) void moba_fwd_kernel(const FwdParams<E> p) 
 #undef MOBA_PIN
 }
 
-// The merge of a row with at most NV slots (parts included), by the row's 16 lanes: the slots' partials are
-// requested at once, before the statistics that say which are present have arrived -- one round trip instead of
-// two.  (An absent slot's bytes are whatever the buffer holds; they are dropped by selection, not multiplied by
-// a zero weight.)  Slots are accumulated in ascending order, as in the general form below.  For up to 8 slots:
-// with 16 in registers too few waves fit a compute unit, and the kernel takes three times as long.
-template <class E, int D, int NV>
-__device__ __forceinline__ void merge_few_slots(const typename E::elem* __restrict__ po, const float* __restrict__ pl,
-                                                const int* __restrict__ ps, typename E::elem* __restrict__ out,
-                                                float* __restrict__ lse, int64_t row, bool row_ok, int c8, int K1,
-                                                int parts, int nvirt, int part_rows) {
+// The merge for rows of NV <= kMostSlotsAtOnce slots (parts included), 16 lanes to a row.  Bound by its instructions unless they
+// are few: every lane reads its row's statistics and picks itself, nothing is divided or searched per lane and the slots'
+// number is a constant: some 200 instructions for a wave's four rows of three slots, where the general form below took 450.
+// General / this, us: 4096 tokens, 4 heads, 3 slots: 5.3 / 4.4; 3 x 2001, 32 heads: 22.9 / 18.9; 8191, 32 heads of 64, 4 slots:
+// 26.3 / 19.0; 20480, 8 heads: 30.9 / 23.6; 302060, 32 heads: 1643 / 1360 (the rate of a copy and a quarter more: 6.6 TB/s);
+// 32768, one head, 2 parts of 3 slots: 14.6 / 10.5; 8192, 4 heads, 10 slots: 17.9 / 14.6; 16384, 8 heads, 12: 46.0 / 41.4;
+// 131072, 32 heads, 12: 1589 / 1546.
+template <class E, int D, int NV, bool kParts>
+__global__ __launch_bounds__(256) void moba_merge_few_kernel(const typename E::elem* __restrict__ part_o,
+                                                             const float* __restrict__ part_lse, const int* __restrict__ sel,
+                                                             typename E::elem* __restrict__ out, float* __restrict__ lse,
+                                                             int K1, int part_rows, const SlotRows which) {
   MOBA_ELEM_TYPES(E)
-  constexpr int kPer = D / 16;  // elements per lane
+  constexpr int kPer = D / 16;
   using vec = typename std::conditional<kPer == 8, elem8, elem4>::type;
-  vec x[NV];
+  const int at = (int)blockIdx.x * 16 + (threadIdx.x >> 4), c8 = threadIdx.x & 15;
+  const int row = slot_row(which, min(at, which.rows - 1));
+  RowSlots<E, D, NV, kParts> slots;
+  slots.request(part_o, row, c8, K1, part_rows);
+  uint32_t bits[NV];  // (of the statistics: selected as integers, as an absent slot's may be those of a NaN)
 #pragma unroll
   for (int u = 0; u < NV; ++u) {
-    const int part = parts == 1 ? 0 : u / K1, j = u - part * K1;
-    if (u < nvirt)
-      x[u] = __builtin_nontemporal_load(reinterpret_cast<const vec*>(po + (int64_t)(part * part_rows + j) * D));
+    const SlotPlace place = slot_place<kParts>(u, K1);
+    bits[u] = reinterpret_cast<const uint32_t*>(part_lse)[(uint32_t)(row * K1) + (uint32_t)(place.part * part_rows + place.j)];
   }
-  const int part = parts == 1 ? 0 : c8 / K1, j = c8 - part * K1;
-  const bool ok = c8 < nvirt && (j == 0 ? part == 0 : ps[j - 1] >= 0);
-  const float l = ok ? pl[(int64_t)part * part_rows + j] : -INFINITY;
-  float mx = l;
+  slots.take_picks(sel, row, K1);
+  float l[NV], mx = -INFINITY;
 #pragma unroll
-  for (int o = 8; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 16));
-  const float wl = ok ? fast_exp2(l - mx) : 0.f;
-  float acc[kPer];
+  for (int u = 0; u < NV; ++u) {
+    l[u] = __builtin_bit_cast(float, slots.present[u] ? bits[u] : 0xff800000u);
+    mx = fmaxf(mx, l[u]);
+  }
+  float acc[kPer], wsum = 0.f;
 #pragma unroll
   for (int e = 0; e < kPer; ++e) acc[e] = 0.f;
-  float wsum = 0.f;
 #pragma unroll
   for (int u = 0; u < NV; ++u) {
-    if (u >= nvirt) break;
-    const float w = __shfl(wl, u, 16);
+    const float w = fast_exp2(l[u] - mx);  // (0 for an absent slot)
     wsum += w;
-#pragma unroll
-    for (int e = 0; e < kPer; ++e) acc[e] += w > 0.f ? w * (float)x[u][e] : 0.f;
+    slots.add(u, w, acc);
   }
-  if (!row_ok) return;
+  if (at >= which.rows) return;
   const float inv = 1.f / wsum;
   vec o;
 #pragma unroll
   for (int e = 0; e < kPer; ++e) o[e] = (elem)(acc[e] * inv);
-  __builtin_nontemporal_store(o, reinterpret_cast<vec*>(out + row * D + c8 * kPer));
+  __builtin_nontemporal_store(o, reinterpret_cast<vec*>(out + (int64_t)row * D + c8 * kPer));
   if (c8 == 0) lse[row] = (mx + fast_log2(wsum)) * 0.6931471805599453f;
 }
 
-// Combine the K1 slots of each (token, head): slot 0 is the self part, slot 1+j the
+// The same for any number of slots.  Combine the K1 slots of each (token, head): slot 0 is the self part, slot 1+j the
 // j-th selected history chunk (present iff sel[row, j] >= 0).  16 lanes per row.
 // With token ranges (mrg_start / mrg_prefix [nranges(+1)]: range b holds the tokens mrg_start[b] + i for
 // i < mrg_prefix[b+1] - mrg_prefix[b]) only the rows of those tokens are merged, `rows` counting them: the others
@@ -715,20 +718,14 @@ template <class E, int D>
 __global__ __launch_bounds__(256) void moba_merge_kernel(const typename E::elem* __restrict__ part_o,
                                                          const float* __restrict__ part_lse,
                                                          const int* __restrict__ sel, typename E::elem* __restrict__ out,
-                                                         float* __restrict__ lse, int64_t rows, int K1, int parts,
-                                                         int64_t all_rows, const int* __restrict__ mrg_start,
-                                                         const int* __restrict__ mrg_prefix, int nranges, int H) {
+                                                         float* __restrict__ lse, int K1, int parts, int part_rows,
+                                                         const SlotRows which) {
   MOBA_ELEM_TYPES(E)
   constexpr int kPer = D / 16;  // elements per lane
   using vec = typename std::conditional<kPer == 8, elem8, elem4>::type;
-  const int64_t row_raw = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
-  const bool row_ok = row_raw < rows;
-  int64_t row = row_ok ? row_raw : rows - 1;  // whole 16-lane groups stay active for the shuffles
-  if (mrg_start) {
-    const int t = (int)(row / H), h = (int)(row - (int64_t)t * H);
-    const int b = upper_row(mrg_prefix, nranges, t);
-    row = (int64_t)(mrg_start[b] + (t - mrg_prefix[b])) * H + h;
-  }
+  const int at_raw = (int)blockIdx.x * 16 + (threadIdx.x >> 4);
+  const bool row_ok = at_raw < which.rows;
+  const int64_t row = slot_row(which, row_ok ? at_raw : which.rows - 1);  // whole 16-lane groups stay active for the shuffles
   const int c8 = threadIdx.x & 15;
   const int K = K1 - 1;
   const float* pl = part_lse + row * K1;
@@ -743,11 +740,6 @@ __global__ __launch_bounds__(256) void moba_merge_kernel(const typename E::elem*
   // The parts are slots like any other: slot v of the parts * K1 is slot v % K1 of part v / K1, at slot row
   // (v / K1) * rows * K1 + v % K1 of the row's first (an int: the buffers hold fewer than 2^31 slot rows).
   const int nvirt = parts * K1;
-  const int part_rows = (int)(all_rows * K1);
-  if (nvirt <= 8) {  // (uniform)
-    merge_few_slots<E, D, 8>(po, pl, ps, out, lse, row, row_ok, c8, K1, parts, nvirt, part_rows);
-    return;
-  }
   float mx = -INFINITY;
   for (int v0 = 0; v0 < nvirt; v0 += 16) {
     const int v = v0 + c8;
@@ -964,6 +956,20 @@ extern "C" int moba_fwd_partials(const void* q, const void* k, const void* v, vo
                                 self_tile_skip, q_tok_shift, kFwdTileRows, redo == nullptr, 1, stream);
 }
 
+template <class E, int D>
+static void launch_merge(const void* part_o, const float* part_lse, const int* sel, void* out, float* lse, int K1, int parts,
+                         int part_rows, const SlotRows& which, hipStream_t st) {
+  typedef typename E::elem elem;
+  const dim3 grid((unsigned)(((int64_t)which.rows + 15) / 16));
+  const bool few = for_slots(K1, parts, [&](auto nv, auto several) {
+    hipLaunchKernelGGL((moba_merge_few_kernel<E, D, decltype(nv)::value, decltype(several)::value>), grid, dim3(256), 0, st,
+                       (const elem*)part_o, part_lse, sel, (elem*)out, lse, K1, part_rows, which);
+  });
+  if (!few)
+    hipLaunchKernelGGL((moba_merge_kernel<E, D>), grid, dim3(256), 0, st, (const elem*)part_o, part_lse, sel, (elem*)out, lse, K1,
+                       parts, part_rows, which);
+}
+
 // mrg_start [nranges], mrg_prefix [nranges + 1], merge_tokens = mrg_prefix[nranges]: the tokens to merge, for a
 // caller whose attention call wrote the other tokens' rows itself (chunk_direct); null, null, 0, S: every token.
 extern "C" int moba_fwd_merge(const void* part_o, const float* part_lse, const int32_t* sel, void* out, float* lse,
@@ -980,16 +986,15 @@ extern "C" int moba_fwd_merge(const void* part_o, const float* part_lse, const i
     return MOBA_ERR_ARG;
   if (merge_tokens == 0) return MOBA_OK;  // every row was written by the attention kernel
   const int64_t rows = merge_tokens * H;
-  const dim3 grid((unsigned)((rows + 15) / 16));
-#define MOBA_MERGE(EL, DIM)                                                                                          \
-  hipLaunchKernelGGL((moba_merge_kernel<EL, DIM>), grid, dim3(256), 0, (hipStream_t)stream, (const EL::elem*)part_o,  \
-                     part_lse, sel, (EL::elem*)out, lse, rows, K + 1, key_split, S * H, mrg_start, mrg_prefix, nranges, H)
-  if (dtype == MOBA_DTYPE_F16) {
-    if (D == 64) MOBA_MERGE(F16, 64); else MOBA_MERGE(F16, 128);
-  } else {
-    if (D == 64) MOBA_MERGE(Bf16, 64); else MOBA_MERGE(Bf16, 128);
-  }
-#undef MOBA_MERGE
+  const SlotRows which = slot_rows(mrg_start, mrg_prefix, nranges, H, rows);
+  auto go = [&](auto elem_c, auto dim_c) {
+    launch_merge<decltype(elem_c), decltype(dim_c)::value>(part_o, part_lse, sel, out, lse, K + 1, key_split,
+                                                           (int)(S * H * (K + 1)), which, (hipStream_t)stream);
+  };
+  using D64 = std::integral_constant<int, 64>;
+  using D128 = std::integral_constant<int, 128>;
+  if (dtype == MOBA_DTYPE_F16) D == 64 ? go(F16{}, D64{}) : go(F16{}, D128{});
+  else D == 64 ? go(Bf16{}, D64{}) : go(Bf16{}, D128{});
   return launch_check.result();
 }
 
