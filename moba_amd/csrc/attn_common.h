@@ -26,7 +26,10 @@ inline Divisor divisor(uint64_t d) {
   while ((1ull << lg) < d) ++lg;
   return {(uint32_t)((1ull << (31 + lg)) / d + 1), lg - 1};
 }
+// (d = 1: no such numbers; {0, 0} stands for it where it may come up)
+inline Divisor divisor_or_one(uint64_t d) { return d == 1 ? Divisor{0, 0} : divisor(d); }
 __device__ __forceinline__ int quotient(int n, Divisor d) { return (int)(__umulhi((uint32_t)n, d.magic) >> d.shift); }
+__device__ __forceinline__ int quotient_or_same(int n, Divisor d) { return d.magic ? quotient(n, d) : n; }  // (d uniform)
 
 // Index tables that define the tiles of one call.
 struct TileTables {
@@ -47,6 +50,7 @@ struct TileTables {
   int S, H, K1, F, N, B;
   int seg_heads, seg_groups;
   Divisor by_hk1, by_k1;        // H*K1 and K1, for the entries of the lists (which exist only with K1 >= 2)
+  Divisor by_groups, by_rep, by_h, by_batch;  // seg_groups, rep, H, batch_rows (divisor_or_one)
   int Hkv, rep;                 // key/value heads and query heads per key/value head (H = Hkv * rep)
   int hist_bound;               // logical tile ids below it are history tiles
   int self_total;               // self_tile_prefix[N] * H
@@ -72,12 +76,12 @@ struct TileTables {
 __device__ __forceinline__ int64_t q_tok_bytes(const TileTables& t, int tok) {
   tok = max(tok - t.q_shift, 0);  // (q holds the rows from q_shift on; row 0 stands in where there is no tile)
   if (t.batch_rows == 0) return (int64_t)tok * t.q_tok_b;
-  const int b = tok / t.batch_rows;
+  const int b = quotient_or_same(tok, t.by_batch);
   return (int64_t)b * t.q_batch_b + (int64_t)(tok - b * t.batch_rows) * t.q_tok_b;
 }
 __device__ __forceinline__ int64_t kv_tok_bytes(const TileTables& t, int tok) {
   if (t.batch_rows == 0) return (int64_t)tok * t.kv_tok_b;
-  const int b = tok / t.batch_rows;
+  const int b = quotient_or_same(tok, t.by_batch);
   return (int64_t)b * t.kv_batch_b + (int64_t)(tok - b * t.batch_rows) * t.kv_tok_b;
 }
 
@@ -94,6 +98,7 @@ inline bool set_layout(TileTables& t, const int64_t* strides) {
   t.self_skip = 0; t.q_shift = 0;
   t.seg_heads = 1; t.seg_groups = t.H;
   t.by_hk1 = divisor((uint64_t)t.H * t.K1); t.by_k1 = divisor(t.K1);
+  t.by_groups = t.by_h = divisor_or_one(t.H); t.by_rep = divisor_or_one(t.rep); t.by_batch = divisor_or_one(1);
   if (!strides) {
     t.q_tok_b = (int64_t)t.H * kHeadDim * 2; t.q_head_b = kHeadDim * 2;
     t.kv_tok_b = (int64_t)t.Hkv * kHeadDim * 2; t.kv_head_b = kHeadDim * 2;
@@ -107,6 +112,7 @@ inline bool set_layout(TileTables& t, const int64_t* strides) {
   if (strides[4] != 0) {
     if (strides[4] < 0 || strides[4] > 0x7fffffffLL || strides[5] <= 0 || strides[6] <= 0 || (strides[5] & 7) || (strides[6] & 7))
       return false;
+    t.by_batch = divisor_or_one(strides[4]);
     t.batch_rows = (int)strides[4]; t.q_batch_b = strides[5] * 2; t.kv_batch_b = strides[6] * 2;
   }
   return true;
@@ -198,7 +204,7 @@ __device__ __forceinline__ TileHeadEntries tile_head_entries(const TileTables& p
     e.a = table_load(p.tile_off + code);
     e.b = table_load(p.seg_off + (kGrouped ? code * p.seg_heads : code));
     e.c = table_load(p.seg_off + (kGrouped ? (code + 1) * p.seg_heads : code + 1));
-    e.d = table_load(p.fchunk_tok + code / (kGrouped ? p.seg_groups : p.H));
+    e.d = table_load(p.fchunk_tok + (kGrouped ? quotient_or_same(code, p.by_groups) : code / p.H));
   } else {
     e.a = table_load(p.self_tile_prefix + code);
     e.b = table_load(p.self_tile_prefix + code + 1);
@@ -220,7 +226,7 @@ __device__ __forceinline__ bool decode_tile_head(const TileTables& p, int logica
   if (logical < p.hist_bound) {
     const int seg = code;
     const int tile = logical - e.a;
-    const int groups = kGrouped ? p.seg_groups : H, f = seg / groups;
+    const int groups = kGrouped ? p.seg_groups : H, f = kGrouped ? quotient_or_same(seg, p.by_groups) : seg / groups;
     t.h = seg - f * groups;
     if constexpr (kGrouped) t.h *= p.seg_heads;
     t.base = e.b + tile * tm;

@@ -240,24 +240,25 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(const BwdParams<E> p) {
   }
   empty_queues = 0;
 
+  const BwdParams<E> pt = kernarg_now<BwdParams<E>>(0);  // (read again for every tile: kept, they are spilled and cost more)
   Tile t;
   const int r = wave * 32 + n;
   // With few tiles per workgroup (self_first) the self tiles take the first ids -- the longest of them are as
   // long as a history tile, and drawn last they would run alone at the end -- and the keys of a history tile
   // are cut into 1 << ks parts that are tiles of their own, each with slot rows of its own for its partial dQ
   // (part g of a slot row lies g * part_stride rows behind part 0; the sum over the slots adds them up).
-  const int hist = p.t.self_first ? id - p.t.self_total : (id < hist_tiles ? id : -1);
-  const int logical = hist >= 0 ? hist >> ks : p.t.hist_bound + (p.t.self_first ? id : id - hist_tiles);
+  const int hist = pt.t.self_first ? id - pt.t.self_total : (id < hist_tiles ? id : -1);
+  const int logical = hist >= 0 ? hist >> ks : pt.t.hist_bound + (pt.t.self_first ? id : id - hist_tiles);
   const int key_part = hist >= 0 ? hist & ((1 << ks) - 1) : 0;
-  decode_tile_head<true>(p.t, logical, t);
+  decode_tile_head<true>(pt.t, logical, t);
   if (t.base >= 0) {
     t.nkeys >>= ks;
     t.kv_tok0 += key_part * t.nkeys;
   }
-  const int entry = decode_tile_row_entry(p.t, r, t);  // (asked for ahead of the first copies)
+  const int entry = decode_tile_row_entry(pt.t, r, t);  // (asked for ahead of the first copies)
   const int h = t.h, nkeys = t.nkeys, kv_tok0 = t.kv_tok0;
-  const int hkv = h / p.t.rep;                                // key/value head of this query head
-  const int64_t row_bytes = p.t.kv_tok_b;                     // from one K or V token to the next
+  const int hkv = quotient_or_same(h, pt.t.by_rep);                                // key/value head of this query head
+  const int64_t row_bytes = pt.t.kv_tok_b;                     // from one K or V token to the next
   const uint32_t lds_base = lds_addr(smem);
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
   const int ld_kin = lane >> 4, ld_pc = lane & 15;
@@ -267,9 +268,9 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(const BwdParams<E> p) {
     const int key = 4 * (4 * i + wave_u) + ld_kin;
     ld_off[i] = (uint32_t)(key * row_bytes + sw_col16(key, ld_pc) * 16);
   }
-  const int64_t kv_off = kv_tok_bytes(p.t, kv_tok0) + hkv * p.t.kv_head_b;
-  const char* k_head = (const char*)p.k + kv_off;
-  const char* v_head = (const char*)p.v + kv_off;
+  const int64_t kv_off = kv_tok_bytes(pt.t, kv_tok0) + hkv * pt.t.kv_head_b;
+  const char* k_head = (const char*)pt.k + kv_off;
+  const char* v_head = (const char*)pt.v + kv_off;
   auto issue_tile = [&](int kt, int buf) __attribute__((always_inline)) {
     const uint32_t kdst = lds_base + buf * kTileBytes;
     const uint32_t vdst = lds_base + (2 + buf) * kTileBytes;
@@ -319,23 +320,23 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(const BwdParams<E> p) {
   // 104.9 ms for a training step of 302060 tokens in 8 sequences)
   issue_tile(0, 0);
 
-  decode_tile_rows<true>(p.t, wave, r, entry, t);
-  t.dest += key_part * p.t.part_stride;
+  decode_tile_rows<true>(pt.t, wave, r, entry, t);
+  t.dest += key_part * pt.t.part_stride;
   const int limit = t.limit;
   const bool row_valid = r < t.row_count;
 
   elem8 bq[8], bdo[8];
   {
-    const int64_t off = ((int64_t)t.tok * H + t.rh) * kHeadDim + 8 * hh;
-    const elem* qsrc = reinterpret_cast<const elem*>((const char*)p.q + q_tok_bytes(p.t, t.tok) + t.rh * p.t.q_head_b) + 8 * hh;
+    const int64_t off = ((int64_t)t.tok * pt.t.H + t.rh) * kHeadDim + 8 * hh;
+    const elem* qsrc = reinterpret_cast<const elem*>((const char*)pt.q + q_tok_bytes(pt.t, t.tok) + t.rh * pt.t.q_head_b) + 8 * hh;
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) {
       bq[ks] = *reinterpret_cast<const elem8*>(qsrc + 16 * ks);
-      bdo[ks] = *reinterpret_cast<const elem8*>(p.dout + off + 16 * ks);
+      bdo[ks] = *reinterpret_cast<const elem8*>(pt.dout + off + 16 * ks);
     }
   }
-  const float lse2 = p.lse[(int64_t)t.tok * H + t.rh] * kLog2e;
-  const float dl = p.delta[(int64_t)t.tok * H + t.rh];
+  const float lse2 = pt.lse[(int64_t)t.tok * pt.t.H + t.rh] * kLog2e;
+  const float dl = pt.delta[(int64_t)t.tok * pt.t.H + t.rh];
 
   wait_vmem();
   scrub_tile(0, 0);
@@ -465,6 +466,7 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(const BwdParams<E> p) {
   }
 
   id = id_of(__builtin_amdgcn_readfirstlane(*id_word));
+  const BwdParams<E> pw = kernarg_now<BwdParams<E>>(0);
   // The accumulators hold dQ^T: element e of lane (n, hh) is dQ[row n][32*db + 8*(e/4) + 4*hh + e%4].  The partial is rounded to
   // the element type, as the per-chunk dQ that flash-attn returns to the reference is; the two lanes of a row exchange
   // halves, and each stores 16 bytes, 32 bytes of a row side by side.
@@ -478,13 +480,13 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(const BwdParams<E> p) {
         for (int i = 0; i < 2; ++i) {
           const int e = 8 * pair + 2 * i;
           // (scaled before the rounding: a partial then overflows fp16 only where dQ itself would)
-          const auto x = __builtin_amdgcn_permlane32_swap(pack2<E>(dqacc[db][e] * p.scale, dqacc[db][e + 1] * p.scale),
-                                                          pack2<E>(dqacc[db][e + 4] * p.scale, dqacc[db][e + 5] * p.scale), false, false);
+          const auto x = __builtin_amdgcn_permlane32_swap(pack2<E>(dqacc[db][e] * pw.scale, dqacc[db][e + 1] * pw.scale),
+                                                          pack2<E>(dqacc[db][e + 4] * pw.scale, dqacc[db][e + 5] * pw.scale), false, false);
           w[2 * db + pair][i] = x[0];
           w[2 * db + pair][2 + i] = x[1];
         }
     // (a tile of a chunk without history slots holds the whole dQ of its rows: nothing to add it to)
-    elem* const row = (t.direct ? p.dq : p.part_dq) + (int64_t)t.dest * kHeadDim + 8 * hh;
+    elem* const row = (t.direct ? pw.dq : pw.part_dq) + (int64_t)t.dest * kHeadDim + 8 * hh;
     if (row_valid) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) *reinterpret_cast<u32x4*>(row + 16 * i) = w[i];
@@ -1260,7 +1262,7 @@ extern "C" int moba_bwd(const void* dout, const void* q, const void* k, const vo
   t.hist_bound = (K > 0) ? (int)hist_bound : 0;
   t.self_total = (int)(self_tiles * H);
   if (!set_layout(t, strides)) return MOBA_ERR_ARG;
-  t.seg_heads = list_heads; t.seg_groups = H / list_heads;
+  t.seg_heads = list_heads; t.seg_groups = H / list_heads; t.by_groups = divisor_or_one(t.seg_groups);
   // the dQ kernel's order of tiles and its parts per history tile (the dK/dV kernel has parts of its own)
   t.self_first = dq_key_split > 1 || total_q < 8 * grid_q;
   while ((1 << t.key_split_log2) < dq_key_split) ++t.key_split_log2;

@@ -923,7 +923,7 @@ extern "C" int moba_fwd_partials_rows(const void* q, const void* k, const void* 
   t.self_total = (int)(self_tiles * H);
   if (!strides && D != kHeadDim) return MOBA_ERR_ARG;  // (packed is said for 128 only)
   if (!set_layout(t, strides)) return MOBA_ERR_ARG;
-  t.seg_heads = list_heads; t.seg_groups = H / list_heads;
+  t.seg_heads = list_heads; t.seg_groups = H / list_heads; t.by_groups = divisor_or_one(t.seg_groups);
   t.key_split_log2 = key_split_log2;
   t.part_stride = (int)(S * H * (K + 1));
   t.xcd_block_log2 = tile_xcd_block_log2(total);

@@ -112,7 +112,7 @@ __global__ __launch_bounds__(NW * 64, (FwdTileShape<D, NW>::kWavesPerSimd)) void
     const int key = Shape::kSlabRows * (NW * i + wave) + ld_kin;
     ld_off[i] = (uint32_t)(key * row_bytes + (ld_pc ^ tile_sw<D>(key)) * 16);
   }
-  const int64_t kv_off = (kTail ? seq * p.t.kv_batch_b : kv_tok_bytes(p.t, t.kv_tok0)) + (h / p.t.rep) * p.t.kv_head_b;
+  const int64_t kv_off = (kTail ? seq * p.t.kv_batch_b : kv_tok_bytes(p.t, t.kv_tok0)) + quotient_or_same(h, p.t.by_rep) * p.t.kv_head_b;
   const char* k_head = (const char*)p.k + kv_off;
   const char* v_head = (const char*)p.v + kv_off;
   auto issue = [&](const char* head, int kt, uint32_t dst) __attribute__((always_inline)) {
@@ -525,7 +525,7 @@ extern "C" int moba_tail_tiles(const void* q, const void* k, const void* v, void
   const int64_t tiles = ((int64_t)nq + tile_rows - 1) / tile_rows, total = heads * tiles;
   TileTables t = {};
   t.S = nq; t.N = (int)tiles; t.q_shift = Skv - nq; t.self_total = (int)total;
-  t.H = H; t.Hkv = Hkv; t.rep = H / Hkv; t.K1 = 1;
+  t.H = H; t.Hkv = Hkv; t.rep = H / Hkv; t.by_rep = divisor_or_one(t.rep); t.K1 = 1;
   t.q_batch_b = strides[0] * 2; t.q_head_b = strides[1] * 2; t.q_tok_b = strides[2] * 2;
   t.kv_batch_b = strides[3] * 2; t.kv_head_b = strides[4] * 2; t.kv_tok_b = strides[5] * 2;
   t.xcd_block_log2 = tile_xcd_block_log2(total);
