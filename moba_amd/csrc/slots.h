@@ -104,7 +104,8 @@ bool for_slots(int K1, int parts, Launch launch) {
   using One = std::false_type;
   using Several = std::true_type;
 #define MOBA_SLOTS(NV, KIND) launch(std::integral_constant<int, NV>{}, KIND{}); return true
-  switch (parts == 1 ? K1 : (K1 >= 2 && K1 * parts <= kMostSlotsAtOnce ? 16 * parts + K1 * parts : 0)) {
+  if ((int64_t)K1 * parts > kMostSlotsAtOnce || (parts > 1 && K1 < 2)) return false;
+  switch ((parts == 1 ? 0 : 16 * parts) + K1 * parts) {
     case 1: MOBA_SLOTS(1, One);
     case 2: MOBA_SLOTS(2, One);
     case 3: MOBA_SLOTS(3, One);

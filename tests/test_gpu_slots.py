@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("dtype,dim", [(torch.bfloat16, 128), (torch.float16, 64)])
 @pytest.mark.parametrize("H", [1, 3])
-@pytest.mark.parametrize("slots,parts", [(1, 1), *((n, 1) for n in range(2, 14)), (2, 2), (3, 2), (4, 2), (5, 2), (6, 2), (7, 2),
+@pytest.mark.parametrize("slots,parts", [(1, 1), *((n, 1) for n in (*range(2, 14), 36, 38, 40, 42, 44, 65)), (2, 2), (3, 2), (4, 2), (5, 2), (6, 2), (7, 2),
                                          (2, 4), (3, 4), (4, 4), (2, 8)])
 def test_merge_of_token_ranges(slots, parts, H, dtype, dim):
     """Random partial results and statistics, a third of the history slots absent (and poisoned), merged for the tokens of
