@@ -7,9 +7,11 @@
 // does not depend on how the chunk is split over workgroups, and the rounded
 // mean is reproducible bit for bit (fp64 -> fp32 -> element type, round to nearest even).
 //
-// One stage (chunk_mean_whole_kernel): one workgroup of 256 to 1024 threads per (chunk, head), D/8 column groups times the
-//          token lanes, their sums added through LDS: one launch instead of two, and no partial sums in memory.  131072 tokens, 8 heads, chunk 4096: 67 -> 44 us; 302060 tokens, 32 heads, chunk 2048: 474 -> 389 us.
-// Two stages where that leaves too few workgroups for too many bytes each (see whole_chunks):
+// One stage (chunk_mean_whole_kernel): one workgroup of 256 to 1024 threads per (chunk, head) or part of its columns
+//          (column_parts_log2), column groups of 8 times the token lanes, their sums added through LDS: one launch instead of
+//          two, and no partial sums in memory.  131072 tokens, 8 heads, chunk 4096: 67 -> 44 us; 302060 tokens, 32 heads,
+//          chunk 2048: 474 -> 389 us; in parts, 32768 tokens, one head, chunk 1024: 9.8 -> 5.8 us.
+// Two stages where that leaves few workgroups for very many bytes each (see whole_chunks):
 //   Stage 1: grid (F, token splits, column blocks); each thread owns 8 adjacent
 //            columns of the [H*D] token row and sums its share of a token split.
 //   Stage 2: sums the splits in order, divides by B, rounds.
@@ -103,28 +105,29 @@ __device__ __forceinline__ float round_to_odd_f32(double x) {
   return f;
 }
 
-// One workgroup of NT threads per (chunk f, head): thread (tl, c) sums the tokens tl, tl + lanes, ... of columns
-// 8c .. 8c + 7.  D8 = D/8 column groups, a power of two up to 16.  NT: about eight tokens per lane or more, so that every
+// One workgroup of NT threads per (chunk f, head, part of the columns): thread (tl, c) sums the tokens tl, tl + lanes, ... of
+// the part's columns 8c .. 8c + 7.  D8 column groups, a power of two up to 16.  NT: about eight tokens per lane or more, so that every
 // lane has its eight rows in flight and the sums' way through LDS stays short against them (65536 tokens, 8 heads, chunk
 // 128: 53 us with 1024 threads, 22 with 256).
 template <class E, int NT>
 __global__ __launch_bounds__(NT) void chunk_mean_whole_kernel(
     const typename E::elem* __restrict__ k, const int* __restrict__ fchunk_tok, typename E::elem* __restrict__ kbar,
     int d8_log2, int B, int64_t row_stride, int64_t head_stride, int batch_rows, int64_t batch_stride,
-    int* __restrict__ clear, int64_t clear_ints) {
+    int* __restrict__ clear, int64_t clear_ints) {  // d8_log2: of the column groups of this workgroup's part
   MOBA_ELEM_TYPES(E)
   __shared__ double red[8][NT / 64][16];  // [element][wave][column group]
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int f = blockIdx.x, head = blockIdx.y, H = gridDim.y;
+  const int f = blockIdx.x, head = blockIdx.y, H = gridDim.y, part = blockIdx.z;
   if (clear) {
-    const int64_t step = (int64_t)gridDim.x * H * NT;
-    for (int64_t i = ((int64_t)head * gridDim.x + f) * NT + tid; i < clear_ints; i += step) clear[i] = 0;
+    const int64_t step = (int64_t)gridDim.x * H * gridDim.z * NT;
+    for (int64_t i = (((int64_t)part * H + head) * gridDim.x + f) * NT + tid; i < clear_ints; i += step) clear[i] = 0;
   }
   const int D8 = 1 << d8_log2, lanes = NT >> d8_log2;
   const int c = tid & (D8 - 1), tl = tid >> d8_log2;
+  const int col0 = part * D8 * 8, D = gridDim.z * D8 * 8;
   const int tok0 = fchunk_tok[f];
   const int be = batch_rows ? tok0 / batch_rows : 0;  // (a chunk lies inside one batch entry)
-  const elem* src = k + be * batch_stride + ((int64_t)(tok0 - be * batch_rows) + tl) * row_stride + head * head_stride + c * 8;
+  const elem* src = k + be * batch_stride + ((int64_t)(tok0 - be * batch_rows) + tl) * row_stride + head * head_stride + col0 + c * 8;
   const int64_t step = (int64_t)lanes * row_stride;
   double acc[8];
 #pragma unroll
@@ -166,7 +169,7 @@ __global__ __launch_bounds__(NT) void chunk_mean_whole_kernel(
   double sum = 0.0;
 #pragma unroll
   for (int w = 0; w < NT / 64; ++w) sum += red[e][w][c];
-  kbar[((int64_t)f * H + head) * (D8 * 8) + c * 8 + e] = (elem)round_to_odd_f32(sum / (double)B);
+  kbar[((int64_t)f * H + head) * D + col0 + c * 8 + e] = (elem)round_to_odd_f32(sum / (double)B);
 }
 
 template <class E>
@@ -231,22 +234,34 @@ extern "C" size_t moba_chunk_mean_workspace_bytes(int H, int D, int F, int B) {
   return (size_t)F * pick_nsplit(HD8, F, B) * HD8 * 8 * sizeof(double);
 }
 
-// Whether one workgroup per (chunk, head) will do: where there are enough of them to keep the memory busy, or so little
-// to read for each that a second launch would take longer.  One workgroup reads its 256 KiB in 9 us, 512 KiB in 15, 1 MiB in
-// 25, alone or not; the two stages take 8 and what the bytes of all take, and more for rows of many heads.  One workgroup
-// each / two stages in us, 128-element heads (heads x chunks, tokens a chunk): 1 x 31, 1024: 9.3 / 8.6; 1 x 64: 9.8 / 10.2;
-// 1 x 15, 2048: 14.1 / 9.9; 1 x 64: 15.8 / 14.5; 2 x 16: 15.5 / 14.8; 2 x 32: 16.8 / 18.2; 4 x 8: 15.9 / 12.2; 4 x 16: 17.1 / 14.3;
-// 8 x 4: 15.9 / 16.6; 1 x 31, 4096: 25.3 / 18.2; 4 x 31: 35.2 / 42.8; 8 x 31: 48.6 / 72.1; 64-element heads: 1 x 31, 2048: 9.5 /
-// 9.2; 4 x 8: 10.2 / 12.9; 1 x 31, 4096: 15.3 / 12.7; 4 x 7: 16.5 / 21.0.
-// Not for very many chunks of at most eight tokens per lane: whole rows of all heads, in the order they lie, then read
-// faster than they add up (65536 tokens, 32 heads, chunk 128: 104 us in two stages, 114 in one; 8 heads: 28 and 22).
+// Into how many parts (log2) the columns of a chunk and head go, each a workgroup's: few chunks leave most of the chip without
+// one, and a workgroup reads its 128 KiB in 7 us, 256 in 9, 512 in 12, alone or not.  Parts of 128 bytes, a line of the caches,
+// are read as well as whole rows; parts of 64 bytes only where all keys together stay in an XCD's second-level cache long
+// enough (17 MB).  1 / 2 / 4 parts, and the two stages below, in us, 128-element heads (heads x chunks, tokens a chunk): 4 x 7,
+// 512: 6.0 / 5.6 / 5.6, 9.2; 1 x 15, 2048: 10.8 / 7.9 / 7.1, 10.0; 1 x 31, 1024: 7.7 / 6.4 / 5.8, 9.8; 4 x 8, 2048: 10.9 / 8.0 /
+// 7.5, 11.7; 1 x 60, 2048: 11.6 / 8.4 / 11.9, 12.7; 8 x 15, 1024: 8.7 / 7.5 / 8.6, 13.6; 1 x 15, 4096: 17.4 / 11.3 / 8.8, 13.3; 1 x 31,
+// 4096: 18.6 / 12.2 / 15.4, 15.9; 4 x 31, 4096: 30.8 / 26.7 / 47.7, 40.1; 8 x 31, 4096: 44.7 / 48.0 / 82, 67; 1 x 3, 16384: 59 / 31 /
+// 20, 32; 64-element heads: 1 x 31, 2048: 7.8 / 7.4, 9.5; 1 x 31, 4096: 11.2 / 9.2, 11.8; 4 x 31, 4096: 17.3 / 24.0, 27.5; 8 x 15,
+// 512: 5.6 / 5.8, 9.6.
+static int column_parts_log2(int H, int D, int F, int B) {
+  const int64_t groups = (int64_t)F * H;
+  int parts = 0, row = 2 * D;
+  if (groups < 192)
+    while (row >= 256) ++parts, row /= 2;
+  if (groups <= 64 && row == 128 && groups * B * D * 2 <= (17 << 20)) ++parts;
+  return parts;
+}
+
+// Whether a chunk's tokens go to one workgroup (a head's columns in parts or not), or to many in two stages: those where a
+// workgroup would read more than 1 MiB and there are few of them, and for very many chunks of at most eight tokens per
+// lane: whole rows of all heads, in the order they lie, then read faster than they add up (65536 tokens, 32 heads, chunk 128:
+// 104 us in two stages, 114 in one; 8 heads: 28 and 22).
 static bool whole_chunks(int H, int D, int F, int B) {
   const int d8 = D / 8;
   if (d8 > 16 || (d8 & (d8 - 1)) || H > 65535) return false;
-  const int64_t groups = (int64_t)F * H, elems = (int64_t)B * D;
+  const int64_t groups = (int64_t)F * H;
   if (B * d8 <= 256 * 8 && groups > 8192) return false;
-  if (groups >= 128 || elems <= 1024 * 128) return true;
-  return elems <= 2048 * 128 && (groups >= 64 || H * 32 > D);
+  return groups >= 128 || ((int64_t)B * D * 2 >> column_parts_log2(H, D, F, B)) <= (1 << 20);
 }
 
 static int launch_chunk_mean(const void* k, const int32_t* fchunk_tok, void* kbar, double* partial, int H, int D,
@@ -256,9 +271,11 @@ static int launch_chunk_mean(const void* k, const int32_t* fchunk_tok, void* kba
   if (!partial) {  // (whole_chunks)
     int d8_log2 = 0;
     while ((8 << d8_log2) < D) ++d8_log2;
-    const dim3 grid(F, H);
+    const int parts_log2 = column_parts_log2(H, D, F, B);
+    d8_log2 -= parts_log2;
+    const dim3 grid(F, H, 1 << parts_log2);
     // threads: as many as eight tokens each would take, to be done soonest, or 256 where there are workgroups enough
-    const int rows = (int64_t)F * H >= 1024 ? 256 : B * (D / 8) / 8;
+    const int rows = (int64_t)F * H >= 1024 ? 256 : B * (D >> (3 + parts_log2)) / 8;
 #define MOBA_MEAN(EL, NT)                                                                                                \
   hipLaunchKernelGGL((chunk_mean_whole_kernel<EL, NT>), grid, dim3(NT), 0, st, (const EL::elem*)k, fchunk_tok,            \
                      (EL::elem*)kbar, d8_log2, B, kts, khs, batch_rows, kbs, clear, clear_ints)
