@@ -539,7 +539,7 @@ __global__ __launch_bounds__(256) void bwd_dq_sum_few_kernel(const typename E::e
 #pragma unroll
   for (int e = 0; e < 8; ++e) acc[e] = 0.f;
 #pragma unroll
-  for (int u = 0; u < NV; ++u) slots.add(u, 1.f, acc);
+  for (int u = 0; u < NV; ++u) slots.add(u, slots.present[u], 1.f, acc);
   if (at >= which.rows) return;
   elem8 o;
 #pragma unroll

@@ -698,7 +698,7 @@ __global__ __launch_bounds__(256) void moba_merge_few_kernel(const typename E::e
   for (int u = 0; u < NV; ++u) {
     const float w = fast_exp2(l[u] - mx);  // (0 for an absent slot)
     wsum += w;
-    slots.add(u, w, acc);
+    slots.add(u, w > 0.f, w, acc);
   }
   if (at >= which.rows) return;
   const float inv = 1.f / wsum;

@@ -59,3 +59,37 @@ def test_results_and_gradients_by_slots(topk, heads, dense):
     from test_gpu_operator import run_case
     print("slots", topk, heads, dense, flush=True)
     run_case(5, 2400, heads, 30, topk, seed=topk, ref_bounds=False, dense=dense)
+
+
+@pytest.mark.parametrize("dtype,dim", [(torch.bfloat16, 128), (torch.float16, 64)])
+@pytest.mark.parametrize("slots,parts", [(2, 1), (3, 1), (8, 1), (9, 1), (12, 1), (3, 2), (6, 2), (2, 4), (3, 4)])
+def test_slots_without_weight(slots, parts, dtype, dim):
+    """A slot whose weight is 0 (its statistic lies 300 below another's) takes no part in its row, whatever its partial result
+    holds: an infinite value of one key stays with the rows that see it."""
+    from moba_amd import _lib
+    print("no weight", slots, parts, dtype, dim, flush=True)
+    lib, S, K = _lib.load(), 37, slots - 1
+    g = torch.Generator().manual_seed(slots + parts)
+    po = torch.randn((parts, S, slots, dim), generator=g).to(dtype)
+    log2 = torch.randn((parts, S, slots), generator=g)
+    none = torch.zeros((parts, S, slots), dtype=torch.bool)
+    none[parts - 1, 0::3, slots - 1] = True    # a history slot, the last part of it,
+    none[0, 1::3, 0] = True                    # the self slot, or none
+    log2[none] -= 300
+    weights = log2.double().exp2()
+    weights[1:, :, 0] = 0                      # (the self slot has part 0 only)
+    weights[none] = 0
+    want = (weights[..., None] * po.double()).sum(dim=(0, 2)) / weights.sum(dim=(0, 2))[:, None]
+    want_lse = weights.sum(dim=(0, 2)).log()
+    values = torch.tensor([math.inf, -math.inf, math.nan], dtype=dtype)
+    po[none] = values[torch.arange(dim) % 3]
+    sel = torch.zeros((S, K), dtype=torch.int32)
+    bufs = [t.cuda() for t in (po, log2.float(), sel)]
+    out, lse = torch.empty((S, dim), dtype=dtype, device="cuda"), torch.empty((S,), device="cuda")
+    p = [t.data_ptr() for t in bufs]
+    _lib.check(lib.moba_fwd_merge(p[0], p[1], p[2], out.data_ptr(), lse.data_ptr(), S, 1, dim, K, parts, None, None, 0, S,
+                                  _lib.DTYPE_F16 if dtype == torch.float16 else _lib.DTYPE_BF16,
+                                  torch.cuda.current_stream().cuda_stream), "moba_fwd_merge")
+    unit = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)   # (as above)
+    assert bool(((out.cpu().double() - want).abs() <= unit * want.abs() + 5 * 2.0 ** -18).all())
+    assert (lse.cpu().double() - want_lse).abs().max() < 2e-5
