@@ -985,6 +985,10 @@ extern "C" int moba_fwd_merge(const void* part_o, const float* part_lse, const i
                 : (mrg_prefix || merge_tokens != S))
     return MOBA_ERR_ARG;
   if (merge_tokens == 0) return MOBA_OK;  // every row was written by the attention kernel
+  // The kernels number the slot rows in 32 bits, as those that write them do (2^31 slot rows with their statistics are more than
+  // the memory holds).  Factor by factor: the product alone could pass 64 bits.
+  constexpr int64_t kMost = 0x7fffffffLL;
+  if (S >= kMost || S * H >= kMost || S * H * (K + 1ll) >= kMost || S * H * (K + 1ll) * key_split >= kMost) return MOBA_ERR_LIMIT;
   const int64_t rows = merge_tokens * H;
   const SlotRows which = slot_rows(mrg_start, mrg_prefix, nranges, H, rows);
   auto go = [&](auto elem_c, auto dim_c) {

@@ -113,3 +113,21 @@ def test_shares_beyond_32_bits_are_refused(lib):
         assert call(*sizes, 4) == -4, sizes
         assert call(*sizes, 0) != -4 and call(*sizes, 4, None) != -4 and call(*sizes, 4, some, 4096) != -4, sizes
     assert call(1 << 19, 64, 1, 1, 4) != -4
+
+
+def test_merges_beyond_32_bit_slot_rows_are_refused(lib):
+    """moba_fwd_merge numbers slot rows in 32 bits: a call with more of them is refused before anything is launched, whichever
+    factor takes it there; one without rows to merge has nothing to number."""
+    from moba_amd import _lib
+    bound = _lib.load()
+    some = 256   # (never read)
+
+    def call(S, H, K, parts, tokens=None, ranges=None):
+        return bound.moba_fwd_merge(some, some, some, some, some, S, H, 128, K, parts, ranges, ranges, 1 if ranges else 0,
+                                    S if tokens is None else tokens, 0, None)
+
+    for S, H, K, parts in ((1 << 31, 1, 2, 1), (1 << 29, 1, 3, 1), (1 << 28, 1, 3, 2), (1 << 20, 1 << 9, 3, 1), (1 << 62, 64, 3, 1),
+                           (1 << 30, 1 << 30, (1 << 30) - 1, 8), ((1 << 31) - 1, 1, 0, 1)):
+        assert call(S, H, K, parts) == -4, (S, H, K, parts)
+        assert call(S, H, K, parts, 1, some) == -4, (S, H, K, parts)
+        assert call(S, H, K, parts, 0, some) == 0, (S, H, K, parts)
