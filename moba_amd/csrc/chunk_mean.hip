@@ -10,8 +10,8 @@
 // One stage (chunk_mean_whole_kernel): one workgroup of 256 to 1024 threads per (chunk, head) or part of its columns
 //          (column_parts_log2), column groups of 8 times the token lanes, their sums added through LDS: one launch instead of
 //          two, and no partial sums in memory.  131072 tokens, 8 heads, chunk 4096: 67 -> 44 us; 302060 tokens, 32 heads,
-//          chunk 2048: 474 -> 389 us; in parts, 32768 tokens, one head, chunk 1024: 9.8 -> 5.8 us.
-// Two stages where that leaves few workgroups for very many bytes each (see whole_chunks):
+//          chunk 2048: 474 -> 389 us; in halves, 32768 tokens, one head, chunk 1024: 10.2 -> 9.2 us (keys just written).
+// Two stages for very many short chunks, and where one would leave few workgroups for very many bytes each (see whole_chunks):
 //   Stage 1: grid (F, token splits, column blocks); each thread owns 8 adjacent
 //            columns of the [H*D] token row and sums its share of a token split.
 //   Stage 2: sums the splits in order, divides by B, rounds.
@@ -234,34 +234,47 @@ extern "C" size_t moba_chunk_mean_workspace_bytes(int H, int D, int F, int B) {
   return (size_t)F * pick_nsplit(HD8, F, B) * HD8 * 8 * sizeof(double);
 }
 
-// Into how many parts (log2) the columns of a chunk and head go, each a workgroup's: few chunks leave most of the chip without
-// one, and a workgroup reads its 128 KiB in 7 us, 256 in 9, 512 in 12, alone or not.  Parts of 128 bytes, a line of the caches,
-// are read as well as whole rows; parts of 64 bytes only where all keys together stay in an XCD's second-level cache long
-// enough (17 MB).  1 / 2 / 4 parts, and the two stages below, in us, 128-element heads (heads x chunks, tokens a chunk): 4 x 7,
-// 512: 6.0 / 5.6 / 5.6, 9.2; 1 x 15, 2048: 10.8 / 7.9 / 7.1, 10.0; 1 x 31, 1024: 7.7 / 6.4 / 5.8, 9.8; 4 x 8, 2048: 10.9 / 8.0 /
-// 7.5, 11.7; 1 x 60, 2048: 11.6 / 8.4 / 11.9, 12.7; 8 x 15, 1024: 8.7 / 7.5 / 8.6, 13.6; 1 x 15, 4096: 17.4 / 11.3 / 8.8, 13.3; 1 x 31,
-// 4096: 18.6 / 12.2 / 15.4, 15.9; 4 x 31, 4096: 30.8 / 26.7 / 47.7, 40.1; 8 x 31, 4096: 44.7 / 48.0 / 82, 67; 1 x 3, 16384: 59 / 31 /
-// 20, 32; 64-element heads: 1 x 31, 2048: 7.8 / 7.4, 9.5; 1 x 31, 4096: 11.2 / 9.2, 11.8; 4 x 31, 4096: 17.3 / 24.0, 27.5; 8 x 15,
-// 512: 5.6 / 5.8, 9.6.
+// Times below: us with the keys last written before 640 MB of other data / just before the call; two stages with both launches.
+//
+// Into how many parts (log2) the columns of a chunk and head go, each a workgroup's.  Halves of 128-element heads below 128
+// (chunk, head) pairs: whole rows leave compute units without a workgroup there, and a workgroup's reads are a chain of its own
+// length; from there on they only make a second round.  Parts of 64 bytes, half a line of the caches, only for up to 64 pairs
+// and 17 MB, and only where the two workgroups of a line share a second-level cache: workgroups go to the eight XCDs in turn
+// and a part's numbers lie F * H behind those of the part before, so where 8 divides that; elsewhere each line is fetched twice.
+// Whole rows / halves / quarters, 128-element heads (heads x chunks, tokens a chunk): 1 x 15, 2048: 17.3 / 14.3, 12.8 / 10.4, 12.8 /
+// 13.0; 1 x 31, 1024: 12.1 / 10.2, 10.4 / 9.2, 10.2 / 10.4; 8 x 1, 4096: 29.1 / 22.2, 21.1 / 14.8, 18.6 / 13.3; 8 x 3, 2048: -, 14.4 /
+// 11.2, 13.7 / 11.1; 8 x 7, 4096: 31.9 / 23.5, 23.7 / 18.6, 21.9 / 27.2; 8 x 15, 1024: 14.1 / 12.8, 12.8 / 12.9, 13.6 / 15.1; 4 x 31,
+// 4096: 35.2 / 35.6, 31.2 / 42.0, 51 / 62; 32 x 5, 1024: 14.6 / 14.2, 19.0 / 18.1, 18.2 / 21.9; 1 x 190, 1024: 15.3 / 15.3, 18.9 / 19.6,
+// 22.9 / 25.6; 64-element heads, whole rows / halves: 8 x 1, 4096: 21.4 / 14.8, 19.0 / 13.3; 8 x 7, 1024: 10.8 / 9.2, 10.2 / 8.7; 1 x 15,
+// 4096: 17.2 / 14.3, 16.0 / 16.6.
 static int column_parts_log2(int H, int D, int F, int B) {
   const int64_t groups = (int64_t)F * H;
-  int parts = 0, row = 2 * D;
-  if (groups < 192)
-    while (row >= 256) ++parts, row /= 2;
-  if (groups <= 64 && row == 128 && groups * B * D * 2 <= (17 << 20)) ++parts;
+  int parts = 0;
+  if (D >= 128 && groups < 128) parts = 1;
+  if (2 * D >> parts == 128 && groups <= 64 && groups % 8 == 0 && groups * B * D * 2 <= 17 << 20) ++parts;
   return parts;
 }
 
-// Whether a chunk's tokens go to one workgroup (a head's columns in parts or not), or to many in two stages: those where a
-// workgroup would read more than 1 MiB and there are few of them, and for very many chunks of at most eight tokens per
-// lane: whole rows of all heads, in the order they lie, then read faster than they add up (65536 tokens, 32 heads, chunk 128:
-// 104 us in two stages, 114 in one; 8 heads: 28 and 22).
+// Whether a chunk's tokens go to one workgroup (a head's columns in parts or not), or to many in two stages.  Those for very
+// many chunks of at most eight tokens per lane: whole rows of all heads, in the order they lie, then read faster than they add
+// up (65536 tokens, 32 heads, chunk 128: 104 us in two stages, 114 in one; 8 heads: 28 and 22).  And where a workgroup would read
+// so much that its chain outlasts them: beyond 2 MiB; for rows of all heads of less than 512 bytes, which the two stages handle
+// faster, beyond 1 MiB, or 384 KiB unless there are many chunks.  Two stages / one, 128-element heads:
+// 1 x 7, 3000: 15.0 / 13.6, 14.8 / 11.9; 1 x 3, 4096: 15.5 / 15.0, 18.3 / 14.5; 1 x 31, 4096: 20.9 / 20.4, 19.3 / 15.6; 1 x 3, 8192: 22.2 /
+// 22.1, 28.9 / 22.5; 1 x 31, 8192: 32.0 / 31.8, 30.9 / 24.5; 2 x 3, 8192: 36.2 / 35.5, 30.9 / 22.6; 8 x 3, 8192: 44.7 / 48.2, 37.6 /
+// 25.4; 1 x 3, 16384: 35.4 / 35.2, 51.6 / 38.2; 2 x 3, 16384: 64.9 / 64.3, 54.6 / 38.6; 4 x 1, 16384: 62.0 / 61.7, 67.6 / 40.9;
+// 64-element heads: 1 x 7, 3000: 13.7 / 12.3, 14.2 / 11.6; 1 x 7, 4096: 13.4 / 13.0, 17.3 / 14.2; 1 x 63, 4096: 18.4 / 18.6, 18.2 / 15.3;
+// 1 x 7, 8192: 16.4 / 16.2, 26.9 / 22.1; 4 x 7, 8192: 39.0 / 38.9, 31.8 / 23.0.
 static bool whole_chunks(int H, int D, int F, int B) {
   const int d8 = D / 8;
   if (d8 > 16 || (d8 & (d8 - 1)) || H > 65535) return false;
   const int64_t groups = (int64_t)F * H;
   if (B * d8 <= 256 * 8 && groups > 8192) return false;
-  return groups >= 128 || ((int64_t)B * D * 2 >> column_parts_log2(H, D, F, B)) <= (1 << 20);
+  if (groups >= 128) return true;
+  const int parts_log2 = column_parts_log2(H, D, F, B);
+  const int64_t bytes = (int64_t)B * D * 2 >> parts_log2;  // of a workgroup
+  if (H * D >= 256) return bytes <= 2 << 20;
+  return bytes <= 384 << 10 || (bytes <= 1 << 20 && (groups << parts_log2) * H * D > 30 * 128);
 }
 
 static int launch_chunk_mean(const void* k, const int32_t* fchunk_tok, void* kbar, double* partial, int H, int D,
