@@ -22,6 +22,7 @@
 // heads, up to 511 candidates, 11 picks: 422 -> 333 us.  Calls of a few microseconds are a chain of round trips to memory:
 // where the counters of the candidates lie is looked up beside Q, and the first block stops at the last candidate (4096
 // tokens, 4 heads: 9.3 -> 8.6 us; 3 x 2001, 32 heads: 15.7 -> 14.5).
+#include <algorithm>
 #include "common.h"
 
 namespace moba {
@@ -330,6 +331,26 @@ using namespace moba;
   else if ((K) <= 64) { CALL(64); }         \
   else return MOBA_ERR_LIMIT;
 
+// What a workgroup's four waves are: heads of the same 64 tokens, whose picks leave as one run per token, or 256 tokens of a head,
+// whose counts leave as one addition.  By tokens in two cases; below by heads / by tokens in us, 2 picks, with the counts, one
+// sequence, Q just written.
+// Waves without a head, a twelfth of all and more, where the chip's 1024 SIMDs have no room for them beside the others at a wave
+// each.  Chunk 128: one head, 16379 tokens: 15.5 / 15.3; 24571: 22.0 / 18.3; 262139: 531 / 191; 2 heads, 16379: 15.8 / 16.1; 24571: 22.3 /
+// 19.2; 3 heads, 16379: 16.2 / 16.6; 21840: 22.2 / 19.5; 5 heads, 52423: 79.8 / 58.5; 13 heads, 20159: 45.6 / 37.7; 22 heads, 2508: 11.5 /
+// 12.2; 2880: 13.5 / 12.4; 11910: 35.8 / 32.7.
+// The additions.  A counter gets one from each wave of its query chunk, B / 64 by heads and a quarter of that by tokens, and a
+// kernel of up to a wave to a SIMD waits for them at its end; with 4 heads, whose counters lie in few cache lines, longer ones
+// with long chunks do too.  Chunks of less than 512 tokens have nothing to gain: a workgroup's tokens then lie in two of them
+// as often as not.  8 heads, 8187 tokens, chunk 128: 13.8 / 14.9; 256: 12.4 / 13.0; 512: 12.4 / 12.0; 2048: 16.0 / 11.8; 4 heads, 32763
+// tokens, 512: 18.5 / 18.0; 2048: 22.5 / 16.2; 65531, 512: 32.5 / 33.9; 2048: 31.9 / 24.8.  More rows of more heads: gain with long chunks
+// of one sequence (8 heads, 16379 tokens, 2048: 20.8 / 15.0), nothing or a loss with several (16 heads, 3 x 5457, 4096: 15.0 / 15.6 and,
+// with Q from memory, 15.9 / 18.3): by heads.
+static bool by_tokens(int64_t S, int H, int B) {
+  const int64_t heads = (H + 3) / 4 * 4ll;  // with those that waves have none for
+  if ((heads - H) * 12 >= heads && (S + 63) / 64 * heads > 1024) return true;
+  return B >= 512 && S * H <= (H == 4 ? std::max<int64_t>(65536, 256ll * B) : 65536);
+}
+
 extern "C" int moba_gate_topk(const void* q, const void* kbar, const int32_t* cu_seqlens, const int32_t* seq_fbase,
                               int32_t* sel, float* scores_out, const int32_t* pair_off, int32_t* cnt, int64_t S, int H,
                               int Hkv, int D, int nseq, int F, int B, int K, int dense_local, const int64_t* strides,
@@ -349,14 +370,7 @@ extern "C" int moba_gate_topk(const void* q, const void* kbar, const int32_t* cu
   const int64_t qbs = strides ? strides[5] : 0;
   if (qts <= 0 || qhs <= 0 || (qts & 7) || (qhs & 7)) return MOBA_ERR_ARG;
   if (qbr < 0 || (qbr > 0 && (qbs <= 0 || (qbs & 7)))) return MOBA_ERR_ARG;
-  // What a workgroup's four waves are: heads of the same 64 tokens, whose picks leave as one run per token, or 256 tokens of a
-  // head, whose counts leave as one addition.  The additions of all workgroups meet in P * H counters, a few cache lines where
-  // there are few heads and chunks, and a short kernel waits for them; beyond that the longer runs count, and below four
-  // heads waves that have no head.  By heads / by tokens, us, with the counts: one head, 32768 tokens, chunk 2048: 14.9 / 8.5,
-  // 262144, chunk 512: 182 / 66; 2 heads, 131072, chunk 512: 68 / 44; 4 heads, 4096 tokens, chunk 512: 8.6 / 7.4, 32768, chunk
-  // 1024: 15.1 / 13.2, 131072, chunk 4096, 11 picks: 65 / 54, 524288: 330 / 335; 8 heads, 8192: 8.6 / 8.5; 32 heads, 2048, chunk
-  // 256: 8.0 / 7.8; 8 heads, 20480 in five sequences, chunk 512: 14.5 / 16.6; 32 heads, 3 x 2001, chunk 256: 14.5 / 16.1.
-  const int one_head = H < 4 || S * H <= (H == 4 ? 1 << 20 : 65536);
+  const int one_head = by_tokens(S, H, B);
   dim3 grid((unsigned)((S + 63) / 64), (unsigned)((H + 3) / 4));
   if (one_head) grid = dim3((unsigned)((S + 255) / 256 * H));
   hipStream_t st = (hipStream_t)stream;
