@@ -60,7 +60,8 @@ struct BwdParams {
   TileTables t;
   float scale_log2;
   float scale;
-  int* queues;        // [16] tile counters, one per XCD, of the dQ kernel and of the dK/dV kernel; zero at the start
+  int* queues;        // [16] tile counters, one per XCD, of the dQ kernel (at the start behind its workgroups' first tiles) and of
+                      // the dK/dV kernel (zero)
   // Problems of few key tiles: the stages of all key tiles of a key/value head, one tile's behind the other's, are cut into equal
   // shares (bwd_dkv_tiles).  share_tiles [Hkv * kv_tiles + 1]: the tiles, head by head, worked out by bwd_delta_kernel; part_dkv:
   // the fp32 sums of the tiles that several shares have parts of, which bwd_dkv_reduce_kernel adds up in the
@@ -148,7 +149,7 @@ __global__ __launch_bounds__(256) void bwd_delta_kernel(const typename E::elem* 
                                                         const typename E::elem* __restrict__ out,
                                                         const float* __restrict__ lse, float* __restrict__ delta,
                                                         float* __restrict__ lse2, int64_t rows,
-                                                        int* __restrict__ queues, const BwdParams<E> p) {
+                                                        int* __restrict__ queues, int dq_first, const BwdParams<E> p) {
   MOBA_ELEM_TYPES(E)
   const int extra = p.dkv_shares ? 1 : 0;
   if (extra && blockIdx.x == 0) {  // the key tiles' first places: a thread adds up some tiles in a row
@@ -178,9 +179,9 @@ __global__ __launch_bounds__(256) void bwd_delta_kernel(const typename E::elem* 
     if (threadIdx.x == 255) p.share_tiles[p.kv_total].begin = at;
     return;
   }
-  // the 16 tile counters of the two kernels that follow start at zero (here: one launch less than a kernel of its
-  // own, and, unlike a memset, safe to record into a graph)
-  if (blockIdx.x == extra && threadIdx.x < 16) queues[threadIdx.x] = 0;
+  // the 16 tile counters of the two kernels that follow: the dQ kernel's start behind the tiles that its workgroups take by
+  // their numbers (here: one launch less than a kernel of its own, and, unlike a memset, safe to record into a graph)
+  if (blockIdx.x == extra && threadIdx.x < 16) queues[threadIdx.x] = threadIdx.x < 8 ? dq_first : 0;
   const int lane = threadIdx.x & 63, g = lane >> 4, c8 = lane & 15;
   const int64_t row0 = ((blockIdx.x - extra) * 4ll + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * (4 * NR);
   if (row0 >= rows) return;
@@ -249,10 +250,12 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(const BwdParams<E> p) {
     const int64_t id = (((int64_t)(x / kXcdBlock) << ql) + queue) * kXcdBlock + (x % kXcdBlock);
     return id < (int64_t)hist_tiles + p.t.self_total ? (int)id : -1;
   };
-  draw();
-  if (tid == 0) *id_word = drawn;
-  __syncthreads();
-  int id = id_of(__builtin_amdgcn_readfirstlane(*id_word));
+  // The first tile goes by the workgroup's number, not by who draws first: numbers are dealt to the units in turn, a second
+  // round behind the first, so a unit's two workgroups start half the grid apart.  Drawn, they may be neighbours, and with few
+  // tiles the unit that has two of the longest ends last; and the draw was a round trip.  Drawn / by number, us: 6 sequences up to
+  // 2627 tokens, 8 heads, chunk 4096 (496 tiles): 91.7 / 78.0; 6 up to 4206, one head: 111 / 94; 2715 + 1980 + 2074, 4 heads, chunk
+  // 512: 43.6 / 35.4; 32768, one head, chunk 2048: 129.6 / 123.8; 20480 in five, 8 heads, chunk 512: 166.2 / 163.9; 302060: equal.
+  int id = id_of(blockIdx.x >> ql);
   while (true) {
   while (id < 0) {  // this queue is empty: the next one (a few draws in the open, at the end of the kernel)
     queue = (queue + 1) & qmask;
@@ -1161,12 +1164,13 @@ static int launch_bwd(const void* dout, const void* q, const void* k, const void
       !allow_dynamic_lds((const void*)dkv_kernels[form], kBwdDkvLds, allowed_dkv[form]))
     return MOBA_ERR_LAUNCH;
   const int64_t rows = S * H;
-  // Four rows to a lane where the chip has workgroups enough that way (163840 rows: 17.2 -> 14.3 us; 32768: 5.2 -> 4.8), one
+  // Four rows to a lane where the chip has workgroups enough that way (163840 rows: 16.3 -> 14.3 us; 32768: 5.4 -> 5.3), one
   // where a second wave is at hand sooner than a lane's second row (1000 rows: 2.9 us, with four 3.6).
   auto* const delta_kernel = rows >= 32768 ? bwd_delta_kernel<E, 4> : bwd_delta_kernel<E, 1>;
   const int delta_rows = rows >= 32768 ? 64 : 16;
   hipLaunchKernelGGL(delta_kernel, dim3((unsigned)((rows + delta_rows - 1) / delta_rows + (dkv_shares ? 1 : 0))), dim3(256), 0,
-                     st, (const elem*)dout, (const elem*)out, lse, delta, delta + S * H, rows, queues, p);
+                     st, (const elem*)dout, (const elem*)out, lse, delta, delta + S * H, rows, queues,
+                     (int)(grid_q >> p.queues_log2), p);
   hipLaunchKernelGGL(bwd_dq_kernel<E>, dim3((unsigned)grid_q), dim3(256), kBwdDqLds, st, p);
   if (merge_tokens > 0) {  // (0: the dQ kernel wrote every row itself)
     const int64_t sum_rows = merge_tokens * H;
@@ -1280,7 +1284,7 @@ extern "C" int moba_bwd(const void* dout, const void* q, const void* k, const vo
   const int cus = resident_compute_units();
   if (cus <= 0) return MOBA_ERR_LAUNCH;
   const int64_t grid_kv = ((int64_t)cus + 7) / 8 * 8;
-  const int64_t grid_q = 2 * grid_kv;  // the dQ kernel fits two workgroups on a CU
+  const int64_t grid_q = 2 * grid_kv;  // the dQ kernel fits two workgroups on a CU (a multiple of 8: as many for every queue)
   if (total_q >= 0x7fffffffLL) return MOBA_ERR_LIMIT;
   TileTables t;
   t.seg_off = seg_off; t.tile_off = tile_off; t.seg_dest = seg_dest; t.fchunk_tok = fchunk_tok;

@@ -1,4 +1,5 @@
-"""Gradients where the delta kernel takes one or four rows to a lane, with rows left over, against 64 bits (GPU only)."""
+"""Gradients where the delta kernel takes one or four rows to a lane, with rows left over, and where the dQ kernel's workgroups
+have a tile each, too few, or some to draw, against 64 bits (GPU only)."""
 
 import pytest
 import torch
@@ -8,7 +9,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("sequences,H", [(1, 1), (1, 2), (2, 5), (3, 3), (4095, 1),   # one row: up to 32767
-                                         (4096, 1), (4099, 1), (1367, 3), (830, 5)])  # four
+                                         (4096, 1), (4099, 1), (1367, 3), (830, 5),  # four
+                                         (511, 1), (512, 1), (513, 1), (257, 2)])    # tiles around the 512 workgroups
 def test_dq_of_short_sequences(sequences, H, dtype):
     from moba_amd import moba_efficient as E
     print("delta", sequences, H, dtype, flush=True)
