@@ -50,7 +50,7 @@ struct TileTables {
   int S, H, K1, F, N, B;
   int seg_heads, seg_groups;
   Divisor by_hk1, by_k1;        // H*K1 and K1, for the entries of the lists (which exist only with K1 >= 2)
-  Divisor by_groups, by_rep, by_h, by_batch;  // seg_groups, rep, H, batch_rows (divisor_or_one)
+  Divisor by_groups, by_rep, by_batch;  // seg_groups, rep, batch_rows (divisor_or_one)
   int Hkv, rep;                 // key/value heads and query heads per key/value head (H = Hkv * rep)
   int hist_bound;               // logical tile ids below it are history tiles
   int self_total;               // self_tile_prefix[N] * H
@@ -98,7 +98,7 @@ inline bool set_layout(TileTables& t, const int64_t* strides) {
   t.self_skip = 0; t.q_shift = 0;
   t.seg_heads = 1; t.seg_groups = t.H;
   t.by_hk1 = divisor((uint64_t)t.H * t.K1); t.by_k1 = divisor(t.K1);
-  t.by_groups = t.by_h = divisor_or_one(t.H); t.by_rep = divisor_or_one(t.rep); t.by_batch = divisor_or_one(1);
+  t.by_groups = divisor_or_one(t.H); t.by_rep = divisor_or_one(t.rep); t.by_batch = divisor_or_one(1);
   if (!strides) {
     t.q_tok_b = (int64_t)t.H * kHeadDim * 2; t.q_head_b = kHeadDim * 2;
     t.kv_tok_b = (int64_t)t.Hkv * kHeadDim * 2; t.kv_head_b = kHeadDim * 2;

@@ -227,7 +227,6 @@ __global__ __launch_bounds__(256, 2) void bwd_dq_kernel(const BwdParams<E> p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int n = lane & 31, hh = lane >> 5;
-  const int H = p.t.H;
 
   // The workgroups (two per CU, all resident) draw their tiles from eight queues, one per XCD: queue x
   // hands out the ids (8i + x) * kXcdBlock + j in order, so that the tiles in flight on an XCD are

@@ -15,7 +15,7 @@
 // milliseconds the chip's power limit decides and the doubled L2 -> LDS traffic costs 3 to 8 %: those stay with
 // moba_fwd_kernel (the rule stands with the caller's choice of the tile height).
 //
-// Heads of 64 elements (the only kernel that takes them unpadded) need half the LDS and 147 registers: three workgroups
+// Heads of 64 elements (the only kernel that takes them unpadded) need half the LDS and 142 registers: three workgroups
 // to a compute unit.  The exponentials weigh twice as much against the products there, so the rate in FLOP/s stays
 // below that of 128 elements, but half the work is gone: 8191 tokens, 32 heads, chunk 512, whole operator: 401 us padded
 // to 128, 205 us here; 131072 tokens, chunk 4096, 12 chunks: 64.8 -> 43.6 ms.

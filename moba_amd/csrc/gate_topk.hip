@@ -10,8 +10,8 @@
 // chunks 0..d of every sequence (which would pick every earlier chunk) get no picks
 // at all: the attention kernels serve them through one causal pass over the prefix.
 //
-// One wave handles 64 consecutive tokens of one head (a workgroup four heads of them, or 256 tokens of one head: the rule stands
-// at the launch): the score tile (32 chunks x 64 tokens) is two 32x32x16 MFMA
+// One wave handles 64 consecutive tokens of one head (a workgroup four heads of them, or 256 tokens of one head: see
+// by_tokens): the score tile (32 chunks x 64 tokens) is two 32x32x16 MFMA
 // accumulators.  Sixteen lane-half swaps leave the 32 scores of token `lane` in lane `lane`; a lane marks those that
 // beat the worst entry of its list (three instructions each, no LDS) and inserts them one per pass, lowest id first, in
 // a top-k held in registers.  Scores never reach HBM (except through the optional debug output).
@@ -94,7 +94,8 @@ __global__ __launch_bounds__(256, KMAX <= 4 ? 3 : (KMAX <= 16 ? 2 : 1)) void gat
     // a token of a dense prefix attends all its earlier chunks through the causal self path: no picks, no counts
     if (c <= dense_local) c = 0;
   }
-  // union of the candidate ranges of the 64 tokens (identical for the 4 waves)
+  // union of the candidate ranges of the wave's 64 tokens (the same for the workgroup's other waves only where they hold other
+  // heads of the same tokens: no barrier may stand under a test of them)
   int flo = c > 0 ? fb : 0x7fffffff;
   int fhi = c > 0 ? fb + c : 0;
 #pragma unroll
@@ -203,11 +204,11 @@ __global__ __launch_bounds__(256, KMAX <= 4 ? 3 : (KMAX <= 16 ? 2 : 1)) void gat
       }
     }
   }
-  // The four waves hold the lists of four consecutive heads of the same 64 tokens: K ints per (token, head) that
-  // lie 4K ints in a row per token in sel.  Through LDS, so that the workgroup stores those runs with consecutive
-  // lanes on consecutive ints (a lane storing its own K ints touches a cache line for 4K bytes of it).
+  // The lists, K ints per (token, head): of four heads that lie side by side, 4K ints in a row per token in sel, or of one head,
+  // K ints in a row every H * K.  Through LDS, so that the workgroup stores those runs with consecutive lanes on consecutive
+  // ints (a lane storing its own K ints touches a cache line for 4K bytes of it).
   __syncthreads();  // (the score tile is read out)
-  int* stage = reinterpret_cast<int*>(&sc[0][0][0]);  // [64 tokens][4 heads][K]
+  int* stage = reinterpret_cast<int*>(&sc[0][0][0]);  // [64 tokens][4 heads][K], or one_head: [256 tokens][K]
   if (4 * 64 * K <= (int)(sizeof(sc) / sizeof(int))) {  // (uniform; K <= 34)
 #pragma unroll
     for (int j = 0; j < KMAX; ++j)
@@ -216,7 +217,7 @@ __global__ __launch_bounds__(256, KMAX <= 4 ? 3 : (KMAX <= 16 ? 2 : 1)) void gat
     if (one_head) {
       const int first = tile * 256;
       for (int i = threadIdx.x; i < 256 * K; i += 256) {
-        const int tk = i / K;  // [256 tokens][K]
+        const int tk = i / K;
         if (first + tk < S) sel[((int64_t)(first + tk) * H + h) * K + i - tk * K] = stage[i];
       }
     } else {
@@ -236,7 +237,8 @@ __global__ __launch_bounds__(256, KMAX <= 4 ? 3 : (KMAX <= 16 ? 2 : 1)) void gat
   }
   // The gather lists' counts as a by-product: how many tokens of a (query chunk, head) picked each earlier chunk,
   // added into cnt[(chunk, head, query chunk)] (integer sums: the order of the additions does not matter).  A
-  // wave's 64 tokens lie in one query chunk, or in a few: one pass per chunk, through a histogram in LDS.
+  // wave's 64 tokens lie in one query chunk, or in a few: one pass per chunk, through a histogram in LDS of the wave's own, or
+  // of all four waves' (one_head) where their tokens lie in one query chunk with up to 64 earlier ones.
   if (!cnt) return;
   constexpr int kHist = (int)(sizeof(sc) / sizeof(int)) / 4;
   int* const hists = reinterpret_cast<int*>(&sc[0][0][0]);

@@ -41,7 +41,8 @@ __device__ __forceinline__ int slot_row(const SlotRows& p, int at) {
 }
 
 // Up to kMostSlotsAtOnce slots of a row (parts included) are requested at once, before the statistics and picks that say which
-// are present have arrived: one round trip to memory instead of two.  (Twelve take 73 registers, seven waves to a SIMD.)
+// are present have arrived: one round trip to memory instead of two.  (The merge of twelve takes 68 registers, seven waves to a
+// SIMD; in parts 82 and five.)
 // NV: slots of a row, all parts; kParts: of several parts -- slot u is slot u % K1 of part u / K1, part_rows slot rows
 // behind part 0 for each; the self slot has part 0 only.
 constexpr int kMostSlotsAtOnce = 12;
