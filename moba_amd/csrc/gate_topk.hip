@@ -66,7 +66,7 @@ __device__ __forceinline__ int find_seq(const int* __restrict__ cu, int nseq, in
 // instructions while others wait; longer lists would spill there: 11 picks, 31 candidates: 422 us held to three, 337 to
 // two)
 template <class E, int KMAX, int D>
-__global__ __launch_bounds__(256, KMAX <= 4 ? 3 : (KMAX <= 16 ? 2 : 1)) void gate_topk_kernel(
+__global__ __launch_bounds__(256, KMAX <= 4 || (KMAX <= 12 && D == 64) ? 3 : (KMAX <= 16 ? 2 : 1)) void gate_topk_kernel(
     const typename E::elem* __restrict__ q, const typename E::elem* __restrict__ kbar, const int* __restrict__ cu_seqlens,
     const int* __restrict__ seq_fbase, int* __restrict__ sel, float* __restrict__ scores_out,
     int S, int H, int Hkv, int nseq, int F, int B, int K, int64_t q_tok_stride, int64_t q_head_stride,
@@ -253,10 +253,11 @@ __global__ __launch_bounds__(256, KMAX <= 4 ? 3 : (KMAX <= 16 ? 2 : 1)) void gat
     }
   };
   auto to_counts = [&](int n, int cc, int cfb, int at) __attribute__((always_inline)) {  // n picks of chunk cfb + at
+    if (n == 0) return;  // (nearly all of many candidates: nothing is looked up for them)
     const int f = cfb + at, l = f - flo;
     int2 pr = my_pairs;
     if (l != lane) pr = make_int2(pair_off[f], pair_off[f + 1]);
-    if (n) atomicAdd(&cnt[pr.x * H + h * (pr.y - pr.x) + (cc - at - 1)], n);
+    atomicAdd(&cnt[pr.x * H + h * (pr.y - pr.x) + (cc - at - 1)], n);
   };
   if (one_head) {
     // the four waves' tokens, if they lie in one query chunk: one histogram, one addition for each count where the waves on
