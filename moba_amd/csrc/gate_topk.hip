@@ -19,9 +19,8 @@
 // Bound: Q is read once (HBM) for few candidates; with many the vector instructions per candidate decide.  Measured at
 // 196608 tokens, 32 heads on 8, up to 767 candidates, 2 picks: 2.20 ms with the tile transposed through LDS and a
 // barrier on either side of it, 1.39 ms here; 302060 tokens, up to 147 candidates: 1.12 -> 0.91 ms; 65536 tokens, 16
-// heads, up to 511 candidates, 11 picks: 422 -> 333 us.  Calls of a few microseconds are a chain of round trips to memory:
-// where the counters of the candidates lie is looked up beside Q, and the first block stops at the last candidate (4096
-// tokens, 4 heads: 9.3 -> 8.6 us; 3 x 2001, 32 heads: 15.7 -> 14.5).
+// heads, up to 511 candidates, 11 picks: 422 -> 333 us.  The first block stops at the last candidate (4096 tokens, 4 heads: 11.0 ->
+// 10.1 us; 8191 tokens, 32 heads of 64: 23.8 -> 21.8).
 #include <algorithm>
 #include "common.h"
 
@@ -106,12 +105,6 @@ __global__ __launch_bounds__(256, KMAX <= 4 || (KMAX <= 12 && D == 64) ? 3 : (KM
 
   TopK<KMAX> top;
   top.init();
-  // where the counts of this lane's chunk start (the first 64 of the wave's candidates; looked up ahead, for the end)
-  int2 my_pairs = make_int2(0, 0);
-  if (cnt && fhi > 0) {
-    const int f = min(flo + lane, F - 1);
-    my_pairs = make_int2(pair_off[f], pair_off[f + 1]);
-  }
 
   if (fhi > 0) {  // wave-uniform
     // Q^T operand: lane (n, hh) holds q[token n (+32)][16*ks + 8*hh .. +7]
@@ -254,10 +247,9 @@ __global__ __launch_bounds__(256, KMAX <= 4 || (KMAX <= 12 && D == 64) ? 3 : (KM
   };
   auto to_counts = [&](int n, int cc, int cfb, int at) __attribute__((always_inline)) {  // n picks of chunk cfb + at
     if (n == 0) return;  // (nearly all of many candidates: nothing is looked up for them)
-    const int f = cfb + at, l = f - flo;
-    int2 pr = my_pairs;
-    if (l != lane) pr = make_int2(pair_off[f], pair_off[f + 1]);
-    atomicAdd(&cnt[pr.x * H + h * (pr.y - pr.x) + (cc - at - 1)], n);
+    const int f = cfb + at;
+    const int q0 = pair_off[f], nq = pair_off[f + 1] - q0;
+    atomicAdd(&cnt[q0 * H + h * nq + (cc - at - 1)], n);
   };
   if (one_head) {
     // the four waves' tokens, if they lie in one query chunk: one histogram, one addition for each count where the waves on
