@@ -330,16 +330,16 @@ using namespace moba;
 // whose counts leave as one addition.  By tokens in two cases; below by heads / by tokens in us, 2 picks, with the counts, one
 // sequence, Q just written.
 // Waves without a head, a twelfth of all and more, where the chip's 1024 SIMDs have no room for them beside the others at a wave
-// each.  Chunk 128: one head, 16379 tokens: 15.5 / 15.3; 24571: 22.0 / 18.3; 262139: 531 / 191; 2 heads, 16379: 15.8 / 16.1; 24571: 22.3 /
-// 19.2; 3 heads, 16379: 16.2 / 16.6; 21840: 22.2 / 19.5; 5 heads, 52423: 79.8 / 58.5; 13 heads, 20159: 45.6 / 37.7; 22 heads, 2508: 11.5 /
+// each.  Chunk 128: one head, 16379 tokens: 15.6 / 15.4; 24571: 22.1 / 18.3; 262139: 541 / 179; 2 heads, 16379: 15.8 / 16.0; 24571: 22.2 /
+// 19.1; 3 heads, 16379: 16.4 / 16.8; 21840: 22.2 / 19.4; 5 heads, 52423: 80.4 / 56.1; 13 heads, 20159: 45.6 / 37.7; 22 heads, 2508: 11.5 /
 // 12.2; 2880: 13.5 / 12.4; 11910: 35.8 / 32.7.
 // The additions.  A counter gets one from each wave of its query chunk, B / 64 by heads and a quarter of that by tokens, and a
 // kernel of up to a wave to a SIMD waits for them at its end; with 4 heads, whose counters lie in few cache lines, longer ones
 // with long chunks do too.  Chunks of less than 512 tokens have nothing to gain: a workgroup's tokens then lie in two of them
-// as often as not.  8 heads, 8187 tokens, chunk 128: 13.8 / 14.9; 256: 12.4 / 13.0; 512: 12.4 / 12.0; 2048: 16.0 / 11.8; 4 heads, 32763
-// tokens, 512: 18.5 / 18.0; 2048: 22.5 / 16.2; 65531, 512: 32.5 / 33.9; 2048: 31.9 / 24.8.  More rows of more heads: gain with long chunks
-// of one sequence (8 heads, 16379 tokens, 2048: 20.8 / 15.0), nothing or a loss with several (16 heads, 3 x 5457, 4096: 15.0 / 15.6 and,
-// with Q from memory, 15.9 / 18.3): by heads.
+// as often as not.  8 heads, 8187 tokens, chunk 128: 13.8 / 14.9; 256: 12.4 / 12.8; 512: 12.3 / 11.9; 2048: 15.9 / 11.6; 4 heads, 32763
+// tokens, 512: 18.6 / 17.8; 2048: 22.4 / 15.5; 65531, 512: 32.6 / 34.0; 2048: 30.9 / 24.6.  More rows of more heads gain with long chunks
+// of one sequence (8 heads, 16379 tokens, 2048: 20.7 / 14.6) and may lose with several (16 heads, 3 x 5457, 4096, Q from memory: 15.9 /
+// 18.3): by heads.
 static bool by_tokens(int64_t S, int H, int B) {
   const int64_t heads = (H + 3) / 4 * 4ll;  // with those that waves have none for
   if ((heads - H) * 12 >= heads && (S + 63) / 64 * heads > 1024) return true;
